@@ -42,28 +42,18 @@
 
 using namespace gss;
 
-// Scratch of the no-allocation record gather (gss_hits_gather): the record
-// offset of every hit chunk the last sweep claimed, then the total.  One copy
-// per device, in this library's code object, held until the process ends.
-// Host code never uses the array's name as an address: every kernel argument
-// takes the per-device address that hipGetSymbolAddress returned for it
-// (scratch_address below, called once per device by gss_engine_create with
-// that device current).  Every call on one device shares the array, and
-// k_chunk_offsets rewrites entries [0, chunks] each time, so nothing in it
-// needs clearing; two gathers that overlap on one device race.
-static constexpr uint32_t kGatherMaxChunks = 262144;  // 2 MiB + 8 B per device
+// gss_hits_gather takes the records of at most this many claimed hit chunks.
+static constexpr uint32_t kGatherMaxChunks = 262144;
 constexpr int kMaxHostRecordBuffers = 4;  // pinned record buffers per step slot
-static __device__ __align__(256) uint64_t scratch[kGatherMaxChunks + 1];
+// records of a step at most this large are written into pinned memory by the
+// step itself: 512 KiB take 9 us over PCIe, about what starting a copy and
+// waiting for it costs (see queue_records_copy)
+constexpr size_t kDirectWords = 64 * 1024;
 
 namespace {
 
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-uint64_t *g_scratch_ptr[kMaxDevices] = {};
-
-// Clauses of at most this many literals read both rows of each literal in one
-// pass (see kernels.hip).
-constexpr int kDefaultFuseLen = 4;
+// literals a step copies straight from its pinned staging
+constexpr int64_t kDirectLits = 16384;
 // steps staging at least this many bytes split their copies over the stage pool
 constexpr size_t kStagePoolMinBytes = 1u << 20;
 
@@ -94,24 +84,6 @@ int set_err(int code, const char *fmt, ...) {
             return set_err(_e == hipErrorOutOfMemory ? GSS_E_NOMEM : GSS_E_HIP, "%s: %s", \
                            #expr, hipGetErrorString(_e));                                  \
     } while (0)
-
-// Device address of `scratch` on `device`, which must be current: taken once
-// per device, then reused.
-int scratch_address(int device, uint64_t **out) {
-    std::lock_guard<std::mutex> g(g_scratch_mu);
-    if (device < 0 || device >= kMaxDevices)
-        return set_err(GSS_E_INVAL, "device %d: at most %d devices", device, kMaxDevices);
-    if (!g_scratch_ptr[device]) {
-        void *p = nullptr;
-        const hipError_t he = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (he != hipSuccess || !p)
-            return set_err(GSS_E_HIP, "hipGetSymbolAddress(scratch) on device %d: %s", device,
-                           hipGetErrorString(he));
-        g_scratch_ptr[device] = (uint64_t *)p;
-    }
-    *out = g_scratch_ptr[device];
-    return GSS_OK;
-}
 
 struct Bucket {
     uint32_t *d = nullptr;
@@ -320,7 +292,7 @@ struct StepSlot {
     Pinned<gss_var_patch> h_patches;
     Pinned<gss_base_update> h_bups;
     Pinned<gss_word_load> h_loads;
-    Pinned<uint32_t> h_out;  // [0] = chunks claimed, [1 + c] = fill of chunk c
+    Pinned<uint32_t> h_out;  // counts of the step (write_counts in kernels.hip)
     DevBuf<StepHeader> d_hdr;
     DevBuf<BucketDesc> d_desc;
     DevBuf<ClauseSeg> d_cls;
@@ -332,7 +304,6 @@ struct StepSlot {
     DevBuf<uint64_t> d_hits;     // chunk_cap chunks of kHitChunk records of rec_words words
     DevBuf<uint32_t> d_fills;
     DevBuf<gss_hit> d_dense;     // compacted records of the last waited step
-    DevBuf<uint64_t> d_offs;     // record offset of each chunk (the graph's compaction)
     uint64_t dense_want = 0;     // records the graph's compaction should hold
     uint64_t step_dense = 0;     // records the last submitted step's graph compacts into
                                  // d_dense (0 = none)
@@ -355,8 +326,13 @@ struct StepSlot {
     bool copy_queued = false;
     int64_t rec_total = 0;  // records of the slot's last waited step
     bool host_ready = false;     // h_hits() holds the last waited step's records
-    Pinned<ScatterSeg> h_cseg;   // compaction segments (one per non-empty chunk)
-    DevBuf<ScatterSeg> d_cseg;
+    // Records of at most kDirectWords words go to pinned memory within the
+    // step: buffer h_direct[direct_at], one more of them than the waits a
+    // step's records stay valid for (h_n), taken in turn by the submits.
+    Pinned<uint64_t> h_direct[kMaxHostRecordBuffers + 1];
+    int direct_at = 0;
+    bool direct = false;  // the last waited step's records are at direct_rec
+    const uint64_t *direct_rec = nullptr;
     uint32_t *d_alloc = nullptr;
     uint32_t chunk_cap = 0;
     // chunks that hold every record the step could make; a buffer sized by
@@ -367,23 +343,24 @@ struct StepSlot {
     bool records_lost = false;  // its recovery could not grow the buffer
     // launch settings of the last submitted step's graph, for a recovery's
     // re-run of its tail
-    int g_blocks = 0, g_tc = 0, g_fuse = 0, g_unroll = 0;
+    int g_blocks = 0, g_tp = 0;
     bool g_serve = false, g_screen = false;
     bool g_agg_full = false;  // screened: the aggregate is rebuilt from the table
+    bool g_agg_fused = false; // screened: the applying and rolling kernels refresh it
     // Graphs captured over this slot's buffers, one per key (everything baked
     // in); a caller alternating between step forms (screened or not, rebuilt
     // aggregate or refreshed) replays them without capturing again.  The
-    // least recently used one goes when a fifth is needed.
+    // least recently used one goes when a ninth is needed.
     struct StepGraph {
         std::vector<const void *> key;
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
-        int blocks = 0, tc = 0, fuse = 0, unroll = 0;
-        bool serve = false, screen = false, agg_full = false;
+        int blocks = 0, tp = 0;
+        bool serve = false, screen = false, agg_full = false, staged = false;
         uint64_t dense = 0;  // records it compacts into d_dense (0 = none)
         uint64_t used = 0;   // submit count at its last use
     };
-    static constexpr size_t kGraphsPerSlot = 4;
+    static constexpr size_t kGraphsPerSlot = 8;
     std::vector<StepGraph> graphs;
     int cur = -1;  // graph of the slot's last submitted step
     uint64_t submits = 0;
@@ -473,22 +450,25 @@ struct gss_engine {
     const BucketDesc *desc_up_at = nullptr;
     std::vector<uint64_t> valid_up;
     Pinned<uint32_t> h_count;  // [0] = chunks claimed, [1], [2] = records (low, high word)
-    uint64_t *gather_scratch = nullptr;  // this device's address of `scratch`
     // host buffers that are only copy endpoints of at least this many bytes
     // are pageable (< 0: no limit); see Pinned
     int64_t page_limit = -1;
     DevBuf<gss_hit> d_hits;
     DevBuf<uint32_t> d_fills;
+    // counters (SweepArgs::alloc) of the sweep alloc_at and of the next one
+    // (8 words on), cleared by the sweep before it
     uint32_t *d_alloc = nullptr;
+    int alloc_at = 0;
+    uint32_t sweep_waves = 0;  // waves of the last sweep
     uint32_t chunk_cap = 0;
-    int nbuckets = 0, ntasks = 0, task_clauses = 0, blocks = 0;
+    int nbuckets = 0, npasses = 0, blocks = 0;
     bool pending = false, waited = false, have_sweep = false;
     int64_t last_hits = 0;
     uint32_t last_chunks = 0;
     float last_ms = 0.f;
     double total_ms = 0.0;
     int64_t nsweeps = 0;
-    int occ[7][9][2][4] = {};  // [log2 words][unroll][fused][sweep mode] resident blocks per CU
+    int occ[7][4] = {};  // [log2 words][sweep mode] resident blocks per CU
 
     // tuning
     int tune_waves_per_cu = 0;
@@ -508,7 +488,6 @@ struct gss_engine {
     int8_t *d_lastpos = nullptr;
     Pinned<int8_t> h_lastpos;
     int64_t applied = 0;  // updates of the last gss_assig_apply, still in d_ups
-    DevBuf<uint64_t> d_offsets;  // record offset of each chunk (dense copies of a sweep)
     DevBuf<gss_hit> d_dense;
     Pinned<gss_hit> h_hits;
 
@@ -529,7 +508,6 @@ struct gss_engine {
     // leaves them out, same records) and by batched steps submitted with
     // GSS_STEP_SCREEN (from the table)
     bool serve_prefilter = true;
-    int serve_vote = 2;  // entries per screening vote (GPUSHARESAT_SERVE_VOTE: 1, 2, 4 or 8)
     DevBuf<uint8_t> serve_agg;         // 2 * vars + 2 bytes, padded to 4
     DevBuf<uint64_t> serve_agg_words;  // [8]
     // state_version right after the last screened batched step was submitted:
@@ -581,21 +559,20 @@ static int settle_steps(gss_engine *e);
 
 namespace {
 
-// Fuse length the kernel runs with: <= 0 selects the variant without the
-// fused schedule.
-int fuse_of(const gss_engine *e) {
-    return e->tune_fuse_len > 0 ? e->tune_fuse_len : e->tune_fuse_len < 0 ? 0 : kDefaultFuseLen;
-}
-
-// Resident 256-thread blocks per CU of the sweep variant the engine runs.
+// Resident 256-thread blocks per CU of the sweep kernel the engine runs.
 int resident_blocks(gss_engine *e, int mode = 0) {
     int l = 0;
     while ((1 << l) < e->words) l++;
-    const int ui = std::min(e->tune_unroll, 8);
-    const int fi = fuse_of(e) > 0;
-    int &o = e->occ[l][ui][fi][mode];
-    if (!o) o = sweep_occupancy(e->words, e->tune_unroll, fi, mode);
+    int &o = e->occ[l][mode];
+    if (!o) o = sweep_occupancy(e->words, mode);
     return o;
+}
+
+// Passes a wave takes at a time: GSS_TUNE_TASK_CLAUSES in passes (0: the
+// kernel's own rule).
+int task_passes(const gss_engine *e, bool screened) {
+    const int cpp = sweep_clauses_per_pass(e->words, screened);
+    return e->tune_task_clauses > 0 ? (e->tune_task_clauses + cpp - 1) / cpp : 0;
 }
 
 int log2_exact(int w) {
@@ -658,31 +635,44 @@ int ensure_bucket_cap(gss_engine *e, int len, int64_t need, bool shrink = false)
     return GSS_OK;
 }
 
+// The hit chunks of the last plain sweep.
+ChunkArgs sweep_chunks(const gss_engine *e) {
+    ChunkArgs c{};
+    c.hits = (const uint64_t *)e->d_hits.p;
+    c.fills = e->d_fills.p;
+    c.alloc = e->d_alloc + 8 * e->alloc_at;
+    c.cap = e->chunk_cap;
+    c.waves = e->sweep_waves;
+    c.rec_words = 3;
+    return c;
+}
+
 // Launches the sweep kernel for the current descriptors (already uploaded).
 int launch_current_sweep(gss_engine *e) {
-    HIP_TRY(launch_reset_u32(e->d_alloc, 1, e->stream));
+    e->alloc_at ^= 1;
+    e->sweep_waves = e->npasses > 0 ? (uint32_t)e->blocks * 4 : 0;
     HIP_TRY(hipEventRecord(e->ev0, e->stream));
-    if (e->ntasks > 0) {
+    if (e->npasses > 0) {
         SweepArgs a{};
         a.dyn = nullptr;  // counts passed by value
         a.buckets = e->d_desc.p;
         a.nbuckets = e->nbuckets;
-        a.ntasks = e->ntasks;
-        a.task_clauses = e->task_clauses;
+        a.npasses = e->npasses;
+        a.task_passes = task_passes(e, false);
         a.table = e->table.p;
         a.sentinel = (uint32_t)(2 * e->vars) << kLitShift;
         a.valid = e->d_valid;
         a.hits = e->d_hits.p;
         a.fills = e->d_fills.p;
-        a.alloc = e->d_alloc;
+        a.alloc = e->d_alloc + 8 * e->alloc_at;
         a.chunk_cap = e->chunk_cap;
-        a.fuse_len = fuse_of(e);
         a.rec_words = 3;
-        HIP_TRY(launch_sweep(a, e->words, e->tune_unroll, e->blocks, e->stream));
+        HIP_TRY(launch_sweep(a, e->words, e->blocks, e->stream));
     }
     HIP_TRY(hipEventRecord(e->ev1, e->stream));
-    // claim counter and record count to pinned memory: the wait reads them there
-    HIP_TRY(launch_count_records(e->d_alloc, e->d_fills.p, e->chunk_cap, e->h_count.p, e->stream));
+    // counts to pinned memory: the wait reads them there
+    HIP_TRY(launch_count_records(sweep_chunks(e), e->h_count.p,
+                                 e->d_alloc + 8 * (e->alloc_at ^ 1), e->stream));
     return GSS_OK;
 }
 
@@ -719,10 +709,6 @@ int gss_engine_create(int device, gss_engine **out) {
         e->stage_threads = std::min(64, std::max(0, std::atoi(st)));
     if (const char *pf = std::getenv("GPUSHARESAT_SERVE_PREFILTER"))
         e->serve_prefilter = std::atoi(pf) != 0;
-    if (const char *sv = std::getenv("GPUSHARESAT_SERVE_VOTE")) {
-        const int v = std::atoi(sv);
-        if (v == 1 || v == 2 || v == 4 || v == 8) e->serve_vote = v;
-    }
     int rc = GSS_OK;
     auto fail = [&](int code) {
         gss_engine_destroy(e);
@@ -730,7 +716,6 @@ int gss_engine_create(int device, gss_engine **out) {
     };
     if (hipDeviceGetAttribute(&e->cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return fail(set_err(GSS_E_HIP, "cannot query CU count"));
-    if ((rc = scratch_address(device, &e->gather_scratch))) return fail(rc);
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(set_err(GSS_E_HIP, "stream creation failed"));
     if (hipEventCreate(&e->ev0) != hipSuccess || hipEventCreate(&e->ev1) != hipSuccess)
@@ -748,7 +733,8 @@ int gss_engine_create(int device, gss_engine **out) {
         hipMalloc((void **)&e->d_halt, 64) != hipSuccess ||
         hipMalloc((void **)&e->d_lastpos, GSS_MAX_WORDS) != hipSuccess)
         return fail(set_err(GSS_E_NOMEM, "device allocation failed"));
-    if (hipMemset(e->d_halt, 0, 64) != hipSuccess)
+    if (hipMemsetAsync(e->d_halt, 0, 64, e->stream) != hipSuccess ||
+        hipMemsetAsync(e->d_alloc, 0, 64, e->stream) != hipSuccess)
         return fail(set_err(GSS_E_HIP, "device memset failed"));
     if ((rc = e->h_valid.reserve(GSS_MAX_WORDS)) || (rc = e->h_lastpos.reserve(GSS_MAX_WORDS)))
         return fail(rc);
@@ -791,9 +777,7 @@ int gss_engine_destroy(gss_engine *e) {
         sl.d_hits.release();
         sl.d_fills.release();
         sl.d_dense.release();
-        sl.d_offs.release();
         sl.d_wcount.release();
-        sl.d_cseg.release();
     }
     for (Bucket &b : e->buckets) {
         if (b.d) (void)hipFreeAsync(b.d, e->stream);
@@ -808,7 +792,6 @@ int gss_engine_destroy(gss_engine *e) {
     e->d_stage.release();
     e->d_segs.release();
     e->d_ups.release();
-    e->d_offsets.release();
     e->d_dense.release();
     e->serve_tail.release();
     e->serve_adm.release();
@@ -1407,22 +1390,19 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
                                     "%lld variables",
                        (long long)e->max_lit, (long long)(e->max_lit >> 1), (long long)e->vars);
     const int W = e->words;
-    const int cpp = sweep_clauses_per_pass(W);
-    int tc = e->tune_task_clauses > 0 ? e->tune_task_clauses : 16 * cpp;
-    tc = std::max(cpp, (tc / cpp) * cpp);
-    e->task_clauses = tc;
+    const int cpp = sweep_clauses_per_pass(W, false);
     // descriptors of non-empty buckets
     int nb = 0;
     for (size_t len = 1; len < e->buckets.size(); len++)
         if (e->buckets[len].count) nb++;
     if ((rc = e->h_desc.reserve(std::max(nb, 1))) || (rc = e->d_desc.reserve(std::max(nb, 1))))
         return rc;
-    int64_t tasks = 0;
+    int64_t passes = 0;
     e->desc_new.clear();
     const size_t nlen = e->buckets.size();
     for (size_t i = 1; i < nlen; i++) {
-        // tasks of long clauses come first (they are the most expensive), so
-        // the persistent waves finish together; schedule 2 reverses that
+        // long clauses come first (they are the most expensive), so the
+        // persistent waves finish together; schedule 2 reverses that
         const size_t len = e->tune_schedule == 2 ? i : nlen - i;
         const Bucket &b = e->buckets[len];
         if (!b.count) continue;
@@ -1434,18 +1414,18 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
         d.lits = b.d;
         d.len = (uint32_t)len;
         d.count = (uint32_t)b.count;
-        d.task_begin = (uint32_t)tasks;
+        d.pass_begin = (uint32_t)passes;
         d.pad = 0;
         e->desc_new.push_back(d);
-        tasks += (b.count + tc - 1) / tc;
+        passes += (b.count + cpp - 1) / cpp;
     }
-    if (tasks > 0x7FFFFFFF) return set_err(GSS_E_INVAL, "too many tasks");
+    if (passes > 0x7FFFFFFF) return set_err(GSS_E_INVAL, "too many clauses");
     e->nbuckets = nb;
-    e->ntasks = (int)tasks;
+    e->npasses = (int)passes;
     int active_words = 0;
     for (int w = 0; w < W; w++)
         if (valid[w]) active_words++;
-    if (!active_words) e->ntasks = 0;  // every clause starts dead: nothing to check
+    if (!active_words) e->npasses = 0;  // every clause starts dead: nothing to check
     // Uploads only when what the device holds differs (the previous sweep has
     // been waited for, so its copies out of the pinned staging are done).
     const bool valid_same = (int)e->valid_up.size() == W &&
@@ -1473,12 +1453,12 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
     int per_cu = resident_blocks(e);
     if (e->tune_waves_per_cu > 0) per_cu = std::max(1, std::min(per_cu, e->tune_waves_per_cu / 4));
     int64_t blocks = (int64_t)e->cu * per_cu;
-    const int64_t need_blocks = (tasks + 3) / 4;
+    const int64_t need_blocks = (passes + 3) / 4;
     blocks = std::max<int64_t>(1, std::min(blocks, need_blocks));
     e->blocks = (int)blocks;
     // Hit capacity: an abandoned chunk holds more than kHitChunk - 64 records
-    // and each wave leaves at most one partial chunk, so this bound is never
-    // exceeded while records <= clauses * active words.
+    // and each wave leaves one partial chunk, so this bound is never exceeded
+    // while records <= clauses * active words.
     const uint64_t ub = (uint64_t)e->total_clauses * (uint64_t)active_words;
     uint64_t chunks = ub / (kHitChunk - 64) + 1 + (uint64_t)blocks * 4;
     size_t free_b = 0, total_b = 0;
@@ -1557,13 +1537,9 @@ int gss_hits_copy(gss_engine *e, gss_hit *out, int64_t cap, int64_t *n) {
     const int64_t want = std::min<int64_t>(cap, e->last_hits);
     if (want <= 0) return GSS_OK;
     if (!out) return set_err(GSS_E_INVAL, "null output");
-    // Compact the claimed chunks into a dense device buffer (offsets and the
-    // copy computed on the device), then one D2H.
-    if ((rc = e->d_dense.reserve((size_t)e->last_hits)) ||
-        (rc = e->d_offsets.reserve((size_t)e->chunk_cap + 1)))
-        return rc;
-    HIP_TRY(launch_compact_records(e->d_alloc, e->d_fills.p, e->chunk_cap, e->d_offsets.p,
-                                   e->d_hits.p, e->d_dense.p, e->d_dense.cap, 3, e->stream));
+    // The chunks into a dense device buffer, then one D2H.
+    if ((rc = e->d_dense.reserve((size_t)e->last_hits))) return rc;
+    HIP_TRY(launch_gather(sweep_chunks(e), e->d_dense.p, e->d_dense.cap, e->stream));
     HIP_TRY(hipMemcpyAsync(out, e->d_dense.p, (size_t)want * sizeof(gss_hit),
                            hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1580,16 +1556,15 @@ int gss_hits_gather(gss_engine *e, gss_hit *d_out, int64_t cap, int64_t *n) {
     if (cap < e->last_hits)
         return set_err(GSS_E_INVAL, "the sweep has %lld records; the output holds %lld",
                        (long long)e->last_hits, (long long)cap);
-    if (e->last_chunks > kGatherMaxChunks)
+    // (the waves' own chunks are there whether or not they hold records)
+    if (e->last_chunks > kGatherMaxChunks + e->sweep_waves)
         return set_err(GSS_E_INVAL,
                        "the sweep claimed %u hit chunks; gss_hits_gather handles at most %u "
                        "(gss_hits_copy has no such limit)",
                        e->last_chunks, kGatherMaxChunks);
     if (!e->last_hits) return GSS_OK;
-    // the same two kernels as gss_hits_copy: chunk offsets into the scratch,
-    // records straight into the caller's array
-    HIP_TRY(launch_compact_records(e->d_alloc, e->d_fills.p, e->chunk_cap, e->gather_scratch,
-                                   e->d_hits.p, d_out, (uint64_t)cap, 3, e->stream));
+    // the same kernel as gss_hits_copy, into the caller's array
+    HIP_TRY(launch_gather(sweep_chunks(e), d_out, (uint64_t)cap, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     return GSS_OK;
 }
@@ -1651,16 +1626,11 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
         int unroll, fuse, task, wpc, sched;
     };
     std::vector<Cfg> grid;
-    // rows in flight per lane: a choice for 16 words and wider, fixed below
-    std::vector<int> unrolls = e->words >= 16 ? std::vector<int>{2, 4} : std::vector<int>{0};
-    const int fuses[] = {-1, 1, 4, 8};
-    const int tasks[] = {0, 32, 128};
-    const int wpcs[] = {0, 24};
-    for (int u : unrolls)
-        for (int f : fuses)
-            for (int t : tasks)
-                for (int w : wpcs)
-                    for (int sc = 1; sc <= 2; sc++) grid.push_back({u, f, t, w, sc});
+    const int tasks[] = {0, 32, 128, 512};
+    const int wpcs[] = {0, 20, 24};
+    for (int t : tasks)
+        for (int w : wpcs)
+            for (int sc = 1; sc <= 2; sc++) grid.push_back({2, -1, t, w, sc});
     const Cfg saved{e->tune_unroll, e->tune_fuse_len, e->tune_task_clauses, e->tune_waves_per_cu,
                     e->tune_schedule};
     auto apply = [&](const Cfg &c) {
@@ -1721,11 +1691,23 @@ static int step_blocks(gss_engine *e, int mode) {
     return (int)std::max<int64_t>(1, (int64_t)e->cu * per_cu);
 }
 
-// Queues the copy of a waited step's `total` records (in `used` chunks) to the
-// slot's pinned h_hits on the slot's stream: one DMA copy when the graph made
+// The hit chunks of a slot's last submitted step, of rw words per record.
+static ChunkArgs step_chunks(const StepSlot &sl, int rw) {
+    ChunkArgs c{};
+    c.hits = sl.d_hits.p;
+    c.fills = sl.d_fills.p;
+    c.alloc = sl.d_alloc;
+    c.cap = sl.chunk_cap;
+    c.waves = (uint32_t)sl.g_blocks * 4;
+    c.rec_words = (uint32_t)rw;
+    return c;
+}
+
+// Queues the copy of a waited step's `total` records to the slot's pinned
+// h_hits on the slot's stream: one DMA copy when the graph made
 // them dense, else a compaction first (and the next capture's dense buffer is
 // sized for this volume).
-static int queue_records_copy(gss_engine *e, StepSlot &sl, int64_t total, uint32_t used) {
+static int queue_records_copy(gss_engine *e, StepSlot &sl, int64_t total) {
     int rc;
     const int rw = sl.res_words;  // 8-byte words per record
     if (!sl.copy) HIP_TRY(hipStreamCreateWithFlags(&sl.copy, hipStreamNonBlocking));
@@ -1799,23 +1781,8 @@ static int queue_records_copy(gss_engine *e, StepSlot &sl, int64_t total, uint32
                               std::max<size_t>(6 * hw, (size_t)1 << 20));
     }
     if ((uint64_t)total > sl.step_dense) {
-        if ((rc = sl.d_dense.reserve_async((size_t)total, cs)) ||
-            (rc = sl.h_cseg.reserve(used)) || (rc = sl.d_cseg.reserve(used)))
-            return rc;
-        int ns = 0;
-        uint64_t acc = 0;
-        for (uint32_t c = 0; c < used; c++) {
-            const uint32_t f = sl.h_out.p[1 + c];
-            if (!f) continue;
-            ScatterSeg &sg = sl.h_cseg.p[ns++];
-            sg.dst = (uint32_t *)((uint64_t *)sl.d_dense.p + acc * rw);
-            sg.src = (uint64_t)c * kHitChunk * rw * 2;
-            sg.count = (uint64_t)f * rw * 2;
-            acc += f;
-        }
-        HIP_TRY(hipMemcpyAsync(sl.d_cseg.p, sl.h_cseg.p, ns * sizeof(ScatterSeg),
-                               hipMemcpyHostToDevice, cs));
-        HIP_TRY(launch_scatter(sl.d_cseg.p, ns, (const uint32_t *)sl.d_hits.p, 0, cs));
+        if ((rc = sl.d_dense.reserve_async((size_t)total, cs))) return rc;
+        HIP_TRY(launch_gather(step_chunks(sl, rw), sl.d_dense.p, (uint64_t)total, cs));
         sl.dense_want = std::max<uint64_t>(sl.dense_want, 2 * (uint64_t)total);
     }
     HIP_TRY(hipMemcpyAsync(sl.h_hits().p, sl.d_dense.p, (size_t)total * rw * sizeof(uint64_t),
@@ -1827,88 +1794,97 @@ static int queue_records_copy(gss_engine *e, StepSlot &sl, int64_t total, uint32
 
 // Chunks a step's hit buffer can hold (the smallest of its parts).
 static uint32_t chunk_room(const StepSlot &sl, int rw) {
-    return (uint32_t)std::min<size_t>(
-        std::min<size_t>(sl.d_fills.cap, sl.d_hits.cap / ((size_t)kHitChunk * rw)),
-        sl.h_out.cap ? sl.h_out.cap - 1 : 0);
+    return (uint32_t)std::min<size_t>(sl.d_fills.cap, sl.d_hits.cap / ((size_t)kHitChunk * rw));
+}
+
+// Chunks for later steps after one that used `used`: one for each of its
+// waves, and twice those it claimed beyond.
+static uint64_t chunks_wanted(uint32_t used, int blocks) {
+    const uint64_t waves = (uint64_t)blocks * 4;
+    return used > waves ? waves + 2 * (used - waves) : waves;
 }
 
 // Publishes the chunks the step hit buffers hold (read by gss_step_stats
 // from any thread).
 static void note_hit_chunks(gss_engine *e) {
     int64_t c = 0;
-    for (const StepSlot &sl : e->slots) c += (int64_t)std::min(sl.d_fills.cap, sl.h_out.cap);
+    for (const StepSlot &sl : e->slots) c += (int64_t)sl.d_fills.cap;
     e->step_hit_chunks.store(c, std::memory_order_relaxed);
 }
 
 // The part of a step after its table updates, over the slot's buffers and
-// the settings of its graph: the sweep, the roll forward (held back if the
-// records overflowed), the chunk fills to the host and the records made
-// dense on the device right after the sweep, so that reading them on the
-// host is one DMA copy (no compute units taken from the next step's sweep;
-// serving steps: grouped by assignment word, so each request's records are
-// one range).
+// the settings of its graph: the sweep, then the roll forward (held back if
+// the records overflowed), the counts to the host and the records made dense
+// on the device, so that reading them on the host is one DMA copy (no compute
+// units taken from the next step's sweep) or, for few, none at all; serving
+// steps: grouped by assignment word, so each request's records are one range.
+// The sweep's counters are clear.
 static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     StepHeader *dh = sl.d_hdr.p;
     SweepArgs a{};
     a.buckets = sl.d_desc.p;
-    a.dyn = &dh->nbuckets;  // {nbuckets, ntasks}
-    a.task_clauses = sl.g_tc;
+    a.dyn = &dh->nbuckets;  // {nbuckets, npasses}
+    a.task_passes = sl.g_tp;
     a.table = e->table.p;
     a.valid = dh->valid;
     a.hits = (gss_hit *)sl.d_hits.p;
     a.fills = sl.d_fills.p;
     a.alloc = sl.d_alloc;
     a.chunk_cap = sl.chunk_cap;
-    a.fuse_len = sl.g_fuse;
     a.sentinel = (uint32_t)(2 * e->vars) << kLitShift;
     a.rec_words = sl.rec_words;
     uint8_t *agg =
         (sl.g_serve && e->serve_prefilter) || sl.g_screen ? e->serve_agg.p : nullptr;
     a.agg = agg;
     a.agg_words = agg ? e->serve_agg_words.p : nullptr;
-    a.agg_vote = e->serve_vote;
-    hipError_t he = launch_reset_u32(sl.d_alloc, 1, s);
-    if (he == hipSuccess) he = launch_sweep(a, e->words, sl.g_unroll, sl.g_blocks, s);
-    if (he == hipSuccess)
-        he = launch_assig_roll_dyn(sl.d_ups.p, &dh->nups, e->table.p, e->words, dh->last_pos,
-                                   sl.d_alloc, sl.chunk_cap, e->d_halt, s);
+    hipError_t he = launch_sweep(a, e->words, sl.g_blocks, s);
+    const ChunkArgs c = step_chunks(sl, sl.rec_words);
+    if (sl.g_serve) {
+        if (he == hipSuccess)
+            he = launch_group_by_word(c, sl.d_wcount.p, sl.d_dense.p, sl.d_dense.cap, sl.h_group.p,
+                                      sl.h_out.p, e->d_halt, s);
+        return he;
+    }
+    StepEndArgs end{};
+    end.dh = dh;
+    end.ups = sl.d_ups.p;
+    end.table = e->table.p;
+    end.words = e->words;
+    end.agg32 = sl.g_agg_fused ? (uint32_t *)agg : nullptr;
+    end.halt = e->d_halt;
+    end.out = sl.h_out.p;
+    end.dense = (uint64_t *)sl.d_dense.p;
+    end.dense_cap = sl.d_dense.cap;
+    end.host_words = kDirectWords;
+    if (he == hipSuccess) he = launch_step_end(c, end, s);
     // screened steps keep the aggregate current through the roll forward
-    if (he == hipSuccess && sl.g_screen)
-        he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, nullptr, false, e->words, agg,
-                                     nullptr, s);
-    if (he == hipSuccess)
-        he = launch_stage_out(sl.d_alloc, sl.d_fills.p, sl.chunk_cap, sl.h_out.p, s);
-    if (he == hipSuccess && sl.d_dense.cap > 0)
-        he = sl.g_serve ? launch_group_by_word(sl.d_alloc, sl.d_fills.p, sl.chunk_cap,
-                                               sl.d_hits.p, sl.rec_words, sl.d_wcount.p,
-                                               sl.d_dense.p, sl.d_dense.cap, sl.h_group.p, s)
-                        : launch_compact_records(sl.d_alloc, sl.d_fills.p, sl.chunk_cap,
-                                                 sl.d_offs.p, sl.d_hits.p, sl.d_dense.p,
-                                                 sl.d_dense.cap, sl.rec_words, s);
+    if (he == hipSuccess && sl.g_screen && !sl.g_agg_fused)
+        he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, nullptr, false, e->words, agg, s);
     return he;
 }
 
 // Captures the step's fixed launch sequence over this slot's buffers into
 // graph entry g (whose previous graph, if any, is destroyed first).
 static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr, int blocks,
-                            int tc, int fuse, bool serve, bool screen, bool agg_full) {
+                            int tp, bool serve, bool screen, bool agg_full, bool staged) {
     if (gr.exec) (void)hipGraphExecDestroy(gr.exec);
     if (gr.graph) (void)hipGraphDestroy(gr.graph);
     gr.exec = nullptr;
     gr.graph = nullptr;
     gr.key.clear();
     sl.g_blocks = blocks;
-    sl.g_tc = tc;
-    sl.g_fuse = fuse;
-    sl.g_unroll = e->tune_unroll;
+    sl.g_tp = tp;
     sl.g_serve = serve;
     sl.g_screen = screen;
     sl.g_agg_full = agg_full;
+    // at most 8 words: a word is its own screening group, so the kernels that
+    // write it know its entries (patches come after the updates: not then)
+    sl.g_agg_fused = screen && e->words <= 8 && !sl.g_patches;
     if (!e->capture_stream)
         HIP_TRY(hipStreamCreateWithFlags(&e->capture_stream, hipStreamNonBlocking));
     hipStream_t cs = e->capture_stream;
     HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    StageArgs st{};
+    StepInArgs st{};
     st.h[kRegHeader] = (const uint32_t *)sl.h_hdr.p;
     st.h[kRegDesc] = (const uint32_t *)sl.h_desc.p;
     st.h[kRegClauses] = (const uint32_t *)sl.h_cls.p;
@@ -1928,9 +1904,18 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     st.halt = e->d_halt;
     StepHeader *dh = sl.d_hdr.p;
     uint8_t *agg = (serve && e->serve_prefilter) || screen ? e->serve_agg.p : nullptr;
-    hipError_t he = hipSuccess;
-    if (he == hipSuccess) he = launch_stage_in(st, cs);
-    if (he == hipSuccess)
+    st.alloc = sl.d_alloc;
+    st.counts = serve ? sl.d_wcount.p : nullptr;
+    st.table = e->table.p;
+    st.words = e->words;
+    // updates come after base updates and word loads, where a step has them
+    st.apply = !sl.g_bases;
+    st.agg32 = sl.g_agg_fused && st.apply && !agg_full ? (uint32_t *)agg : nullptr;
+    st.agg_words = screen ? e->serve_agg_words.p : nullptr;
+    st.clauses = !staged;
+    st.shift = kLitShift;
+    hipError_t he = launch_step_in(st, cs);
+    if (he == hipSuccess && staged)
         he = launch_scatter_clauses(sl.d_cls.p, &dh->nclauses, sl.d_lits.p, kLitShift, cs);
     if (he == hipSuccess && sl.g_bases)
         he = launch_base_apply_dyn(sl.d_bups.p, &dh->nbups, e->bases.p, e->bases_vw, cs);
@@ -1950,19 +1935,19 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     if (he == hipSuccess && agg && serve)
         he = launch_serve_agg(e->serve, dh, sl.d_loads.p, e->bases.p, e->bases_vw, e->vars, agg,
                               e->serve_agg_words.p, cs);
-    if (he == hipSuccess) he = launch_assig_apply_dyn(sl.d_ups.p, &dh->nups, e->table.p, e->words, cs);
+    if (he == hipSuccess && !st.apply && !serve)
+        he = launch_assig_apply_dyn(sl.d_ups.p, &dh->nups, e->table.p, e->words, cs);
     if (he == hipSuccess && sl.g_patches)
         he = serve ? launch_serve_patch(e->serve, dh, e->table.p, e->words, agg, cs)
                    : launch_assig_patch_dyn(sl.d_patches.p, &dh->npatches, e->table.p, e->words,
                                             cs);
     // batched steps: the aggregate of the table as the sweep will read it,
     // rebuilt, or refreshed where this step's updates and patches changed it
-    if (he == hipSuccess && screen)
-        he = agg_full ? launch_table_agg(e->table.p, dh, e->vars, e->words, agg,
-                                         e->serve_agg_words.p, cs)
-                      : launch_table_agg_update(e->table.p, dh, sl.d_ups.p, sl.d_patches.p,
-                                                sl.g_patches, e->words, agg,
-                                                e->serve_agg_words.p, cs);
+    if (he == hipSuccess && screen && agg_full)
+        he = launch_table_agg(e->table.p, dh, e->vars, e->words, agg, cs);
+    else if (he == hipSuccess && screen && !st.agg32)
+        he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, sl.d_patches.p, sl.g_patches,
+                                     e->words, agg, cs);
     if (he == hipSuccess) he = launch_step_tail(e, sl, cs);
     hipGraph_t g = nullptr;
     hipError_t he2 = hipStreamEndCapture(cs, &g);
@@ -1974,12 +1959,11 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     gr.graph = g;
     HIP_TRY(hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0));
     gr.blocks = blocks;
-    gr.tc = tc;
-    gr.fuse = fuse;
-    gr.unroll = e->tune_unroll;
+    gr.tp = tp;
     gr.serve = serve;
     gr.screen = screen;
     gr.agg_full = agg_full;
+    gr.staged = staged;
     gr.dense = sl.d_dense.cap;
     e->graph_captures.fetch_add(1, std::memory_order_relaxed);
     return GSS_OK;
@@ -2010,20 +1994,21 @@ static int recover_step(gss_engine *e, size_t at, uint32_t used) {
     int rc = GSS_OK;
     if (want > chunk_room(sl, rw) &&
         ((rc = sl.d_hits.reserve_async((size_t)want * kHitChunk * rw, es)) ||
-         (rc = sl.d_fills.reserve_async((size_t)want, es)) || (rc = sl.h_out.reserve(want + 1))))
+         (rc = sl.d_fills.reserve_async((size_t)want, es))))
         sl.records_lost = true;
-    if (!sl.records_lost) {
-        sl.chunk_cap = chunk_room(sl, rw);
-        if ((rc = sl.d_offs.reserve_async((size_t)sl.chunk_cap + 1, es))) sl.records_lost = true;
-    }
+    if (!sl.records_lost) sl.chunk_cap = chunk_room(sl, rw);
     note_hit_chunks(e);
     HIP_TRY(launch_reset_u32(e->d_halt, 1, es));
     if (sl.records_lost) {
-        // no room: roll the table forward (the gate passes with no limit)
+        // no room: only roll the table forward
         HIP_TRY(launch_assig_roll_dyn(sl.d_ups.p, &sl.d_hdr.p->nups, e->table.p, e->words,
-                                      sl.d_hdr.p->last_pos, sl.d_alloc, UINT32_MAX, e->d_halt,
-                                      es));
+                                      sl.d_hdr.p->last_pos, es));
+        if (sl.g_screen)
+            HIP_TRY(launch_table_agg_update(e->table.p, sl.d_hdr.p, sl.d_ups.p, nullptr, false,
+                                            e->words, e->serve_agg.p, es));
     } else {
+        HIP_TRY(launch_reset_u32(sl.d_alloc, 2, es));
+        if (sl.g_serve) HIP_TRY(launch_reset_u32(sl.d_wcount.p, 2 * GSS_MAX_WORDS, es));
         HIP_TRY(launch_step_tail(e, sl, es));
     }
     HIP_TRY(hipEventRecord(sl.t1, es));
@@ -2035,7 +2020,7 @@ static int recover_step(gss_engine *e, size_t at, uint32_t used) {
         HIP_TRY(hipEventRecord(nx.t1, es));
         nx.settled = false;
     }
-    e->step_hit_want = std::max<uint64_t>(e->step_hit_want, 2 * (uint64_t)used);
+    e->step_hit_want = std::max(e->step_hit_want, chunks_wanted(used, sl.g_blocks));
     e->step_recoveries++;
     return sl.records_lost ? set_err(GSS_E_NOMEM, "a step's hit buffer overflowed (%u chunks) and "
                                                   "could not grow: its records are lost",
@@ -2347,26 +2332,25 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
             if (per[len] && (rc = ensure_bucket_cap(e, len, e->buckets[len].count + per[len])))
                 return rc;
     }
-    const int cpp = sweep_clauses_per_pass(W);
-    int tc = e->tune_task_clauses > 0 ? e->tune_task_clauses : 16 * cpp;
-    tc = std::max(cpp, (tc / cpp) * cpp);
+    const bool use_agg = (serve && e->serve_prefilter) || screen;
+    const int cpp = sweep_clauses_per_pass(W, use_agg);
     const size_t nlen = std::max(e->buckets.size(), per.size());
     auto rows_after = [&](size_t len) -> int64_t {
         const int64_t c = len < e->buckets.size() ? e->buckets[len].count : 0;
         return c + (len < per.size() ? per[len] : 0);
     };
     int nb = 0;
-    int64_t tasks = 0;
+    int64_t passes = 0;
     for (size_t len = 1; len < nlen; len++) {
         const int64_t c = rows_after(len);
         if (c > 0x7FFFFFFFll)
             return set_err(GSS_E_INVAL, "bucket %zu would hold %lld rows (at most 2^31 - 1)", len,
                            (long long)c);
         if (c) nb++;
-        tasks += (c + tc - 1) / tc;
+        passes += (c + cpp - 1) / cpp;
     }
-    if (tasks > 0x7FFFFFFF) return set_err(GSS_E_INVAL, "too many tasks");
-    const int blocks = step_blocks(e, ((serve && e->serve_prefilter) || screen ? 1 : 0) +
+    if (passes > 0x7FFFFFFF) return set_err(GSS_E_INVAL, "too many clauses");
+    const int blocks = step_blocks(e, (use_agg ? 1 : 0) +
                                           (desc->records == GSS_RECORDS_CLAUSES ? 2 : 0));
     // an abandoned chunk holds more than kHitChunk - 64 records and each wave
     // leaves at most one partial chunk: records <= clauses * active words
@@ -2390,8 +2374,15 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     if (sl.copy_queued) HIP_TRY(hipStreamWaitEvent(es, sl.ev_copied, 0));
     if (serve && ((rc = sl.h_report.reserve(1)) || (rc = sl.h_group.reserve(GSS_MAX_WORDS + 2))))
         return rc;
+    if ((rc = sl.h_out.reserve(4))) return rc;
+    // the pinned buffer that takes this step's records if they are few; a
+    // page-locked limit below its size rules it out
+    const int nd = sl.h_n + 1;
+    sl.direct_at = (sl.direct_at + 1) % nd;
+    const bool can_direct =
+        !serve && (e->page_limit < 0 || (int64_t)(kDirectWords * 8) < e->page_limit);
+    if (can_direct && (rc = sl.h_direct[sl.direct_at].reserve(kDirectWords))) return rc;
     if (serve && (rc = sl.d_wcount.reserve_async(2 * GSS_MAX_WORDS, e->stream))) return rc;
-    const bool use_agg = (serve && e->serve_prefilter) || screen;
     // a screened step rebuilds the aggregate unless the last change to the
     // table was a screened step's (word loads change whole words: rebuilt)
     const bool agg_full =
@@ -2420,8 +2411,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     if (want > chunk_room(sl, rw)) {
         const uint64_t chunks = e->tune_max_chunks > 0 ? want : 2 * want;
         if ((rc = sl.d_hits.reserve_async((size_t)chunks * kHitChunk * rw, e->stream)) ||
-            (rc = sl.d_fills.reserve_async((size_t)chunks, e->stream)) ||
-            (rc = sl.h_out.reserve(chunks + 1)))
+            (rc = sl.d_fills.reserve_async((size_t)chunks, e->stream)))
             return rc;
         note_hit_chunks(e);
     }
@@ -2431,14 +2421,16 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
                        : chunk_room(sl, rw);
     sl.worst_chunks = worst;
     sl.rec_words = rw;
-    if ((rc = sl.d_offs.reserve_async((size_t)sl.chunk_cap + 1, es))) return rc;
     if (sl.dense_want > sl.d_dense.cap && (rc = sl.d_dense.reserve_async(sl.dense_want, es)))
         return rc;
     if (!sl.d_alloc) HIP_TRY(hipMalloc((void **)&sl.d_alloc, 64));
     if (!sl.t0) HIP_TRY(hipEventCreate(&sl.t0));
     if (!sl.t1) HIP_TRY(hipEventCreate(&sl.t1));
     // ---- graph over exactly these buffers and settings
-    const int fuse = fuse_of(e);
+    const int tp = task_passes(e, use_agg);
+    // Few literals go straight from the staging to their rows (32-byte reads
+    // over PCIe); more are copied first and scattered by a kernel of its own.
+    const bool staged = total > kDirectLits;
     sl.g_bases |= serve || n_bups > 0 || n_loads > 0;
     sl.g_patches |= serve || n_patches > 0;
     std::vector<const void *> key = {
@@ -2446,17 +2438,16 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         sl.h_patches.p, sl.h_bups.p, sl.h_loads.p,
         sl.d_hdr.p, sl.d_desc.p, sl.d_cls.p, sl.d_lits.p, sl.d_ups.p, sl.d_hits.p,
         sl.d_patches.p, sl.d_bups.p, sl.d_loads.p,
-        sl.d_fills.p, sl.d_offs.p, sl.d_dense.p, (const void *)(intptr_t)sl.d_dense.cap,
+        sl.d_fills.p, sl.d_dense.p, (const void *)(intptr_t)sl.d_dense.cap,
         e->table.p, e->bases.p, (const void *)(intptr_t)e->bases_vw,
         (const void *)(intptr_t)W, (const void *)(intptr_t)e->vars,
-        (const void *)(intptr_t)e->tune_unroll, (const void *)(intptr_t)blocks,
-        (const void *)(intptr_t)tc, (const void *)(intptr_t)fuse,
+        (const void *)(intptr_t)blocks, (const void *)(intptr_t)tp,
         (const void *)(intptr_t)sl.chunk_cap, (const void *)(intptr_t)sl.rec_words,
         (const void *)(intptr_t)serve, sl.h_report.p, serve ? (const void *)e->serve.reqs : nullptr,
         sl.h_group.p, sl.d_wcount.p, (const void *)(intptr_t)(sl.g_bases + 2 * sl.g_patches),
         use_agg ? (const void *)e->serve_agg.p : nullptr,
         use_agg ? (const void *)e->serve_agg_words.p : nullptr,
-        (const void *)(intptr_t)(screen ? (agg_full ? 1 : 2) : 0)};
+        (const void *)(intptr_t)((screen ? (agg_full ? 1 : 2) : 0) + (staged ? 4 : 0))};
     int gi = -1;
     for (size_t i = 0; i < sl.graphs.size(); i++)
         if (sl.graphs[i].exec && sl.graphs[i].key == key) gi = (int)i;
@@ -2471,7 +2462,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         }
         StepSlot::StepGraph &gr = sl.graphs[gi];
         const auto t0 = std::chrono::steady_clock::now();
-        if ((rc = build_step_graph(e, sl, gr, blocks, tc, fuse, serve, screen, agg_full))) return rc;
+        if ((rc = build_step_graph(e, sl, gr, blocks, tp, serve, screen, agg_full, staged))) return rc;
         gss::log_stall("step graph capture", std::chrono::duration<double, std::milli>(
                                                   std::chrono::steady_clock::now() - t0)
                                                   .count());
@@ -2481,12 +2472,11 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     gr.used = ++sl.submits;
     sl.cur = gi;
     sl.g_blocks = gr.blocks;
-    sl.g_tc = gr.tc;
-    sl.g_fuse = gr.fuse;
-    sl.g_unroll = gr.unroll;
+    sl.g_tp = gr.tp;
     sl.g_serve = gr.serve;
     sl.g_screen = gr.screen;
     sl.g_agg_full = gr.agg_full;
+    sl.g_agg_fused = gr.screen && W <= 8 && !sl.g_patches;
     sl.step_dense = gr.dense;
     // ---- stage this step (the slot is idle) and commit it to the DB: one
     // record per clause (the device copies it to its bucket row)
@@ -2533,16 +2523,16 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         d.lits = b.d;
         d.len = (uint32_t)len;
         d.count = (uint32_t)b.count;
-        d.task_begin = (uint32_t)t;
+        d.pass_begin = (uint32_t)t;
         d.pad = 0;
-        t += (b.count + tc - 1) / tc;
+        t += (b.count + cpp - 1) / cpp;
     }
     StepHeader &h = *sl.h_hdr.p;
     std::memset(&h, 0, sizeof h);
     h.nbuckets = k;
     // with no valid slot every clause starts dead: the sweep has no work (a
     // serving step's admission decides that on the device)
-    h.ntasks = active_words ? (int32_t)t : 0;
+    h.npasses = active_words ? (int32_t)t : 0;
     h.nclauses = (int32_t)n;
     h.nups = n_ups;
     h.npatches = n_patches;
@@ -2560,6 +2550,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         h.valid[w] = w < W ? valid[w] : 0;
         h.last_pos[w] = (w < W && last_pos) ? last_pos[w] : -1;
     }
+    h.host_rec = can_direct ? sl.h_direct[sl.direct_at].p : nullptr;
     e->state_version++;
     e->table_agg_at = screen ? e->state_version : 0;
     HIP_TRY(hipEventRecord(sl.t0, e->stream));
@@ -2571,10 +2562,22 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     sl.serve = serve;
     // the previous records of this slot stay readable only if their copy
     // was queued (or there were none)
-    if (sl.rec_total > 0 && !sl.copy_queued) sl.results = false;
+    if (sl.rec_total > 0 && !sl.copy_queued && !sl.direct) sl.results = false;
     e->inflight.push_back(S);
     e->next_slot ^= 1;
     return GSS_OK;
+}
+
+// The last waited step's records of a slot, and the wait for their copy.
+static const void *records_at(StepSlot &sl) {
+    return sl.direct ? (const void *)sl.direct_rec : (const void *)sl.h_hits().p;
+}
+
+static hipError_t records_on_host(StepSlot &sl, int64_t total) {
+    const hipError_t he =
+        !sl.direct && !sl.host_ready && total > 0 ? hipEventSynchronize(sl.ev_copied) : hipSuccess;
+    if (he == hipSuccess) sl.host_ready = true;
+    return he;
 }
 
 extern "C" {
@@ -2611,9 +2614,8 @@ int gss_step_wait(gss_engine *e, int64_t *n_hits, float *step_ms) {
                              sl.chunk_cap);
     }
     // the next steps' buffers hold twice the most chunks a step has claimed
-    e->step_hit_want = std::max<uint64_t>(e->step_hit_want, 2 * (uint64_t)used);
-    int64_t tot = 0;
-    for (uint32_t c = 0; c < used; c++) tot += sl.h_out.p[1 + c];
+    e->step_hit_want = std::max(e->step_hit_want, chunks_wanted(used, sl.g_blocks));
+    const int64_t tot = (int64_t)((uint64_t)sl.h_out.p[1] | ((uint64_t)sl.h_out.p[2] << 32));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, sl.t0, sl.t1));
     sl.results = false;
@@ -2623,13 +2625,15 @@ int gss_step_wait(gss_engine *e, int64_t *n_hits, float *step_ms) {
     // the slot's next capture compacts into a buffer with room to spare once
     // the records pass half of the current one (a step whose records do not
     // fit is compacted, or grouped, outside the graph)
-    if (2 * (uint64_t)tot > sl.step_dense)
+    sl.direct = sl.h_hdr.p->host_rec && (uint64_t)tot * sl.rec_words <= kDirectWords;
+    sl.direct_rec = sl.h_hdr.p->host_rec;
+    if (!sl.direct && 2 * (uint64_t)tot > sl.step_dense)
         sl.dense_want = std::max<uint64_t>(sl.dense_want, 4 * (uint64_t)tot);
     e->last_step_slot = S;
     e->last_step_hits = tot;
     e->last_step_chunks = used;
     e->last_step_ms = ms;
-    if (tot > 0 && (rc = queue_records_copy(e, sl, tot, used))) return rc;
+    if (tot > 0 && !sl.direct && (rc = queue_records_copy(e, sl, tot))) return rc;
     sl.results = true;
     if (n_hits) *n_hits = tot;
     if (step_ms) *step_ms = ms;
@@ -2662,9 +2666,8 @@ int gss_step_hits_map(gss_engine *e, const gss_hit **out, int64_t *n) {
                                     "(gss_step_ids_map, gss_step_clauses_map)");
     const int64_t total = e->last_step_hits;
     if (n) *n = total;
-    if (!sl.host_ready && total > 0) HIP_TRY(hipEventSynchronize(sl.ev_copied));
-    sl.host_ready = true;
-    *out = sl.h_hits().p;
+    HIP_TRY(records_on_host(sl, total));
+    *out = (const gss_hit *)records_at(sl);
     return GSS_OK;
 }
 
@@ -2680,9 +2683,8 @@ int gss_step_ids_map(gss_engine *e, const gss_hit_id **out, int64_t *n) {
         return set_err(GSS_E_STATE, "the last waited step recorded another form");
     const int64_t total = e->last_step_hits;
     if (n) *n = total;
-    if (!sl.host_ready && total > 0) HIP_TRY(hipEventSynchronize(sl.ev_copied));
-    sl.host_ready = true;
-    *out = (const gss_hit_id *)sl.h_hits().p;
+    HIP_TRY(records_on_host(sl, total));
+    *out = (const gss_hit_id *)records_at(sl);
     return GSS_OK;
 }
 
@@ -2698,9 +2700,8 @@ int gss_step_clauses_map(gss_engine *e, const gss_hit_clause **out, int64_t *n) 
         return set_err(GSS_E_STATE, "the last waited step recorded another form");
     const int64_t total = e->last_step_hits;
     if (n) *n = total;
-    if (!sl.host_ready && total > 0) HIP_TRY(hipEventSynchronize(sl.ev_copied));
-    sl.host_ready = true;
-    *out = (const gss_hit_clause *)sl.h_hits().p;
+    HIP_TRY(records_on_host(sl, total));
+    *out = (const gss_hit_clause *)records_at(sl);
     return GSS_OK;
 }
 

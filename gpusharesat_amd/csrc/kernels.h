@@ -16,26 +16,25 @@ struct BucketDesc {
                            // row offsets (literal << 7)
     uint32_t len;
     uint32_t count;        // rows
-    uint32_t task_begin;   // first task index of this bucket
+    uint32_t pass_begin;   // first wave pass of this bucket
     uint32_t pad;
 };
 
 struct SweepArgs {
     const BucketDesc *buckets;
     int nbuckets;
-    int ntasks;
-    int task_clauses;        // clauses per task (multiple of clauses per wave pass)
+    int npasses;             // wave passes over all buckets (sweep_clauses_per_pass clauses each)
+    int task_passes;         // passes a wave takes at a time (0: see kTaskRounds in kernels.hip)
     const uint64_t *table;   // [2 * vars + 2][words]: row l = slots where literal l is not
                              // false; rows 2*vars (zeros), 2*vars+1 (ones) are sentinels
     const uint64_t *valid;   // [words]
     gss_hit *hits;           // chunk_cap * kHitChunk records
-    uint32_t *fills;         // [chunk_cap] records used in each claimed chunk
-    uint32_t *alloc;         // number of chunks claimed (may exceed chunk_cap)
+    uint32_t *fills;         // [chunk_cap] records used in each chunk
+    uint32_t *alloc;         // zero before the sweep: [0] chunks claimed past the waves' own
+                             // (wave g starts in chunk g), [1] chunks past chunk_cap with records
     uint32_t chunk_cap;
-    int fuse_len;            // clauses of at most this many literals use the fused schedule
-                             // (<= 0: none, and the kernel without that path runs)
     uint32_t sentinel;       // stored row offset of the sentinel literal
-    const int32_t *dyn;      // if set, {nbuckets, ntasks} are read here (graph replays)
+    const int32_t *dyn;      // if set, {nbuckets, npasses} are read here (graph replays)
     int rec_words;           // 8-byte words per record: 3 (gss_hit), 1 (gss_hit_id) or 2
                              // (gss_hit_clause: one record per clause, its words as a mask)
     // Serving and screened batched steps (null otherwise): bit b of agg[l]
@@ -49,7 +48,6 @@ struct SweepArgs {
     // other words.  4 MB at 2M variables: the votes are served from L2.
     const uint8_t *agg;
     const uint64_t *agg_words;  // [8]
-    int agg_vote;               // aggregate entries read together per vote: 1, 2, 4 or 8
 };
 
 // Staged regions of a batched step, copied host -> device by k_stage_in.
@@ -69,7 +67,7 @@ enum StepRegion {
 // pinned staging slot and copied to the device by k_stage_in.
 struct StepHeader {
     int32_t nbuckets;
-    int32_t ntasks;
+    int32_t npasses;
     int32_t nclauses;
     // 1 in the device copy when the step found the engine halted: every
     // count is then 0 and the step does nothing (it is replayed later)
@@ -78,15 +76,49 @@ struct StepHeader {
     int64_t region_words[kStageRegions];  // uint32 words of each region to copy
     uint64_t valid[GSS_MAX_WORDS];
     int8_t last_pos[GSS_MAX_WORDS];
+    uint64_t *host_rec;  // pinned memory that takes the step's records if they fit there
 };
 
-struct StageArgs {
+struct StepEndArgs {
+    const StepHeader *dh;
+    const gss_var_update *ups;
+    uint64_t *table;
+    int words;
+    uint32_t *agg32;      // as in StepInArgs
+    uint32_t *halt;       // set if records were dropped
+    uint32_t *out;        // counts for the host: see write_counts in kernels.hip
+    uint64_t *dense;
+    uint64_t dense_cap;   // records
+    uint64_t host_words;  // 8-byte words at StepHeader::host_rec
+};
+
+// The hit chunks a sweep of `waves` waves left (SweepArgs).
+struct ChunkArgs {
+    const uint64_t *hits;
+    const uint32_t *fills;
+    const uint32_t *alloc;
+    uint32_t cap;        // chunks in the buffer
+    uint32_t waves;
+    uint32_t rec_words;  // 8-byte words per record
+};
+
+struct StepInArgs {
     const uint32_t *h[kStageRegions];  // pinned host (h[kRegHeader] = the header)
     uint32_t *d[kStageRegions];        // device
     // device word, nonzero while the engine is halted: an earlier step's
     // records overflowed its hit buffer and its sweep is to be re-run before
     // the table moves on
     const uint32_t *halt;
+    uint32_t *alloc;      // the sweep's counters, cleared
+    uint32_t *counts;     // serving: 2 * 64 counters of the grouping, cleared (else null)
+    uint64_t *table;
+    uint32_t *agg32;      // apply with at most 8 words: screening entries to keep current
+                          // (null: none, or a later kernel does it)
+    uint64_t *agg_words;  // screened steps: [8], written from the header (else null)
+    int words;
+    int apply;            // apply the updates (else they are copied for a later kernel)
+    int clauses;          // copy the clauses to their rows (else to the staged regions)
+    int shift;            // of a literal on its way to its row
 };
 
 struct ScatterSeg {
@@ -158,19 +190,17 @@ hipError_t launch_serve_admit(const ServeRing &r, StepHeader *dh, gss_word_load 
 // SweepArgs::agg): group b = words [b * words / 8, (b + 1) * words / 8) (one
 // word per group below 8 words); bit b of agg[l] set if row l is all ones on
 // every slot of group b's words (valid or not: all ones there implies all
-// ones on the valid slots); agg_words[b] = the group's words with a valid
-// slot in this step.  Reads the table once.
+// ones on the valid slots).  Reads the table once.
 hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t vars, int words,
-                            uint8_t *agg, uint64_t *agg_words, hipStream_t s);
+                            uint8_t *agg, hipStream_t s);
 // Keeps such entries current without reading the table: for each of the
 // step's updates (and patches, if with_patches) the bit of the update's word
 // group in both literals of its variable, from the table as it is when the
-// kernel runs; agg_words as above if not null.  Run after the updates are
-// applied and again after the roll forward.
+// kernel runs.  Run after the updates are applied and again after the roll
+// forward.
 hipError_t launch_table_agg_update(const uint64_t *table, const StepHeader *dh,
                                    const gss_var_update *ups, const gss_var_patch *patches,
-                                   bool with_patches, int words, uint8_t *agg,
-                                   uint64_t *agg_words, hipStream_t s);
+                                   bool with_patches, int words, uint8_t *agg, hipStream_t s);
 // Copies the admitted requests' patches from the pinned ring to r.dpatches
 // (consecutive lanes read consecutive 4-byte words: one pass over PCIe).
 hipError_t launch_serve_stage_patches(const ServeRing &r, const StepHeader *dh, hipStream_t s);
@@ -197,14 +227,13 @@ struct CompactRef {
     uint32_t pad;
 };
 
-// words is the table row width (power of two, 1..64); unroll selects the
-// number of rows in flight per lane for 16 words and wider (0 = default).
-hipError_t launch_sweep(const SweepArgs &a, int words, int unroll, int blocks, hipStream_t s);
-int sweep_clauses_per_pass(int words);
-// Max resident 256-thread blocks per CU for the sweep kernel variant (with or
-// without the fused schedule; mode 0: plain, 1: screened, 2: clause records,
-// 3: screened with clause records).
-int sweep_occupancy(int words, int unroll, bool fused, int mode = 0);
+// words is the table row width (power of two, 1..64); a.agg and a.rec_words
+// choose the kernel.
+hipError_t launch_sweep(const SweepArgs &a, int words, int blocks, hipStream_t s);
+int sweep_clauses_per_pass(int words, bool screened);
+// Resident 256-thread blocks per CU of a sweep kernel (mode 0: plain, 1:
+// screened, 2: clause records, 3: screened with clause records).
+int sweep_occupancy(int words, int mode);
 
 hipError_t launch_reset_u32(uint32_t *p, int n, hipStream_t s);
 hipError_t launch_scatter(const ScatterSeg *segs, int nseg, const uint32_t *src, int shift,
@@ -217,46 +246,37 @@ hipError_t launch_fill_u64(uint64_t *p, int64_t n, uint64_t v, hipStream_t s);
 
 // Fixed-shape launches of a batched step (counts read from the device header,
 // so a captured graph can be replayed with new data).  While the engine is
-// halted k_stage_in writes a header with no work and `halted` set instead of
+// halted k_step_in writes a header with no work and `halted` set instead of
 // staging: every later kernel of the step then has nothing to do (the
 // serving kernels and k_table_agg, whose work is not counted by the header,
 // test `halted` themselves).
-hipError_t launch_stage_in(const StageArgs &a, hipStream_t s);
+hipError_t launch_step_in(const StepInArgs &a, hipStream_t s);
+hipError_t launch_step_end(const ChunkArgs &c, const StepEndArgs &a, hipStream_t s);
 // Copies each staged clause (n read on the device) to its bucket row,
 // shifting literals left by `shift`.
 hipError_t launch_scatter_clauses(const ClauseSeg *cls, const int32_t *n, const uint32_t *src,
                                   int shift, hipStream_t s);
 hipError_t launch_assig_apply_dyn(const gss_var_update *ups, const int64_t *n, uint64_t *table,
                                   int words, hipStream_t s);
-// Rolls the step's updated entries forward -- unless the sweep before it
-// claimed more than `cap` hit chunks: then the table stays as the sweep read
-// it and *halt is set, so that the sweep can be re-run with room for every
-// record.
+// Rolls the step's updated entries forward (k_step_end does, after a sweep
+// that kept its records).
 hipError_t launch_assig_roll_dyn(const gss_var_update *ups, const int64_t *n, uint64_t *table,
-                                 int words, const int8_t *last_pos, const uint32_t *alloc,
-                                 uint32_t cap, uint32_t *halt, hipStream_t s);
-hipError_t launch_stage_out(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                            uint32_t *h_out, hipStream_t s);
-// Chunks claimed and records of a sweep to pinned host memory: h_out[0] =
-// claims, h_out[1] / h_out[2] = low / high word of the record count.
-hipError_t launch_count_records(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                                uint32_t *h_out, hipStream_t s);
+                                 int words, const int8_t *last_pos, hipStream_t s);
+// Counts of a plain sweep to pinned host memory (write_counts in
+// kernels.hip); next = the counters of the sweep after it, cleared.
+hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, hipStream_t s);
 // Dense copy of a sweep's records (chunk order, the records of a chunk in
-// place): offs = exclusive prefix of the fills of the claimed chunks (cap + 1
-// entries), dense = the records, when they all fit in dense_cap records;
-// counts are read on the device.  Records are rec_words 8-byte words (3: a
-// gss_hit, 1: a gss_hit_id, 2: a gss_hit_clause); chunk c starts at word
-// c * kHitChunk * rec_words.
-hipError_t launch_compact_records(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                                  uint64_t *offs, const void *hits, void *dense,
-                                  uint64_t dense_cap, int rec_words, hipStream_t s);
+// place) when they all fit in dense_cap records; counts are read on the
+// device.  Chunk c starts at word c * kHitChunk * rec_words.
+hipError_t launch_gather(const ChunkArgs &c, void *dense, uint64_t dense_cap, hipStream_t s);
 // Dense copy of a sweep's records grouped by assignment word, ascending:
-// counts = 2 * 64 uint32 of device scratch (cleared here), group = 66 uint64:
+// counts = 2 * 64 uint32 of device scratch (zero), group = 66 uint64:
 // group[w] = first record of word w, group[64] = all, group[65] = 1 if they
-// fitted in dense_cap records (else nothing moved).
-hipError_t launch_group_by_word(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                                const void *hits, int rec_words, uint32_t *counts,
-                                void *dense, uint64_t dense_cap, uint64_t *group, hipStream_t s);
+// fitted in dense_cap records (else nothing moved); out = the counts for the
+// host, *halt set if records were dropped.
+hipError_t launch_group_by_word(const ChunkArgs &c, uint32_t *counts, void *dense,
+                                uint64_t dense_cap, uint64_t *group, uint32_t *out,
+                                uint32_t *halt, hipStream_t s);
 // Solver base planes: bases[(2 b) * vw + i] / bases[(2 b + 1) * vw + i] hold
 // bit (v mod 64) of word i = v / 64 of base b's is_def / is_true.
 hipError_t launch_base_apply_dyn(const gss_base_update *u, const int64_t *n, uint64_t *bases,

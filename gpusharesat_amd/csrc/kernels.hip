@@ -13,20 +13,14 @@
 //   true    nt = AND over the clause of nf_{l^1} (no literal is true)
 //   report  falsified = ~c1;  unit = c1 & ~c2 & nt
 //
-// A slot with c2 set, or outside nt, can never report, so a clause stops once
-// every valid slot of every word of its group is dead.  Two schedules give the
-// same answer:
-//   two-pass  pass 1 reads only rows nf_l (1 bit per slot per literal) and
-//             stops on c2; pass 2 reads rows nf_{l^1} only if some slot has
-//             exactly one non-false occurrence, and stops once those slots are
-//             resolved;
-//   fused     one pass reads both rows of each literal (adjacent in memory)
-//             and stops on c2 | ~nt.
-// A clause of at most `fuse_len` literals uses the fused schedule, longer
-// ones the two-pass one.  Duplicate literals are separate occurrences, as in
-// the reference (GpuRunner.cu:68-89 walks the literal list), so "x, x" with x
-// undefined is not unit.  tests/test_oracle.py and the GPU parity tests check
-// the forms agree.
+// A slot with c2 set can never report, so a clause stops once every valid
+// slot is dead.  The check reads the rows nf_l first (1 bit per slot per
+// literal) until then; a slot that ends with exactly one non-false occurrence
+// needs nt, and there only the row nf_{l^1} of that one literal can hold a
+// zero, so only those negated rows are read.  Duplicate literals are separate
+// occurrences, as in the reference (GpuRunner.cu:68-89 walks the literal
+// list), so "x, x" with x undefined is not unit.  tests/test_oracle.py and the
+// GPU parity tests check the forms agree.
 //
 // Clause literals are stored on the device as row offsets: literal l as
 // l << 7, the byte offset of its row in a table of 16 words (scaled by the
@@ -34,31 +28,32 @@
 // the end of a clause hold the offset of a sentinel row pair (nf = 0, and
 // all ones for its negation) that contributes nothing, so they need no mask.
 //
-// Work mapping.  A group of 16 lanes owns one clause.  Up to 16 words, lane
-// (s, w) of the group handles table word w and literal sub-lane s (G = W*S =
-// 16); at 32 and 64 words each lane handles K = W/16 consecutive words, read
-// with 16-byte loads, so every width checks 4 clauses per wave pass and keeps
-// 4*U row reads per wave in flight.  The group loads G literals of the
-// clause at once (lane q holds literal q of the chunk; the first chunk of the
-// next clause is prefetched while the current one is checked) and hands them
-// out with DPP row broadcasts (G = 16: a group is one 16-lane DPP row) or
-// shuffles; each step a lane issues U row reads (U independent loads in
-// flight), the S sub-lanes' counts are merged with a butterfly, then the group
-// votes on early exit.  With W = 16 (1024 slots) a row read by the 16 lanes of
-// a group is one coalesced 128-byte line.  A wave holds 64/G groups; a task is
-// a run of clauses of one length bucket (its parameters are wave-uniform and
-// live in scalar registers); waves are persistent and take tasks round-robin.
+// Work mapping.  k_sweep: W lanes check one clause, one table word each, 64 / W
+// clauses per wave pass, literals handed out with DPP (no LDS); k_sweep_screened:
+// one clause per lane against the aggregate, then one surviving (clause, word)
+// per lane.  Waves are persistent and walk the clauses in tasks of passes.
+//
+// What bounds it is the row reads: 128-byte lines of a table that the L2s do
+// not hold, ~6.9 TB/s of them at any size past 32 MB.  Measured on one MI355X,
+// kernel alone, before (16 lanes per clause at every width, 4 rows per step,
+// all negated rows of a clause left with a candidate, both rows of every
+// literal up to 4 literals) and now:
+//   16 words, 4M clauses, 1M variables, random values   711 -> 618 us
+//   16 words, 2M clauses, 500k variables, planted       204 -> 119 us
+//   64 words, 400k clauses, 200k variables, planted     140 ->  87 us
+//    8 words, 1M clauses, 100k variables, planted       109 ->  45 us
+//    1 word,  100k clauses, 10k variables, random        32 ->  10 us
+// Rows read per clause, counted on the CPU: 7.97 -> 6.95 (random), 4.54 -> 2.77
+// (planted).
 //
 // Hits.  A clause/word with a report becomes one 24-byte record (gss_hit:
 // clause, word and both masks), or, for delivery to the solvers, which never
 // read the masks, one 8-byte record (gss_hit_id: the first word of the
-// gss_hit).  Each wave compacts its records with a ballot + mbcnt prefix and
-// appends them to a private chunk of kHitChunk records claimed with one
-// atomic (non-temporal stores: records are never re-read by the sweep); a
-// chunk is abandoned (fill recorded) when the next pass does not fit.  Capacity is
-// sized on the host so that nothing is dropped (the reference drops on
-// overflow, gpuShareLib/Reporter.cuh:46-48); if it ever is exceeded the claim
-// counter still counts and the host re-runs the sweep.
+// gss_hit), or one gss_hit_clause per clause.  Each wave compacts its records
+// with a ballot + mbcnt prefix into chunks of kHitChunk records of its own
+// (HitWriter).  Capacity is sized on the host so that nothing is dropped (the
+// reference drops on overflow, gpuShareLib/Reporter.cuh:46-48); if it ever is
+// exceeded the counters tell, and the host re-runs the sweep.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -92,14 +87,9 @@ __device__ __forceinline__ uint32_t prefix_count(unsigned long long bal) {
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-template <int G>
-__device__ __forceinline__ bool group_any(bool pred, uint64_t gmask) {
-    const unsigned long long b = __ballot(pred);
-    if constexpr (G == 64) {
-        return b != 0;
-    } else {
-        return (b & gmask) != 0;
-    }
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+    return (uint64_t)(uint32_t)uniform((int)(uint32_t)x) |
+           ((uint64_t)(uint32_t)uniform((int)(uint32_t)(x >> 32)) << 32);
 }
 
 // Byte offset inside the table of row word w, from a stored row offset
@@ -111,56 +101,6 @@ __device__ __forceinline__ uint32_t scale_offset(uint32_t stored) {
     else return stored >> (W == 8 ? 1 : W == 4 ? 2 : W == 2 ? 3 : 4);
 }
 
-// Address of row word w of the literal at chunk position J, for every lane of
-// the group.  With G = 16 a group is one DPP row, so the literal is a row
-// broadcast (no LDS), fused with the add of the lane's word offset.
-template <int W, int G, int J>
-__device__ __forceinline__ uint32_t chunk_addr(uint32_t litreg, int gbase, uint32_t w8) {
-    if constexpr (G == 16 && W == 16) {
-        return (uint32_t)__builtin_amdgcn_mov_dpp((int)litreg, 0x150 + J, 0xF, 0xF, false) | w8;
-    } else if constexpr (G == 16) {
-        return scale_offset<W>(
-                   (uint32_t)__builtin_amdgcn_mov_dpp((int)litreg, 0x150 + J, 0xF, 0xF, false)) |
-               w8;
-    } else {
-        return scale_offset<W>((uint32_t)__shfl((int)litreg, gbase + J)) | w8;
-    }
-}
-
-typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-
-// K consecutive table words of one row (K = 1, 2 or 4), read with 8- or
-// 16-byte loads.
-template <int K>
-struct Words {
-    uint64_t v[K];
-};
-
-template <int K>
-__device__ __forceinline__ Words<K> load_words(const uint64_t *__restrict__ table, uint32_t off) {
-    Words<K> r;
-    const char *p = (const char *)table + off;
-    if constexpr (K == 1) {
-        r.v[0] = *(const uint64_t *)p;
-    } else {
-#pragma unroll
-        for (int i = 0; i < K; i += 2) {
-            const u64x2 x = *(const u64x2 *)(p + 8 * i);
-            r.v[i] = x.x;
-            r.v[i + 1] = x.y;
-        }
-    }
-    return r;
-}
-
-// Clause state of one lane for its K words: saturating count of non-false
-// occurrences per slot (c1: >= 1, c2: >= 2) and the slots where no literal is
-// true (nt).
-template <int K>
-struct ClauseState {
-    uint64_t c1[K], c2[K], nt[K];
-};
-
 // Offset of the negated literal's row: stored offsets are literal << 7, so the
 // negation flips bit 7, scaled like the offset.
 template <int W>
@@ -168,392 +108,542 @@ __device__ __forceinline__ uint32_t neg_bit() {
     return scale_offset<W>(128u);
 }
 
-// One step: U literals per lane.  The chunk holds the group's literals
-// [base, base + G), sentinel past the clause end; this step covers chunk
-// positions [ST, ST + S*U).  The U row reads are issued back to back, folded
-// into the state, and for S > 1 the S sub-lanes are merged with a butterfly.
-template <int W, int S, int U, int K, int ST, bool ROWS_F, bool ROWS_T>
-__device__ __forceinline__ void step_rows(uint32_t litreg, int gbase, int sub, uint32_t w8,
-                                          const uint64_t *__restrict__ table,
-                                          ClauseState<K> &cs, bool live) {
-    constexpr int LW = W / K;  // lanes across one row
-    constexpr int G = LW * S;
-    Words<K> f[U], t[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        uint32_t off;
-        if constexpr (S == 1 && U <= 4) {
-            off = u == 0 ? chunk_addr<W, G, ST + 0>(litreg, gbase, w8)
-                : u == 1 ? chunk_addr<W, G, (ST + 1) % G>(litreg, gbase, w8)
-                : u == 2 ? chunk_addr<W, G, (ST + 2) % G>(litreg, gbase, w8)
-                         : chunk_addr<W, G, (ST + 3) % G>(litreg, gbase, w8);
-        } else if constexpr (S == 1) {
-            off = scale_offset<W>((uint32_t)__shfl((int)litreg, gbase + ST + u)) | w8;
-        } else {
-            off = scale_offset<W>((uint32_t)__shfl((int)litreg, gbase + ST + sub * U + u)) | w8;
-        }
-        // A lane whose slots are all settled skips its reads (wide rows:
-        // lines of settled lanes are not fetched; at one word per lane a
-        // partial line is fetched whole, so 16-word rows do not skip);
-        // all-ones rows leave its state's report masks unchanged.
-        if (live) {
-            if (ROWS_F) f[u] = load_words<K>(table, off);
-            if (ROWS_T) t[u] = load_words<K>(table, off ^ neg_bit<W>());
-        } else {
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                if (ROWS_F) f[u].v[k] = ~0ull;
-                if (ROWS_T) t[u].v[k] = ~0ull;
-            }
-        }
-    }
-    if constexpr (S == 1) {
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                if (ROWS_F) {
-                    cs.c2[k] |= cs.c1[k] & f[u].v[k];
-                    cs.c1[k] |= f[u].v[k];
-                }
-                if (ROWS_T) cs.nt[k] &= t[u].v[k];
-            }
-        }
+__device__ __forceinline__ uint64_t load_word(const uint64_t *__restrict__ table, uint32_t off) {
+    return *(const uint64_t *)((const char *)table + off);
+}
+
+// Clause literals: a global-memory pointer (made from the bucket descriptor's
+// address, which the compiler would otherwise read with FLAT loads).
+typedef const __attribute__((address_space(1))) uint32_t *LitPtr;
+
+// A clause is checked by W lanes (lane w: table word w), which share its
+// literals: a literal register holds G = min(W, 16) consecutive literals of
+// the clause, one per lane of each G-lane group, and kRegs of them hold the
+// first kHeld literals.  Wider clauses repeat the group (every 16-lane DPP
+// row holds the same 16 literals), so a literal is always handed out inside
+// one DPP row.
+template <int W>
+struct Lits {
+    static constexpr int G = W < 16 ? W : 16;
+    static constexpr int kRegs = W >= 4 ? 1 : 4 / W;
+    static constexpr int kHeld = G * kRegs;  // 16, 8 (W = 8) or 4
+    uint32_t r[kRegs];
+};
+
+// The literal at position J of the held ones, in every lane of the group: a
+// DPP broadcast (row_newbcast for 16 lanes, two of them under bank masks for
+// 8, quad_perm for 4 and 2), so no LDS.  All 64 lanes must call it.
+template <int W, int J>
+__device__ __forceinline__ uint32_t lit_at(const Lits<W> &l) {
+    constexpr int G = Lits<W>::G, R = J / G, Q = J % G;
+    const int x = (int)l.r[R];
+    if constexpr (G == 16) {
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x150 + Q, 0xF, 0xF, false);
+    } else if constexpr (G == 8) {
+        const int lo = __builtin_amdgcn_mov_dpp(x, 0x150 + Q, 0xF, 0xF, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp(lo, x, 0x150 + 8 + Q, 0xF, 0xC, false);
+    } else if constexpr (G == 4) {
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, Q * 0x55, 0xF, 0xF, false);
+    } else if constexpr (G == 2) {
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, Q * 0x55 + 0xA0, 0xF, 0xF, false);
     } else {
-        static_assert(K == 1, "sub-lanes split narrow rows only");
-        uint64_t m1 = 0, m2 = 0, tt = ~0ull;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (ROWS_F) {
-                m2 |= m1 & f[u].v[0];
-                m1 |= f[u].v[0];
-            }
-            if (ROWS_T) tt &= t[u].v[0];
-        }
-#pragma unroll
-        for (int d = W; d < G; d <<= 1) {
-            if (ROWS_F) {
-                const uint64_t p1 = __shfl_xor(m1, d);
-                const uint64_t p2 = __shfl_xor(m2, d);
-                m2 = m2 | p2 | (m1 & p1);
-                m1 |= p1;
-            }
-            if (ROWS_T) tt &= __shfl_xor(tt, d);
-        }
-        if (ROWS_F) {
-            cs.c2[0] |= m2 | (cs.c1[0] & m1);
-            cs.c1[0] |= m1;
-        }
-        if (ROWS_T) cs.nt[0] &= tt;
+        return (uint32_t)x;
     }
 }
 
-// Runs the steps of one preloaded chunk while they start before the clause
-// end and `more(cs)` holds.  Returns false if it stopped early.
-template <int W, int S, int U, int K, bool ROWS_F, bool ROWS_T, typename More, typename Live>
-__device__ __forceinline__ bool chunk_steps(uint32_t litreg, int gbase, int sub, uint32_t w8,
-                                            int base, int len,
-                                            const uint64_t *__restrict__ table,
-                                            ClauseState<K> &cs, More &&more, Live &&live) {
-    constexpr int G = (W / K) * S;
-    constexpr int LPS = S * U;
-    bool go = true;
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-        ((go = go && (base + I * LPS < len) &&
-               [&] {
-                   step_rows<W, S, U, K, I * LPS, ROWS_F, ROWS_T>(
-                       litreg, gbase, sub, w8, table, cs, K > 1 ? live(cs) : true);
-                   return more(cs);
-               }()),
-         ...);
-    }(std::make_integer_sequence<int, G / LPS>{});
-    return go;
+// Literals [base, base + kHeld) of the clause whose row starts at cl (lane q
+// of its group holds literals base + q + G * r), the sentinel past its end
+// and for lanes without a clause (on = false).
+template <int W>
+__device__ __forceinline__ Lits<W> load_lits(LitPtr cl, int base, int len,
+                                             int q, bool on, uint32_t sentinel) {
+    Lits<W> l;
+#pragma unroll
+    for (int r = 0; r < Lits<W>::kRegs; r++) {
+        const int j = base + r * Lits<W>::G + q;
+        l.r[r] = on && j < len ? cl[j] : sentinel;
+    }
+    return l;
 }
 
-// Evaluates one clause for this lane's K words.  All G lanes of the group call
-// it together (group-uniform control flow).  first_chunk holds literal q of
-// the clause in lane q of the group (the sentinel past the end), already
-// loaded by the caller.
-template <int W, int S, int U, int K, bool FUSE>
-__device__ __forceinline__ void check_clause(const uint32_t *__restrict__ cl, int len,
-                                             uint32_t first_chunk, uint32_t sentinel,
-                                             const uint64_t *__restrict__ table, int q,
-                                             uint64_t gmask, int gbase, uint32_t w8, int sub,
-                                             const uint64_t (&valid)[K], int fuse_len,
-                                             uint64_t (&fm)[K], uint64_t (&um)[K]) {
-    constexpr int G = (W / K) * S;
-    // invalid slots start dead
-    ClauseState<K> cs;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        cs.c1[k] = ~valid[k];
-        cs.c2[k] = ~valid[k];
-        cs.nt[k] = ~0ull;
+// Bucket of pass p: the last one whose first pass is <= p.  One lane per
+// bucket (a binary search is a chain of 6-9 dependent scalar loads).
+__device__ __forceinline__ int find_bucket(const BucketDesc *__restrict__ b, int nb, int p,
+                                           int lane) {
+    int n = 0;
+    for (int i = 0; i < nb; i += 64) {
+        const bool le = i + lane < nb && (int)b[i + lane].pass_begin <= p;
+        n += __popcll(__ballot(le));
     }
-    // FUSE = false compiles the two-pass schedule only (its registers are
-    // then not sized for the fused path's two rows per literal)
-    const bool fused = FUSE && len <= fuse_len;
-    auto lane_alive = [&](const ClauseState<K> &c) {
-        uint64_t x = 0;
-#pragma unroll
-        for (int k = 0; k < K; k++) x |= c.nt[k] & ~c.c2[k];
-        return x != 0;
-    };
-    auto alive = [&](const ClauseState<K> &c) { return group_any<G>(lane_alive(c), gmask); };
-    uint32_t litreg = first_chunk;
-    for (int base = 0; base < len; base += G) {
-        if (base) litreg = base + q < len ? cl[base + q] : sentinel;
-        const bool go =
-            fused ? chunk_steps<W, S, U, K, true, true>(litreg, gbase, sub, w8, base, len, table,
-                                                       cs, alive, lane_alive)
-                  : chunk_steps<W, S, U, K, true, false>(litreg, gbase, sub, w8, base, len, table,
-                                                        cs, alive, lane_alive);
-        if (!go) break;  // dead, or the clause ended inside this chunk
+    return uniform(n - 1);
+}
+
+// 7 blocks of 4 waves per CU need at most 96 scalar registers: the device
+// counts them in sixteens, with sixteen more per wave than the kernel's own
+// (measured: kernels of 97-106 ran 6 blocks per CU, of 81-96 seven).
+#define GSS_SWEEP_BOUNDS __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256)
+constexpr int kSweepBlocksPerCu = 7;
+
+// How a wave walks the clauses: the passes of all buckets (CPW clauses of one
+// length each) form one sequence, cut into tasks of `tp` passes that the
+// persistent waves take round-robin.  tp gives every wave kTaskRounds tasks
+// of the same number of passes, so the waves finish together whatever the
+// number of clauses (tasks of a fixed 64 clauses left 4.4 tasks per wave on 2M
+// clauses: some waves had 5), and a wave reads its literals in long runs.
+constexpr int kTaskRounds = 4;
+
+struct Passes {
+    int nbuckets, total, tp, gw, nw;
+
+    __device__ __forceinline__ explicit Passes(const SweepArgs &a) {
+        nbuckets = a.nbuckets;
+        total = a.npasses;
+        if (a.dyn) {
+            nbuckets = uniform(a.dyn[0]);
+            total = uniform(a.dyn[1]);
+        }
+        gw = uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));  // 256-thread blocks
+        nw = (int)gridDim.x * 4;
+        tp = a.task_passes;
+        if (tp <= 0) tp = (total - 1) / (nw * kTaskRounds) + 1;
     }
-    uint64_t cand[K], any = 0;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        fm[k] = ~cs.c1[k];
-        cand[k] = cs.c1[k] & ~cs.c2[k] & cs.nt[k];
-        any |= cand[k];
+};
+
+// Appends a wave's records to its hit chunks.  A wave's first chunk is the
+// one of its own number, so a sweep with few records claims nothing (one
+// device-scope atomic costs ~10 ns and they all meet on one address: claims
+// of the first chunk by ~8,000 waves took 80 us); a full chunk is replaced by
+// one claimed past those.  Chunks past the buffer take no records: alloc[1]
+// counts them, and the host re-runs the sweep with room.
+struct HitWriter {
+    gss_hit *hits;
+    uint32_t *fills;
+    uint32_t *alloc;  // [0] chunks claimed past the waves' own, [1] chunks past the buffer
+    uint32_t cap;     // chunks in the buffer
+    int waves;        // first claimable chunk
+    int chunk;
+    int fill = 0;
+
+    __device__ __forceinline__ HitWriter(const SweepArgs &a, const Passes &ps)
+        : hits(a.hits), fills(a.fills), alloc(a.alloc), cap(a.chunk_cap), waves(ps.nw),
+          chunk(ps.gw) {}
+
+    // Room for n more records (n <= 64): true if they may be written.
+    __device__ __forceinline__ bool room(int n, int lane) {
+        if (fill + n > kHitChunk) {
+            if (lane == 0 && (uint32_t)chunk < cap) fills[chunk] = (uint32_t)fill;
+            uint32_t c = 0;
+            if (lane == 0) c = atomicAdd(alloc, 1u);
+            chunk = waves + uniform((int)__shfl(c, 0));
+            fill = 0;
+        }
+        if ((uint32_t)chunk < cap) return true;
+        if (fill == 0 && lane == 0) atomicAdd(alloc + 1, 1u);
+        return false;
     }
-    if (!fused && group_any<G>(any != 0, gmask)) {
-        auto lane_open = [&](const ClauseState<K> &c) {
-            uint64_t x = 0;
-#pragma unroll
-            for (int k = 0; k < K; k++) x |= cand[k] & c.nt[k];
-            return x != 0;
+
+    __device__ __forceinline__ void end(int lane) {
+        if (lane == 0 && (uint32_t)chunk < cap) fills[chunk] = (uint32_t)fill;
+    }
+
+    // One record per lane with a report: a gss_hit (rec_words 3) or its first
+    // word.  Records are streamed out and never read by the sweep:
+    // non-temporal stores keep them from displacing table rows in L2 and the
+    // memory-side cache.
+    __device__ __forceinline__ void words(bool hit, uint32_t row, int len, int word, uint64_t fm,
+                                          uint64_t um, int rec_words, int lane) {
+        const unsigned long long bal = __ballot(hit);
+        if (!bal) return;
+        const int n = __popcll(bal);
+        if (room(n, lane) && hit) {
+            const size_t r = (size_t)chunk * kHitChunk + fill + prefix_count(bal);
+            uint64_t *dst = (uint64_t *)hits + r * (size_t)rec_words;
+            __builtin_nontemporal_store(
+                (uint64_t)row | ((uint64_t)len << 32) | ((uint64_t)word << 48), dst);
+            if (rec_words == 3) {
+                __builtin_nontemporal_store(fm, dst + 1);
+                __builtin_nontemporal_store(um, dst + 2);
+            }
+        }
+        fill += n;
+    }
+
+    // One gss_hit_clause per lane with hit set: its clause and the words with
+    // a report.
+    __device__ __forceinline__ void clause(bool hit, uint32_t row, int len, uint64_t wm,
+                                           int lane) {
+        const unsigned long long bal = __ballot(hit);
+        if (!bal) return;
+        const int n = __popcll(bal);
+        if (room(n, lane) && hit) {
+            const size_t r = (size_t)chunk * kHitChunk + fill + prefix_count(bal);
+            uint64_t *dst = (uint64_t *)hits + r * 2;
+            __builtin_nontemporal_store((uint64_t)row | ((uint64_t)len << 32), dst);
+            __builtin_nontemporal_store(wm, dst + 1);
+        }
+        fill += n;
+    }
+};
+
+// Passes [first, first + n) of one bucket.
+struct Run {
+    LitPtr lits;  // of the bucket
+    int len, count, first, n;
+};
+
+// Calls run(Run) for every run of passes that belongs to this wave.
+template <int CPW, typename F>
+__device__ __forceinline__ void walk(const SweepArgs &a, const Passes &ps, int lane, F &&run) {
+    for (int64_t t = ps.gw;; t += ps.nw) {
+        const int64_t first = t * ps.tp;
+        if (first >= ps.total) break;
+        int p = (int)first;
+        const int end = ps.total - p < ps.tp ? ps.total : p + ps.tp;
+        int bi = find_bucket(a.buckets, ps.nbuckets, p, lane);
+        while (p < end) {
+            const BucketDesc d = a.buckets[bi];
+            Run r;
+            r.lits = (LitPtr)uniform64((uint64_t)d.lits);
+            r.len = uniform((int)d.len);
+            r.count = uniform((int)d.count);
+            r.first = p - uniform((int)d.pass_begin);
+            const int have = (r.count - 1) / CPW + 1 - r.first;
+            r.n = end - p < have ? end - p : have;
+            const int n = r.n;
+            run(r);
+            p += n;
+            bi++;
+        }
+    }
+}
+
+// Every clause checked.  W lanes check one clause, one table word per lane,
+// 64 / W clauses per wave pass; a lane stops reading rows once its 64 slots
+// are dead (the line of a row is fetched while any of its lanes is alive) and
+// the pass ends when every lane is.
+//
+// The rows are the traffic (a line per row and 16 words), so the schedule
+// reads few of them: the first two prefetched during the pass before, then two
+// per step up to the sixth, then one (random 1024-slot clauses of 8 literals
+// and more die after the sixth to eighth: 642 us with pairs throughout, 618 so);
+// and, only for lanes left with a slot of exactly one non-false literal, the
+// negated row of that literal alone (the first kKeep literals' rows are kept in
+// registers for it; past those every negated row is read).  A per-step choice
+// by the number of live lanes read as few rows but spilled: 845 us.
+template <int W, bool CLAUSES>
+__global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
+    using L = Lits<W>;
+    constexpr int CPW = 64 / W;  // clauses per wave pass
+    constexpr int H = L::kHeld;
+    constexpr int kKeep = H < 8 ? H : 8;
+    const int lane = (int)__lane_id();
+    const int c = lane / W;           // clause of the pass
+    const int w = lane % W;           // table word
+    const int q = lane % L::G;        // literal of the group's registers
+    const uint32_t w8 = (uint32_t)w * 8u;
+    const uint64_t valid = a.valid[w];
+    const uint64_t *__restrict__ table = a.table;
+    const Passes ps(a);
+    HitWriter out(a, ps);
+
+    walk<CPW>(a, ps, lane, [&](const Run &run) {
+        const int len = run.len, n = run.n;
+        const int row0 = run.first * CPW;   // of the run's first pass
+        const int left = run.count - row0;  // rows from there on
+        const LitPtr cl = run.lits + (size_t)row0 * len;
+        auto clause = [&](int pass) {
+            return cl + (size_t)(uint32_t)(pass * CPW + c) * (uint32_t)len;
         };
-        auto open = [&](const ClauseState<K> &c) { return group_any<G>(lane_open(c), gmask); };
-        litreg = first_chunk;
-        for (int base = 0; base < len; base += G) {
-            if (base) litreg = base + q < len ? cl[base + q] : sentinel;
-            if (!chunk_steps<W, S, U, K, false, true>(litreg, gbase, sub, w8, base, len, table,
-                                                      cs, open, lane_open))
-                break;
+        auto lits_of = [&](int pass) {
+            return load_lits<W>(clause(pass), 0, len, q, pass < n && pass * CPW + c < left,
+                                a.sentinel);
+        };
+        auto row = [&]<int J>(const Lits<W> &l) {
+            return load_word(table, scale_offset<W>(lit_at<W, J>(l)) | w8);
+        };
+        // One pass: its held literals and first two rows.
+        auto check = [&](int pass, const Lits<W> &cur, uint64_t x0, uint64_t x1) {
+            const int r = pass * CPW + c;
+            const bool on = r < left;
+            // invalid slots (and lanes without a clause) start dead
+            uint64_t c2 = on ? ~valid : ~0ull, c1 = c2;
+            uint64_t f[kKeep];
+            f[0] = x0;
+            f[1] = x1;
+            auto fold = [&](uint64_t x) {
+                c2 |= c1 & x;
+                c1 |= x;
+            };
+            fold(x0);
+            fold(x1);
+            // two rows from position J of the literals l; rows kept when J is
+            // among the first kKeep of the clause
+            auto step = [&]<int J, bool KEEP>(const Lits<W> &l) {
+                const uint32_t o0 = scale_offset<W>(lit_at<W, J>(l)) | w8;
+                const uint32_t o1 = scale_offset<W>(lit_at<W, J + 1>(l)) | w8;
+                if (c2 != ~0ull) {
+                    const uint64_t y0 = load_word(table, o0), y1 = load_word(table, o1);
+                    if constexpr (KEEP) {
+                        f[J % kKeep] = y0;
+                        f[(J + 1) % kKeep] = y1;
+                    }
+                    fold(y0);
+                    fold(y1);
+                }
+                return __ballot(c2 != ~0ull) != 0;
+            };
+            auto step1 = [&]<int J, bool KEEP>(const Lits<W> &l) {
+                const uint32_t o0 = scale_offset<W>(lit_at<W, J>(l)) | w8;
+                if (c2 != ~0ull) {
+                    const uint64_t y0 = load_word(table, o0);
+                    if constexpr (KEEP) f[J % kKeep] = y0;
+                    fold(y0);
+                }
+                return __ballot(c2 != ~0ull) != 0;
+            };
+            bool go = len > 2 && __ballot(c2 != ~0ull) != 0;
+            constexpr int P2 = H / 2 - 1 < 2 ? H / 2 - 1 : 2;
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ((go = go && 2 * I + 2 < len &&
+                       step.template operator()<2 * I + 2, (2 * I + 2 < kKeep)>(cur)),
+                 ...);
+            }(std::make_integer_sequence<int, P2>{});
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ((go = go && 2 + 2 * P2 + I < len &&
+                       step1.template operator()<2 + 2 * P2 + I, (2 + 2 * P2 + I < kKeep)>(cur)),
+                 ...);
+            }(std::make_integer_sequence<int, H - 2 - 2 * P2>{});
+            if (go && len > H) {
+                for (int base = H; base < len && go; base += H) {
+                    const Lits<W> l = load_lits<W>(clause(pass), base, len, q, on, a.sentinel);
+                    [&]<int... I>(std::integer_sequence<int, I...>) {
+                        ((go = go && base + 2 * I < len &&
+                               step.template operator()<2 * I, false>(l)),
+                         ...);
+                    }(std::make_integer_sequence<int, H / 2>{});
+                }
+            }
+            const uint64_t fm = ~c1;
+            uint64_t um = c1 & ~c2;  // exactly one non-false literal
+            if (__ballot(um != 0)) {
+                // a slot's one non-false literal must not be true there
+                auto neg_row = [&]<int J>(const Lits<W> &l, bool need) {
+                    const uint32_t o = (scale_offset<W>(lit_at<W, J>(l)) ^ neg_bit<W>()) | w8;
+                    return need ? load_word(table, o) : ~0ull;
+                };
+                [&]<int... I>(std::integer_sequence<int, I...>) {
+                    uint64_t rest = um, t[kKeep];
+                    ((t[I] = I < len ? neg_row.template operator()<I>(cur, (f[I] & um) != 0)
+                                     : ~0ull),
+                     ...);
+                    ((rest &= I < len ? ~f[I] : ~0ull), ...);
+                    ((um &= t[I]), ...);
+                    // positions past the kept rows, for the slots left over
+                    for (int base = kKeep; base < len && __ballot((rest & um) != 0);
+                         base += kKeep) {
+                        const Lits<W> l = load_lits<W>(clause(pass), base, len, q, on, a.sentinel);
+                        const bool need = (rest & um) != 0;
+                        ((t[I] = base + I < len ? neg_row.template operator()<I>(l, need) : ~0ull),
+                         ...);
+                        ((um &= ~rest | t[I]), ...);
+                    }
+                }(std::make_integer_sequence<int, kKeep>{});
+            }
+            const bool hit = (fm | um) != 0;
+            if constexpr (CLAUSES) {
+                const unsigned long long bw = __ballot(hit);
+                if (bw) {
+                    const uint64_t wm =
+                        W == 64 ? bw : (bw >> (c * W)) & ((1ull << (W & 63)) - 1ull);
+                    out.clause(w == 0 && wm != 0, (uint32_t)(row0 + r), len, wm, lane);
+                }
+            } else {
+                out.words(hit, (uint32_t)(row0 + r), len, w, fm, um, a.rec_words, lane);
+            }
+        };
+        // Two passes per turn: the rows of one are in flight while the other
+        // is checked, and the literals of the next two (separate registers: a
+        // rotation would wait for what it copies).
+        Lits<W> la = lits_of(0), lb = lits_of(1);
+        uint64_t a0 = row.template operator()<0>(la), a1 = row.template operator()<1>(la);
+        for (int pass = 0; pass < n; pass += 2) {
+            const uint64_t b0 = row.template operator()<0>(lb), b1 = row.template operator()<1>(lb);
+            const Lits<W> na = lits_of(pass + 2), nb = lits_of(pass + 3);
+            check(pass, la, a0, a1);
+            a0 = row.template operator()<0>(na);
+            a1 = row.template operator()<1>(na);
+            if (pass + 1 < n) check(pass + 1, lb, b0, b1);
+            la = na;
+            lb = nb;
         }
-    }
-#pragma unroll
-    for (int k = 0; k < K; k++) um[k] = cand[k] & cs.nt[k];
+    });
+    out.end(lane);
 }
 
-// Serving steps, one clause per lane: the request groups in which fewer
-// than two literal occurrences of the clause (its row of len stored
-// offsets) are non-false in every valid slot (SweepArgs::agg), i.e. the only
-// groups where it can report; 0 once none is left.  `vote` literals and then
-// their entries are read together per vote (1, 2, 4 or 8), so a wave keeps
-// up to 64 * vote loads in flight.
-__device__ __forceinline__ uint32_t lane_agg(const uint32_t *__restrict__ row, int len,
-                                             const uint8_t *__restrict__ agg, int vote,
-                                             uint32_t gdead) {
-    constexpr int kMaxVote = 8;
+// ---- screened sweeps -----------------------------------------------------------
+
+// One clause per lane: the groups in which fewer than two literal occurrences
+// of the clause (its row of len stored offsets) are non-false in every valid
+// slot (SweepArgs::agg), i.e. the only groups where it can report; 0 once none
+// is left.  Two literals and then their entries are read per vote.
+__device__ __forceinline__ uint32_t lane_agg(LitPtr row, int len,
+                                             const uint8_t *__restrict__ agg, uint32_t gdead) {
     uint32_t a1 = 0, a2 = gdead;  // groups with >= 1 / >= 2 such occurrences (empty: dead)
-    for (int j = 0; j < len; j += vote) {
-        uint32_t l[kMaxVote], x[kMaxVote];
-#pragma unroll
-        for (int u = 0; u < kMaxVote; u++) l[u] = (u < vote && j + u < len) ? row[j + u] : 0u;
-#pragma unroll
-        for (int u = 0; u < kMaxVote; u++) x[u] = (u < vote && j + u < len) ? agg[l[u] >> 7] : 0u;
-#pragma unroll
-        for (int u = 0; u < kMaxVote; u++) {
-            a2 |= a1 & x[u];
-            a1 |= x[u];
-        }
+    for (int j = 0; j < len; j += 2) {
+        const uint32_t l0 = row[j], l1 = j + 1 < len ? row[j + 1] : 0u;
+        const uint32_t x0 = agg[l0 >> 7], x1 = j + 1 < len ? agg[l1 >> 7] : 0u;
+        a2 |= a1 & x0;
+        a1 |= x0;
+        a2 |= a1 & x1;
+        a1 |= x1;
         if ((a2 & 0xFFu) == 0xFFu) return 0;
     }
     return ~a2 & 0xFFu;
 }
 
-__device__ __forceinline__ int find_bucket(const BucketDesc *__restrict__ b, int nb, int task) {
-    int lo = 0, hi = nb;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if ((int)b[mid].task_begin <= task) lo = mid;
-        else hi = mid;
+// Position of set bit number r (r < popcount(m)) of m.
+__device__ __forceinline__ int nth_bit(uint64_t m, int r) {
+    int pos = 0;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        const int k = __popcll(m & ((1ull << s) - 1ull));
+        if (r >= k) {
+            r -= k;
+            m >>= s;
+            pos += s;
+        }
     }
-    return lo;
+    return pos;
 }
 
-// MODE: 0 = every clause checked, records per (clause, word) (full or id
-// form, a.rec_words); 1 = clauses screened against a.agg first (serving and
-// screened steps), same record forms; 2 = every clause checked, one record
-// per clause with its words (a.rec_words = 2); 3 = screened, one record per
-// clause (screened steps).
-template <int W, int S, int U, bool FUSE, int MODE>
-__global__ __launch_bounds__(256) void k_sweep(SweepArgs a) {
-    constexpr bool AGG = MODE == 1 || MODE == 3;
-    constexpr bool CLAUSE_RECORDS = MODE == 2 || MODE == 3;
-    constexpr int K = W > 16 ? W / 16 : 1;  // table words per lane
-    constexpr int LW = W / K;               // lanes across one row
-    constexpr int G = LW * S;
-    constexpr int CPW = 64 / G;  // clauses per wave pass
-    const int lane = (int)__lane_id();
-    const int g = lane / G;
-    const int q = lane % G;
-    const int sub = q / LW;
-    const int lw = lane % LW;
-    const int gbase = g * G;
-    const uint64_t gmask = G == 64 ? ~0ull : (((1ull << G) - 1ull) << gbase);
-    const uint32_t w8 = (uint32_t)(lw * K) * 8u;
-    uint64_t valid[K];
+// One (clause, word) per lane: the clause's len stored offsets at cl, table
+// word w8 / 8, the slots not in dead.  All 64 lanes call it (len is uniform).
+// Same schedule as k_sweep, with every lane's literals its own.
+template <int W>
+__device__ __forceinline__ void check_word(LitPtr cl, int len,
+                                           const uint64_t *__restrict__ table, uint32_t w8,
+                                           uint64_t dead, uint64_t &fm, uint64_t &um) {
+    constexpr int kKeep = 4;
+    uint64_t c1 = dead, c2 = dead, f[kKeep] = {};
+    bool alive = dead != ~0ull;
+    uint32_t l0 = alive ? cl[0] : 0u, l1 = alive && len > 1 ? cl[1] : 0u;
+    auto step = [&](int j, uint64_t &x0, uint64_t &x1) {
+        if (alive) {
+            x0 = load_word(table, scale_offset<W>(l0) | w8);
+            x1 = j + 1 < len ? load_word(table, scale_offset<W>(l1) | w8) : 0ull;
+            if (j + 2 < len) l0 = cl[j + 2];
+            if (j + 3 < len) l1 = cl[j + 3];
+            c2 |= c1 & x0;
+            c1 |= x0;
+            c2 |= c1 & x1;
+            c1 |= x1;
+            alive = c2 != ~0ull;
+        }
+    };
+    step(0, f[0], f[1]);
+    if (len > 2 && __ballot(alive)) {
+        step(2, f[2], f[3]);
+        for (int j = kKeep; j < len && __ballot(alive); j += 2) {
+            uint64_t x0, x1;
+            step(j, x0, x1);
+        }
+    }
+    fm = ~c1;
+    um = c1 & ~c2;
+    if (__ballot(um != 0)) {
+        uint64_t rest = um, t[kKeep];
 #pragma unroll
-    for (int k = 0; k < K; k++) valid[k] = a.valid[lw * K + k];
-    uint32_t gdead = 0xFFu;  // serving steps: request groups without a word
-    if constexpr (AGG)
-        for (int b = 0; b < 8; b++)
-            if (a.agg_words[b]) gdead &= ~(1u << b);
-    // wave id and count are wave-uniform: keep the task walk scalar
-    const int gw = uniform((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    const int nw = (int)((gridDim.x * blockDim.x) >> 6);
+        for (int i = 0; i < kKeep; i++) {
+            t[i] = ~0ull;
+            if (i < len && (f[i] & um) != 0)
+                t[i] = load_word(table, (scale_offset<W>(cl[i]) ^ neg_bit<W>()) | w8);
+            rest &= ~f[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kKeep; i++) um &= t[i];
+        for (int j = kKeep; j < len && __ballot((rest & um) != 0); j += 2) {
+            if ((rest & um) != 0) {
+                um &= ~rest | load_word(table, (scale_offset<W>(cl[j]) ^ neg_bit<W>()) | w8);
+                if (j + 1 < len)
+                    um &= ~rest | load_word(table, (scale_offset<W>(cl[j + 1]) ^ neg_bit<W>()) | w8);
+            }
+        }
+    }
+}
 
-    int nbuckets = a.nbuckets, ntasks = a.ntasks;
-    if (a.dyn) {
-        nbuckets = uniform(a.dyn[0]);
-        ntasks = uniform(a.dyn[1]);
-    }
-    int chunk = -1;
-    int fill = 0;
-    // Appends this pass's records (all lanes call it; `active` marks the
-    // groups that checked a clause).
-    auto claim = [&](unsigned long long bal) {
-        const int n = __popcll(bal);
-        if (chunk < 0 || fill + n > kHitChunk) {
-            if (chunk >= 0 && lane == 0 && (uint32_t)chunk < a.chunk_cap)
-                a.fills[chunk] = (uint32_t)fill;
-            uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(a.alloc, 1u);
-            chunk = uniform((int)__shfl(c, 0));
-            fill = 0;
-        }
-    };
-    auto emit = [&](bool active, int64_t row, int len, const uint64_t (&fm)[K],
-                    const uint64_t (&um)[K]) {
-        if constexpr (CLAUSE_RECORDS) {
-            // one record per clause: the words with a report of the group
-            uint64_t wm = 0;
-            if constexpr (K == 1) {
-                // word lw is lane gbase + lw (sub-lane 0): one ballot
-                const unsigned long long bw =
-                    __ballot(active && sub == 0 && (fm[0] | um[0]) != 0);
-                wm = (bw >> gbase) & (LW == 64 ? ~0ull : ((1ull << LW) - 1ull));
-            } else {
-                // each lane holds K consecutive words: OR over the group's lanes
+// Clauses screened against a.agg first (serving and screened steps).  A wave
+// screens 64 clauses, one per lane; the (clause, word) pairs that are left
+// are then spread one per lane over the wave, whatever clause they belong to,
+// and checked exactly.  Giving each surviving clause a group of 16 lanes (as
+// many words each as it takes) kept most lanes idle: a clause survives in one
+// or two of its eight word groups.
+template <int W, bool CLAUSES>
+__global__ GSS_SWEEP_BOUNDS void k_sweep_screened(SweepArgs a) {
+    __shared__ uint64_t s_valid[W], s_words[4][64], s_hit[4][64];
+    __shared__ uint32_t s_start[4][64];
+    const int lane = (int)__lane_id(), wv = (int)(threadIdx.x >> 6);
+    if (threadIdx.x < W) s_valid[threadIdx.x] = a.valid[threadIdx.x];
+    __syncthreads();
+    uint32_t gdead = 0;  // groups without a word
+    for (int b = 0; b < 8; b++)
+        if (!a.agg_words[b]) gdead |= 1u << b;
+    const Passes ps(a);
+    HitWriter out(a, ps);
+
+    walk<64>(a, ps, lane, [&](const Run &run) {
+        const int len = run.len, count = run.count;
+        for (int pass = 0; pass < run.n; pass++) {
+            const int row0 = (run.first + pass) * 64;
+            const LitPtr cl = run.lits + (size_t)row0 * len;
+            const uint32_t grp =
+                row0 + lane < count
+                    ? lane_agg(cl + (size_t)lane * len, len, a.agg, gdead)
+                    : 0u;
+            if (!__ballot(grp != 0)) continue;
+            uint64_t m = 0;  // table words to check
 #pragma unroll
-                for (int k = 0; k < K; k++)
-                    if (active && (fm[k] | um[k]) != 0) wm |= 1ull << (lw * K + k);
+            for (int b = 0; b < 8; b++)
+                if ((grp >> b) & 1u) m |= a.agg_words[b];
+            const int cnt = __popcll(m);
+            int incl = cnt;
 #pragma unroll
-                for (int d = 1; d < G; d <<= 1) wm |= __shfl_xor(wm, d);
+            for (int d = 1; d < 64; d <<= 1) {
+                const int y = __shfl_up(incl, d);
+                if (lane >= d) incl += y;
             }
-            const bool hit = active && q == 0 && wm != 0;
-            const unsigned long long bal = __ballot(hit);
-            if (bal) {
-                claim(bal);
-                if (hit && (uint32_t)chunk < a.chunk_cap) {
-                    const size_t r = (size_t)chunk * kHitChunk + fill + prefix_count(bal);
-                    uint64_t *dst = (uint64_t *)a.hits + r * 2;
-                    __builtin_nontemporal_store((uint64_t)(uint32_t)row | ((uint64_t)len << 32),
-                                                dst);
-                    __builtin_nontemporal_store(wm, dst + 1);
-                }
-                fill += __popcll(bal);
-            }
-        } else {
+            const int total = uniform(__shfl(incl, 63));
+            s_start[wv][lane] = (uint32_t)(incl - cnt);
+            s_words[wv][lane] = m;
+            if constexpr (CLAUSES) s_hit[wv][lane] = 0;
+            __builtin_amdgcn_wave_barrier();
+            for (int base = 0; base < total; base += 64) {
+                const int item = base + lane;
+                const bool on = item < total;
+                // the clause it belongs to: the last one that starts at or before it
+                int i = 0;
 #pragma unroll
-            for (int k = 0; k < K; k++) {
-                const bool hit = active && sub == 0 && (fm[k] | um[k]) != 0;
-                const unsigned long long bal = __ballot(hit);
-                if (bal) {
-                    const int n = __popcll(bal);
-                    claim(bal);
-                    if (hit && (uint32_t)chunk < a.chunk_cap) {
-                        // Records are streamed out and never read by the
-                        // kernel: non-temporal stores keep them from
-                        // displacing table rows in L2 and the memory-side
-                        // cache.
-                        const uint64_t id = (uint64_t)(uint32_t)row | ((uint64_t)len << 32) |
-                                            ((uint64_t)(lw * K + k) << 48);
-                        const size_t r = (size_t)chunk * kHitChunk + fill + prefix_count(bal);
-                        uint64_t *dst = (uint64_t *)a.hits + r * (size_t)a.rec_words;
-                        __builtin_nontemporal_store(id, dst);
-                        if (a.rec_words == 3) {
-                            __builtin_nontemporal_store(fm[k], dst + 1);
-                            __builtin_nontemporal_store(um[k], dst + 2);
-                        }
-                    }
-                    fill += n;
+                for (int s = 32; s > 0; s >>= 1)
+                    if (i + s < 64 && (int)s_start[wv][i + s] <= item) i += s;
+                const int w = on ? nth_bit(s_words[wv][i], item - (int)s_start[wv][i]) : 0;
+                uint64_t fm, um;
+                check_word<W>(cl + (size_t)i * len, len, a.table, (uint32_t)w * 8u,
+                              on ? ~s_valid[w] : ~0ull, fm, um);
+                const bool hit = (fm | um) != 0;
+                if constexpr (CLAUSES) {
+                    if (hit) atomicOr((unsigned long long *)&s_hit[wv][i], 1ull << w);
+                } else {
+                    out.words(hit, (uint32_t)(row0 + i), len, w, fm, um, a.rec_words, lane);
                 }
             }
-        }
-    };
-    for (int task = gw; task < ntasks; task += nw) {
-        const int bi = uniform(find_bucket(a.buckets, nbuckets, task));
-        const BucketDesc bd = a.buckets[bi];
-        const int len = uniform((int)bd.len);
-        const int64_t row0 = (int64_t)(task - uniform((int)bd.task_begin)) * a.task_clauses;
-        const int64_t rem = (int64_t)uniform((int)bd.count) - row0;
-        const int nrows = rem < a.task_clauses ? (int)rem : a.task_clauses;
-        const uint32_t *rows_base = bd.lits + (size_t)row0 * len;
-        if constexpr (AGG) {
-            // Serving steps: each lane screens one clause against the
-            // aggregate entries; the groups then check the survivors exactly,
-            // CPW at a time, on the words of their surviving request groups.
-            for (int it = 0; it < nrows; it += 64) {
-                const int c = it + lane;
-                const uint32_t grp =
-                    c < nrows ? lane_agg(rows_base + (size_t)c * len, len, a.agg, a.agg_vote, gdead)
-                              : 0u;
-                unsigned long long left = __ballot(grp != 0);
-                while (left) {
-                    unsigned long long m = left;
-                    for (int k = 0; k < g && m; k++) m &= m - 1;  // group g: the g-th survivor
-                    const int src = m ? (int)__builtin_ctzll(m) : 0;
-                    const bool active = m != 0;
-                    for (int k = 0; k < CPW && left; k++) left &= left - 1;
-                    const uint32_t gr = (uint32_t)__shfl((int)grp, src);  // the survivor's lane
-                    const int64_t row = row0 + it + src;
-                    uint64_t fm[K], um[K];
-#pragma unroll
-                    for (int k = 0; k < K; k++) fm[k] = um[k] = 0;
-                    if (active) {
-                        uint64_t alive = 0;
-                        for (int b = 0; b < 8; b++)
-                            if ((gr >> b) & 1u) alive |= a.agg_words[b];
-                        uint64_t vk[K];
-#pragma unroll
-                        for (int k = 0; k < K; k++)
-                            vk[k] = ((alive >> (lw * K + k)) & 1ull) ? valid[k] : 0ull;
-                        const uint32_t *cl = bd.lits + (size_t)row * len;
-                        const uint32_t chunk0 = q < len ? cl[q] : a.sentinel;
-                        check_clause<W, S, U, K, FUSE>(cl, len, chunk0, a.sentinel, a.table, q,
-                                                       gmask, gbase, w8, sub, vk, a.fuse_len, fm,
-                                                       um);
-                    }
-                    emit(active, row, len, fm, um);
-                }
+            __builtin_amdgcn_wave_barrier();
+            if constexpr (CLAUSES) {
+                const uint64_t wm = s_hit[wv][lane];
+                out.clause(wm != 0, (uint32_t)(row0 + lane), len, wm, lane);
             }
-        } else {
-            // literal q of the group's first clause chunk, prefetched one pass ahead
-            uint32_t next_chunk =
-                (g < nrows && q < len) ? rows_base[(size_t)g * len + q] : a.sentinel;
-            for (int it = 0; it < nrows; it += CPW) {
-                const bool active = it + g < nrows;
-                const int64_t row = row0 + it + g;
-                const uint32_t chunk0 = next_chunk;
-                const int nxt = it + CPW + g;
-                next_chunk =
-                    (nxt < nrows && q < len) ? rows_base[(size_t)nxt * len + q] : a.sentinel;
-                uint64_t fm[K], um[K];
-#pragma unroll
-                for (int k = 0; k < K; k++) fm[k] = um[k] = 0;
-                if (active)
-                    check_clause<W, S, U, K, FUSE>(bd.lits + (size_t)row * len, len, chunk0,
-                                                   a.sentinel, a.table, q, gmask, gbase, w8, sub,
-                                                   valid, a.fuse_len, fm, um);
-                emit(active, row, len, fm, um);
-            }
+            __builtin_amdgcn_wave_barrier();
         }
-    }
-    if (chunk >= 0 && lane == 0 && (uint32_t)chunk < a.chunk_cap) a.fills[chunk] = (uint32_t)fill;
+    });
+    out.end(lane);
 }
 
 __global__ void k_reset_u32(uint32_t *p, int n) {
@@ -604,11 +694,32 @@ __global__ void k_assig_roll(const gss_var_update *__restrict__ ups, int64_t n,
     table[base + words] = ((t >> p) & 1ull) ? ~0ull : 0ull;
 }
 
+// Screening entries of a variable where a word is its own group (at most 8
+// words): bit `word` of both literals' bytes, from the variable's rows f and t.
+__device__ __forceinline__ void agg_word_bits(uint32_t *agg32, uint32_t var, uint32_t word,
+                                              uint64_t f, uint64_t t) {
+    const uint32_t sh = (var & 1u) * 16u + word;  // entries 2 var, 2 var + 1 of word var / 2
+    const uint32_t bf = 1u << sh, bt = 1u << (sh + 8u);
+    const uint32_t set = (f == ~0ull ? bf : 0u) | (t == ~0ull ? bt : 0u);
+    const uint32_t clr = (bf | bt) & ~set;
+    if (set) atomicOr(agg32 + (var >> 1), set);
+    if (clr) atomicAnd(agg32 + (var >> 1), ~clr);
+}
+
 // ---- batched steps: fixed launch shapes, counts from device memory --------
 
-// Copies a step's staged inputs from pinned host memory to the device.  The
-// region sizes are read once per block from the pinned header.
-__global__ void k_stage_in(StageArgs a) {
+// A step's inputs from pinned host memory: the header and the regions a later
+// kernel reads are copied, the counters of its sweep cleared, and -- straight
+// from the staging, each byte crossing PCIe once -- its clauses copied to
+// their rows (a.clauses) and its updates applied (a.apply).  Staging first and
+// applying in kernels after it took 3 launches more, 3-5 us each on a step of
+// few updates.
+//
+// Updates go through LDS, 256 at a time, so that the 24-byte records are read
+// in whole lines.
+__global__ __launch_bounds__(256) void k_step_in(StepInArgs a) {
+    if (blockIdx.x == 0 && threadIdx.x < 2) a.alloc[threadIdx.x] = 0;
+    if (a.counts && blockIdx.x == 1 && threadIdx.x < 2 * GSS_MAX_WORDS) a.counts[threadIdx.x] = 0;
     if (*a.halt) {
         // halted: a header with no work (and `halted` set) instead of the step
         if (blockIdx.x == 0) {
@@ -619,17 +730,65 @@ __global__ void k_stage_in(StageArgs a) {
         }
         return;
     }
-    __shared__ int64_t n[kStageRegions];
-    if (threadIdx.x < kStageRegions)
-        n[threadIdx.x] = ((const StepHeader *)a.h[kRegHeader])->region_words[threadIdx.x];
+    __shared__ int64_t s_n[kStageRegions];
+    __shared__ int64_t s_nups;
+    __shared__ int32_t s_ncls;
+    __shared__ uint64_t s_up[3 * 256];
+    const StepHeader *h = (const StepHeader *)a.h[kRegHeader];
+    if (threadIdx.x < kStageRegions) s_n[threadIdx.x] = h->region_words[threadIdx.x];
+    if (threadIdx.x == 64) s_nups = h->nups;
+    if (threadIdx.x == 65) s_ncls = h->nclauses;
+    // words of each screening group with a valid slot
+    if (a.agg_words && blockIdx.x == 1 && threadIdx.x >= 128 && threadIdx.x < 136) {
+        const int b = (int)threadIdx.x - 128, gw = a.words < 8 ? 1 : a.words / 8;
+        uint64_t m = 0;
+        for (int w = b * gw; w < (b + 1) * gw && w < a.words; w++)
+            if (h->valid[w]) m |= 1ull << w;
+        a.agg_words[b] = m;
+    }
     __syncthreads();
     const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 #pragma unroll
     for (int r = 0; r < kStageRegions; r++) {
+        if (r == kRegUps && a.apply) continue;
+        if ((r == kRegClauses || r == kRegLits) && a.clauses) continue;
         const uint32_t *src = a.h[r];
         uint32_t *dst = a.d[r];
-        for (int64_t i = tid; i < n[r]; i += stride) dst[i] = src[i];
+        for (int64_t i = tid; i < s_n[r]; i += stride) dst[i] = src[i];
+    }
+    if (a.clauses) {  // eight lanes per clause
+        const ClauseSeg *cls = (const ClauseSeg *)a.h[kRegClauses];
+        const uint32_t *lits = a.h[kRegLits];
+        for (int64_t i = tid >> 3; i < s_ncls; i += stride >> 3) {
+            const ClauseSeg c = cls[i];
+            for (uint32_t j = threadIdx.x & 7; j < c.len; j += 8)
+                c.dst[j] = lits[(uint64_t)c.src + j] << a.shift;
+        }
+    }
+    if (a.apply) {
+        const uint64_t *src = (const uint64_t *)a.h[kRegUps];
+        uint64_t *dst = (uint64_t *)a.d[kRegUps];
+        for (int64_t t = (int64_t)blockIdx.x * 256; t < s_nups; t += (int64_t)gridDim.x * 256) {
+            const int n = s_nups - t < 256 ? (int)(s_nups - t) : 256;
+            for (int i = (int)threadIdx.x; i < 3 * n; i += 256) {
+                const uint64_t x = src[3 * t + i];
+                s_up[i] = x;
+                dst[3 * t + i] = x;
+            }
+            __syncthreads();
+            if ((int)threadIdx.x < n) {
+                const uint64_t vw = s_up[3 * threadIdx.x];  // {var, word}
+                const uint64_t def = s_up[3 * threadIdx.x + 1], tru = s_up[3 * threadIdx.x + 2];
+                const uint32_t var = (uint32_t)vw, word = (uint32_t)(vw >> 32);
+                const size_t base = (size_t)var * 2 * a.words + word;
+                const uint64_t f = ~(def & ~tru), t1 = ~(def & tru);
+                a.table[base] = f;
+                a.table[base + a.words] = t1;
+                if (a.agg32) agg_word_bits(a.agg32, var, word, f, t1);
+            }
+            __syncthreads();
+        }
     }
 }
 
@@ -762,133 +921,180 @@ __global__ void k_assig_apply_dyn(const gss_var_update *__restrict__ ups, const 
     }
 }
 
+// One update rolled forward: every slot of its word takes the value of slot
+// last_pos[word] (none if negative).
+__device__ __forceinline__ void roll_update(const gss_var_update *__restrict__ ups, int64_t i,
+                                            uint64_t *__restrict__ table, int words,
+                                            const int8_t *__restrict__ last_pos,
+                                            uint32_t *agg32) {
+    const uint32_t var = ups[i].var, word = ups[i].word;
+    const int p = last_pos[word];
+    if (p < 0) return;
+    const size_t base = (size_t)var * 2 * words + word;
+    const uint64_t f = ((table[base] >> p) & 1ull) ? ~0ull : 0ull;
+    const uint64_t t = ((table[base + words] >> p) & 1ull) ? ~0ull : 0ull;
+    table[base] = f;
+    table[base + words] = t;
+    if (agg32) agg_word_bits(agg32, var, word, f, t);
+}
+
 __global__ void k_assig_roll_dyn(const gss_var_update *__restrict__ ups, const int64_t *n_p,
                                  uint64_t *__restrict__ table, int words,
-                                 const int8_t *__restrict__ last_pos, const uint32_t *alloc,
-                                 uint32_t cap, uint32_t *halt) {
-    if (*alloc > cap) {
-        // records were dropped: keep the table as the sweep read it, and halt
-        if (blockIdx.x == 0 && threadIdx.x == 0) *halt = 1u;
-        return;
-    }
+                                 const int8_t *__restrict__ last_pos) {
     const int64_t n = *n_p;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const gss_var_update u = ups[i];
-        const int p = last_pos[u.word];
-        if (p < 0) continue;
-        const size_t base = (size_t)u.var * 2 * words + u.word;
-        const uint64_t f = table[base], t = table[base + words];
-        table[base] = ((f >> p) & 1ull) ? ~0ull : 0ull;
-        table[base + words] = ((t >> p) & 1ull) ? ~0ull : 0ull;
+         i += (int64_t)gridDim.x * blockDim.x)
+        roll_update(ups, i, table, words, last_pos, nullptr);
+}
+
+// ---- records made dense ---------------------------------------------------------
+
+// Chunks of a sweep of `waves` waves that hold records (at most its buffer's).
+__device__ __forceinline__ uint32_t chunks_held(const ChunkArgs &c) {
+    const uint32_t used = c.waves + c.alloc[0];
+    return used < c.cap ? used : c.cap;
+}
+
+// What the host reads: out[0] = the chunks, more than the buffer's if records
+// were dropped; out[1], out[2] = low and high word of the records kept.
+__device__ __forceinline__ void write_counts(const ChunkArgs &c, uint64_t total, uint32_t *out) {
+    out[0] = c.alloc[1] ? c.waves + c.alloc[0] : chunks_held(c);
+    out[1] = (uint32_t)total;
+    out[2] = (uint32_t)(total >> 32);
+}
+
+// Sums of fills[0, at) and fills[0, n) over a block of 256 threads.
+__device__ __forceinline__ void sum_fills(const uint32_t *__restrict__ fills, uint32_t at,
+                                          uint32_t n, uint64_t &before, uint64_t &total) {
+    __shared__ uint64_t s_sum[2][4];
+    uint64_t x = 0, y = 0;
+    for (uint32_t i = threadIdx.x; i < n; i += 256u * 4) {
+        uint32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = i + 256u * u < n ? fills[i + 256u * u] : 0u;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            y += v[u];
+            if (i + 256u * u < at) x += v[u];
+        }
     }
-}
-
-// Writes the claim count and the fill of every claimed chunk to pinned host
-// memory: h_out[0] = claimed chunks, h_out[1 + c] = fill of chunk c.
-__global__ void k_stage_out(const uint32_t *alloc, const uint32_t *__restrict__ fills,
-                            uint32_t cap, uint32_t *h_out) {
-    const uint32_t used = *alloc;
-    const uint32_t n = used < cap ? used : cap;
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid == 0) h_out[0] = used;
-    for (uint32_t i = tid; i < n; i += gridDim.x * blockDim.x) h_out[1 + i] = fills[i];
-}
-
-// Exclusive prefix of the chunk fills: offs[c] = records before chunk c for
-// the chunks [0, n) a sweep claimed (n = min(*alloc, cap), read on the device
-// so a graph replay needs no host count), offs[n] = all records.  One block:
-// each thread sums a contiguous run of chunks, the 1024 sums are scanned in
-// LDS, then each thread writes its run's prefixes.
-__global__ __launch_bounds__(1024) void k_chunk_offsets(const uint32_t *alloc,
-                                                        const uint32_t *__restrict__ fills,
-                                                        uint32_t cap, uint64_t *__restrict__ offs) {
-    __shared__ uint64_t part[1024];
-    const uint32_t used = *alloc;
-    const uint32_t n = used < cap ? used : cap;
-    const uint32_t t = threadIdx.x;
-    const uint32_t per = (n + 1023u) / 1024u;
-    const uint32_t b = (uint64_t)t * per < n ? t * per : n;
-    const uint32_t e = b + per < n ? b + per : n;
-    uint64_t sum = 0;
-    for (uint32_t i = b; i < e; i++) sum += fills[i];
-    part[t] = sum;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        x += __shfl_xor(x, d);
+        y += __shfl_xor(y, d);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_sum[0][threadIdx.x >> 6] = x;
+        s_sum[1][threadIdx.x >> 6] = y;
+    }
     __syncthreads();
-    for (uint32_t d = 1; d < 1024u; d <<= 1) {
-        const uint64_t v = t >= d ? part[t - d] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    uint64_t acc = t ? part[t - 1] : 0;
-    for (uint32_t i = b; i < e; i++) {
-        offs[i] = acc;
-        acc += fills[i];
-    }
-    if (t == 1023u) offs[n] = part[1023];
+    before = s_sum[0][0] + s_sum[0][1] + s_sum[0][2] + s_sum[0][3];
+    total = s_sum[1][0] + s_sum[1][1] + s_sum[1][2] + s_sum[1][3];
 }
 
-// Copies the records of every claimed chunk to its place in a dense array
-// (three 8-byte words per record), or nothing when they would not all fit in
-// dense_cap records (the host then compacts them itself).
-__global__ __launch_bounds__(256) void k_gather_chunks(const uint32_t *alloc,
-                                                       const uint32_t *__restrict__ fills,
-                                                       uint32_t cap,
-                                                       const uint64_t *__restrict__ offs,
-                                                       const uint64_t *__restrict__ hits,
-                                                       uint64_t *__restrict__ dense,
-                                                       uint64_t dense_cap, uint32_t rec_words) {
-    const uint32_t used = *alloc;
-    const uint32_t n = used < cap ? used : cap;
-    if (offs[n] > dense_cap) return;
-    for (uint32_t c = blockIdx.x; c < n; c += gridDim.x) {
-        const uint32_t words = fills[c] * rec_words;
-        const uint64_t *src = hits + (uint64_t)c * kHitChunk * rec_words;
-        uint64_t *dst = dense + offs[c] * rec_words;
-        for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
+// Block `blk` of `blocks` (256 threads) of the dense copy: its share of the
+// chunks, one wave per chunk, each to its place in the dense array.  Every
+// block sums the fills itself (32 KB from L2 for a sweep of ~8,000 waves): an
+// offsets kernel before this one took longer, on one CU, than the sums do.
+// Records go straight to `host` when they take at most host_words there (the
+// wait then has no copy to start), else to `dense` if they fit.
+__device__ __forceinline__ void gather_block(const ChunkArgs &c, uint32_t blk, uint32_t blocks,
+                                             uint64_t *dense, uint64_t dense_cap, uint64_t *host,
+                                             uint64_t host_words, uint32_t *out) {
+    const uint32_t n = chunks_held(c);
+    const uint32_t per = (n + blocks - 1) / blocks;
+    const uint32_t c0 = blk * per < n ? blk * per : n, c1 = c0 + per < n ? c0 + per : n;
+    if (blk != 0 && c0 == c1) return;
+    uint64_t at, total;
+    sum_fills(c.fills, c0, n, at, total);
+    if (out && blk == 0 && threadIdx.x == 0) write_counts(c, total, out);
+    if (c.alloc[1]) return;  // records were dropped: the sweep runs again
+    const uint32_t rw = c.rec_words;
+    uint64_t *to = host && total * rw <= host_words ? host : total <= dense_cap ? dense : nullptr;
+    if (!to) return;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (uint32_t k = c0; k < c1; k++) {
+        const uint32_t f = c.fills[k];
+        if (f && (k & 3) == wv) {
+            const uint64_t *__restrict__ src = c.hits + (uint64_t)k * kHitChunk * rw;
+            uint64_t *__restrict__ dst = to + at * rw;
+            const uint32_t m = f * rw;
+            uint32_t i = lane;
+            for (; i + 64 * 3 < m; i += 64 * 4) {
+                uint64_t v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) v[u] = src[i + 64 * u];
+#pragma unroll
+                for (int u = 0; u < 4; u++) dst[i + 64 * u] = v[u];
+            }
+            for (; i < m; i += 64) dst[i] = src[i];
+        }
+        at += f;
     }
 }
 
-// Claim counter and record total of a sweep to pinned host memory:
-// out[0] = chunks claimed, out[1] / out[2] = low / high word of the records
-// in the chunks that fit (one block).
-__global__ __launch_bounds__(1024) void k_count_records(const uint32_t *alloc,
-                                                        const uint32_t *__restrict__ fills,
-                                                        uint32_t cap, uint32_t *out) {
-    __shared__ uint64_t part[1024];
-    const uint32_t used = *alloc;
-    const uint32_t n = used < cap ? used : cap;
+__global__ __launch_bounds__(256) void k_gather(ChunkArgs c, uint64_t *dense, uint64_t dense_cap) {
+    gather_block(c, blockIdx.x, gridDim.x, dense, dense_cap, nullptr, 0, nullptr);
+}
+
+// Counts of a plain sweep to pinned memory.  The counters are read by the
+// gather after it; the next sweep starts from `next`, cleared here.
+__global__ __launch_bounds__(1024) void k_count_records(ChunkArgs c, uint32_t *out,
+                                                        uint32_t *next) {
+    __shared__ uint64_t part[16];
+    const uint32_t n = chunks_held(c);
     uint64_t sum = 0;
-    for (uint32_t i = threadIdx.x; i < n; i += 1024u) sum += fills[i];
-    part[threadIdx.x] = sum;
-    __syncthreads();
-    for (uint32_t d = 512; d > 0; d >>= 1) {
-        if (threadIdx.x < d) part[threadIdx.x] += part[threadIdx.x + d];
-        __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += 4096u) {
+        uint32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = i + 1024u * u < n ? c.fills[i + 1024u * u] : 0u;
+        sum += (uint64_t)v[0] + v[1] + v[2] + v[3];
     }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
+    __syncthreads();
     if (threadIdx.x == 0) {
-        out[0] = used;
-        out[1] = (uint32_t)part[0];
-        out[2] = (uint32_t)(part[0] >> 32);
+        uint64_t t = 0;
+        for (int i = 0; i < 16; i++) t += part[i];
+        write_counts(c, t, out);
+        next[0] = next[1] = 0;
     }
+}
+
+// What follows a step's sweep, in one launch: the first kGatherBlocks blocks
+// make its records dense (and write its counts for the host), the others roll
+// its updates forward -- unless records were dropped: then the table stays as
+// the sweep read it and the engine halts.
+constexpr unsigned kGatherBlocks = 512, kRollBlocks = 512;
+__global__ __launch_bounds__(256) void k_step_end(ChunkArgs c, StepEndArgs a) {
+    if (blockIdx.x < kGatherBlocks) {
+        gather_block(c, blockIdx.x, kGatherBlocks, a.dense, a.dense_cap, a.dh->host_rec,
+                     a.host_words, a.out);
+        return;
+    }
+    if (c.alloc[1]) {
+        if (blockIdx.x == kGatherBlocks && threadIdx.x == 0) *a.halt = 1u;
+        return;
+    }
+    const int64_t n = a.dh->nups;
+    for (int64_t i = (blockIdx.x - kGatherBlocks) * (int64_t)256 + threadIdx.x; i < n;
+         i += (int64_t)kRollBlocks * 256)
+        roll_update(a.ups, i, a.table, a.words, a.dh->last_pos, a.agg32);
 }
 
 // ---- records grouped by assignment word (serving steps) ----------------------
 
 // Records per word over the claimed chunks (word = the top 16 bits of a
 // record's first word); counts[64] must start at zero.
-__global__ __launch_bounds__(256) void k_word_count(const uint32_t *alloc,
-                                                    const uint32_t *__restrict__ fills,
-                                                    uint32_t cap, const uint64_t *__restrict__ hits,
-                                                    uint32_t rec_words, uint32_t *counts) {
+__global__ __launch_bounds__(256) void k_word_count(ChunkArgs ch, uint32_t *counts) {
     __shared__ uint32_t h[GSS_MAX_WORDS];
     if (threadIdx.x < GSS_MAX_WORDS) h[threadIdx.x] = 0;
     __syncthreads();
-    const uint32_t used = *alloc;
-    const uint32_t n = used < cap ? used : cap;
+    const uint32_t n = chunks_held(ch), rec_words = ch.rec_words;
     for (uint32_t c = blockIdx.x; c < n; c += gridDim.x) {
-        const uint32_t f = fills[c];
-        const uint64_t *src = hits + (uint64_t)c * kHitChunk * rec_words;
+        const uint32_t f = ch.fills[c];
+        const uint64_t *src = ch.hits + (uint64_t)c * kHitChunk * rec_words;
         for (uint32_t i = threadIdx.x; i < f; i += blockDim.x)
             atomicAdd(&h[(uint32_t)(src[(uint64_t)i * rec_words] >> 48) & (GSS_MAX_WORDS - 1)], 1u);
     }
@@ -902,14 +1108,11 @@ __global__ __launch_bounds__(256) void k_word_count(const uint32_t *alloc,
 // cursor, then places them.  group[w] = first record of word w, group[64] =
 // all records, group[65] = 1 when they fitted in dense_cap (else nothing is
 // moved and the host groups the records itself).  cursor[64] starts at zero.
-__global__ __launch_bounds__(256) void k_word_scatter(const uint32_t *alloc,
-                                                      const uint32_t *__restrict__ fills,
-                                                      uint32_t cap,
-                                                      const uint64_t *__restrict__ hits,
-                                                      uint32_t rec_words,
+__global__ __launch_bounds__(256) void k_word_scatter(ChunkArgs ch,
                                                       const uint32_t *__restrict__ counts,
                                                       uint32_t *cursor, uint64_t *__restrict__ dense,
-                                                      uint64_t dense_cap, uint64_t *group) {
+                                                      uint64_t dense_cap, uint64_t *group,
+                                                      uint32_t *out, uint32_t *halt) {
     __shared__ uint64_t base[GSS_MAX_WORDS + 1];
     __shared__ uint32_t lc[GSS_MAX_WORDS], lbase[GSS_MAX_WORDS];
     if (threadIdx.x == 0) {
@@ -921,17 +1124,21 @@ __global__ __launch_bounds__(256) void k_word_scatter(const uint32_t *alloc,
         base[GSS_MAX_WORDS] = acc;
     }
     __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        write_counts(ch, base[GSS_MAX_WORDS], out);
+        if (ch.alloc[1]) *halt = 1u;  // records were dropped: the step is re-run
+    }
     const bool fits = base[GSS_MAX_WORDS] <= dense_cap;
     if (blockIdx.x == 0 && threadIdx.x <= GSS_MAX_WORDS + 1)
         group[threadIdx.x] = threadIdx.x <= GSS_MAX_WORDS ? base[threadIdx.x] : (fits ? 1ull : 0ull);
     if (!fits) return;  // the same for every thread of every block
-    const uint32_t used = *alloc;
-    const uint32_t n = used < cap ? used : cap;
+    const uint32_t n = chunks_held(ch), rec_words = ch.rec_words;
     for (uint32_t c = blockIdx.x; c < n; c += gridDim.x) {
+        const uint32_t f = ch.fills[c];
+        if (!f) continue;  // uniform in the block
         if (threadIdx.x < GSS_MAX_WORDS) lc[threadIdx.x] = 0;
         __syncthreads();
-        const uint32_t f = fills[c];
-        const uint64_t *src = hits + (uint64_t)c * kHitChunk * rec_words;
+        const uint64_t *src = ch.hits + (uint64_t)c * kHitChunk * rec_words;
         for (uint32_t i = threadIdx.x; i < f; i += blockDim.x)
             atomicAdd(&lc[(uint32_t)(src[(uint64_t)i * rec_words] >> 48) & (GSS_MAX_WORDS - 1)], 1u);
         __syncthreads();
@@ -1022,7 +1229,7 @@ __global__ __launch_bounds__(64) void k_serve_admit(ServeRing r, StepHeader *dh,
         *r.adm_count = (uint32_t)count;
         dh->nloads = (int64_t)total_words;
         dh->npatches = count > 0 ? (int64_t)total_patches : 0;
-        if (count == 0) dh->ntasks = 0;  // nothing to check
+        if (count == 0) dh->npasses = 0;  // nothing to check
         *r.tail = tail + (uint64_t)count;
         report->first = tail;
         report->count = (uint32_t)count;
@@ -1068,19 +1275,6 @@ struct TableGroups {
 };
 
 template <int W>
-__device__ __forceinline__ void table_agg_words(const StepHeader *__restrict__ dh,
-                                                uint64_t *__restrict__ agg_words) {
-    constexpr int NG = TableGroups<W>::NG, GW = TableGroups<W>::GW;
-    if (blockIdx.x == 0 && (int)threadIdx.x < 8) {
-        uint64_t m = 0;
-        if ((int)threadIdx.x < NG)
-            for (int w = (int)threadIdx.x * GW; w < ((int)threadIdx.x + 1) * GW; w++)
-                if (dh->valid[w]) m |= 1ull << w;
-        agg_words[threadIdx.x] = m;
-    }
-}
-
-template <int W>
 __device__ __forceinline__ bool group_all_ones(const uint64_t *__restrict__ row, int b) {
     constexpr int GW = TableGroups<W>::GW;
     uint64_t x = ~0ull;
@@ -1091,11 +1285,9 @@ __device__ __forceinline__ bool group_all_ones(const uint64_t *__restrict__ row,
 
 template <int W>
 __global__ void k_table_agg(const uint64_t *__restrict__ table, const StepHeader *__restrict__ dh,
-                            int64_t rows, uint8_t *__restrict__ agg,
-                            uint64_t *__restrict__ agg_words) {
+                            int64_t rows, uint8_t *__restrict__ agg) {
     constexpr int NG = TableGroups<W>::NG;
     if (dh->halted) return;  // the aggregate stays the halted step's
-    table_agg_words<W>(dh, agg_words);
     for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; l < rows;
          l += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t *row = table + (size_t)l * W;
@@ -1117,11 +1309,9 @@ __global__ void k_table_agg_update(const uint64_t *__restrict__ table,
                                    const StepHeader *__restrict__ dh,
                                    const gss_var_update *__restrict__ ups,
                                    const gss_var_patch *__restrict__ patches, int with_patches,
-                                   uint32_t *__restrict__ agg32,
-                                   uint64_t *__restrict__ agg_words) {
+                                   uint32_t *__restrict__ agg32) {
     constexpr int GW = TableGroups<W>::GW;
     if (dh->halted) return;
-    if (agg_words) table_agg_words<W>(dh, agg_words);
     const int64_t nu = dh->nups, n = nu + (with_patches ? dh->npatches : 0);
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
@@ -1269,105 +1459,58 @@ __global__ void k_compact_move(const CompactRef *__restrict__ refs, int nb, int6
     }
 }
 
-template <int W, int S, int U>
-hipError_t launch_sweep_t(const SweepArgs &a, int blocks, hipStream_t s) {
+template <int W>
+hipError_t launch_sweep_w(const SweepArgs &a, int blocks, hipStream_t s) {
     const dim3 g(blocks), b(256);
-    const bool fused = a.fuse_len > 0;
-    const int mode = (a.agg ? 1 : 0) + (a.rec_words == 2 ? 2 : 0);
-#define GSS_LAUNCH(F_, M_)                                                     \
-    if (fused == F_ && mode == M_) {                                           \
-        hipLaunchKernelGGL((k_sweep<W, S, U, F_, M_>), g, b, 0, s, a);         \
-        return hipGetLastError();                                              \
+    const bool clauses = a.rec_words == 2;
+    if (a.agg) {
+        if (clauses) hipLaunchKernelGGL((k_sweep_screened<W, true>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((k_sweep_screened<W, false>), g, b, 0, s, a);
+    } else {
+        if (clauses) hipLaunchKernelGGL((k_sweep<W, true>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((k_sweep<W, false>), g, b, 0, s, a);
     }
-    GSS_LAUNCH(true, 0)
-    GSS_LAUNCH(false, 0)
-    GSS_LAUNCH(true, 1)
-    GSS_LAUNCH(false, 1)
-    GSS_LAUNCH(true, 2)
-    GSS_LAUNCH(false, 2)
-    GSS_LAUNCH(true, 3)
-    GSS_LAUNCH(false, 3)
-#undef GSS_LAUNCH
-    return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
-template <int W, int S, int U>
-int occupancy_t(bool fused, int mode) {
+// Resident blocks per CU: as the runtime counts them, which leaves the scalar
+// registers out, at most kSweepBlocksPerCu.  A persistent grid of one block
+// per CU more than is resident runs that block's share alone at the end
+// (k_sweep at 16 words, 4M clauses: 640 -> 773 us).
+template <int W>
+int occupancy_w(int mode) {
     int nb = 0;
     hipError_t e = hipErrorInvalidValue;
-#define GSS_OCC(F_, M_)                                                                     \
-    if (fused == F_ && mode == M_)                                                          \
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sweep<W, S, U, F_, M_>, 256, 0);
-    GSS_OCC(true, 0)
-    GSS_OCC(false, 0)
-    GSS_OCC(true, 1)
-    GSS_OCC(false, 1)
-    GSS_OCC(true, 2)
-    GSS_OCC(false, 2)
-    GSS_OCC(true, 3)
-    GSS_OCC(false, 3)
-#undef GSS_OCC
-    if (e != hipSuccess) return 1;
-    return nb > 0 ? nb : 1;
+    if (mode == 0)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sweep<W, false>, 256, 0);
+    else if (mode == 1)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sweep_screened<W, false>, 256, 0);
+    else if (mode == 2)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sweep<W, true>, 256, 0);
+    else if (mode == 3)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sweep_screened<W, true>, 256, 0);
+    if (e != hipSuccess || nb < 1) return 1;
+    return nb < kSweepBlocksPerCu ? nb : kSweepBlocksPerCu;
 }
 
-// Kernel variants: (W, S, U), each with and without the fused schedule
-// (fuse_len <= 0 selects the one without), in the four modes of k_sweep.  `unroll` selects U for W >= 16
-// (0 = default).
-#define GSS_SWEEP_VARIANTS(X)                  \
-    X(1, 16, 1)                                \
-    X(2, 8, 2)                                 \
-    X(4, 4, 4)                                 \
-    X(8, 2, 4)                                 \
-    X(16, 1, 4)                                \
-    X(16, 1, 1)                                \
-    X(16, 1, 2)                                \
-    X(16, 1, 8)                                \
-    X(32, 1, 2)                                \
-    X(32, 1, 4)                                \
-    X(64, 1, 1)                                \
-    X(64, 1, 2)                                \
-    X(64, 1, 4)
-
-struct Variant {
-    int w, s, u;
-};
-
-Variant pick(int words, int unroll) {
-    switch (words) {
-        case 1: return {1, 16, 1};
-        case 2: return {2, 8, 2};
-        case 4: return {4, 4, 4};
-        case 8: return {8, 2, 4};
-        case 16:
-            if (unroll == 1 || unroll == 2 || unroll == 8) return {16, 1, unroll};
-            return {16, 1, 4};
-        case 32: return {32, 1, unroll == 2 ? 2 : 4};
-        case 64: return {64, 1, unroll == 1 || unroll == 4 ? unroll : 2};
-        default: return {0, 0, 0};
-    }
-}
+#define GSS_WORDS(X) X(1) X(2) X(4) X(8) X(16) X(32) X(64)
 
 }  // namespace
 
-// Every variant gives a clause a group of 16 lanes (W*S = 16 for W <= 16, 16
-// lanes of W/16 words each above), so a wave pass checks 4 clauses.
-int sweep_clauses_per_pass(int) { return 4; }
+int sweep_clauses_per_pass(int words, bool screened) { return screened ? 64 : 64 / words; }
 
-hipError_t launch_sweep(const SweepArgs &a, int words, int unroll, int blocks, hipStream_t s) {
-    const Variant v = pick(words, unroll);
-#define X(W_, S_, U_) \
-    if (v.w == W_ && v.s == S_ && v.u == U_) return launch_sweep_t<W_, S_, U_>(a, blocks, s);
-    GSS_SWEEP_VARIANTS(X)
+hipError_t launch_sweep(const SweepArgs &a, int words, int blocks, hipStream_t s) {
+#define X(W_) \
+    if (words == W_) return launch_sweep_w<W_>(a, blocks, s);
+    GSS_WORDS(X)
 #undef X
     return hipErrorInvalidValue;
 }
 
-int sweep_occupancy(int words, int unroll, bool fused, int mode) {
-    const Variant v = pick(words, unroll);
-#define X(W_, S_, U_) \
-    if (v.w == W_ && v.s == S_ && v.u == U_) return occupancy_t<W_, S_, U_>(fused, mode);
-    GSS_SWEEP_VARIANTS(X)
+int sweep_occupancy(int words, int mode) {
+#define X(W_) \
+    if (words == W_) return occupancy_w<W_>(mode);
+    GSS_WORDS(X)
 #undef X
     return 1;
 }
@@ -1402,8 +1545,13 @@ hipError_t launch_assig_apply(const gss_var_update *ups, int64_t n, uint64_t *ta
     return hipGetLastError();
 }
 
-hipError_t launch_stage_in(const StageArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL(k_stage_in, dim3(512), dim3(256), 0, s, a);
+hipError_t launch_step_in(const StepInArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(k_step_in, dim3(512), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_step_end(const ChunkArgs &c, const StepEndArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(k_step_end, dim3(kGatherBlocks + kRollBlocks), dim3(256), 0, s, c, a);
     return hipGetLastError();
 }
 
@@ -1450,51 +1598,32 @@ hipError_t launch_assig_apply_dyn(const gss_var_update *ups, const int64_t *n, u
 }
 
 hipError_t launch_assig_roll_dyn(const gss_var_update *ups, const int64_t *n, uint64_t *table,
-                                 int words, const int8_t *last_pos, const uint32_t *alloc,
-                                 uint32_t cap, uint32_t *halt, hipStream_t s) {
+                                 int words, const int8_t *last_pos, hipStream_t s) {
     hipLaunchKernelGGL(k_assig_roll_dyn, dim3(1024), dim3(256), 0, s, ups, n, table, words,
-                       last_pos, alloc, cap, halt);
+                       last_pos);
     return hipGetLastError();
 }
 
-hipError_t launch_stage_out(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                            uint32_t *h_out, hipStream_t s) {
-    hipLaunchKernelGGL(k_stage_out, dim3(256), dim3(256), 0, s, alloc, fills, cap, h_out);
+hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, hipStream_t s) {
+    hipLaunchKernelGGL(k_count_records, dim3(1), dim3(1024), 0, s, c, out, next);
     return hipGetLastError();
 }
 
-hipError_t launch_count_records(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                                uint32_t *h_out, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_records, dim3(1), dim3(1024), 0, s, alloc, fills, cap, h_out);
+hipError_t launch_gather(const ChunkArgs &c, void *dense, uint64_t dense_cap, hipStream_t s) {
+    if (c.rec_words < 1 || c.rec_words > 3) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_gather, dim3(2048), dim3(256), 0, s, c, (uint64_t *)dense, dense_cap);
     return hipGetLastError();
 }
 
-hipError_t launch_compact_records(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                                  uint64_t *offs, const void *hits, void *dense,
-                                  uint64_t dense_cap, int rec_words, hipStream_t s) {
-    if (rec_words < 1 || rec_words > 3) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_chunk_offsets, dim3(1), dim3(1024), 0, s, alloc, fills, cap, offs);
+hipError_t launch_group_by_word(const ChunkArgs &c, uint32_t *counts, void *dense,
+                                uint64_t dense_cap, uint64_t *group, uint32_t *out,
+                                uint32_t *halt, hipStream_t s) {
+    if (c.rec_words != 1 && c.rec_words != 3) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_word_count, dim3(1024), dim3(256), 0, s, c, counts);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_gather_chunks, dim3(2048), dim3(256), 0, s, alloc, fills, cap,
-                       (const uint64_t *)offs, (const uint64_t *)hits, (uint64_t *)dense,
-                       dense_cap, (uint32_t)rec_words);
-    return hipGetLastError();
-}
-
-hipError_t launch_group_by_word(const uint32_t *alloc, const uint32_t *fills, uint32_t cap,
-                                const void *hits, int rec_words, uint32_t *counts,
-                                void *dense, uint64_t dense_cap, uint64_t *group, hipStream_t s) {
-    if (rec_words != 1 && rec_words != 3) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_reset_u32, dim3(1), dim3(256), 0, s, counts, 2 * GSS_MAX_WORDS);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_word_count, dim3(1024), dim3(256), 0, s, alloc, fills, cap,
-                       (const uint64_t *)hits, (uint32_t)rec_words, counts);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_word_scatter, dim3(1024), dim3(256), 0, s, alloc, fills, cap,
-                       (const uint64_t *)hits, (uint32_t)rec_words, counts,
-                       counts + GSS_MAX_WORDS, (uint64_t *)dense, dense_cap, group);
+    hipLaunchKernelGGL(k_word_scatter, dim3(1024), dim3(256), 0, s, c, counts,
+                       counts + GSS_MAX_WORDS, (uint64_t *)dense, dense_cap, group, out, halt);
     return hipGetLastError();
 }
 
@@ -1505,13 +1634,13 @@ hipError_t launch_serve_admit(const ServeRing &r, StepHeader *dh, gss_word_load 
 }
 
 hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t vars, int words,
-                            uint8_t *agg, uint64_t *agg_words, hipStream_t s) {
+                            uint8_t *agg, hipStream_t s) {
     const int64_t rows = 2 * vars + 2;
     const unsigned blocks = (unsigned)std::min<int64_t>((rows + 255) / 256, 8192);
 #define GSS_TABLE_AGG(W_)                                                                   \
     if (words == W_) {                                                                      \
         hipLaunchKernelGGL(k_table_agg<W_>, dim3(blocks), dim3(256), 0, s, table, dh, rows, \
-                           agg, agg_words);                                                 \
+                           agg);                                                            \
         return hipGetLastError();                                                           \
     }
     GSS_TABLE_AGG(1)
@@ -1527,14 +1656,13 @@ hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t
 
 hipError_t launch_table_agg_update(const uint64_t *table, const StepHeader *dh,
                                    const gss_var_update *ups, const gss_var_patch *patches,
-                                   bool with_patches, int words, uint8_t *agg,
-                                   uint64_t *agg_words, hipStream_t s) {
+                                   bool with_patches, int words, uint8_t *agg, hipStream_t s) {
     uint32_t *agg32 = (uint32_t *)agg;
     const int wp = with_patches ? 1 : 0;
 #define GSS_TABLE_AGG_UP(W_)                                                                 \
     if (words == W_) {                                                                       \
         hipLaunchKernelGGL(k_table_agg_update<W_>, dim3(1024), dim3(256), 0, s, table, dh,   \
-                           ups, patches, wp, agg32, agg_words);                              \
+                           ups, patches, wp, agg32);                                         \
         return hipGetLastError();                                                            \
     }
     GSS_TABLE_AGG_UP(1)

@@ -223,13 +223,9 @@ int gss_hits_copy(gss_engine *e, gss_hit *out, int64_t cap, int64_t *n);
  * the last waited sweep densely into d_out, caller DEVICE memory of cap
  * records (record order unspecified, as gss_hits_copy), and *n = their
  * number; with d_out NULL and cap 0 only *n is set.  Calls no hipMalloc,
- * hipFree or other allocating routine: its only working memory is a static
- * per-device array of 262,145 uint64 (2 MiB, held by every device the library
- * runs on until the process ends) for the chunk offsets, so a sweep that
- * claimed more than 262,144 hit chunks of 1024 records is refused with
- * GSS_E_INVAL, as is cap below the record count.  Synchronous.  Every call on
- * one device shares that array: calls that overlap on one device (from two
- * threads or two engines) race. */
+ * hipFree or other allocating routine and needs no working memory.  A sweep
+ * that claimed more than 262,144 hit chunks of 1024 records is refused with
+ * GSS_E_INVAL, as is cap below the record count.  Synchronous. */
 int gss_hits_gather(gss_engine *e, gss_hit *d_out, int64_t cap, int64_t *n);
 /* Duration in ms of the sweep kernel of the last waited sweep, measured with
  * HIP events recorded on the engine's stream around the kernel launch. */
@@ -241,30 +237,26 @@ int gss_sweep_kernel_stats(gss_engine *e, double *total_ms, int64_t *count, int 
  * results never depend on them. */
 int gss_set_tuning(gss_engine *e, int key, int value);
 #define GSS_TUNE_WAVES_PER_CU 1   /* persistent waves per CU (0 = occupancy) */
-#define GSS_TUNE_TASK_CLAUSES 2   /* clauses per task */
+#define GSS_TUNE_TASK_CLAUSES 2   /* clauses a wave takes at a time (0 = a
+                                     quarter of its share of the DB) */
 #define GSS_TUNE_MAX_HIT_CHUNKS 3 /* cap on the hit buffer a sweep starts with
                                      (0 = sized to the worst case, for steps
                                      by the records seen); a sweep that needs
                                      more re-runs with a larger one.  Steps are
                                      held to it on every submit */
-#define GSS_TUNE_UNROLL 4         /* table rows in flight per lane: 1, 2, 4 or 8
-                                     at 16 words (default 4), 2 or 4 at 32
-                                     (default 4), 1, 2 or 4 at 64 (default 2);
-                                     fixed below 16 words */
-#define GSS_TUNE_FUSE_LEN 5       /* clauses of at most this many literals read
-                                     both rows of a literal in one pass
-                                     (0 = default 4; -1 = none, which runs the
-                                     kernel built without that pass and its
-                                     registers) */
+#define GSS_TUNE_UNROLL 4         /* 0, 1, 2, 4 or 8: accepted, without effect (the
+                                     sweep reads two rows per step, then one) */
+#define GSS_TUNE_FUSE_LEN 5       /* accepted, without effect (the negated row of a
+                                     literal is read only where a slot needs it) */
 #define GSS_TUNE_SCHEDULE 6       /* wave-to-bucket schedule: tasks of long
                                      clauses first (0 = default, 1), or short
                                      clauses first (2) */
 
 /* Autotuner: times the sweep on the current clause DB and assignment table
- * under a grid of (rows in flight, fuse length, clauses per task, waves per
- * CU, schedule) settings, `reps` sweeps each, and keeps the fastest.  The
- * chosen values are written to best[0..4] in that order (may be NULL) and
- * the best average kernel time to *best_ms.  Replaces the reference's fixed
+ * under a grid of (clauses per task, waves per CU, schedule) settings, `reps`
+ * sweeps each, and keeps the fastest.  The rows in flight (2), the fuse
+ * length (-1: none) and the chosen values are written to best[0..4] in that
+ * order (may be NULL) and the best average kernel time to *best_ms.  Replaces the reference's fixed
  * launch guidelines (GpuClauseSharerImpl.cu:50-57). */
 int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, float *best_ms);
 

@@ -508,7 +508,7 @@ struct gss_engine {
     // leaves them out, same records) and by batched steps submitted with
     // GSS_STEP_SCREEN (from the table)
     bool serve_prefilter = true;
-    DevBuf<uint8_t> serve_agg;         // 2 * vars + 2 bytes, padded to 4
+    DevBuf<uint32_t> serve_agg;        // one word per variable (SweepArgs::agg)
     DevBuf<uint64_t> serve_agg_words;  // [8]
     // state_version right after the last screened batched step was submitted:
     // while it still holds, serve_agg is that step's aggregate kept current
@@ -1833,7 +1833,7 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     a.chunk_cap = sl.chunk_cap;
     a.sentinel = (uint32_t)(2 * e->vars) << kLitShift;
     a.rec_words = sl.rec_words;
-    uint8_t *agg =
+    uint32_t *agg =
         (sl.g_serve && e->serve_prefilter) || sl.g_screen ? e->serve_agg.p : nullptr;
     a.agg = agg;
     a.agg_words = agg ? e->serve_agg_words.p : nullptr;
@@ -1850,7 +1850,7 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     end.ups = sl.d_ups.p;
     end.table = e->table.p;
     end.words = e->words;
-    end.agg32 = sl.g_agg_fused ? (uint32_t *)agg : nullptr;
+    end.agg = sl.g_agg_fused ? agg : nullptr;
     end.halt = e->d_halt;
     end.out = sl.h_out.p;
     end.dense = (uint64_t *)sl.d_dense.p;
@@ -1903,14 +1903,14 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     st.d[kRegLoads] = (uint32_t *)sl.d_loads.p;
     st.halt = e->d_halt;
     StepHeader *dh = sl.d_hdr.p;
-    uint8_t *agg = (serve && e->serve_prefilter) || screen ? e->serve_agg.p : nullptr;
+    uint32_t *agg = (serve && e->serve_prefilter) || screen ? e->serve_agg.p : nullptr;
     st.alloc = sl.d_alloc;
     st.counts = serve ? sl.d_wcount.p : nullptr;
     st.table = e->table.p;
     st.words = e->words;
     // updates come after base updates and word loads, where a step has them
     st.apply = !sl.g_bases;
-    st.agg32 = sl.g_agg_fused && st.apply && !agg_full ? (uint32_t *)agg : nullptr;
+    st.agg = sl.g_agg_fused && st.apply && !agg_full ? agg : nullptr;
     st.agg_words = screen ? e->serve_agg_words.p : nullptr;
     st.clauses = !staged;
     st.shift = kLitShift;
@@ -1945,7 +1945,7 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     // rebuilt, or refreshed where this step's updates and patches changed it
     if (he == hipSuccess && screen && agg_full)
         he = launch_table_agg(e->table.p, dh, e->vars, e->words, agg, cs);
-    else if (he == hipSuccess && screen && !st.agg32)
+    else if (he == hipSuccess && screen && !st.agg)
         he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, sl.d_patches.p, sl.g_patches,
                                      e->words, agg, cs);
     if (he == hipSuccess) he = launch_step_tail(e, sl, cs);
@@ -2387,7 +2387,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     // table was a screened step's (word loads change whole words: rebuilt)
     const bool agg_full =
         screen && (e->table_agg_at == 0 || e->table_agg_at != e->state_version || n_loads > 0);
-    if (use_agg && ((rc = e->serve_agg.reserve_async((size_t)((2 * e->vars + 2 + 3) / 4 * 4), es)) ||
+    if (use_agg && ((rc = e->serve_agg.reserve_async((size_t)e->vars + 1, es)) ||
                     (rc = e->serve_agg_words.reserve_async(8, es))))
         return rc;
     if ((rc = sl.d_hdr.reserve_async(1, es)) || (rc = sl.d_lits.reserve_async(sl.h_lits.cap, es)) ||

@@ -37,16 +37,17 @@ struct SweepArgs {
     const int32_t *dyn;      // if set, {nbuckets, npasses} are read here (graph replays)
     int rec_words;           // 8-byte words per record: 3 (gss_hit), 1 (gss_hit_id) or 2
                              // (gss_hit_clause: one record per clause, its words as a mask)
-    // Serving and screened batched steps (null otherwise): bit b of agg[l]
-    // is set only if literal l is non-false in every valid slot of group b --
-    // serving: the step's admitted requests r with r % 8 = b; screened steps:
-    // word group b, the row all ones over its slots (launch_table_agg);
-    // 2 * vars + 2 bytes (padded to 4).  agg_words[b] = the table words of
-    // group b (serving: of its requests; screened: with a valid slot).  In a
-    // group where two literal occurrences of a clause are so marked no slot
+    // Serving and screened batched steps (null otherwise): for each literal l
+    // a 16-bit entry (two per variable in one 32-bit word, literal 2v low);
+    // bit b is set only if l is non-false in every valid slot of group b, bit
+    // 8 + b only if it is true there -- serving: the step's admitted requests r
+    // with r % 8 = b; screened steps: word group b, over all its slots
+    // (launch_table_agg).  agg_words[b] = the table words of group b (serving:
+    // of its requests; screened: with a valid slot).  Where a literal of a
+    // clause is true, or two occurrences are non-false, no slot of the group
     // can report, so the exact check reads table rows only for the clause's
-    // other words.  4 MB at 2M variables: the votes are served from L2.
-    const uint8_t *agg;
+    // other words.
+    const uint32_t *agg;
     const uint64_t *agg_words;  // [8]
 };
 
@@ -84,7 +85,7 @@ struct StepEndArgs {
     const gss_var_update *ups;
     uint64_t *table;
     int words;
-    uint32_t *agg32;      // as in StepInArgs
+    uint32_t *agg;        // as in StepInArgs
     uint32_t *halt;       // set if records were dropped
     uint32_t *out;        // counts for the host: see write_counts in kernels.hip
     uint64_t *dense;
@@ -112,7 +113,7 @@ struct StepInArgs {
     uint32_t *alloc;      // the sweep's counters, cleared
     uint32_t *counts;     // serving: 2 * 64 counters of the grouping, cleared (else null)
     uint64_t *table;
-    uint32_t *agg32;      // apply with at most 8 words: screening entries to keep current
+    uint32_t *agg;        // apply with at most 8 words: screening entries to keep current
                           // (null: none, or a later kernel does it)
     uint64_t *agg_words;  // screened steps: [8], written from the header (else null)
     int words;
@@ -186,21 +187,19 @@ constexpr int kServeMaxRequests = 64;  // one admission wave: at most 64 request
 // the report.  One wave.
 hipError_t launch_serve_admit(const ServeRing &r, StepHeader *dh, gss_word_load *loads,
                               ServeReport *report, int words, hipStream_t s);
-// Aggregate entries of a batched step from the table itself (see
-// SweepArgs::agg): group b = words [b * words / 8, (b + 1) * words / 8) (one
-// word per group below 8 words); bit b of agg[l] set if row l is all ones on
-// every slot of group b's words (valid or not: all ones there implies all
-// ones on the valid slots).  Reads the table once.
+// Screening entries of a batched step from the table itself (SweepArgs::agg):
+// group b = words [b * words / 8, (b + 1) * words / 8) (one word per group
+// below 8 words), over every slot of its words (valid or not: what holds in
+// all of them holds in the valid ones).  Reads the table once.
 hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t vars, int words,
-                            uint8_t *agg, hipStream_t s);
+                            uint32_t *agg, hipStream_t s);
 // Keeps such entries current without reading the table: for each of the
-// step's updates (and patches, if with_patches) the bit of the update's word
-// group in both literals of its variable, from the table as it is when the
-// kernel runs.  Run after the updates are applied and again after the roll
+// step's updates (and patches, if with_patches) the bits of the update's word
+// group, from the table as it is when the kernel runs.  Run after the updates are applied and again after the roll
 // forward.
 hipError_t launch_table_agg_update(const uint64_t *table, const StepHeader *dh,
                                    const gss_var_update *ups, const gss_var_patch *patches,
-                                   bool with_patches, int words, uint8_t *agg, hipStream_t s);
+                                   bool with_patches, int words, uint32_t *agg, hipStream_t s);
 // Copies the admitted requests' patches from the pinned ring to r.dpatches
 // (consecutive lanes read consecutive 4-byte words: one pass over PCIe).
 hipError_t launch_serve_stage_patches(const ServeRing &r, const StepHeader *dh, hipStream_t s);
@@ -208,13 +207,13 @@ hipError_t launch_serve_stage_patches(const ServeRing &r, const StepHeader *dh, 
 // agg_words from the solver bases its admitted requests were loaded from:
 // one pass over the variables, after the admission and the base updates.
 hipError_t launch_serve_agg(const ServeRing &r, const StepHeader *dh, const gss_word_load *loads,
-                            const uint64_t *bases, int64_t vw, int64_t vars, uint8_t *agg,
+                            const uint64_t *bases, int64_t vw, int64_t vars, uint32_t *agg,
                             uint64_t *agg_words, hipStream_t s);
 // Applies the admitted requests' patches (staged in r.dpatches) with their
-// words shifted to where each request landed; with agg, clears the group bit
-// of every literal a patch makes false in a valid slot.
+// words shifted to where each request landed; with agg, clears the group's
+// bits that a patch undoes in a valid slot.
 hipError_t launch_serve_patch(const ServeRing &r, const StepHeader *dh, uint64_t *table,
-                              int words, uint8_t *agg, hipStream_t s);
+                              int words, uint32_t *agg, hipStream_t s);
 
 // One non-empty bucket of a tagged DB during compaction.
 struct CompactRef {

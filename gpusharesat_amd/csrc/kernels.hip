@@ -482,19 +482,19 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
 
 // ---- screened sweeps -----------------------------------------------------------
 
-// One clause per lane: the groups in which fewer than two literal occurrences
-// of the clause (its row of len stored offsets) are non-false in every valid
-// slot (SweepArgs::agg), i.e. the only groups where it can report; 0 once none
-// is left.  Two literals and then their entries are read per vote.
+// One clause per lane: the groups in which it can report, i.e. where none of
+// its literals (its row of len stored offsets) is true in every valid slot and
+// fewer than two occurrences are non-false in every valid slot (SweepArgs::agg);
+// 0 once none is left.  Two literals and then their entries are read per vote.
 __device__ __forceinline__ uint32_t lane_agg(LitPtr row, int len,
-                                             const uint8_t *__restrict__ agg, uint32_t gdead) {
-    uint32_t a1 = 0, a2 = gdead;  // groups with >= 1 / >= 2 such occurrences (empty: dead)
+                                             const uint16_t *__restrict__ agg, uint32_t gdead) {
+    uint32_t a1 = 0, a2 = gdead;  // groups with a non-false occurrence / that cannot report
     for (int j = 0; j < len; j += 2) {
         const uint32_t l0 = row[j], l1 = j + 1 < len ? row[j + 1] : 0u;
         const uint32_t x0 = agg[l0 >> 7], x1 = j + 1 < len ? agg[l1 >> 7] : 0u;
-        a2 |= a1 & x0;
+        a2 |= (a1 & x0) | (x0 >> 8);
         a1 |= x0;
-        a2 |= a1 & x1;
+        a2 |= (a1 & x1) | (x1 >> 8);
         a1 |= x1;
         if ((a2 & 0xFFu) == 0xFFu) return 0;
     }
@@ -597,7 +597,7 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep_screened(SweepArgs a) {
             const LitPtr cl = run.lits + (size_t)row0 * len;
             const uint32_t grp =
                 row0 + lane < count
-                    ? lane_agg(cl + (size_t)lane * len, len, a.agg, gdead)
+                    ? lane_agg(cl + (size_t)lane * len, len, (const uint16_t *)a.agg, gdead)
                     : 0u;
             if (!__ballot(grp != 0)) continue;
             uint64_t m = 0;  // table words to check
@@ -644,6 +644,19 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep_screened(SweepArgs a) {
         }
     });
     out.end(lane);
+}
+
+// Bit b of a variable's screening entries (SweepArgs::agg; one 32-bit word per
+// variable): literal v non-false / true, literal ~v non-false / true in every
+// slot of group b.
+__device__ __forceinline__ void agg_set(uint32_t *entry, uint32_t b, bool nf, bool tr, bool nfn,
+                                        bool trn) {
+    const uint32_t m = 0x01010101u << b;
+    const uint32_t x =
+        ((nf ? 1u : 0u) | (tr ? 0x100u : 0u) | (nfn ? 0x10000u : 0u) | (trn ? 0x1000000u : 0u))
+        << b;
+    if (x) atomicOr(entry, x);
+    if (x != m) atomicAnd(entry, ~(m & ~x));
 }
 
 __global__ void k_reset_u32(uint32_t *p, int n) {
@@ -695,15 +708,10 @@ __global__ void k_assig_roll(const gss_var_update *__restrict__ ups, int64_t n,
 }
 
 // Screening entries of a variable where a word is its own group (at most 8
-// words): bit `word` of both literals' bytes, from the variable's rows f and t.
-__device__ __forceinline__ void agg_word_bits(uint32_t *agg32, uint32_t var, uint32_t word,
+// words): the word's bits, from the variable's rows f and t there.
+__device__ __forceinline__ void agg_word_bits(uint32_t *agg, uint32_t var, uint32_t word,
                                               uint64_t f, uint64_t t) {
-    const uint32_t sh = (var & 1u) * 16u + word;  // entries 2 var, 2 var + 1 of word var / 2
-    const uint32_t bf = 1u << sh, bt = 1u << (sh + 8u);
-    const uint32_t set = (f == ~0ull ? bf : 0u) | (t == ~0ull ? bt : 0u);
-    const uint32_t clr = (bf | bt) & ~set;
-    if (set) atomicOr(agg32 + (var >> 1), set);
-    if (clr) atomicAnd(agg32 + (var >> 1), ~clr);
+    agg_set(agg + var, word, f == ~0ull, t == 0, t == ~0ull, f == 0);
 }
 
 // ---- batched steps: fixed launch shapes, counts from device memory --------
@@ -785,7 +793,7 @@ __global__ __launch_bounds__(256) void k_step_in(StepInArgs a) {
                 const uint64_t f = ~(def & ~tru), t1 = ~(def & tru);
                 a.table[base] = f;
                 a.table[base + a.words] = t1;
-                if (a.agg32) agg_word_bits(a.agg32, var, word, f, t1);
+                if (a.agg) agg_word_bits(a.agg, var, word, f, t1);
             }
             __syncthreads();
         }
@@ -926,7 +934,7 @@ __global__ void k_assig_apply_dyn(const gss_var_update *__restrict__ ups, const 
 __device__ __forceinline__ void roll_update(const gss_var_update *__restrict__ ups, int64_t i,
                                             uint64_t *__restrict__ table, int words,
                                             const int8_t *__restrict__ last_pos,
-                                            uint32_t *agg32) {
+                                            uint32_t *agg) {
     const uint32_t var = ups[i].var, word = ups[i].word;
     const int p = last_pos[word];
     if (p < 0) return;
@@ -935,7 +943,7 @@ __device__ __forceinline__ void roll_update(const gss_var_update *__restrict__ u
     const uint64_t t = ((table[base + words] >> p) & 1ull) ? ~0ull : 0ull;
     table[base] = f;
     table[base + words] = t;
-    if (agg32) agg_word_bits(agg32, var, word, f, t);
+    if (agg) agg_word_bits(agg, var, word, f, t);
 }
 
 __global__ void k_assig_roll_dyn(const gss_var_update *__restrict__ ups, const int64_t *n_p,
@@ -1080,7 +1088,7 @@ __global__ __launch_bounds__(256) void k_step_end(ChunkArgs c, StepEndArgs a) {
     const int64_t n = a.dh->nups;
     for (int64_t i = (blockIdx.x - kGatherBlocks) * (int64_t)256 + threadIdx.x; i < n;
          i += (int64_t)kRollBlocks * 256)
-        roll_update(a.ups, i, a.table, a.words, a.dh->last_pos, a.agg32);
+        roll_update(a.ups, i, a.table, a.words, a.dh->last_pos, a.agg);
 }
 
 // ---- records grouped by assignment word (serving steps) ----------------------
@@ -1263,53 +1271,61 @@ __global__ void k_serve_stage_patches(ServeRing r, const StepHeader *__restrict_
     }
 }
 
-// Batched-step aggregate: bit b of a literal row's entry is set if the row is
-// all ones over every slot of word group b (valid or not, so that the entry
-// follows the table alone and a step's updates refresh it).  All ones on
-// every slot implies all ones on the valid ones, which is what the screening
-// needs.  agg_words[b] = the group's words with a valid slot in this step.
+// Screening entries of a batched step (SweepArgs::agg), over every slot of a
+// group's words, valid or not, so that they follow the table alone and a
+// step's updates refresh them: all of them implies the valid ones.
 template <int W>
 struct TableGroups {
     static constexpr int NG = W < 8 ? W : 8;  // word groups
     static constexpr int GW = W / NG;         // words per group
 };
 
+// AND and OR of group b of a row.
 template <int W>
-__device__ __forceinline__ bool group_all_ones(const uint64_t *__restrict__ row, int b) {
+__device__ __forceinline__ void group_fold(const uint64_t *__restrict__ row, int b, uint64_t &all,
+                                           uint64_t &any) {
     constexpr int GW = TableGroups<W>::GW;
-    uint64_t x = ~0ull;
+    all = ~0ull;
+    any = 0;
 #pragma unroll
-    for (int w = 0; w < GW; w++) x &= row[b * GW + w];
-    return x == ~0ull;
+    for (int w = 0; w < GW; w++) {
+        const uint64_t x = row[b * GW + w];
+        all &= x;
+        any |= x;
+    }
 }
 
 template <int W>
 __global__ void k_table_agg(const uint64_t *__restrict__ table, const StepHeader *__restrict__ dh,
-                            int64_t rows, uint8_t *__restrict__ agg) {
+                            int64_t vars, uint32_t *__restrict__ agg) {
     constexpr int NG = TableGroups<W>::NG;
     if (dh->halted) return;  // the aggregate stays the halted step's
-    for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; l < rows;
-         l += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t *row = table + (size_t)l * W;
-        uint32_t bits = 0xFFu;
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < vars;
+         v += (int64_t)gridDim.x * blockDim.x) {
+        const uint64_t *f = table + (size_t)v * 2 * W, *t = f + W;
+        uint32_t x = 0;
 #pragma unroll
-        for (int b = 0; b < NG; b++)
-            if (!group_all_ones<W>(row, b)) bits &= ~(1u << b);
-        agg[l] = (uint8_t)bits;
+        for (int b = 0; b < NG; b++) {
+            uint64_t fa, fo, ta, to;
+            group_fold<W>(f, b, fa, fo);
+            group_fold<W>(t, b, ta, to);
+            x |= ((fa == ~0ull ? 1u : 0u) | (to == 0 ? 0x100u : 0u) |
+                  (ta == ~0ull ? 0x10000u : 0u) | (fo == 0 ? 0x1000000u : 0u))
+                 << b;
+        }
+        agg[v] = x;
     }
 }
 
-// Refreshes the aggregate bits that the step's updates (and patches) may have
-// changed: for each (var, word), the bit of the word's group in the entries
-// of both literals of var, from the table as it is now.  Entries are bytes,
-// four to a 32-bit word: bits change with 32-bit atomics.  Two updates of one
-// (var, group) write the same bit.
+// Refreshes the entries that the step's updates (and patches) may have
+// changed: for each (var, word), the bits of the word's group, from the table
+// as it is now.  Two updates of one (var, group) write the same bits.
 template <int W>
 __global__ void k_table_agg_update(const uint64_t *__restrict__ table,
                                    const StepHeader *__restrict__ dh,
                                    const gss_var_update *__restrict__ ups,
                                    const gss_var_patch *__restrict__ patches, int with_patches,
-                                   uint32_t *__restrict__ agg32) {
+                                   uint32_t *__restrict__ agg) {
     constexpr int GW = TableGroups<W>::GW;
     if (dh->halted) return;
     const int64_t nu = dh->nups, n = nu + (with_patches ? dh->npatches : 0);
@@ -1324,25 +1340,22 @@ __global__ void k_table_agg_update(const uint64_t *__restrict__ table,
             word = patches[i - nu].word;
         }
         const int b = (int)(word / GW);
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const uint64_t l = 2ull * var + s;
-            const uint32_t bit = 1u << (b + 8 * (int)(l & 3));
-            if (group_all_ones<W>(table + l * W, b)) atomicOr(agg32 + (l >> 2), bit);
-            else atomicAnd(agg32 + (l >> 2), ~bit);
-        }
+        const uint64_t *f = table + (size_t)var * 2 * W;
+        uint64_t fa, fo, ta, to;
+        group_fold<W>(f, b, fa, fo);
+        group_fold<W>(f + W, b, ta, to);
+        agg_set(agg + var, (uint32_t)b, fa == ~0ull, to == 0, ta == ~0ull, fo == 0);
     }
 }
 
-// Aggregate entries of a serving step: bit b of agg[2v] (agg[2v + 1]) is set
-// if literal v (~v) is not false in the bases of all of group b's requests
-// (r % 8 = b), or if the group is empty.  A request's words are loaded whole
-// from its solver's base, so until its patches (k_serve_patch clears what
-// they make false) the base value holds in all its slots.
+// Screening entries of a serving step: group b = the admitted requests r with
+// r % 8 = b, from their solvers' bases (a request's words are loaded whole from
+// its base, so until its patches the base value holds in all its slots;
+// k_serve_patch clears what a patch undoes).  Bits of empty groups are not read.
 __global__ void k_serve_agg(ServeRing r, const StepHeader *__restrict__ dh,
                             const gss_word_load *__restrict__ loads,
                             const uint64_t *__restrict__ bases, int64_t vw, int64_t vars,
-                            uint8_t *__restrict__ agg, uint64_t *__restrict__ agg_words) {
+                            uint32_t *__restrict__ agg, uint64_t *__restrict__ agg_words) {
     if (dh->halted) return;  // the aggregate stays the halted step's
     __shared__ uint32_t s_base[kServeMaxRequests];
     const int cnt = (int)*r.adm_count;
@@ -1358,30 +1371,26 @@ __global__ void k_serve_agg(ServeRing r, const StepHeader *__restrict__ dh,
         agg_words[threadIdx.x] = m;
     }
     __syncthreads();
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v <= vars;
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < vars;
          v += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t pos = 0xFFu, neg = 0xFFu;
-        if (v < vars) {
-            const uint64_t bit = 1ull << (v & 63);
-            const int64_t i = v >> 6;
-            for (int q = 0; q < cnt; q++) {
-                const uint64_t *def = bases + (size_t)(2 * s_base[q]) * vw;
-                const bool d = (def[i] & bit) != 0;
-                const bool t = (def[vw + i] & bit) != 0;
-                const uint32_t gb = 1u << (q & 7);
-                if (d && !t) pos &= ~gb;  // v is false in this base
-                if (d && t) neg &= ~gb;   // ~v is false in this base
-            }
-        } else {  // sentinel pair: the padding entry contributes nothing
-            pos = 0u;
+        uint32_t x = ~0u;
+        const uint64_t bit = 1ull << (v & 63);
+        const int64_t i = v >> 6;
+        for (int q = 0; q < cnt; q++) {
+            const uint64_t *def = bases + (size_t)(2 * s_base[q]) * vw;
+            const bool d = (def[i] & bit) != 0;
+            const bool t = (def[vw + i] & bit) != 0;
+            // true: v non-false and true; false: ~v; undefined: both non-false
+            const uint32_t keep = !d ? 0x00010001u : t ? 0x00000101u : 0x01010000u;
+            x &= ~((0x01010101u & ~keep) << (q & 7));
         }
-        ((uint16_t *)agg)[v] = (uint16_t)(pos | (neg << 8));
+        agg[v] = x;
     }
 }
 
 __global__ void k_serve_patch(ServeRing r, const StepHeader *__restrict__ dh,
                               uint64_t *__restrict__ table, int words,
-                              uint32_t *__restrict__ agg32) {
+                              uint32_t *__restrict__ agg) {
     const int64_t n = dh->npatches;
     const int cnt = (int)*r.adm_count;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
@@ -1395,14 +1404,16 @@ __global__ void k_serve_patch(ServeRing r, const StepHeader *__restrict__ dh,
         const size_t base = (size_t)var * 2 * words + word;
         table[base] = (table[base] & ~m) | (~(d & ~t) & m);
         table[base + words] = (table[base + words] & ~m) | (~(d & t) & m);
-        if (agg32 && word < 64u) {
+        if (agg && word < 64u) {
+            // the request's group keeps what holds in the patched slots too
             const uint64_t vm = m & dh->valid[word];
-            const uint32_t gb = 1u << (q & 7);
-            // entries 2 var and 2 var + 1 are bytes 2 (var & 1) and +1 of
-            // 4-byte word var / 2
-            const uint32_t sh = (var & 1u) * 16u;
-            if (d & ~t & vm) atomicAnd(&agg32[var >> 1], ~(gb << sh));
-            if (d & t & vm) atomicAnd(&agg32[var >> 1], ~(gb << (sh + 8u)));
+            const uint64_t fal = d & ~t & vm, tru = d & t & vm;
+            uint32_t clr = 0;
+            if (fal) clr |= 0x1u;               // v non-false
+            if (vm & ~tru) clr |= 0x100u;       // v true
+            if (tru) clr |= 0x10000u;           // ~v non-false
+            if (vm & ~fal) clr |= 0x1000000u;   // ~v true
+            if (clr) atomicAnd(agg + var, ~(clr << (q & 7)));
         }
     }
 }
@@ -1634,45 +1645,32 @@ hipError_t launch_serve_admit(const ServeRing &r, StepHeader *dh, gss_word_load 
 }
 
 hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t vars, int words,
-                            uint8_t *agg, hipStream_t s) {
-    const int64_t rows = 2 * vars + 2;
-    const unsigned blocks = (unsigned)std::min<int64_t>((rows + 255) / 256, 8192);
-#define GSS_TABLE_AGG(W_)                                                                   \
+                            uint32_t *agg, hipStream_t s) {
+    const unsigned blocks = (unsigned)std::min<int64_t>((vars + 255) / 256, 8192);
+    if (vars <= 0) return hipSuccess;
+#define X(W_)                                                                               \
     if (words == W_) {                                                                      \
-        hipLaunchKernelGGL(k_table_agg<W_>, dim3(blocks), dim3(256), 0, s, table, dh, rows, \
+        hipLaunchKernelGGL(k_table_agg<W_>, dim3(blocks), dim3(256), 0, s, table, dh, vars, \
                            agg);                                                            \
         return hipGetLastError();                                                           \
     }
-    GSS_TABLE_AGG(1)
-    GSS_TABLE_AGG(2)
-    GSS_TABLE_AGG(4)
-    GSS_TABLE_AGG(8)
-    GSS_TABLE_AGG(16)
-    GSS_TABLE_AGG(32)
-    GSS_TABLE_AGG(64)
-#undef GSS_TABLE_AGG
+    GSS_WORDS(X)
+#undef X
     return hipErrorInvalidValue;
 }
 
 hipError_t launch_table_agg_update(const uint64_t *table, const StepHeader *dh,
                                    const gss_var_update *ups, const gss_var_patch *patches,
-                                   bool with_patches, int words, uint8_t *agg, hipStream_t s) {
-    uint32_t *agg32 = (uint32_t *)agg;
+                                   bool with_patches, int words, uint32_t *agg, hipStream_t s) {
     const int wp = with_patches ? 1 : 0;
-#define GSS_TABLE_AGG_UP(W_)                                                                 \
-    if (words == W_) {                                                                       \
-        hipLaunchKernelGGL(k_table_agg_update<W_>, dim3(1024), dim3(256), 0, s, table, dh,   \
-                           ups, patches, wp, agg32);                                         \
-        return hipGetLastError();                                                            \
+#define X(W_)                                                                              \
+    if (words == W_) {                                                                     \
+        hipLaunchKernelGGL(k_table_agg_update<W_>, dim3(1024), dim3(256), 0, s, table, dh, \
+                           ups, patches, wp, agg);                                         \
+        return hipGetLastError();                                                          \
     }
-    GSS_TABLE_AGG_UP(1)
-    GSS_TABLE_AGG_UP(2)
-    GSS_TABLE_AGG_UP(4)
-    GSS_TABLE_AGG_UP(8)
-    GSS_TABLE_AGG_UP(16)
-    GSS_TABLE_AGG_UP(32)
-    GSS_TABLE_AGG_UP(64)
-#undef GSS_TABLE_AGG_UP
+    GSS_WORDS(X)
+#undef X
     return hipErrorInvalidValue;
 }
 
@@ -1682,7 +1680,7 @@ hipError_t launch_serve_stage_patches(const ServeRing &r, const StepHeader *dh, 
 }
 
 hipError_t launch_serve_agg(const ServeRing &r, const StepHeader *dh, const gss_word_load *loads,
-                            const uint64_t *bases, int64_t vw, int64_t vars, uint8_t *agg,
+                            const uint64_t *bases, int64_t vw, int64_t vars, uint32_t *agg,
                             uint64_t *agg_words, hipStream_t s) {
     hipLaunchKernelGGL(k_serve_agg, dim3(2048), dim3(256), 0, s, r, dh, loads, bases, vw, vars,
                        agg, agg_words);
@@ -1690,9 +1688,9 @@ hipError_t launch_serve_agg(const ServeRing &r, const StepHeader *dh, const gss_
 }
 
 hipError_t launch_serve_patch(const ServeRing &r, const StepHeader *dh, uint64_t *table,
-                              int words, uint8_t *agg, hipStream_t s) {
+                              int words, uint32_t *agg, hipStream_t s) {
     hipLaunchKernelGGL(k_serve_patch, dim3(1024), dim3(256), 0, s, r, dh, table, words,
-                       (uint32_t *)agg);
+                       agg);
     return hipGetLastError();
 }
 

@@ -11,13 +11,11 @@
 // approxNthAct, gpuShareLib/Clauses.cu:484-525) and compacts the DB on the
 // device.
 //
-// The MLP kernels: training runs one sample per wave (lane i = hidden unit i
-// of both 64-unit layers, the parameters staged in LDS) and writes the
-// activations and the back-propagated deltas; the weight gradient is a sum of
-// per-sample outer products, computed per (parameter, chunk of 32 samples)
-// and reduced in a fixed order, so gradients are deterministic.  Scoring runs
-// one clause per thread.  ReLU'(0) = 0.  Loss: weighted logistic, mean over
-// the batch.
+// The MLP kernels: a training pass (k_mlp_pass) computes 64 samples per block
+// on the FP32 matrix units, forward, deltas and weight gradients, and leaves
+// one partial gradient per block, reduced in a fixed order, so gradients are
+// deterministic.  Scoring runs one clause per thread.  ReLU'(0) = 0.  Loss:
+// weighted logistic, mean over the batch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,8 +45,7 @@ constexpr int OW1 = 0, OB1 = H * F, OW2 = OB1 + H, OB2 = OW2 + H * H, OW3 = OB2 
 static_assert(OB3 + 1 == P, "parameter layout");
 constexpr int kBuckets = 20000;
 constexpr float kRescale = 1e19f;  // RESCALE_CONST, gpuShareLib/Clauses.cuh:39
-constexpr int kGradChunk = 32;     // samples per partial gradient
-
+constexpr size_t kGradDirect = 4u << 20;  // floats gss_res_grad passes through pinned memory
 int set_err(int code, const char *fmt, ...) {
     char buf[512];
     va_list ap;
@@ -348,136 +345,240 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// Forward + backward, one sample per wave: lane i is hidden unit i of both
-// layers (H = 64 = the wave).  W2 is staged in LDS in both orientations, so
-// the forward (row j by lane j) and the backward (column i by lane i) read
-// consecutive words.  A wave hands its layer's outputs to all its lanes
-// through its own LDS row.  Writes a1, a2 (activations), d1, d2 (deltas at
-// the hidden pre-activations), d3 (at the output logit), already multiplied
-// by the sample weight.
-__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(
-    const float *__restrict__ params, const float *__restrict__ x, const float *__restrict__ y,
-    const float *__restrict__ wt, const uint32_t *__restrict__ idx, int64_t n, float w_pos,
-    float w_neg, float *__restrict__ a1o, float *__restrict__ a2o, float *__restrict__ d1o,
-    float *__restrict__ d2o, float *__restrict__ d3o, float *loss_sum) {
-    static_assert(H == 64, "one hidden unit per lane of a wave");
-    __shared__ float w1[H * F], b1[H], w2[H * H], w2t[H * H], b2[H], w3[H];
-    __shared__ float row[4][H];
-    __shared__ float b3s, blk;
-    const int tid = threadIdx.x;
-    for (int i = tid; i < H * F; i += blockDim.x) w1[i] = params[OW1 + i];
-    for (int i = tid; i < H * H; i += blockDim.x) {
-        const float v = params[OW2 + i];
-        w2[i] = v;
-        w2t[(i % H) * H + i / H] = v;
+// Forward, backward and weight gradients of the whole network in one kernel, on
+// the FP32 matrix units: a block of 4 waves takes 64 samples at a time, wave w
+// the forward and the deltas of samples 16 w .. 16 w + 15, then (all deltas in
+// LDS) the gradient rows of hidden units 16 w .. 16 w + 15, which stay in its
+// accumulators until the block's last tile.  Each product is a chain of
+// 16x16x4 tiles: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and, of the
+// result, rows 4 (l / 16) + r of column l % 16.
+//
+// 880 of those instructions per 64 samples, ~3 us a block; what is left is
+// latency (8,192 samples: 128 blocks, one tile each).  One sample per wave with
+// the activations and deltas going through memory, and the gradients in a
+// second kernel, took 47 + 32 us for 8,192 samples; this takes 24, the samples
+// read from pinned memory.
+//
+// Row strides of 68 and 20 words keep the A operands' 16 rows x 4 columns on
+// different LDS banks.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kTile = 64;     // samples
+constexpr int kLd = H + 4;    // row stride of the 64-column LDS arrays
+constexpr int kLdx = 20;      // of the inputs and W1 (12 columns, the bias, padding)
+constexpr int kPartial = P + 1;  // floats per block: the gradient, the loss
+constexpr int kMlpBlocks = 256;  // most blocks (partial gradients) of a pass
+
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ params,
+                                                  const float *__restrict__ x,
+                                                  const float *__restrict__ y,
+                                                  const float *__restrict__ wt,
+                                                  const uint32_t *__restrict__ idx, int64_t n,
+                                                  float w_pos, float w_neg,
+                                                  float *__restrict__ partial) {
+    static_assert(H == 64 && F == 12, "four 16-unit tiles, three 16-byte loads per sample");
+    __shared__ float s_w1[H * kLdx], s_w2[H * kLd], s_b2[H], s_w3[H];
+    __shared__ float s_x[kTile * kLdx], s_y[kTile], s_sw[kTile];
+    __shared__ float s_a1[kTile * kLd], s_d1[kTile * kLd], s_d2[kTile * kLd];
+    __shared__ float s_sum[4][2 * H + 2];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int lc = lane & 15, lr = lane >> 4;
+    for (int i = tid; i < H * 16; i += 256) {
+        const int u = i >> 4, k = i & 15;
+        s_w1[u * kLdx + k] = k < F ? params[OW1 + u * F + k] : k == F ? params[OB1 + u] : 0.f;
     }
+    for (int i = tid; i < H * H; i += 256) s_w2[(i >> 6) * kLd + (i & 63)] = params[OW2 + i];
     if (tid < H) {
-        b1[tid] = params[OB1 + tid];
-        b2[tid] = params[OB2 + tid];
-        w3[tid] = params[OW3 + tid];
+        s_b2[tid] = params[OB2 + tid];
+        s_w3[tid] = params[OW3 + tid];
     }
-    if (tid == 0) {
-        b3s = params[OB3];
-        blk = 0.f;
-    }
-    __syncthreads();
-    const int lane = tid & 63, wv = tid >> 6;
-    float my_loss = 0.f;
-    for (int64_t b = (int64_t)blockIdx.x * 4 + wv; b < n; b += (int64_t)gridDim.x * 4) {
-        const int64_t src = idx ? (int64_t)idx[b] : b;
-        float z1 = b1[lane];
+    const float b3 = params[OB3];
+    f32x4 g1 = {}, g2[4] = {};             // gradient rows 16 wv .. of W1 (and b1), W2
+    float gw3[4] = {}, gb2[4] = {};        // of this lane's rows
+    float gb3 = 0.f, loss = 0.f;
+    const int r0 = 16 * wv;                // the wave's first sample / gradient row
+    for (int64_t t0 = (int64_t)blockIdx.x * kTile; t0 < n; t0 += (int64_t)gridDim.x * kTile) {
+        // inputs: 12 columns, a one for the bias; rows past n are zero.  Three
+        // 16-byte loads per sample (x may lie in pinned memory: whole lines).
+        if (tid < 3 * kTile) {
+            const int s = tid / 3, k = 4 * (tid % 3);
+            f32x4 v = {};
+            if (t0 + s < n) {
+                const int64_t src = idx ? (int64_t)idx[t0 + s] : t0 + s;
+                v = *(const f32x4 *)(x + src * F + k);
+            }
 #pragma unroll
-        for (int k = 0; k < F; k++) z1 = fmaf(w1[lane * F + k], x[src * F + k], z1);
-        const float a1 = z1 > 0.f ? z1 : 0.f;
-        a1o[b * H + lane] = a1;
-        row[wv][lane] = a1;
-        __builtin_amdgcn_wave_barrier();
-        float z2 = b2[lane];
-#pragma unroll 16
-        for (int i = 0; i < H; i++) z2 = fmaf(w2t[i * H + lane], row[wv][i], z2);
-        const float a2 = z2 > 0.f ? z2 : 0.f;
-        a2o[b * H + lane] = a2;
-        const float z3 = b3s + wave_sum(w3[lane] * a2);
-        const float yv = y[src];
-        const float sw = (wt ? wt[src] : 1.f) * (yv > 0.5f ? w_pos : w_neg);
-        const float d3 = sw * (sigmoidf(z3) - yv);
-        if (lane == 0) {
-            d3o[b] = d3;
-            my_loss += sw * logistic_loss(z3, yv);
+            for (int u = 0; u < 4; u++) s_x[s * kLdx + k + u] = v[u];
+        } else {
+            const int s = tid - 3 * kTile;
+            const bool on = t0 + s < n;
+            const int64_t src = on && idx ? (int64_t)idx[t0 + s] : t0 + s;
+            const float yv = on ? y[src] : 0.f;
+            const float w = on && wt ? wt[src] : 1.f;
+            s_y[s] = yv;
+            s_sw[s] = on ? w * (yv > 0.5f ? w_pos : w_neg) : 0.f;
+            s_x[s * kLdx + F] = on ? 1.f : 0.f;
+#pragma unroll
+            for (int k = F + 1; k < 16; k++) s_x[s * kLdx + k] = 0.f;
+        }
+        __syncthreads();
+        f32x4 a1[4] = {}, a2[4];
+#pragma unroll
+        for (int k = 0; k < 16; k += 4) {
+            const float a = s_x[(r0 + lc) * kLdx + k + lr];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                a1[c] = mfma(a, s_w1[(16 * c + lc) * kLdx + k + lr], a1[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                a1[c][r] = fmaxf(a1[c][r], 0.f);
+                s_a1[(r0 + 4 * lr + r) * kLd + 16 * c + lc] = a1[c][r];
+            }
+        __builtin_amdgcn_wave_barrier();  // the wave's own rows
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float b = s_b2[16 * c + lc];
+            a2[c] = f32x4{b, b, b, b};
+        }
+#pragma unroll 4
+        for (int k = 0; k < H; k += 4) {
+            const float a = s_a1[(r0 + lc) * kLd + k + lr];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                a2[c] = mfma(a, s_w2[(16 * c + lc) * kLd + k + lr], a2[c]);
+        }
+        f32x4 z3 = {};
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float w3 = s_w3[16 * c + lc];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                a2[c][r] = fmaxf(a2[c][r], 0.f);
+                z3[r] = fmaf(w3, a2[c][r], z3[r]);
+            }
+        }
+        float d3[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float z = z3[r];
+#pragma unroll
+            for (int d = 1; d < 16; d <<= 1) z += __shfl_xor(z, d);
+            z += b3;
+            const float yv = s_y[r0 + 4 * lr + r], sw = s_sw[r0 + 4 * lr + r];
+            d3[r] = sw * (sigmoidf(z) - yv);
+            if (lc == 0) {
+                gb3 += d3[r];
+                loss += sw * logistic_loss(z, yv);
+            }
         }
         // d2_j = d3 w3_j relu'(z2_j); d1_i = relu'(z1_i) sum_j W2[j][i] d2_j
-        const float d2 = a2 > 0.f ? d3 * w3[lane] : 0.f;
-        d2o[b * H + lane] = d2;
-        __builtin_amdgcn_wave_barrier();  // every lane has read a1 from the row
-        row[wv][lane] = d2;
-        __builtin_amdgcn_wave_barrier();
-        float acc = 0.f;
-#pragma unroll 16
-        for (int j = 0; j < H; j++) acc = fmaf(w2[j * H + lane], row[wv][j], acc);
-        d1o[b * H + lane] = a1 > 0.f ? acc : 0.f;
-        __builtin_amdgcn_wave_barrier();  // the next sample rewrites the row
-    }
-    atomicAdd(&blk, my_loss);
-    __syncthreads();
-    if (tid == 0) atomicAdd(loss_sum, blk);
-}
-
-// Partial gradient of every parameter over one chunk of samples.
-__global__ void k_mlp_grad_partial(const float *__restrict__ x, const uint32_t *__restrict__ idx,
-                                   const float *__restrict__ a1, const float *__restrict__ a2,
-                                   const float *__restrict__ d1, const float *__restrict__ d2,
-                                   const float *__restrict__ d3, int64_t n,
-                                   float *__restrict__ partial) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t b0 = (int64_t)blockIdx.y * kGradChunk;
-    const int64_t b1 = min<int64_t>(n, b0 + kGradChunk);
-    if (p >= P) return;
-    float g = 0.f;
-    if (p < OB1) {
-        const int i = p / F, k = p % F;
-        for (int64_t b = b0; b < b1; b++) {
-            const int64_t src = idx ? (int64_t)idx[b] : b;
-            g = fmaf(d1[b * H + i], x[src * F + k], g);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float w3 = s_w3[16 * c + lc];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float d2 = a2[c][r] > 0.f ? d3[r] * w3 : 0.f;
+                gw3[c] = fmaf(d3[r], a2[c][r], gw3[c]);
+                gb2[c] += d2;
+                s_d2[(r0 + 4 * lr + r) * kLd + 16 * c + lc] = d2;
+            }
         }
-    } else if (p < OW2) {
-        const int i = p - OB1;
-        for (int64_t b = b0; b < b1; b++) g += d1[b * H + i];
-    } else if (p < OB2) {
-        const int q = p - OW2, j = q / H, i = q % H;
-        for (int64_t b = b0; b < b1; b++) g = fmaf(d2[b * H + j], a1[b * H + i], g);
-    } else if (p < OW3) {
-        const int j = p - OB2;
-        for (int64_t b = b0; b < b1; b++) g += d2[b * H + j];
-    } else if (p < OB3) {
-        const int j = p - OW3;
-        for (int64_t b = b0; b < b1; b++) g = fmaf(d3[b], a2[b * H + j], g);
-    } else {
-        for (int64_t b = b0; b < b1; b++) g += d3[b];
+        __builtin_amdgcn_wave_barrier();
+        f32x4 d1[4] = {};
+#pragma unroll 4
+        for (int k = 0; k < H; k += 4) {
+            const float a = s_d2[(r0 + lc) * kLd + k + lr];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                d1[c] = mfma(a, s_w2[(k + lr) * kLd + 16 * c + lc], d1[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                s_d1[(r0 + 4 * lr + r) * kLd + 16 * c + lc] = a1[c][r] > 0.f ? d1[c][r] : 0.f;
+        __syncthreads();
+        // gradients over the tile's 64 samples: rows r0 .. r0 + 15
+#pragma unroll 4
+        for (int k = 0; k < kTile; k += 4) {
+            const float a = s_d2[(k + lr) * kLd + r0 + lc];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                g2[c] = mfma(a, s_a1[(k + lr) * kLd + 16 * c + lc], g2[c]);
+            g1 = mfma(s_d1[(k + lr) * kLd + r0 + lc], s_x[(k + lr) * kLdx + lc], g1);
+        }
+        __syncthreads();  // the next tile overwrites the arrays
     }
-    partial[(size_t)blockIdx.y * P + p] = g;
+    float *out = partial + (size_t)blockIdx.x * kPartial;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int u = r0 + 4 * lr + r;
+        if (lc < F) out[OW1 + u * F + lc] = g1[r];
+        else if (lc == F) out[OB1 + u] = g1[r];
+#pragma unroll
+        for (int c = 0; c < 4; c++) out[OW2 + u * H + 16 * c + lc] = g2[c][r];
+    }
+    // column sums: over the lanes of a column, then over the waves in order
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        float u = gb2[c], v = gw3[c];
+        u += __shfl_xor(u, 16);
+        u += __shfl_xor(u, 32);
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+        if (lr == 0) {
+            s_sum[wv][16 * c + lc] = u;
+            s_sum[wv][H + 16 * c + lc] = v;
+        }
+    }
+    const float g = wave_sum(gb3), l = wave_sum(loss);
+    if (lane == 0) {
+        s_sum[wv][2 * H] = g;
+        s_sum[wv][2 * H + 1] = l;
+    }
+    __syncthreads();
+    if (tid < 2 * H + 2) {
+        const float v = s_sum[0][tid] + s_sum[1][tid] + s_sum[2][tid] + s_sum[3][tid];
+        out[tid < H ? OB2 + tid : tid < 2 * H ? OW3 + tid - H : tid == 2 * H ? OB3 : P] = v;
+    }
 }
 
-// grad = scale * sum of the partials (fixed order); with lr != 0 also a
-// momentum step: m = mu m + grad, w -= lr m.
-__global__ void k_mlp_reduce_step(const float *__restrict__ partial, int nchunks, float scale,
-                                  float *__restrict__ grad, float *__restrict__ params,
-                                  float *__restrict__ mom, float lr, float mu) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= P) return;
-    // loads issued eight at a time, summed in chunk order (deterministic)
+// grad = scale * sum of the blocks' partials (fixed order: four runs of blocks,
+// one per thread, then the four); with lr != 0 also a momentum step: m = mu m +
+// grad, w -= lr m.  host (pinned, may be null) takes the gradient and the loss.
+__global__ __launch_bounds__(256) void k_mlp_reduce_step(const float *__restrict__ partial,
+                                                         int blocks, float scale,
+                                                         float *__restrict__ params,
+                                                         float *__restrict__ mom, float lr,
+                                                         float mu, float *host) {
+    __shared__ float s[4][64];
+    const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + c;
     float g = 0.f;
-    int c = 0;
-    for (; c + 8 <= nchunks; c += 8) {
-        float v[8];
+    if (p < kPartial) {
+        int b = blocks * q / 4;
+        const int e = blocks * (q + 1) / 4;
+        for (; b + 16 <= e; b += 16) {
+            float v[16];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = partial[(size_t)(c + u) * P + p];
+            for (int u = 0; u < 16; u++) v[u] = partial[(size_t)(b + u) * kPartial + p];
 #pragma unroll
-        for (int u = 0; u < 8; u++) g += v[u];
+            for (int u = 0; u < 16; u++) g += v[u];
+        }
+        for (; b < e; b++) g += partial[(size_t)b * kPartial + p];
     }
-    for (; c < nchunks; c++) g += partial[(size_t)c * P + p];
-    g *= scale;
-    grad[p] = g;
-    if (lr != 0.f) {
+    s[q][c] = g;
+    __syncthreads();
+    if (q != 0 || p >= kPartial) return;
+    g = (s[0][c] + s[1][c] + s[2][c] + s[3][c]) * scale;
+    if (host) host[p] = g;
+    if (lr != 0.f && p < P) {
         const float m = mu * mom[p] + g;
         mom[p] = m;
         params[p] -= lr * m;
@@ -584,8 +685,9 @@ struct gss_res {
     Buf<float> ema_f, ema_s, tot, act, score;
     Buf<uint8_t> alive_d, keep, evicted;
     // MLP
-    Buf<float> params, mom, grad, partial;
-    Buf<float> a1, a2, d1, d2, d3, loss;
+    Buf<float> params, mom, partial;
+    float *h_in = nullptr, *h_res = nullptr;  // pinned: samples of gss_res_grad, a pass's results
+    size_t h_in_cap = 0;
     Buf<float> xs, ys, ws;
     Buf<uint32_t> idx;
     // scratch
@@ -610,35 +712,27 @@ int check(gss_res *r) {
     return engine_activate(r->e);
 }
 
-// Runs forward/backward + gradient (+ optional SGD step) on n samples
-// already in r->xs / ys / ws, in the order of idx (null = identity).
+// Runs forward/backward + gradient (+ optional SGD step) on n samples x / y /
+// wt (device or pinned memory), in the order of idx (null = identity).  With
+// wait, r->h_res then holds the gradient and, at [P], the mean loss.
 int run_batch(gss_res *r, hipStream_t st, const float *x, const float *y, const float *wt,
-              const uint32_t *idx, int64_t n, float w_pos, float w_neg, float lr, float *loss) {
+              const uint32_t *idx, int64_t n, float w_pos, float w_neg, float lr, bool wait) {
     int rc;
-    const int nchunks = (int)((n + kGradChunk - 1) / kGradChunk);
-    if ((rc = r->a1.reserve((size_t)n * H)) || (rc = r->a2.reserve((size_t)n * H)) ||
-        (rc = r->d1.reserve((size_t)n * H)) || (rc = r->d2.reserve((size_t)n * H)) ||
-        (rc = r->d3.reserve((size_t)n)) || (rc = r->loss.reserve(1)) ||
-        (rc = r->partial.reserve((size_t)nchunks * P)))
-        return rc;
-    RES_HIP(hipMemsetAsync(r->loss.p, 0, sizeof(float), st));
-    const unsigned fb_blocks = (unsigned)std::min<int64_t>((n + 3) / 4, 4096);
-    hipLaunchKernelGGL(k_mlp_fwd_bwd, dim3(std::max(fb_blocks, 1u)), dim3(256), 0, st, r->params.p, x,
-                       y, wt, idx, n, w_pos, w_neg, r->a1.p, r->a2.p, r->d1.p, r->d2.p, r->d3.p,
-                       r->loss.p);
-    RES_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_grad_partial, dim3((P + 255) / 256, nchunks), dim3(256), 0, st, x,
-                       idx, r->a1.p, r->a2.p, r->d1.p, r->d2.p, r->d3.p, n, r->partial.p);
-    RES_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_mlp_reduce_step, dim3((P + 255) / 256), dim3(256), 0, st, r->partial.p,
-                       nchunks, 1.0f / (float)n, r->grad.p, r->params.p, r->mom.p, lr, 0.9f);
-    RES_HIP(hipGetLastError());
-    if (loss) {
-        float l = 0.f;
-        RES_HIP(hipMemcpyAsync(&l, r->loss.p, sizeof(float), hipMemcpyDeviceToHost, st));
-        RES_HIP(hipStreamSynchronize(st));
-        *loss = l / (float)n;
+    if ((rc = r->partial.reserve((size_t)kMlpBlocks * kPartial))) return rc;
+    if (!r->h_res && hipHostMalloc((void **)&r->h_res, kPartial * sizeof(float),
+                                   hipHostMallocDefault) != hipSuccess) {
+        r->h_res = nullptr;
+        return set_err(GSS_E_NOMEM, "pinned host allocation failed");
     }
+    const int blocks = (int)std::min<int64_t>((n + kTile - 1) / kTile, kMlpBlocks);
+    hipLaunchKernelGGL(k_mlp_pass, dim3(blocks), dim3(256), 0, st, r->params.p, x, y, wt, idx, n,
+                       w_pos, w_neg, r->partial.p);
+    RES_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_mlp_reduce_step, dim3((kPartial + 63) / 64), dim3(256), 0, st,
+                       r->partial.p, blocks, 1.0f / (float)n, r->params.p, r->mom.p, lr, 0.9f,
+                       wait ? r->h_res : (float *)nullptr);
+    RES_HIP(hipGetLastError());
+    if (wait) RES_HIP(hipStreamSynchronize(st));
     return GSS_OK;
 }
 
@@ -667,7 +761,7 @@ int gss_res_create(gss_engine *e, int64_t max_tags, float decay, uint64_t seed, 
         (rc = r->ema_s.reserve(n)) || (rc = r->tot.reserve(n)) || (rc = r->act.reserve(n)) ||
         (rc = r->score.reserve(n)) || (rc = r->alive_d.reserve(n)) || (rc = r->keep.reserve(n)) ||
         (rc = r->evicted.reserve(n)) || (rc = r->params.reserve(P)) || (rc = r->mom.reserve(P)) ||
-        (rc = r->grad.reserve(P)) || (rc = r->hist.reserve(kBuckets)) ||
+        (rc = r->hist.reserve(kBuckets)) ||
         (rc = r->maxbits.reserve(1)) || (rc = r->counters.reserve(2))) {
         gss_res_destroy(r);
         return rc;
@@ -709,9 +803,10 @@ int gss_res_destroy(gss_res *r) {
     r->lens_in.release();
     r->solv.release();
     r->solv_cum.release();
+    if (r->h_in) (void)hipHostFree(r->h_in);
+    if (r->h_res) (void)hipHostFree(r->h_res);
     for (auto *b : {&r->ema_f, &r->ema_s, &r->tot, &r->act, &r->score, &r->params, &r->mom,
-                    &r->grad, &r->partial, &r->a1, &r->a2, &r->d1, &r->d2, &r->d3, &r->loss,
-                    &r->xs, &r->ys, &r->ws, &r->act_in, &r->fout})
+                    &r->partial, &r->xs, &r->ys, &r->ws, &r->act_in, &r->fout})
         b->release();
     r->alive_d.release();
     r->keep.release();
@@ -890,11 +985,11 @@ int gss_res_train(gss_res *r, int32_t round, int horizon, int epochs, int batch,
         int nb = 0;
         for (int64_t b0 = 0; b0 < n; b0 += batch) {
             const int64_t m = std::min<int64_t>(batch, n - b0);
-            float l = 0.f;
+            const bool wait = ep == epochs - 1;
             if ((rc = run_batch(r, st, sn.x.p, r->ys.p, r->ws.p, r->idx.p + b0, m, w_pos, w_neg,
-                                lr, ep == epochs - 1 ? &l : nullptr)))
+                                lr, wait)))
                 return rc;
-            acc += l;
+            if (wait) acc += r->h_res[P];
             nb++;
         }
         if (ep == epochs - 1) last = (float)(acc / std::max(nb, 1));
@@ -1024,18 +1119,44 @@ int gss_res_grad(gss_res *r, int64_t n, const float *x, const float *y, const fl
     if (rc) return rc;
     if (n <= 0 || !x || !y || !grad) return set_err(GSS_E_INVAL, "bad arguments");
     hipStream_t st = engine_stream(r->e);
-    if ((rc = r->xs.reserve((size_t)n * F)) || (rc = r->ys.reserve(n)) || (rc = r->ws.reserve(n)))
-        return rc;
-    RES_HIP(hipMemcpyAsync(r->xs.p, x, (size_t)n * F * 4, hipMemcpyHostToDevice, st));
-    RES_HIP(hipMemcpyAsync(r->ys.p, y, (size_t)n * 4, hipMemcpyHostToDevice, st));
-    if (wt) RES_HIP(hipMemcpyAsync(r->ws.p, wt, (size_t)n * 4, hipMemcpyHostToDevice, st));
-    float l = 0.f;
-    if ((rc = run_batch(r, st, r->xs.p, r->ys.p, wt ? r->ws.p : nullptr, nullptr, n, 1.f, 1.f,
-                        0.f, &l)))
-        return rc;
-    RES_HIP(hipMemcpyAsync(grad, r->grad.p, P * 4, hipMemcpyDeviceToHost, st));
-    RES_HIP(hipStreamSynchronize(st));
-    if (loss) *loss = l;
+    // the kernel reads each sample once: straight from pinned memory, one pass
+    // over PCIe under its arithmetic (three copies from pageable memory and
+    // their waits took as long as all the kernels)
+    const size_t need = (size_t)n * (F + 1 + (wt ? 1 : 0));
+    const float *dx, *dy, *dw = nullptr;
+    if (need <= kGradDirect) {
+        if (need > r->h_in_cap) {
+            if (r->h_in) (void)hipHostFree(r->h_in);
+            r->h_in = nullptr;
+            r->h_in_cap = 0;
+            const size_t cap = std::min(kGradDirect, 2 * need);
+            if (hipHostMalloc((void **)&r->h_in, cap * sizeof(float), hipHostMallocDefault) !=
+                hipSuccess) {
+                r->h_in = nullptr;
+                return set_err(GSS_E_NOMEM, "pinned host allocation failed");
+            }
+            r->h_in_cap = cap;
+        }
+        std::memcpy(r->h_in, x, (size_t)n * F * 4);
+        std::memcpy(r->h_in + (size_t)n * F, y, (size_t)n * 4);
+        if (wt) std::memcpy(r->h_in + (size_t)n * (F + 1), wt, (size_t)n * 4);
+        dx = r->h_in;
+        dy = r->h_in + (size_t)n * F;
+        if (wt) dw = r->h_in + (size_t)n * (F + 1);
+    } else {
+        if ((rc = r->xs.reserve((size_t)n * F)) || (rc = r->ys.reserve(n)) ||
+            (rc = r->ws.reserve(n)))
+            return rc;
+        RES_HIP(hipMemcpyAsync(r->xs.p, x, (size_t)n * F * 4, hipMemcpyHostToDevice, st));
+        RES_HIP(hipMemcpyAsync(r->ys.p, y, (size_t)n * 4, hipMemcpyHostToDevice, st));
+        if (wt) RES_HIP(hipMemcpyAsync(r->ws.p, wt, (size_t)n * 4, hipMemcpyHostToDevice, st));
+        dx = r->xs.p;
+        dy = r->ys.p;
+        if (wt) dw = r->ws.p;
+    }
+    if ((rc = run_batch(r, st, dx, dy, dw, nullptr, n, 1.f, 1.f, 0.f, true))) return rc;
+    std::memcpy(grad, r->h_res, P * 4);
+    if (loss) *loss = r->h_res[P];
     return GSS_OK;
 }
 

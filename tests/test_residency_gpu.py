@@ -249,3 +249,25 @@ def test_learned_policy_gains_over_activity_policy():
     print(f"activity {act.hits_per_gb:.4e}, learned {lrn.hits_per_gb:.4e} hit pairs/GB", flush=True)
     assert lrn.reductions > 0 and act.reductions > 0
     assert lrn.hits_per_gb >= 1.02 * act.hits_per_gb
+
+
+@pytest.mark.parametrize("n, weighted", [(1, True), (63, False), (64, True), (65, True),
+                                         (16385, True), (310_000, True)])
+def test_mlp_gradient_at_tile_edges(engine_factory, n, weighted):
+    """Sample counts around the 64-sample tile, past one tile for each of the
+    256 blocks, and past what goes through pinned memory.  Every sum is a chain
+    of at most ~200 FP32 additions within a block and 256 blocks: relative
+    error at most ~500 * 2^-24 = 3e-5 of the gradient's norm."""
+    _, r = make_res(engine_factory)
+    rng = np.random.default_rng(50 + n)
+    p = rng.normal(0, 0.25, rs.PARAMS).astype(np.float32)
+    r.params = p
+    x = rng.normal(0, 1, (n, 12)).astype(np.float32)
+    y = (rng.random(n) < 0.3).astype(np.float32)
+    wt = (rng.random(n) + 0.5).astype(np.float32) if weighted else None
+    loss, g = r.grad(x, y, wt)
+    loss_ref, g_ref = ref.loss_and_grad(p, x, y, wt)
+    print(f"{n} samples: off by {np.linalg.norm(g - g_ref) / np.linalg.norm(g_ref):.2g}",
+          flush=True)
+    assert abs(loss - loss_ref) <= 3e-5 * abs(loss_ref)
+    assert np.linalg.norm(g - g_ref) <= 3e-5 * np.linalg.norm(g_ref)

@@ -52,6 +52,11 @@ constexpr size_t kDirectWords = 64 * 1024;
 
 namespace {
 
+// Steps of at most this many kernels are launched one by one, longer ones as a
+// graph.  Launching and waiting for 3 / 5 / 10 small kernels takes 17 / 22 / 38
+// us one by one and 37 / 35 / 38 us as a graph, the host's part 10 / 16 / 30 us
+// and 28 us.
+constexpr int kDirectLaunches = 8;
 // literals a step copies straight from its pinned staging
 constexpr int64_t kDirectLits = 16384;
 // steps staging at least this many bytes split their copies over the stage pool
@@ -280,9 +285,21 @@ struct DevBuf {
     bool async = false;
 };
 
+// The launches of a step beside its data (which they read from the device
+// header): see launch_step.
+struct StepPlan {
+    int blocks = 0, tp = 0;
+    bool serve = false, screen = false;
+    bool agg_full = false;   // screened: the entries are rebuilt from the table
+    bool agg_fused = false;  // screened: the applying and rolling kernels refresh them
+    bool staged = false;     // clauses are copied by a kernel of their own
+    bool bases = false;      // base updates and word loads
+    bool patches = false;
+};
+
 // One of the two ping-pong slots of batched steps: pinned staging the host
 // fills, the device copies the step's kernels read, this slot's hit buffer,
-// and the graph captured over exactly these buffers.
+// and graphs captured over exactly these buffers.
 struct StepSlot {
     Pinned<StepHeader> h_hdr;
     Pinned<BucketDesc> h_desc;
@@ -341,12 +358,7 @@ struct StepSlot {
     uint64_t worst_chunks = 0;
     bool settled = false;       // the step in flight is known to have kept its records
     bool records_lost = false;  // its recovery could not grow the buffer
-    // launch settings of the last submitted step's graph, for a recovery's
-    // re-run of its tail
-    int g_blocks = 0, g_tp = 0;
-    bool g_serve = false, g_screen = false;
-    bool g_agg_full = false;  // screened: the aggregate is rebuilt from the table
-    bool g_agg_fused = false; // screened: the applying and rolling kernels refresh it
+    StepPlan plan;  // the last submitted step's launches
     // Graphs captured over this slot's buffers, one per key (everything baked
     // in); a caller alternating between step forms (screened or not, rebuilt
     // aggregate or refreshed) replays them without capturing again.  The
@@ -355,19 +367,16 @@ struct StepSlot {
         std::vector<const void *> key;
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
-        int blocks = 0, tp = 0;
-        bool serve = false, screen = false, agg_full = false, staged = false;
-        uint64_t dense = 0;  // records it compacts into d_dense (0 = none)
         uint64_t used = 0;   // submit count at its last use
     };
     static constexpr size_t kGraphsPerSlot = 8;
     std::vector<StepGraph> graphs;
-    int cur = -1;  // graph of the slot's last submitted step
+    int cur = -1;  // graph of the slot's last submitted step (-1: launched directly)
     uint64_t submits = 0;
     hipEvent_t t0 = nullptr, t1 = nullptr;
     bool busy = false;
     bool serve = false;    // the slot's last step admitted requests from the serving ring
-    // the slot's graph holds the base-plane nodes (base updates, word loads)
+    // a graph of the slot holds the base-plane nodes (base updates, word loads)
     // and the patch node once a step of the slot needed them (then always:
     // a caller alternating between step kinds does not re-capture each time)
     bool g_bases = false, g_patches = false;
@@ -1698,7 +1707,7 @@ static ChunkArgs step_chunks(const StepSlot &sl, int rw) {
     c.fills = sl.d_fills.p;
     c.alloc = sl.d_alloc;
     c.cap = sl.chunk_cap;
-    c.waves = (uint32_t)sl.g_blocks * 4;
+    c.waves = (uint32_t)sl.plan.blocks * 4;
     c.rec_words = (uint32_t)rw;
     return c;
 }
@@ -1824,7 +1833,7 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     SweepArgs a{};
     a.buckets = sl.d_desc.p;
     a.dyn = &dh->nbuckets;  // {nbuckets, npasses}
-    a.task_passes = sl.g_tp;
+    a.task_passes = sl.plan.tp;
     a.table = e->table.p;
     a.valid = dh->valid;
     a.hits = (gss_hit *)sl.d_hits.p;
@@ -1834,12 +1843,12 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     a.sentinel = (uint32_t)(2 * e->vars) << kLitShift;
     a.rec_words = sl.rec_words;
     uint32_t *agg =
-        (sl.g_serve && e->serve_prefilter) || sl.g_screen ? e->serve_agg.p : nullptr;
+        (sl.plan.serve && e->serve_prefilter) || sl.plan.screen ? e->serve_agg.p : nullptr;
     a.agg = agg;
     a.agg_words = agg ? e->serve_agg_words.p : nullptr;
-    hipError_t he = launch_sweep(a, e->words, sl.g_blocks, s);
+    hipError_t he = launch_sweep(a, e->words, sl.plan.blocks, s);
     const ChunkArgs c = step_chunks(sl, sl.rec_words);
-    if (sl.g_serve) {
+    if (sl.plan.serve) {
         if (he == hipSuccess)
             he = launch_group_by_word(c, sl.d_wcount.p, sl.d_dense.p, sl.d_dense.cap, sl.h_group.p,
                                       sl.h_out.p, e->d_halt, s);
@@ -1850,7 +1859,7 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     end.ups = sl.d_ups.p;
     end.table = e->table.p;
     end.words = e->words;
-    end.agg = sl.g_agg_fused ? agg : nullptr;
+    end.agg = sl.plan.agg_fused ? agg : nullptr;
     end.halt = e->d_halt;
     end.out = sl.h_out.p;
     end.dense = (uint64_t *)sl.d_dense.p;
@@ -1858,32 +1867,15 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     end.host_words = kDirectWords;
     if (he == hipSuccess) he = launch_step_end(c, end, s);
     // screened steps keep the aggregate current through the roll forward
-    if (he == hipSuccess && sl.g_screen && !sl.g_agg_fused)
+    if (he == hipSuccess && sl.plan.screen && !sl.plan.agg_fused)
         he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, nullptr, false, e->words, agg, s);
     return he;
 }
 
-// Captures the step's fixed launch sequence over this slot's buffers into
-// graph entry g (whose previous graph, if any, is destroyed first).
-static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr, int blocks,
-                            int tp, bool serve, bool screen, bool agg_full, bool staged) {
-    if (gr.exec) (void)hipGraphExecDestroy(gr.exec);
-    if (gr.graph) (void)hipGraphDestroy(gr.graph);
-    gr.exec = nullptr;
-    gr.graph = nullptr;
-    gr.key.clear();
-    sl.g_blocks = blocks;
-    sl.g_tp = tp;
-    sl.g_serve = serve;
-    sl.g_screen = screen;
-    sl.g_agg_full = agg_full;
-    // at most 8 words: a word is its own screening group, so the kernels that
-    // write it know its entries (patches come after the updates: not then)
-    sl.g_agg_fused = screen && e->words <= 8 && !sl.g_patches;
-    if (!e->capture_stream)
-        HIP_TRY(hipStreamCreateWithFlags(&e->capture_stream, hipStreamNonBlocking));
-    hipStream_t cs = e->capture_stream;
-    HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+// The launches of a step of plan sl.plan over the slot's buffers, in order.
+static hipError_t launch_step(gss_engine *e, StepSlot &sl, hipStream_t cs) {
+    const StepPlan &pl = sl.plan;
+    const bool serve = pl.serve, screen = pl.screen;
     StepInArgs st{};
     st.h[kRegHeader] = (const uint32_t *)sl.h_hdr.p;
     st.h[kRegDesc] = (const uint32_t *)sl.h_desc.p;
@@ -1909,15 +1901,15 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     st.table = e->table.p;
     st.words = e->words;
     // updates come after base updates and word loads, where a step has them
-    st.apply = !sl.g_bases;
-    st.agg = sl.g_agg_fused && st.apply && !agg_full ? agg : nullptr;
+    st.apply = !pl.bases;
+    st.agg = pl.agg_fused && st.apply && !pl.agg_full ? agg : nullptr;
     st.agg_words = screen ? e->serve_agg_words.p : nullptr;
-    st.clauses = !staged;
+    st.clauses = !pl.staged;
     st.shift = kLitShift;
     hipError_t he = launch_step_in(st, cs);
-    if (he == hipSuccess && staged)
+    if (he == hipSuccess && pl.staged)
         he = launch_scatter_clauses(sl.d_cls.p, &dh->nclauses, sl.d_lits.p, kLitShift, cs);
-    if (he == hipSuccess && sl.g_bases)
+    if (he == hipSuccess && pl.bases)
         he = launch_base_apply_dyn(sl.d_bups.p, &dh->nbups, e->bases.p, e->bases_vw, cs);
     // serving: the published requests that fit are admitted here, on the
     // device, when the step starts (their loads, valid slots and counts)
@@ -1926,7 +1918,7 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     if (he == hipSuccess && serve) he = launch_serve_stage_patches(e->serve, dh, cs);
     // a serving step's words follow its loads and the rest are invalid in it,
     // so it writes whole table lines
-    if (he == hipSuccess && sl.g_bases)
+    if (he == hipSuccess && pl.bases)
         he = serve && e->words % 2 == 0
                  ? launch_words_load_lines(sl.d_loads.p, &dh->nloads, e->bases.p, e->bases_vw,
                                            e->table.p, e->words, e->vars, cs)
@@ -1937,20 +1929,47 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
                               e->serve_agg_words.p, cs);
     if (he == hipSuccess && !st.apply && !serve)
         he = launch_assig_apply_dyn(sl.d_ups.p, &dh->nups, e->table.p, e->words, cs);
-    if (he == hipSuccess && sl.g_patches)
+    if (he == hipSuccess && pl.patches)
         he = serve ? launch_serve_patch(e->serve, dh, e->table.p, e->words, agg, cs)
                    : launch_assig_patch_dyn(sl.d_patches.p, &dh->npatches, e->table.p, e->words,
                                             cs);
     // batched steps: the aggregate of the table as the sweep will read it,
     // rebuilt, or refreshed where this step's updates and patches changed it
-    if (he == hipSuccess && screen && agg_full)
+    if (he == hipSuccess && screen && pl.agg_full)
         he = launch_table_agg(e->table.p, dh, e->vars, e->words, agg, cs);
     else if (he == hipSuccess && screen && !st.agg)
-        he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, sl.d_patches.p, sl.g_patches,
+        he = launch_table_agg_update(e->table.p, dh, sl.d_ups.p, sl.d_patches.p, pl.patches,
                                      e->words, agg, cs);
     if (he == hipSuccess) he = launch_step_tail(e, sl, cs);
+    return he;
+}
+
+// Launches launch_step makes for a plan.
+static int step_launches(const gss_engine *e, const StepPlan &p) {
+    const bool agg = (p.serve && e->serve_prefilter) || p.screen;
+    int n = 3 + p.staged + 2 * p.bases + p.patches;  // in, sweep, end
+    if (p.serve) return n + 3 + agg;                 // admission, patches, word count
+    if (p.bases) n++;                                // the updates, after the loads
+    if (p.screen && (p.agg_full || p.bases || !p.agg_fused)) n++;
+    if (p.screen && !p.agg_fused) n++;
+    return n;
+}
+
+// Captures launch_step into graph entry gr (whose previous graph, if any, is
+// destroyed first).
+static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr) {
+    if (gr.exec) (void)hipGraphExecDestroy(gr.exec);
+    if (gr.graph) (void)hipGraphDestroy(gr.graph);
+    gr.exec = nullptr;
+    gr.graph = nullptr;
+    gr.key.clear();
+    if (!e->capture_stream)
+        HIP_TRY(hipStreamCreateWithFlags(&e->capture_stream, hipStreamNonBlocking));
+    hipStream_t cs = e->capture_stream;
+    HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+    const hipError_t he = launch_step(e, sl, cs);
     hipGraph_t g = nullptr;
-    hipError_t he2 = hipStreamEndCapture(cs, &g);
+    const hipError_t he2 = hipStreamEndCapture(cs, &g);
     if (he != hipSuccess) {
         if (g) (void)hipGraphDestroy(g);
         return set_err(GSS_E_HIP, "step capture failed: %s", hipGetErrorString(he));
@@ -1958,15 +1977,13 @@ static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr
     if (he2 != hipSuccess) return set_err(GSS_E_HIP, "step capture: %s", hipGetErrorString(he2));
     gr.graph = g;
     HIP_TRY(hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0));
-    gr.blocks = blocks;
-    gr.tp = tp;
-    gr.serve = serve;
-    gr.screen = screen;
-    gr.agg_full = agg_full;
-    gr.staged = staged;
-    gr.dense = sl.d_dense.cap;
     e->graph_captures.fetch_add(1, std::memory_order_relaxed);
     return GSS_OK;
+}
+
+// Runs the slot's step (again): its launches, or its graph.
+static hipError_t run_step(gss_engine *e, StepSlot &sl, hipStream_t s) {
+    return sl.cur >= 0 ? hipGraphLaunch(sl.graphs[sl.cur].exec, s) : launch_step(e, sl, s);
 }
 
 // Recovers step `at` of the steps in flight, whose sweep claimed `used`
@@ -2003,12 +2020,12 @@ static int recover_step(gss_engine *e, size_t at, uint32_t used) {
         // no room: only roll the table forward
         HIP_TRY(launch_assig_roll_dyn(sl.d_ups.p, &sl.d_hdr.p->nups, e->table.p, e->words,
                                       sl.d_hdr.p->last_pos, es));
-        if (sl.g_screen)
+        if (sl.plan.screen)
             HIP_TRY(launch_table_agg_update(e->table.p, sl.d_hdr.p, sl.d_ups.p, nullptr, false,
                                             e->words, e->serve_agg.p, es));
     } else {
         HIP_TRY(launch_reset_u32(sl.d_alloc, 2, es));
-        if (sl.g_serve) HIP_TRY(launch_reset_u32(sl.d_wcount.p, 2 * GSS_MAX_WORDS, es));
+        if (sl.plan.serve) HIP_TRY(launch_reset_u32(sl.d_wcount.p, 2 * GSS_MAX_WORDS, es));
         HIP_TRY(launch_step_tail(e, sl, es));
     }
     HIP_TRY(hipEventRecord(sl.t1, es));
@@ -2016,11 +2033,11 @@ static int recover_step(gss_engine *e, size_t at, uint32_t used) {
     for (size_t i = at + 1; i < e->inflight.size(); i++) {
         StepSlot &nx = e->slots[e->inflight[i]];
         HIP_TRY(hipEventRecord(nx.t0, es));
-        HIP_TRY(hipGraphLaunch(nx.graphs[nx.cur].exec, es));
+        HIP_TRY(run_step(e, nx, es));
         HIP_TRY(hipEventRecord(nx.t1, es));
         nx.settled = false;
     }
-    e->step_hit_want = std::max(e->step_hit_want, chunks_wanted(used, sl.g_blocks));
+    e->step_hit_want = std::max(e->step_hit_want, chunks_wanted(used, sl.plan.blocks));
     e->step_recoveries++;
     return sl.records_lost ? set_err(GSS_E_NOMEM, "a step's hit buffer overflowed (%u chunks) and "
                                                   "could not grow: its records are lost",
@@ -2426,58 +2443,72 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     if (!sl.d_alloc) HIP_TRY(hipMalloc((void **)&sl.d_alloc, 64));
     if (!sl.t0) HIP_TRY(hipEventCreate(&sl.t0));
     if (!sl.t1) HIP_TRY(hipEventCreate(&sl.t1));
-    // ---- graph over exactly these buffers and settings
-    const int tp = task_passes(e, use_agg);
+    // ---- the step's launches
+    StepPlan &pl = sl.plan;
+    pl.blocks = blocks;
+    pl.tp = task_passes(e, use_agg);
+    pl.serve = serve;
+    pl.screen = screen;
+    pl.agg_full = agg_full;
     // Few literals go straight from the staging to their rows (32-byte reads
     // over PCIe); more are copied first and scattered by a kernel of its own.
-    const bool staged = total > kDirectLits;
-    sl.g_bases |= serve || n_bups > 0 || n_loads > 0;
-    sl.g_patches |= serve || n_patches > 0;
-    std::vector<const void *> key = {
-        sl.h_hdr.p, sl.h_desc.p, sl.h_cls.p, sl.h_lits.p, sl.h_ups.p, sl.h_out.p,
-        sl.h_patches.p, sl.h_bups.p, sl.h_loads.p,
-        sl.d_hdr.p, sl.d_desc.p, sl.d_cls.p, sl.d_lits.p, sl.d_ups.p, sl.d_hits.p,
-        sl.d_patches.p, sl.d_bups.p, sl.d_loads.p,
-        sl.d_fills.p, sl.d_dense.p, (const void *)(intptr_t)sl.d_dense.cap,
-        e->table.p, e->bases.p, (const void *)(intptr_t)e->bases_vw,
-        (const void *)(intptr_t)W, (const void *)(intptr_t)e->vars,
-        (const void *)(intptr_t)blocks, (const void *)(intptr_t)tp,
-        (const void *)(intptr_t)sl.chunk_cap, (const void *)(intptr_t)sl.rec_words,
-        (const void *)(intptr_t)serve, sl.h_report.p, serve ? (const void *)e->serve.reqs : nullptr,
-        sl.h_group.p, sl.d_wcount.p, (const void *)(intptr_t)(sl.g_bases + 2 * sl.g_patches),
-        use_agg ? (const void *)e->serve_agg.p : nullptr,
-        use_agg ? (const void *)e->serve_agg_words.p : nullptr,
-        (const void *)(intptr_t)((screen ? (agg_full ? 1 : 2) : 0) + (staged ? 4 : 0))};
-    int gi = -1;
-    for (size_t i = 0; i < sl.graphs.size(); i++)
-        if (sl.graphs[i].exec && sl.graphs[i].key == key) gi = (int)i;
-    if (gi < 0) {
-        if (sl.graphs.size() < StepSlot::kGraphsPerSlot) {
-            sl.graphs.emplace_back();
-            gi = (int)sl.graphs.size() - 1;
-        } else {
-            gi = 0;
-            for (size_t i = 1; i < sl.graphs.size(); i++)
-                if (sl.graphs[i].used < sl.graphs[gi].used) gi = (int)i;
+    pl.staged = total > kDirectLits;
+    pl.bases = serve || n_bups > 0 || n_loads > 0;
+    pl.patches = serve || n_patches > 0;
+    sl.g_bases |= pl.bases;
+    sl.g_patches |= pl.patches;
+    auto fused = [&] {
+        // at most 8 words: a word is its own screening group, so the kernels
+        // that write it know its entries (patches come after the updates: not
+        // then)
+        pl.agg_fused = screen && W <= 8 && !pl.patches;
+    };
+    fused();
+    sl.step_dense = sl.d_dense.cap;
+    sl.cur = -1;
+    if (step_launches(e, pl) > kDirectLaunches) {
+        // a graph over exactly these buffers and settings
+        pl.bases = sl.g_bases;
+        pl.patches = sl.g_patches;
+        fused();
+        std::vector<const void *> key = {
+            sl.h_hdr.p, sl.h_desc.p, sl.h_cls.p, sl.h_lits.p, sl.h_ups.p, sl.h_out.p,
+            sl.h_patches.p, sl.h_bups.p, sl.h_loads.p,
+            sl.d_hdr.p, sl.d_desc.p, sl.d_cls.p, sl.d_lits.p, sl.d_ups.p, sl.d_hits.p,
+            sl.d_patches.p, sl.d_bups.p, sl.d_loads.p,
+            sl.d_fills.p, sl.d_dense.p, (const void *)(intptr_t)sl.d_dense.cap,
+            e->table.p, e->bases.p, (const void *)(intptr_t)e->bases_vw,
+            (const void *)(intptr_t)W, (const void *)(intptr_t)e->vars,
+            (const void *)(intptr_t)pl.blocks, (const void *)(intptr_t)pl.tp,
+            (const void *)(intptr_t)sl.chunk_cap, (const void *)(intptr_t)sl.rec_words,
+            (const void *)(intptr_t)serve, sl.h_report.p, serve ? (const void *)e->serve.reqs : nullptr,
+            sl.h_group.p, sl.d_wcount.p, (const void *)(intptr_t)(pl.bases + 2 * pl.patches),
+            use_agg ? (const void *)e->serve_agg.p : nullptr,
+            use_agg ? (const void *)e->serve_agg_words.p : nullptr,
+            (const void *)(intptr_t)((screen ? (agg_full ? 1 : 2) : 0) + (pl.staged ? 4 : 0))};
+        int gi = -1;
+        for (size_t i = 0; i < sl.graphs.size(); i++)
+            if (sl.graphs[i].exec && sl.graphs[i].key == key) gi = (int)i;
+        if (gi < 0) {
+            if (sl.graphs.size() < StepSlot::kGraphsPerSlot) {
+                sl.graphs.emplace_back();
+                gi = (int)sl.graphs.size() - 1;
+            } else {
+                gi = 0;
+                for (size_t i = 1; i < sl.graphs.size(); i++)
+                    if (sl.graphs[i].used < sl.graphs[gi].used) gi = (int)i;
+            }
+            StepSlot::StepGraph &gr = sl.graphs[gi];
+            const auto t0 = std::chrono::steady_clock::now();
+            if ((rc = build_step_graph(e, sl, gr))) return rc;
+            gss::log_stall("step graph capture", std::chrono::duration<double, std::milli>(
+                                                      std::chrono::steady_clock::now() - t0)
+                                                      .count());
+            gr.key = key;
         }
-        StepSlot::StepGraph &gr = sl.graphs[gi];
-        const auto t0 = std::chrono::steady_clock::now();
-        if ((rc = build_step_graph(e, sl, gr, blocks, tp, serve, screen, agg_full, staged))) return rc;
-        gss::log_stall("step graph capture", std::chrono::duration<double, std::milli>(
-                                                  std::chrono::steady_clock::now() - t0)
-                                                  .count());
-        gr.key = key;
+        sl.graphs[gi].used = ++sl.submits;
+        sl.cur = gi;
     }
-    StepSlot::StepGraph &gr = sl.graphs[gi];
-    gr.used = ++sl.submits;
-    sl.cur = gi;
-    sl.g_blocks = gr.blocks;
-    sl.g_tp = gr.tp;
-    sl.g_serve = gr.serve;
-    sl.g_screen = gr.screen;
-    sl.g_agg_full = gr.agg_full;
-    sl.g_agg_fused = gr.screen && W <= 8 && !sl.g_patches;
-    sl.step_dense = gr.dense;
     // ---- stage this step (the slot is idle) and commit it to the DB: one
     // record per clause (the device copies it to its bucket row)
     {
@@ -2554,7 +2585,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     e->state_version++;
     e->table_agg_at = screen ? e->state_version : 0;
     HIP_TRY(hipEventRecord(sl.t0, e->stream));
-    HIP_TRY(hipGraphLaunch(sl.graphs[sl.cur].exec, e->stream));
+    HIP_TRY(run_step(e, sl, e->stream));
     HIP_TRY(hipEventRecord(sl.t1, e->stream));
     sl.busy = true;
     sl.settled = false;
@@ -2614,7 +2645,7 @@ int gss_step_wait(gss_engine *e, int64_t *n_hits, float *step_ms) {
                              sl.chunk_cap);
     }
     // the next steps' buffers hold twice the most chunks a step has claimed
-    e->step_hit_want = std::max(e->step_hit_want, chunks_wanted(used, sl.g_blocks));
+    e->step_hit_want = std::max(e->step_hit_want, chunks_wanted(used, sl.plan.blocks));
     const int64_t tot = (int64_t)((uint64_t)sl.h_out.p[1] | ((uint64_t)sl.h_out.p[2] << 32));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, sl.t0, sl.t1));

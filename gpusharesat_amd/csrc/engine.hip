@@ -52,11 +52,6 @@ constexpr size_t kDirectWords = 64 * 1024;
 
 namespace {
 
-// Steps of at most this many kernels are launched one by one, longer ones as a
-// graph.  Launching and waiting for 3 / 5 / 10 small kernels takes 17 / 22 / 38
-// us one by one and 37 / 35 / 38 us as a graph, the host's part 10 / 16 / 30 us
-// and 28 us.
-constexpr int kDirectLaunches = 8;
 // literals a step copies straight from its pinned staging
 constexpr int64_t kDirectLits = 16384;
 // steps staging at least this many bytes split their copies over the stage pool
@@ -293,13 +288,12 @@ struct StepPlan {
     bool agg_full = false;   // screened: the entries are rebuilt from the table
     bool agg_fused = false;  // screened: the applying and rolling kernels refresh them
     bool staged = false;     // clauses are copied by a kernel of their own
-    bool bases = false;      // base updates and word loads
+    bool loads = false;      // word loads
     bool patches = false;
 };
 
 // One of the two ping-pong slots of batched steps: pinned staging the host
-// fills, the device copies the step's kernels read, this slot's hit buffer,
-// and graphs captured over exactly these buffers.
+// fills, the device copies the step's kernels read, and this slot's hit buffer.
 struct StepSlot {
     Pinned<StepHeader> h_hdr;
     Pinned<BucketDesc> h_desc;
@@ -316,17 +310,16 @@ struct StepSlot {
     DevBuf<uint32_t> d_lits;
     DevBuf<gss_var_update> d_ups;
     DevBuf<gss_var_patch> d_patches;
-    DevBuf<gss_base_update> d_bups;
     DevBuf<gss_word_load> d_loads;
     DevBuf<uint64_t> d_hits;     // chunk_cap chunks of kHitChunk records of rec_words words
     DevBuf<uint32_t> d_fills;
     DevBuf<gss_hit> d_dense;     // compacted records of the last waited step
-    uint64_t dense_want = 0;     // records the graph's compaction should hold
-    uint64_t step_dense = 0;     // records the last submitted step's graph compacts into
+    uint64_t dense_want = 0;     // records the step's compaction should hold
+    uint64_t step_dense = 0;     // records the last submitted step compacts into
                                  // d_dense (0 = none)
     // The records of a waited step go to a pinned host buffer on the slot's
     // own stream as soon as gss_step_wait has seen the step end (one DMA copy
-    // when the graph compacted them); the slot's next graph waits for that
+    // when the step compacted them); the slot's next step waits for that
     // copy on the engine stream, so the records stay valid until the slot's
     // next step is waited and the host can stage that step while they travel.
     // With h_n > 1 buffers (serving engines) the waits rotate through them,
@@ -359,27 +352,9 @@ struct StepSlot {
     bool settled = false;       // the step in flight is known to have kept its records
     bool records_lost = false;  // its recovery could not grow the buffer
     StepPlan plan;  // the last submitted step's launches
-    // Graphs captured over this slot's buffers, one per key (everything baked
-    // in); a caller alternating between step forms (screened or not, rebuilt
-    // aggregate or refreshed) replays them without capturing again.  The
-    // least recently used one goes when a ninth is needed.
-    struct StepGraph {
-        std::vector<const void *> key;
-        hipGraph_t graph = nullptr;
-        hipGraphExec_t exec = nullptr;
-        uint64_t used = 0;   // submit count at its last use
-    };
-    static constexpr size_t kGraphsPerSlot = 8;
-    std::vector<StepGraph> graphs;
-    int cur = -1;  // graph of the slot's last submitted step (-1: launched directly)
-    uint64_t submits = 0;
     hipEvent_t t0 = nullptr, t1 = nullptr;
     bool busy = false;
     bool serve = false;    // the slot's last step admitted requests from the serving ring
-    // a graph of the slot holds the base-plane nodes (base updates, word loads)
-    // and the patch node once a step of the slot needed them (then always:
-    // a caller alternating between step kinds does not re-capture each time)
-    bool g_bases = false, g_patches = false;
     Pinned<ServeReport> h_report;  // what that step admitted (serving steps)
     // serving steps: records made dense grouped by assignment word, and where
     // each word's records start (h_group[w], [64] = all, [65] = 1 if grouped)
@@ -414,7 +389,6 @@ struct gss_engine {
     int device = 0;
     int cu = 0;
     hipStream_t stream = nullptr;
-    hipStream_t capture_stream = nullptr;  // records step graphs (never executes work)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 
     std::vector<Bucket> buckets;  // index = clause length
@@ -534,7 +508,6 @@ struct gss_engine {
     int64_t last_step_hits = 0;
     uint32_t last_step_chunks = 0;
     float last_step_ms = 0.f;
-    std::atomic<int64_t> graph_captures{0};  // step graphs captured (read by other threads)
     // Step hit buffers are sized by the records steps have made: twice the
     // most chunks a step claimed (at least a floor), never beyond the worst
     // case.  A step that overflows its buffer sets d_halt (device, zero while
@@ -766,10 +739,6 @@ int gss_engine_destroy(gss_engine *e) {
     e->prefetch.reset();  // its thread may be filling a slot's spare buffer
     for (StepSlot &sl : e->slots) {
         if (sl.copy) (void)hipStreamSynchronize(sl.copy);
-        for (StepSlot::StepGraph &g : sl.graphs) {
-            if (g.exec) (void)hipGraphExecDestroy(g.exec);
-            if (g.graph) (void)hipGraphDestroy(g.graph);
-        }
         if (sl.t0) (void)hipEventDestroy(sl.t0);
         if (sl.t1) (void)hipEventDestroy(sl.t1);
         if (sl.ev_copied) (void)hipEventDestroy(sl.ev_copied);
@@ -781,7 +750,6 @@ int gss_engine_destroy(gss_engine *e) {
         sl.d_lits.release();
         sl.d_ups.release();
         sl.d_patches.release();
-        sl.d_bups.release();
         sl.d_loads.release();
         sl.d_hits.release();
         sl.d_fills.release();
@@ -815,7 +783,6 @@ int gss_engine_destroy(gss_engine *e) {
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->stream) (void)hipStreamDestroy(e->stream);
-    if (e->capture_stream) (void)hipStreamDestroy(e->capture_stream);
     delete e;
     return GSS_OK;
 }
@@ -1692,8 +1659,7 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
 /* ---- batched steps -------------------------------------------------------- */
 
 // Persistent grid of a step: the resident maximum of 4-wave blocks, whatever
-// the tasks (waves without a task end at once), so a growing DB never
-// re-captures the graph for its grid.
+// the tasks (waves without a task end at once).
 static int step_blocks(gss_engine *e, int mode) {
     int per_cu = resident_blocks(e, mode);
     if (e->tune_waves_per_cu > 0) per_cu = std::max(1, std::min(per_cu, e->tune_waves_per_cu / 4));
@@ -1713,8 +1679,8 @@ static ChunkArgs step_chunks(const StepSlot &sl, int rw) {
 }
 
 // Queues the copy of a waited step's `total` records to the slot's pinned
-// h_hits on the slot's stream: one DMA copy when the graph made
-// them dense, else a compaction first (and the next capture's dense buffer is
+// h_hits on the slot's stream: one DMA copy when the step made
+// them dense, else a compaction first (and the next step's dense buffer is
 // sized for this volume).
 static int queue_records_copy(gss_engine *e, StepSlot &sl, int64_t total) {
     int rc;
@@ -1822,7 +1788,7 @@ static void note_hit_chunks(gss_engine *e) {
 }
 
 // The part of a step after its table updates, over the slot's buffers and
-// the settings of its graph: the sweep, then the roll forward (held back if
+// its plan: the sweep, then the roll forward (held back if
 // the records overflowed), the counts to the host and the records made dense
 // on the device, so that reading them on the host is one DMA copy (no compute
 // units taken from the next step's sweep) or, for few, none at all; serving
@@ -1872,12 +1838,15 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     return he;
 }
 
-// The launches of a step of plan sl.plan over the slot's buffers, in order.
+// The launches of a step of plan sl.plan over the slot's buffers, in order: 3
+// for a plain step, 6 for a serving one, at most 9.  One by one: launching and
+// waiting for 3 / 5 / 10 small kernels takes 17 / 22 / 38 us so and 37 / 35 / 38
+// us as a captured graph, the host's part 10 / 16 / 30 us and 28 us.
 static hipError_t launch_step(gss_engine *e, StepSlot &sl, hipStream_t cs) {
     const StepPlan &pl = sl.plan;
     const bool serve = pl.serve, screen = pl.screen;
     StepInArgs st{};
-    st.h[kRegHeader] = (const uint32_t *)sl.h_hdr.p;
+    st.header = *sl.h_hdr.p;
     st.h[kRegDesc] = (const uint32_t *)sl.h_desc.p;
     st.h[kRegClauses] = (const uint32_t *)sl.h_cls.p;
     st.h[kRegLits] = sl.h_lits.p;
@@ -1891,7 +1860,6 @@ static hipError_t launch_step(gss_engine *e, StepSlot &sl, hipStream_t cs) {
     st.d[kRegLits] = sl.d_lits.p;
     st.d[kRegUps] = (uint32_t *)sl.d_ups.p;
     st.d[kRegPatches] = (uint32_t *)sl.d_patches.p;
-    st.d[kRegBaseUps] = (uint32_t *)sl.d_bups.p;
     st.d[kRegLoads] = (uint32_t *)sl.d_loads.p;
     st.halt = e->d_halt;
     StepHeader *dh = sl.d_hdr.p;
@@ -1900,33 +1868,27 @@ static hipError_t launch_step(gss_engine *e, StepSlot &sl, hipStream_t cs) {
     st.counts = serve ? sl.d_wcount.p : nullptr;
     st.table = e->table.p;
     st.words = e->words;
-    // updates come after base updates and word loads, where a step has them
-    st.apply = !pl.bases;
+    // updates come after word loads, where a step has them
+    st.apply = !pl.loads;
     st.agg = pl.agg_fused && st.apply && !pl.agg_full ? agg : nullptr;
     st.agg_words = screen ? e->serve_agg_words.p : nullptr;
     st.clauses = !pl.staged;
     st.shift = kLitShift;
+    st.bases = e->bases.p;
+    st.bases_vw = e->bases_vw;
+    if (serve) {  // the published requests that fit are admitted when the step starts
+        st.serve = e->serve;
+        st.report = sl.h_report.p;
+    }
     hipError_t he = launch_step_in(st, cs);
     if (he == hipSuccess && pl.staged)
         he = launch_scatter_clauses(sl.d_cls.p, &dh->nclauses, sl.d_lits.p, kLitShift, cs);
-    if (he == hipSuccess && pl.bases)
-        he = launch_base_apply_dyn(sl.d_bups.p, &dh->nbups, e->bases.p, e->bases_vw, cs);
-    // serving: the published requests that fit are admitted here, on the
-    // device, when the step starts (their loads, valid slots and counts)
     if (he == hipSuccess && serve)
-        he = launch_serve_admit(e->serve, dh, sl.d_loads.p, sl.h_report.p, e->words, cs);
-    if (he == hipSuccess && serve) he = launch_serve_stage_patches(e->serve, dh, cs);
-    // a serving step's words follow its loads and the rest are invalid in it,
-    // so it writes whole table lines
-    if (he == hipSuccess && pl.bases)
-        he = serve && e->words % 2 == 0
-                 ? launch_words_load_lines(sl.d_loads.p, &dh->nloads, e->bases.p, e->bases_vw,
-                                           e->table.p, e->words, e->vars, cs)
-                 : launch_words_load_dyn(sl.d_loads.p, &dh->nloads, e->bases.p, e->bases_vw,
-                                         e->table.p, e->words, e->vars, cs);
-    if (he == hipSuccess && agg && serve)
-        he = launch_serve_agg(e->serve, dh, sl.d_loads.p, e->bases.p, e->bases_vw, e->vars, agg,
-                              e->serve_agg_words.p, cs);
+        he = launch_serve_load(e->serve, dh, sl.d_loads.p, e->bases.p, e->bases_vw, e->table.p,
+                               e->words, e->vars, agg, e->serve_agg_words.p, cs);
+    else if (he == hipSuccess && pl.loads)
+        he = launch_words_load_dyn(sl.d_loads.p, &dh->nloads, e->bases.p, e->bases_vw, e->table.p,
+                                   e->words, e->vars, cs);
     if (he == hipSuccess && !st.apply && !serve)
         he = launch_assig_apply_dyn(sl.d_ups.p, &dh->nups, e->table.p, e->words, cs);
     if (he == hipSuccess && pl.patches)
@@ -1944,51 +1906,9 @@ static hipError_t launch_step(gss_engine *e, StepSlot &sl, hipStream_t cs) {
     return he;
 }
 
-// Launches launch_step makes for a plan.
-static int step_launches(const gss_engine *e, const StepPlan &p) {
-    const bool agg = (p.serve && e->serve_prefilter) || p.screen;
-    int n = 3 + p.staged + 2 * p.bases + p.patches;  // in, sweep, end
-    if (p.serve) return n + 3 + agg;                 // admission, patches, word count
-    if (p.bases) n++;                                // the updates, after the loads
-    if (p.screen && (p.agg_full || p.bases || !p.agg_fused)) n++;
-    if (p.screen && !p.agg_fused) n++;
-    return n;
-}
-
-// Captures launch_step into graph entry gr (whose previous graph, if any, is
-// destroyed first).
-static int build_step_graph(gss_engine *e, StepSlot &sl, StepSlot::StepGraph &gr) {
-    if (gr.exec) (void)hipGraphExecDestroy(gr.exec);
-    if (gr.graph) (void)hipGraphDestroy(gr.graph);
-    gr.exec = nullptr;
-    gr.graph = nullptr;
-    gr.key.clear();
-    if (!e->capture_stream)
-        HIP_TRY(hipStreamCreateWithFlags(&e->capture_stream, hipStreamNonBlocking));
-    hipStream_t cs = e->capture_stream;
-    HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    const hipError_t he = launch_step(e, sl, cs);
-    hipGraph_t g = nullptr;
-    const hipError_t he2 = hipStreamEndCapture(cs, &g);
-    if (he != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return set_err(GSS_E_HIP, "step capture failed: %s", hipGetErrorString(he));
-    }
-    if (he2 != hipSuccess) return set_err(GSS_E_HIP, "step capture: %s", hipGetErrorString(he2));
-    gr.graph = g;
-    HIP_TRY(hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0));
-    e->graph_captures.fetch_add(1, std::memory_order_relaxed);
-    return GSS_OK;
-}
-
-// Runs the slot's step (again): its launches, or its graph.
-static hipError_t run_step(gss_engine *e, StepSlot &sl, hipStream_t s) {
-    return sl.cur >= 0 ? hipGraphLaunch(sl.graphs[sl.cur].exec, s) : launch_step(e, sl, s);
-}
-
 // Recovers step `at` of the steps in flight, whose sweep claimed `used`
 // chunks, more than its buffer held (the steps before it kept their
-// records).  Its graph left the table as the sweep read it and halted the
+// records).  It left the table as the sweep read it and halted the
 // engine, so the later step in flight (if any) staged nothing.  Grows the
 // buffer to what the sweep claimed, re-runs the step's sweep and what follows
 // it, and replays the later step.  If the buffer cannot grow, the table
@@ -2033,7 +1953,7 @@ static int recover_step(gss_engine *e, size_t at, uint32_t used) {
     for (size_t i = at + 1; i < e->inflight.size(); i++) {
         StepSlot &nx = e->slots[e->inflight[i]];
         HIP_TRY(hipEventRecord(nx.t0, es));
-        HIP_TRY(run_step(e, nx, es));
+        HIP_TRY(launch_step(e, nx, es));
         HIP_TRY(hipEventRecord(nx.t1, es));
         nx.settled = false;
     }
@@ -2127,10 +2047,6 @@ int gss::engine_set_record_buffers(gss_engine *e, int n) {
     return GSS_OK;
 }
 
-int64_t gss::engine_graph_captures(const gss_engine *e) {
-    return e ? e->graph_captures.load(std::memory_order_relaxed) : 0;
-}
-
 int gss::engine_serve_attach(gss_engine *e, const ServeReq *reqs, uint32_t req_cap,
                              const gss_var_patch *patches, uint64_t patch_cap,
                              const uint64_t *head) {
@@ -2162,7 +2078,7 @@ int gss::step_word_groups(gss_engine *e, uint64_t *offs, bool *grouped) {
     if (!e || !offs || !grouped) return set_err(GSS_E_INVAL, "null argument");
     if (e->last_step_slot < 0) return set_err(GSS_E_STATE, "no waited step");
     const StepSlot &sl = e->slots[e->last_step_slot];
-    // grouped only if the graph's dense buffer held them (else the records
+    // grouped only if the step's dense buffer held them (else the records
     // reached the host in chunk order)
     *grouped = sl.serve && sl.h_group.p && sl.rec_total > 0 &&
                (uint64_t)sl.rec_total <= sl.step_dense && sl.h_group.p[GSS_MAX_WORDS + 1] == 1;
@@ -2382,7 +2298,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         (rc = sl.h_bups.reserve(std::max<int64_t>(n_bups, 1))) ||
         (rc = sl.h_loads.reserve(std::max<int64_t>(n_loads, 1))))
         return rc;
-    // the slot's device copies are read only by its own graph, on the engine
+    // the slot's device copies are read only by its own step, on the engine
     // stream: they grow in stream order, without stalling the other slot.
     // The copy of this slot's previous records (its own stream) still reads
     // d_hits and d_dense: the engine stream waits for it before anything of
@@ -2412,7 +2328,6 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         (rc = sl.d_ups.reserve_async(sl.h_ups.cap, es)) ||
         (rc = sl.d_desc.reserve_async(sl.h_desc.cap, es)) ||
         (rc = sl.d_patches.reserve_async(sl.h_patches.cap, es)) ||
-        (rc = sl.d_bups.reserve_async(sl.h_bups.cap, es)) ||
         (rc = sl.d_loads.reserve_async(std::max<size_t>(sl.h_loads.cap, GSS_MAX_WORDS), es)))
         return rc;
     // The hit buffer holds chunks of records of this step's form, as many as
@@ -2453,62 +2368,12 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     // Few literals go straight from the staging to their rows (32-byte reads
     // over PCIe); more are copied first and scattered by a kernel of its own.
     pl.staged = total > kDirectLits;
-    pl.bases = serve || n_bups > 0 || n_loads > 0;
+    pl.loads = serve || n_loads > 0;
     pl.patches = serve || n_patches > 0;
-    sl.g_bases |= pl.bases;
-    sl.g_patches |= pl.patches;
-    auto fused = [&] {
-        // at most 8 words: a word is its own screening group, so the kernels
-        // that write it know its entries (patches come after the updates: not
-        // then)
-        pl.agg_fused = screen && W <= 8 && !pl.patches;
-    };
-    fused();
+    // at most 8 words: a word is its own screening group, so the kernels that
+    // write it know its entries (patches come after the updates: not then)
+    pl.agg_fused = screen && W <= 8 && !pl.patches;
     sl.step_dense = sl.d_dense.cap;
-    sl.cur = -1;
-    if (step_launches(e, pl) > kDirectLaunches) {
-        // a graph over exactly these buffers and settings
-        pl.bases = sl.g_bases;
-        pl.patches = sl.g_patches;
-        fused();
-        std::vector<const void *> key = {
-            sl.h_hdr.p, sl.h_desc.p, sl.h_cls.p, sl.h_lits.p, sl.h_ups.p, sl.h_out.p,
-            sl.h_patches.p, sl.h_bups.p, sl.h_loads.p,
-            sl.d_hdr.p, sl.d_desc.p, sl.d_cls.p, sl.d_lits.p, sl.d_ups.p, sl.d_hits.p,
-            sl.d_patches.p, sl.d_bups.p, sl.d_loads.p,
-            sl.d_fills.p, sl.d_dense.p, (const void *)(intptr_t)sl.d_dense.cap,
-            e->table.p, e->bases.p, (const void *)(intptr_t)e->bases_vw,
-            (const void *)(intptr_t)W, (const void *)(intptr_t)e->vars,
-            (const void *)(intptr_t)pl.blocks, (const void *)(intptr_t)pl.tp,
-            (const void *)(intptr_t)sl.chunk_cap, (const void *)(intptr_t)sl.rec_words,
-            (const void *)(intptr_t)serve, sl.h_report.p, serve ? (const void *)e->serve.reqs : nullptr,
-            sl.h_group.p, sl.d_wcount.p, (const void *)(intptr_t)(pl.bases + 2 * pl.patches),
-            use_agg ? (const void *)e->serve_agg.p : nullptr,
-            use_agg ? (const void *)e->serve_agg_words.p : nullptr,
-            (const void *)(intptr_t)((screen ? (agg_full ? 1 : 2) : 0) + (pl.staged ? 4 : 0))};
-        int gi = -1;
-        for (size_t i = 0; i < sl.graphs.size(); i++)
-            if (sl.graphs[i].exec && sl.graphs[i].key == key) gi = (int)i;
-        if (gi < 0) {
-            if (sl.graphs.size() < StepSlot::kGraphsPerSlot) {
-                sl.graphs.emplace_back();
-                gi = (int)sl.graphs.size() - 1;
-            } else {
-                gi = 0;
-                for (size_t i = 1; i < sl.graphs.size(); i++)
-                    if (sl.graphs[i].used < sl.graphs[gi].used) gi = (int)i;
-            }
-            StepSlot::StepGraph &gr = sl.graphs[gi];
-            const auto t0 = std::chrono::steady_clock::now();
-            if ((rc = build_step_graph(e, sl, gr))) return rc;
-            gss::log_stall("step graph capture", std::chrono::duration<double, std::milli>(
-                                                      std::chrono::steady_clock::now() - t0)
-                                                      .count());
-            gr.key = key;
-        }
-        sl.graphs[gi].used = ++sl.submits;
-        sl.cur = gi;
-    }
     // ---- stage this step (the slot is idle) and commit it to the DB: one
     // record per clause (the device copies it to its bucket row)
     {
@@ -2575,7 +2440,6 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     h.region_words[kRegLits] = total;
     h.region_words[kRegUps] = n_ups * (int64_t)(sizeof(gss_var_update) / 4);
     h.region_words[kRegPatches] = n_patches * (int64_t)(sizeof(gss_var_patch) / 4);
-    h.region_words[kRegBaseUps] = n_bups * (int64_t)(sizeof(gss_base_update) / 4);
     h.region_words[kRegLoads] = n_loads * (int64_t)(sizeof(gss_word_load) / 4);
     for (int w = 0; w < GSS_MAX_WORDS; w++) {
         h.valid[w] = w < W ? valid[w] : 0;
@@ -2585,7 +2449,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     e->state_version++;
     e->table_agg_at = screen ? e->state_version : 0;
     HIP_TRY(hipEventRecord(sl.t0, e->stream));
-    HIP_TRY(run_step(e, sl, e->stream));
+    HIP_TRY(launch_step(e, sl, e->stream));
     HIP_TRY(hipEventRecord(sl.t1, e->stream));
     sl.busy = true;
     sl.settled = false;
@@ -2653,9 +2517,9 @@ int gss_step_wait(gss_engine *e, int64_t *n_hits, float *step_ms) {
     sl.host_ready = false;
     sl.rec_total = tot;
     sl.res_words = sl.rec_words;
-    // the slot's next capture compacts into a buffer with room to spare once
+    // the slot's next step compacts into a buffer with room to spare once
     // the records pass half of the current one (a step whose records do not
-    // fit is compacted, or grouped, outside the graph)
+    // fit is compacted, or grouped, afterwards)
     sl.direct = sl.h_hdr.p->host_rec && (uint64_t)tot * sl.rec_words <= kDirectWords;
     sl.direct_rec = sl.h_hdr.p->host_rec;
     if (!sl.direct && 2 * (uint64_t)tot > sl.step_dense)

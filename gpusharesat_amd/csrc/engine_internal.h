@@ -29,8 +29,6 @@ hipStream_t engine_stream(gss_engine *e);
 // Pinned record buffers per step slot (1 .. 4): a waited step's records then
 // stay in place for that many waits of its slot (2n steps with two slots).
 int engine_set_record_buffers(gss_engine *e, int n);
-// Step graphs captured by the engine so far.
-int64_t engine_graph_captures(const gss_engine *e);
 int engine_serve_attach(gss_engine *e, const ServeReq *reqs, uint32_t req_cap,
                         const gss_var_patch *patches, uint64_t patch_cap, const uint64_t *head);
 // gss_step_submit, or with serve a step that admits requests from the ring

@@ -9,6 +9,6 @@ int record_error(int code, const char *msg);
 // first such check, when GPUSHARESAT_LOG_STALLS_MS is set and ms reaches it
 // (host calls that can hold a serving thread or an engine's allocator
 // thread: step submits and waits, record buffer allocations and releases,
-// clause bucket growth, step graph captures).
+// clause bucket growth).
 void log_stall(const char *what, double ms);
 }  // namespace gss

@@ -34,7 +34,7 @@ struct SweepArgs {
                              // (wave g starts in chunk g), [1] chunks past chunk_cap with records
     uint32_t chunk_cap;
     uint32_t sentinel;       // stored row offset of the sentinel literal
-    const int32_t *dyn;      // if set, {nbuckets, npasses} are read here (graph replays)
+    const int32_t *dyn;      // if set, {nbuckets, npasses} are read here (steps)
     int rec_words;           // 8-byte words per record: 3 (gss_hit), 1 (gss_hit_id) or 2
                              // (gss_hit_clause: one record per clause, its words as a mask)
     // Serving and screened batched steps (null otherwise): for each literal l
@@ -51,7 +51,7 @@ struct SweepArgs {
     const uint64_t *agg_words;  // [8]
 };
 
-// Staged regions of a batched step, copied host -> device by k_stage_in.
+// Staged regions of a batched step, read by k_step_in.
 enum StepRegion {
     kRegHeader = 0,
     kRegDesc,
@@ -65,7 +65,7 @@ enum StepRegion {
 };
 
 // Per-step inputs of a batched step (gss_step_*), written by the host into a
-// pinned staging slot and copied to the device by k_stage_in.
+// pinned staging slot and copied to the device by k_step_in.
 struct StepHeader {
     int32_t nbuckets;
     int32_t npasses;
@@ -101,25 +101,6 @@ struct ChunkArgs {
     uint32_t cap;        // chunks in the buffer
     uint32_t waves;
     uint32_t rec_words;  // 8-byte words per record
-};
-
-struct StepInArgs {
-    const uint32_t *h[kStageRegions];  // pinned host (h[kRegHeader] = the header)
-    uint32_t *d[kStageRegions];        // device
-    // device word, nonzero while the engine is halted: an earlier step's
-    // records overflowed its hit buffer and its sweep is to be re-run before
-    // the table moves on
-    const uint32_t *halt;
-    uint32_t *alloc;      // the sweep's counters, cleared
-    uint32_t *counts;     // serving: 2 * 64 counters of the grouping, cleared (else null)
-    uint64_t *table;
-    uint32_t *agg;        // apply with at most 8 words: screening entries to keep current
-                          // (null: none, or a later kernel does it)
-    uint64_t *agg_words;  // screened steps: [8], written from the header (else null)
-    int words;
-    int apply;            // apply the updates (else they are copied for a later kernel)
-    int clauses;          // copy the clauses to their rows (else to the staged regions)
-    int shift;            // of a literal on its way to its row
 };
 
 struct ScatterSeg {
@@ -180,13 +161,35 @@ struct ServeRing {
 };
 constexpr int kServeMaxRequests = 64;  // one admission wave: at most 64 requests per step
 
-// Admits, in sequence order, the published requests whose words fit the
-// table (FIFO: the first that does not fit waits for the next step): writes
-// the step's word loads, valid masks, load and patch counts (and no tasks
-// when nothing was admitted) into the device header, the admitted list, and
-// the report.  One wave.
-hipError_t launch_serve_admit(const ServeRing &r, StepHeader *dh, gss_word_load *loads,
-                              ServeReport *report, int words, hipStream_t s);
+struct StepInArgs {
+    StepHeader header;                 // read over PCIe it cost k_step_in ~2 us more
+    const uint32_t *h[kStageRegions];  // pinned host (the header's unused)
+    uint32_t *d[kStageRegions];        // device
+    // device word, nonzero while the engine is halted: an earlier step's
+    // records overflowed its hit buffer and its sweep is to be re-run before
+    // the table moves on
+    const uint32_t *halt;
+    uint32_t *alloc;      // the sweep's counters, cleared
+    uint32_t *counts;     // serving: 2 * 64 counters of the grouping, cleared (else null)
+    uint64_t *table;
+    uint32_t *agg;        // apply with at most 8 words: screening entries to keep current
+                          // (null: none, or a later kernel does it)
+    uint64_t *agg_words;  // screened steps: [8], written from the header (else null)
+    int words;
+    int apply;            // apply the updates (else they are copied for a later kernel)
+    int clauses;          // copy the clauses to their rows (else to the staged regions)
+    int shift;            // of a literal on its way to its row
+    uint64_t *bases;      // solver base planes (see launch_words_load_dyn)
+    int64_t bases_vw;
+    // Serving steps (report null otherwise): the published requests whose words
+    // fit the table are admitted in sequence order (FIFO: the first that does
+    // not fit waits for the next step).  The step's word loads, valid masks,
+    // load and patch counts go to the device header and loads (and no passes
+    // when nothing was admitted), the admitted list to serve.adm.
+    ServeRing serve;
+    ServeReport *report;  // pinned
+};
+
 // Screening entries of a batched step from the table itself (SweepArgs::agg):
 // group b = words [b * words / 8, (b + 1) * words / 8) (one word per group
 // below 8 words), over every slot of its words (valid or not: what holds in
@@ -200,15 +203,13 @@ hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t
 hipError_t launch_table_agg_update(const uint64_t *table, const StepHeader *dh,
                                    const gss_var_update *ups, const gss_var_patch *patches,
                                    bool with_patches, int words, uint32_t *agg, hipStream_t s);
-// Copies the admitted requests' patches from the pinned ring to r.dpatches
-// (consecutive lanes read consecutive 4-byte words: one pass over PCIe).
-hipError_t launch_serve_stage_patches(const ServeRing &r, const StepHeader *dh, hipStream_t s);
-// Builds the aggregate entries of a serving step (see SweepArgs::agg) and
-// agg_words from the solver bases its admitted requests were loaded from:
-// one pass over the variables, after the admission and the base updates.
-hipError_t launch_serve_agg(const ServeRing &r, const StepHeader *dh, const gss_word_load *loads,
-                            const uint64_t *bases, int64_t vw, int64_t vars, uint32_t *agg,
-                            uint64_t *agg_words, hipStream_t s);
+// After the admission (launch_step_in): copies the admitted requests' patches
+// from the pinned ring to r.dpatches, sets the words they took from their
+// solvers' bases (and the rest of the rows' lines to all ones), and builds the
+// step's screening entries and agg_words (none if agg is null).
+hipError_t launch_serve_load(const ServeRing &r, const StepHeader *dh, const gss_word_load *loads,
+                             const uint64_t *bases, int64_t vw, uint64_t *table, int words,
+                             int64_t vars, uint32_t *agg, uint64_t *agg_words, hipStream_t s);
 // Applies the admitted requests' patches (staged in r.dpatches) with their
 // words shifted to where each request landed; with agg, clears the group's
 // bits that a patch undoes in a valid slot.
@@ -244,7 +245,7 @@ hipError_t launch_assig_roll(const gss_var_update *ups, int64_t n, uint64_t *tab
 hipError_t launch_fill_u64(uint64_t *p, int64_t n, uint64_t v, hipStream_t s);
 
 // Fixed-shape launches of a batched step (counts read from the device header,
-// so a captured graph can be replayed with new data).  While the engine is
+// which a serving step's admission sets there).  While the engine is
 // halted k_step_in writes a header with no work and `halted` set instead of
 // staging: every later kernel of the step then has nothing to do (the
 // serving kernels and k_table_agg, whose work is not counted by the header,
@@ -276,21 +277,12 @@ hipError_t launch_gather(const ChunkArgs &c, void *dense, uint64_t dense_cap, hi
 hipError_t launch_group_by_word(const ChunkArgs &c, uint32_t *counts, void *dense,
                                 uint64_t dense_cap, uint64_t *group, uint32_t *out,
                                 uint32_t *halt, hipStream_t s);
-// Solver base planes: bases[(2 b) * vw + i] / bases[(2 b + 1) * vw + i] hold
-// bit (v mod 64) of word i = v / 64 of base b's is_def / is_true.
-hipError_t launch_base_apply_dyn(const gss_base_update *u, const int64_t *n, uint64_t *bases,
-                                 int64_t vw, hipStream_t s);
-// Sets word w of every variable's two rows from base b, for each load.
+// Sets word w of every variable's two rows from base b, for each load.  Solver
+// base planes: bases[(2 b) * vw + i] / bases[(2 b + 1) * vw + i] hold bit (v
+// mod 64) of word i = v / 64 of base b's is_def / is_true.
 hipError_t launch_words_load_dyn(const gss_word_load *loads, const int64_t *n,
                                  const uint64_t *bases, int64_t vw, uint64_t *table, int words,
                                  int64_t vars, hipStream_t s);
-// Serving steps (loads[k].word == k, words the step does not load invalid in
-// it): sets words [0, n) of every variable's two rows from their loads and
-// words [n, L) to all ones, L = n rounded up to 16 (at most words), so rows
-// are written in whole lines.  words even; vw = (vars + 63) / 64.
-hipError_t launch_words_load_lines(const gss_word_load *loads, const int64_t *n,
-                                   const uint64_t *bases, int64_t vw, uint64_t *table, int words,
-                                   int64_t vars, hipStream_t s);
 hipError_t launch_assig_patch_dyn(const gss_var_patch *p, const int64_t *n, uint64_t *table,
                                   int words, hipStream_t s);
 

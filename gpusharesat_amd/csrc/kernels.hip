@@ -716,59 +716,163 @@ __device__ __forceinline__ void agg_word_bits(uint32_t *agg, uint32_t var, uint3
 
 // ---- batched steps: fixed launch shapes, counts from device memory --------
 
-// A step's inputs from pinned host memory: the header and the regions a later
-// kernel reads are copied, the counters of its sweep cleared, and -- straight
-// from the staging, each byte crossing PCIe once -- its clauses copied to
-// their rows (a.clauses) and its updates applied (a.apply).  Staging first and
-// applying in kernels after it took 3 launches more, 3-5 us each on a step of
-// few updates.
+__device__ __forceinline__ void base_update(const gss_base_update &x, uint64_t *bases,
+                                            int64_t vw) {
+    const uint64_t bit = 1ull << (x.var & 63);
+    unsigned long long *def = (unsigned long long *)bases + (size_t)(2 * x.base) * vw + x.var / 64;
+    unsigned long long *tru = def + vw;
+    if (x.is_def) atomicOr(def, bit);
+    else atomicAnd(def, ~bit);
+    if (x.is_def && x.is_true) atomicOr(tru, bit);
+    else atomicAnd(tru, ~bit);
+}
+
+__device__ __forceinline__ uint64_t wave_incl_scan(uint64_t x, int lane) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t y = __shfl_up(x, d);
+        if (lane >= d) x += y;
+    }
+    return x;
+}
+
+// Admission of a serving step: in sequence order, the published requests whose
+// words fit the table.  One wave reads the ring (two reads over PCIe, one
+// after the other) while the header is on its way, and fills the header in
+// once it is there.
+struct ServePending {
+    uint64_t tail, patch_off;
+    uint32_t solver, k, n_patches;
+    int avail;
+};
+
+__device__ __forceinline__ ServePending serve_pending(const ServeRing &r, int lane) {
+    ServePending p{};
+    p.tail = *r.tail;
+    // published by the host with a release store after the entries
+    uint64_t head = 0;
+    if (lane == 0) head = __hip_atomic_load(r.head, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM);
+    head = uniform64(head);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");  // later reads see the published entries
+    const uint64_t pend = head > p.tail ? head - p.tail : 0;
+    p.avail = (int)(pend < (uint64_t)kServeMaxRequests ? pend : kServeMaxRequests);
+    if (lane < p.avail) {
+        const volatile ServeReq *q = r.reqs + (p.tail + lane) % r.req_cap;
+        p.solver = q->solver;
+        p.k = q->k;
+        p.n_patches = q->n_patches;
+        p.patch_off = q->patch_off;
+    }
+    return p;
+}
+
+__device__ __forceinline__ void serve_admit(const ServePending &p, const ServeRing &r,
+                                            StepHeader *dh, gss_word_load *loads,
+                                            ServeReport *report, int words, int lane) {
+    const int avail = p.avail;
+    const uint32_t k = p.k, np = p.n_patches;
+    const uint64_t nw = lane < avail ? (k + 63u) / 64u : 0;
+    const uint64_t end = wave_incl_scan(nw, lane);
+    // end grows with the lane (every request takes at least one word), so
+    // the requests that fit are a prefix
+    const bool fits = lane < avail && end <= (uint64_t)words;
+    const unsigned long long bal = __ballot(fits);
+    const int count = __popcll(bal);
+    const uint64_t pend_p = wave_incl_scan(fits ? (uint64_t)np : 0, lane);
+    const uint64_t used = __shfl(end, count > 0 ? count - 1 : 0);
+    const uint64_t total_words = count > 0 ? used : 0;
+    const uint64_t total_patches = __shfl(pend_p, count > 0 ? count - 1 : 0);
+    if (fits) {
+        const uint32_t w0 = (uint32_t)(end - nw);
+        ServeAdmitted a;
+        a.patch_off = p.patch_off;
+        a.patch_pfx = pend_p - np;
+        a.n_patches = np;
+        a.w0 = w0;
+        r.adm[lane] = a;
+        for (uint32_t j = 0; j < (uint32_t)nw; j++) {
+            gss_word_load ld;
+            ld.word = (uint16_t)(w0 + j);
+            ld.base = (uint16_t)p.solver;
+            loads[w0 + j] = ld;
+            const uint32_t last = k - 64u * j;  // slots of this word
+            dh->valid[w0 + j] = last >= 64u ? ~0ull : ((1ull << last) - 1ull);
+        }
+    }
+    // words no request took are not checked
+    if ((uint64_t)lane < (uint64_t)GSS_MAX_WORDS && (uint64_t)lane >= total_words)
+        dh->valid[lane] = 0ull;
+    if (lane == 0) {
+        *r.adm_count = (uint32_t)count;
+        dh->nloads = (int64_t)total_words;
+        dh->npatches = count > 0 ? (int64_t)total_patches : 0;
+        if (count == 0) dh->npasses = 0;  // nothing to check
+        *r.tail = p.tail + (uint64_t)count;
+        report->first = p.tail;
+        report->count = (uint32_t)count;
+        report->words = (uint32_t)total_words;
+    }
+}
+
+// A step's inputs from pinned host memory: the header (which comes with the
+// launch) and the regions a later kernel reads are copied, the counters of its
+// sweep cleared, and -- straight from the staging, each byte crossing PCIe once
+// -- its clauses copied to their rows (a.clauses), its base updates and its
+// updates applied (a.apply).  Staging first and applying in kernels after it
+// took 3 launches more, 3-5 us each on a step of few updates.  A serving step's
+// requests are admitted by the first block.
 //
 // Updates go through LDS, 256 at a time, so that the 24-byte records are read
 // in whole lines.
 __global__ __launch_bounds__(256) void k_step_in(StepInArgs a) {
+    const StepHeader &h = a.header;
+    static_assert(sizeof(StepHeader) / 4 <= 192, "three waves copy the header");
     if (blockIdx.x == 0 && threadIdx.x < 2) a.alloc[threadIdx.x] = 0;
     if (a.counts && blockIdx.x == 1 && threadIdx.x < 2 * GSS_MAX_WORDS) a.counts[threadIdx.x] = 0;
     if (*a.halt) {
         // halted: a header with no work (and `halted` set) instead of the step
-        if (blockIdx.x == 0) {
-            uint32_t *d = a.d[kRegHeader];
-            constexpr int kFlag = (int)(offsetof(StepHeader, halted) / 4);
-            for (int i = (int)threadIdx.x; i < (int)(sizeof(StepHeader) / 4); i += (int)blockDim.x)
-                d[i] = i == kFlag ? 1u : 0u;
-        }
+        constexpr int kFlag = (int)(offsetof(StepHeader, halted) / 4);
+        if (blockIdx.x == 0 && threadIdx.x < sizeof(StepHeader) / 4)
+            a.d[kRegHeader][threadIdx.x] = threadIdx.x == kFlag ? 1u : 0u;
         return;
     }
-    __shared__ int64_t s_n[kStageRegions];
-    __shared__ int64_t s_nups;
-    __shared__ int32_t s_ncls;
     __shared__ uint64_t s_up[3 * 256];
-    const StepHeader *h = (const StepHeader *)a.h[kRegHeader];
-    if (threadIdx.x < kStageRegions) s_n[threadIdx.x] = h->region_words[threadIdx.x];
-    if (threadIdx.x == 64) s_nups = h->nups;
-    if (threadIdx.x == 65) s_ncls = h->nclauses;
+    if (blockIdx.x == 0) {
+        ServePending p{};
+        if (threadIdx.x < sizeof(StepHeader) / 4)
+            a.d[kRegHeader][threadIdx.x] = ((const uint32_t *)&h)[threadIdx.x];
+        else if (threadIdx.x >= 192 && a.report)
+            p = serve_pending(a.serve, (int)threadIdx.x & 63);
+        __syncthreads();
+        if (threadIdx.x >= 192 && a.report)
+            serve_admit(p, a.serve, (StepHeader *)a.d[kRegHeader], (gss_word_load *)a.d[kRegLoads],
+                        a.report, a.words, (int)threadIdx.x & 63);
+    }
     // words of each screening group with a valid slot
     if (a.agg_words && blockIdx.x == 1 && threadIdx.x >= 128 && threadIdx.x < 136) {
         const int b = (int)threadIdx.x - 128, gw = a.words < 8 ? 1 : a.words / 8;
         uint64_t m = 0;
         for (int w = b * gw; w < (b + 1) * gw && w < a.words; w++)
-            if (h->valid[w]) m |= 1ull << w;
+            if (h.valid[w]) m |= 1ull << w;
         a.agg_words[b] = m;
     }
-    __syncthreads();
     const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 #pragma unroll
-    for (int r = 0; r < kStageRegions; r++) {
+    for (int r = kRegHeader + 1; r < kStageRegions; r++) {
+        if (r == kRegBaseUps) continue;  // applied below
         if (r == kRegUps && a.apply) continue;
         if ((r == kRegClauses || r == kRegLits) && a.clauses) continue;
         const uint32_t *src = a.h[r];
         uint32_t *dst = a.d[r];
-        for (int64_t i = tid; i < s_n[r]; i += stride) dst[i] = src[i];
+        for (int64_t i = tid; i < h.region_words[r]; i += stride) dst[i] = src[i];
     }
+    const gss_base_update *bups = (const gss_base_update *)a.h[kRegBaseUps];
+    for (int64_t i = tid; i < h.nbups; i += stride) base_update(bups[i], a.bases, a.bases_vw);
     if (a.clauses) {  // eight lanes per clause
         const ClauseSeg *cls = (const ClauseSeg *)a.h[kRegClauses];
         const uint32_t *lits = a.h[kRegLits];
-        for (int64_t i = tid >> 3; i < s_ncls; i += stride >> 3) {
+        for (int64_t i = tid >> 3; i < h.nclauses; i += stride >> 3) {
             const ClauseSeg c = cls[i];
             for (uint32_t j = threadIdx.x & 7; j < c.len; j += 8)
                 c.dst[j] = lits[(uint64_t)c.src + j] << a.shift;
@@ -777,8 +881,8 @@ __global__ __launch_bounds__(256) void k_step_in(StepInArgs a) {
     if (a.apply) {
         const uint64_t *src = (const uint64_t *)a.h[kRegUps];
         uint64_t *dst = (uint64_t *)a.d[kRegUps];
-        for (int64_t t = (int64_t)blockIdx.x * 256; t < s_nups; t += (int64_t)gridDim.x * 256) {
-            const int n = s_nups - t < 256 ? (int)(s_nups - t) : 256;
+        for (int64_t t = (int64_t)blockIdx.x * 256; t < h.nups; t += (int64_t)gridDim.x * 256) {
+            const int n = h.nups - t < 256 ? (int)(h.nups - t) : 256;
             for (int i = (int)threadIdx.x; i < 3 * n; i += 256) {
                 const uint64_t x = src[3 * t + i];
                 s_up[i] = x;
@@ -800,22 +904,6 @@ __global__ __launch_bounds__(256) void k_step_in(StepInArgs a) {
     }
 }
 
-__global__ void k_base_apply_dyn(const gss_base_update *__restrict__ u, const int64_t *n_p,
-                                 uint64_t *bases, int64_t vw) {
-    const int64_t n = *n_p;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const gss_base_update x = u[i];
-        const uint64_t bit = 1ull << (x.var & 63);
-        unsigned long long *def = (unsigned long long *)bases + (size_t)(2 * x.base) * vw + x.var / 64;
-        unsigned long long *tru = def + vw;
-        if (x.is_def) atomicOr(def, bit);
-        else atomicAnd(def, ~bit);
-        if (x.is_def && x.is_true) atomicOr(tru, bit);
-        else atomicAnd(tru, ~bit);
-    }
-}
-
 // Element i covers variable i / nloads and load i % nloads, so the lanes of
 // a wave write neighbouring words of the same rows.
 __global__ void k_words_load_dyn(const gss_word_load *__restrict__ loads, const int64_t *n_p,
@@ -834,60 +922,6 @@ __global__ void k_words_load_dyn(const gss_word_load *__restrict__ loads, const 
         const size_t row = (size_t)v * 2 * words + ld.word;
         table[row] = (d && !t) ? 0ull : ~0ull;     // literal v is false where v is false
         table[row + words] = (d && t) ? 0ull : ~0ull;  // literal ~v is false where v is true
-    }
-}
-
-// Serving steps: load k (0 <= k < n) sets word k from loads[k].base (the
-// admission hands out words 0..n-1 in order), and the words a serving step
-// does not load are not valid in it.  So each row is written in whole
-// 128-byte lines: words [0, L), L = n rounded up to 16 (at most `words`),
-// with words n..L-1 set to all ones.  Written word by word (k_words_load_dyn),
-// 1 to 12 words of a 64-word table cost 0.19-0.29 ms at 2M variables: each
-// row line was written in part.  Whole lines, 16-byte stores: a serving
-// step's device time fell from 0.435 to 0.327 ms at 2M variables, ~1.3
-// requests per step.  One workgroup per 64 variables: the
-// bases' 64-variable words go through LDS, then each lane writes 16 bytes
-// (2 words) of a variable's F row and of its T row, neighbouring lanes
-// neighbouring words.  `words` is even (16-byte stores stay aligned).
-__global__ __launch_bounds__(256) void k_words_load_lines(const gss_word_load *__restrict__ loads,
-                                                          const int64_t *n_p,
-                                                          const uint64_t *__restrict__ bases,
-                                                          int64_t vw, uint64_t *__restrict__ table,
-                                                          int words, int64_t vars) {
-    const int nl = (int)*n_p;
-    if (nl <= 0) return;
-    __shared__ uint64_t s_bits[2 * GSS_MAX_WORDS];  // [2k] def, [2k + 1] true of load k
-    const int64_t blk = blockIdx.x;                   // variables [64 blk, 64 blk + 64)
-    const int tid = (int)threadIdx.x;
-    if (tid < 2 * nl) {
-        const gss_word_load ld = loads[tid >> 1];
-        s_bits[tid] = bases[(size_t)(2 * ld.base + (tid & 1)) * vw + blk];
-    }
-    __syncthreads();
-    int L = (nl + 15) & ~15;
-    if (L > words) L = words;
-    const int pairs = L >> 1;  // 16-byte stores per row
-    for (int it = tid; it < 64 * pairs; it += 256) {
-        const int vi = it / pairs, p = it - vi * pairs;
-        const int64_t v = blk * 64 + vi;
-        if (v >= vars) break;  // it grows with vi
-        const uint64_t bit = 1ull << vi;
-        uint64_t f[2], t[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int w = 2 * p + h;
-            f[h] = ~0ull;
-            t[h] = ~0ull;
-            if (w < nl) {
-                const bool d = (s_bits[2 * w] & bit) != 0;
-                const bool tr = (s_bits[2 * w + 1] & bit) != 0;
-                if (d && !tr) f[h] = 0ull;  // literal v is false where v is false
-                if (d && tr) t[h] = 0ull;   // literal ~v is false where v is true
-            }
-        }
-        uint64_t *row = table + (size_t)v * 2 * words + 2 * p;
-        *(ulonglong2 *)row = make_ulonglong2(f[0], f[1]);
-        *(ulonglong2 *)(row + words) = make_ulonglong2(t[0], t[1]);
     }
 }
 
@@ -1093,157 +1127,101 @@ __global__ __launch_bounds__(256) void k_step_end(ChunkArgs c, StepEndArgs a) {
 
 // ---- records grouped by assignment word (serving steps) ----------------------
 
-// Records per word over the claimed chunks (word = the top 16 bits of a
-// record's first word); counts[64] must start at zero.
+// f(record) for every record of the block's share of the chunks, a thread per
+// record: with a wave per chunk, the chunks' few records each (thousands of
+// chunks, ~10 records in one) were a chain of reads per wave.
+template <typename F>
+__device__ __forceinline__ void for_records(const ChunkArgs &ch, F &&f) {
+    __shared__ uint32_t s_end[64];  // records up to and with the group's chunk k
+    const uint32_t n = chunks_held(ch), rw = ch.rec_words;
+    const uint32_t per = (n + gridDim.x - 1) / gridDim.x;
+    const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < n ? c0 + per : n;
+    for (uint32_t c = c0; c < c1; c += 64) {
+        if (threadIdx.x < 64) {
+            const uint32_t fill = c + threadIdx.x < c1 ? ch.fills[c + threadIdx.x] : 0u;
+            s_end[threadIdx.x] = (uint32_t)wave_incl_scan(fill, (int)threadIdx.x);
+        }
+        __syncthreads();
+        const uint32_t total = s_end[63];
+        for (uint32_t i = threadIdx.x; i < total; i += 256) {
+            uint32_t k = 0;  // the first chunk that ends after record i
+#pragma unroll
+            for (uint32_t d = 32; d > 0; d >>= 1)
+                if (s_end[k + d - 1] <= i) k += d;
+            const uint32_t at = i - (k ? s_end[k - 1] : 0u);
+            f(ch.hits + ((uint64_t)(c + k) * kHitChunk + at) * rw);
+        }
+        __syncthreads();
+    }
+}
+
+// The word a record is of: the top 16 bits of its first word.
+__device__ __forceinline__ uint32_t record_word(const uint64_t *r) {
+    return (uint32_t)(r[0] >> 48) & (GSS_MAX_WORDS - 1);
+}
+
+// Records per word; counts[64] must start at zero.  The two grouping kernels
+// run kGroupBlocks blocks, and a block adds to a word's counter once:
+// device-scope atomics on one address take ~10 ns each.  With one per chunk and
+// word, over the 1,024 blocks' chunks, the kernels took 12 and 14 us.
+constexpr unsigned kGroupBlocks = 128;
 __global__ __launch_bounds__(256) void k_word_count(ChunkArgs ch, uint32_t *counts) {
     __shared__ uint32_t h[GSS_MAX_WORDS];
     if (threadIdx.x < GSS_MAX_WORDS) h[threadIdx.x] = 0;
     __syncthreads();
-    const uint32_t n = chunks_held(ch), rec_words = ch.rec_words;
-    for (uint32_t c = blockIdx.x; c < n; c += gridDim.x) {
-        const uint32_t f = ch.fills[c];
-        const uint64_t *src = ch.hits + (uint64_t)c * kHitChunk * rec_words;
-        for (uint32_t i = threadIdx.x; i < f; i += blockDim.x)
-            atomicAdd(&h[(uint32_t)(src[(uint64_t)i * rec_words] >> 48) & (GSS_MAX_WORDS - 1)], 1u);
-    }
+    for_records(ch, [&](const uint64_t *r) { atomicAdd(&h[record_word(r)], 1u); });
     __syncthreads();
     if (threadIdx.x < GSS_MAX_WORDS && h[threadIdx.x]) atomicAdd(&counts[threadIdx.x], h[threadIdx.x]);
 }
 
 // Moves the records into `dense` grouped by word, ascending (within a word in
-// no set order): a block takes one chunk at a time, counts its records per
-// word in LDS, reserves each word's share with one atomic on that word's
-// cursor, then places them.  group[w] = first record of word w, group[64] =
-// all records, group[65] = 1 when they fitted in dense_cap (else nothing is
-// moved and the host groups the records itself).  cursor[64] starts at zero.
+// no set order): a block counts its records per word in LDS, reserves each
+// word's share with one atomic on that word's cursor, then places them.
+// group[w] = first record of word w, group[64] = all records, group[65] = 1
+// when they fitted in dense_cap (else nothing is moved and the host groups the
+// records itself).  cursor[64] starts at zero.
 __global__ __launch_bounds__(256) void k_word_scatter(ChunkArgs ch,
                                                       const uint32_t *__restrict__ counts,
                                                       uint32_t *cursor, uint64_t *__restrict__ dense,
                                                       uint64_t dense_cap, uint64_t *group,
                                                       uint32_t *out, uint32_t *halt) {
     __shared__ uint64_t base[GSS_MAX_WORDS + 1];
-    __shared__ uint32_t lc[GSS_MAX_WORDS], lbase[GSS_MAX_WORDS];
-    if (threadIdx.x == 0) {
-        uint64_t acc = 0;
-        for (int w = 0; w < GSS_MAX_WORDS; w++) {
-            base[w] = acc;
-            acc += counts[w];
-        }
-        base[GSS_MAX_WORDS] = acc;
+    __shared__ uint32_t lc[GSS_MAX_WORDS];
+    const int tid = (int)threadIdx.x;
+    if (tid < GSS_MAX_WORDS) {
+        static_assert(GSS_MAX_WORDS == 64, "one wave");
+        const uint64_t k = counts[tid], end = wave_incl_scan(k, tid);
+        base[tid] = end - k;
+        if (tid == GSS_MAX_WORDS - 1) base[GSS_MAX_WORDS] = end;
+        lc[tid] = 0;
     }
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        write_counts(ch, base[GSS_MAX_WORDS], out);
+    const uint64_t total = base[GSS_MAX_WORDS];
+    const bool fits = total <= dense_cap;
+    if (blockIdx.x == 0 && tid == 0) {
+        write_counts(ch, total, out);
         if (ch.alloc[1]) *halt = 1u;  // records were dropped: the step is re-run
     }
-    const bool fits = base[GSS_MAX_WORDS] <= dense_cap;
-    if (blockIdx.x == 0 && threadIdx.x <= GSS_MAX_WORDS + 1)
-        group[threadIdx.x] = threadIdx.x <= GSS_MAX_WORDS ? base[threadIdx.x] : (fits ? 1ull : 0ull);
+    if (blockIdx.x == 0 && tid <= GSS_MAX_WORDS + 1)
+        group[tid] = tid <= GSS_MAX_WORDS ? base[tid] : (fits ? 1ull : 0ull);
     if (!fits) return;  // the same for every thread of every block
-    const uint32_t n = chunks_held(ch), rec_words = ch.rec_words;
-    for (uint32_t c = blockIdx.x; c < n; c += gridDim.x) {
-        const uint32_t f = ch.fills[c];
-        if (!f) continue;  // uniform in the block
-        if (threadIdx.x < GSS_MAX_WORDS) lc[threadIdx.x] = 0;
-        __syncthreads();
-        const uint64_t *src = ch.hits + (uint64_t)c * kHitChunk * rec_words;
-        for (uint32_t i = threadIdx.x; i < f; i += blockDim.x)
-            atomicAdd(&lc[(uint32_t)(src[(uint64_t)i * rec_words] >> 48) & (GSS_MAX_WORDS - 1)], 1u);
-        __syncthreads();
-        if (threadIdx.x < GSS_MAX_WORDS) {
-            const uint32_t k = lc[threadIdx.x];
-            lbase[threadIdx.x] = k ? atomicAdd(&cursor[threadIdx.x], k) : 0u;
-            lc[threadIdx.x] = 0;
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < f; i += blockDim.x) {
-            const uint64_t *r = src + (uint64_t)i * rec_words;
-            const uint32_t w = (uint32_t)(r[0] >> 48) & (GSS_MAX_WORDS - 1);
-            const uint64_t pos = base[w] + lbase[w] + atomicAdd(&lc[w], 1u);
-            for (uint32_t q = 0; q < rec_words; q++) dense[pos * rec_words + q] = r[q];
-        }
-        __syncthreads();
+    for_records(ch, [&](const uint64_t *r) { atomicAdd(&lc[record_word(r)], 1u); });
+    __syncthreads();
+    if (tid < GSS_MAX_WORDS) {
+        const uint32_t k = lc[tid];
+        if (k) base[tid] += atomicAdd(&cursor[tid], k);
+        lc[tid] = 0;
     }
+    __syncthreads();
+    const uint32_t rw = ch.rec_words;
+    for_records(ch, [&](const uint64_t *r) {
+        const uint32_t w = record_word(r);
+        const uint64_t pos = base[w] + atomicAdd(&lc[w], 1u);
+        for (uint32_t q = 0; q < rw; q++) dense[pos * rw + q] = r[q];
+    });
 }
 
 // ---- serving: requests admitted on the device ---------------------------------
-
-__device__ __forceinline__ uint64_t wave_incl_scan(uint64_t x, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t y = __shfl_up(x, d);
-        if (lane >= d) x += y;
-    }
-    return x;
-}
-
-__global__ __launch_bounds__(64) void k_serve_admit(ServeRing r, StepHeader *dh,
-                                                    gss_word_load *loads, ServeReport *report,
-                                                    int words) {
-    if (dh->halted) return;  // the ring waits for the step's replay
-    const int lane = (int)threadIdx.x;
-    __shared__ uint64_t s_head;
-    if (lane == 0) {
-        // published by the host with a release store after the entries
-        s_head = __hip_atomic_load(r.head, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");  // later reads see the published entries
-    const uint64_t tail = *r.tail;
-    const uint64_t head = s_head;
-    const uint64_t pend = head > tail ? head - tail : 0;
-    const int avail = (int)(pend < (uint64_t)kServeMaxRequests ? pend : kServeMaxRequests);
-    uint32_t solver = 0, k = 0, np = 0;
-    uint64_t poff = 0;
-    if (lane < avail) {
-        const volatile ServeReq *q = r.reqs + (tail + lane) % r.req_cap;
-        solver = q->solver;
-        k = q->k;
-        np = q->n_patches;
-        poff = q->patch_off;
-    }
-    const uint64_t nw = lane < avail ? (k + 63u) / 64u : 0;
-    const uint64_t end = wave_incl_scan(nw, lane);
-    // end grows with the lane (every request takes at least one word), so
-    // the requests that fit are a prefix
-    const bool fits = lane < avail && end <= (uint64_t)words;
-    const unsigned long long bal = __ballot(fits);
-    const int count = __popcll(bal);
-    const uint64_t pend_p = wave_incl_scan(fits ? (uint64_t)np : 0, lane);
-    const uint64_t used = __shfl(end, count > 0 ? count - 1 : 0);
-    const uint64_t total_words = count > 0 ? used : 0;
-    const uint64_t total_patches = __shfl(pend_p, count > 0 ? count - 1 : 0);
-    if (fits) {
-        const uint32_t w0 = (uint32_t)(end - nw);
-        ServeAdmitted a;
-        a.patch_off = poff;
-        a.patch_pfx = pend_p - np;
-        a.n_patches = np;
-        a.w0 = w0;
-        r.adm[lane] = a;
-        for (uint32_t j = 0; j < (uint32_t)nw; j++) {
-            gss_word_load ld;
-            ld.word = (uint16_t)(w0 + j);
-            ld.base = (uint16_t)solver;
-            loads[w0 + j] = ld;
-            const uint32_t last = k - 64u * j;  // slots of this word
-            dh->valid[w0 + j] = last >= 64u ? ~0ull : ((1ull << last) - 1ull);
-        }
-    }
-    // words no request took are not checked
-    if ((uint64_t)lane < (uint64_t)GSS_MAX_WORDS && (uint64_t)lane >= total_words)
-        dh->valid[lane] = 0ull;
-    if (lane == 0) {
-        *r.adm_count = (uint32_t)count;
-        dh->nloads = (int64_t)total_words;
-        dh->npatches = count > 0 ? (int64_t)total_patches : 0;
-        if (count == 0) dh->npasses = 0;  // nothing to check
-        *r.tail = tail + (uint64_t)count;
-        report->first = tail;
-        report->count = (uint32_t)count;
-        report->words = (uint32_t)total_words;
-    }
-}
 
 // The admitted request (index into r.adm) of the step's i-th patch.
 __device__ __forceinline__ int admitted_of(const ServeRing &r, int cnt, int64_t i) {
@@ -1254,21 +1232,6 @@ __device__ __forceinline__ int admitted_of(const ServeRing &r, int cnt, int64_t 
         else hi = mid;
     }
     return lo;
-}
-
-__global__ void k_serve_stage_patches(ServeRing r, const StepHeader *__restrict__ dh) {
-    constexpr int kWords = (int)(sizeof(gss_var_patch) / 4);
-    const int64_t n = dh->npatches * kWords;
-    const int cnt = (int)*r.adm_count;
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n;
-         k += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t i = k / kWords;
-        const int f = (int)(k - i * kWords);
-        const ServeAdmitted a = r.adm[admitted_of(r, cnt, i)];
-        const uint64_t j = (uint64_t)(i - (int64_t)a.patch_pfx);
-        const uint32_t *src = (const uint32_t *)(r.patches + (a.patch_off + j) % r.patch_cap);
-        ((uint32_t *)(r.dpatches + i))[f] = src[f];
-    }
 }
 
 // Screening entries of a batched step (SweepArgs::agg), over every slot of a
@@ -1348,43 +1311,100 @@ __global__ void k_table_agg_update(const uint64_t *__restrict__ table,
     }
 }
 
-// Screening entries of a serving step: group b = the admitted requests r with
+// A serving step's table words, screening entries and patches, in one launch.
+//
+// Load k (0 <= k < n) sets word k from loads[k].base (the admission hands out
+// words 0..n-1 in order), and the words a serving step does not load are not
+// valid in it.  So each row is written in whole 128-byte lines: words [0, L), L
+// = n rounded up to 16 (at most `words`), words n..L-1 all ones.  Written word
+// by word, 1 to 12 words of a 64-word table cost 0.19-0.29 ms at 2M variables:
+// each row line was written in part.
+//
+// Screening entries (SweepArgs::agg): group b = the admitted requests r with
 // r % 8 = b, from their solvers' bases (a request's words are loaded whole from
 // its base, so until its patches the base value holds in all its slots;
 // k_serve_patch clears what a patch undoes).  Bits of empty groups are not read.
-__global__ void k_serve_agg(ServeRing r, const StepHeader *__restrict__ dh,
-                            const gss_word_load *__restrict__ loads,
-                            const uint64_t *__restrict__ bases, int64_t vw, int64_t vars,
-                            uint32_t *__restrict__ agg, uint64_t *__restrict__ agg_words) {
-    if (dh->halted) return;  // the aggregate stays the halted step's
-    __shared__ uint32_t s_base[kServeMaxRequests];
-    const int cnt = (int)*r.adm_count;
-    if ((int)threadIdx.x < cnt) s_base[threadIdx.x] = loads[r.adm[threadIdx.x].w0].base;
-    if (blockIdx.x == 0 && threadIdx.x < 8) {
-        const int64_t nl = dh->nloads;
-        uint64_t m = 0;
-        for (int q = (int)threadIdx.x; q < cnt; q += 8) {
-            const uint32_t w0 = r.adm[q].w0;
-            const uint32_t w1 = q + 1 < cnt ? r.adm[q + 1].w0 : (uint32_t)nl;
-            for (uint32_t w = w0; w < w1 && w < 64u; w++) m |= 1ull << w;
+//
+// The first kPatchBlocks blocks copy the admitted requests' patches from the
+// pinned ring (consecutive lanes read consecutive 4-byte words: one pass over
+// PCIe); each other block covers 64 variables: the bases' 64-variable words go
+// through LDS, then each lane writes 16 bytes (2 words) of a variable's F row
+// and of its T row, neighbouring lanes neighbouring words.
+constexpr unsigned kPatchBlocks = 128;
+__global__ __launch_bounds__(256) void k_serve_load(ServeRing r, const StepHeader *__restrict__ dh,
+                                                    const gss_word_load *__restrict__ loads,
+                                                    const uint64_t *__restrict__ bases,
+                                                    int64_t vw, uint64_t *__restrict__ table,
+                                                    int words, int64_t vars,
+                                                    uint32_t *__restrict__ agg,
+                                                    uint64_t *__restrict__ agg_words) {
+    if (dh->halted) return;  // the words and the entries stay the halted step's
+    const int nl = (int)dh->nloads, cnt = (int)*r.adm_count;
+    const int tid = (int)threadIdx.x;
+    if (blockIdx.x < kPatchBlocks) {
+        if (agg && blockIdx.x == 0 && tid < 8) {
+            uint64_t m = 0;
+            for (int q = tid; q < cnt; q += 8) {
+                const uint32_t w0 = r.adm[q].w0;
+                const uint32_t w1 = q + 1 < cnt ? r.adm[q + 1].w0 : (uint32_t)nl;
+                for (uint32_t w = w0; w < w1 && w < 64u; w++) m |= 1ull << w;
+            }
+            agg_words[tid] = m;
         }
-        agg_words[threadIdx.x] = m;
+        constexpr int kWords = (int)(sizeof(gss_var_patch) / 4);
+        const int64_t n = dh->npatches * kWords;
+        for (int64_t k = blockIdx.x * (int64_t)256 + tid; k < n; k += kPatchBlocks * 256) {
+            const int64_t i = k / kWords;
+            const int f = (int)(k - i * kWords);
+            const ServeAdmitted a = r.adm[admitted_of(r, cnt, i)];
+            const uint64_t j = (uint64_t)(i - (int64_t)a.patch_pfx);
+            const uint32_t *src = (const uint32_t *)(r.patches + (a.patch_off + j) % r.patch_cap);
+            ((uint32_t *)(r.dpatches + i))[f] = src[f];
+        }
+        return;
     }
+    if (nl <= 0) return;
+    __shared__ uint64_t s_bits[2 * GSS_MAX_WORDS];  // [2k] def, [2k + 1] true of load k
+    __shared__ uint32_t s_w0[kServeMaxRequests];
+    const int64_t blk = blockIdx.x - kPatchBlocks;  // variables [64 blk, 64 blk + 64)
+    if (tid < 2 * nl) s_bits[tid] = bases[(size_t)(2 * loads[tid >> 1].base + (tid & 1)) * vw + blk];
+    if (tid >= 192 && tid - 192 < cnt) s_w0[tid - 192] = r.adm[tid - 192].w0;
     __syncthreads();
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < vars;
-         v += (int64_t)gridDim.x * blockDim.x) {
+    if (agg && tid < 64 && blk * 64 + tid < vars) {
         uint32_t x = ~0u;
-        const uint64_t bit = 1ull << (v & 63);
-        const int64_t i = v >> 6;
         for (int q = 0; q < cnt; q++) {
-            const uint64_t *def = bases + (size_t)(2 * s_base[q]) * vw;
-            const bool d = (def[i] & bit) != 0;
-            const bool t = (def[vw + i] & bit) != 0;
+            const bool d = (s_bits[2 * s_w0[q]] >> tid) & 1ull;
+            const bool t = (s_bits[2 * s_w0[q] + 1] >> tid) & 1ull;
             // true: v non-false and true; false: ~v; undefined: both non-false
             const uint32_t keep = !d ? 0x00010001u : t ? 0x00000101u : 0x01010000u;
             x &= ~((0x01010101u & ~keep) << (q & 7));
         }
-        agg[v] = x;
+        agg[blk * 64 + tid] = x;
+    }
+    // literal v is false where v is false, ~v where v is true
+    const auto word = [&](int w, int vi, uint64_t &f, uint64_t &t) {
+        f = t = ~0ull;
+        if (w < nl && ((s_bits[2 * w] >> vi) & 1ull))
+            (((s_bits[2 * w + 1] >> vi) & 1ull) ? t : f) = 0ull;
+    };
+    if (words == 1) {
+        const int64_t v = blk * 64 + tid;
+        if (tid < 64 && v < vars) word(0, tid, table[2 * v], table[2 * v + 1]);
+        return;
+    }
+    int L = (nl + 15) & ~15;
+    if (L > words) L = words;
+    const int pairs = L >> 1;  // 16-byte stores per row; words is a power of two
+    for (int it = tid; it < 64 * pairs; it += 256) {
+        const int vi = it / pairs, p = it - vi * pairs;
+        const int64_t v = blk * 64 + vi;
+        if (v >= vars) break;  // it grows with vi
+        uint64_t f[2], t[2];
+        word(2 * p, vi, f[0], t[0]);
+        word(2 * p + 1, vi, f[1], t[1]);
+        uint64_t *row = table + (size_t)v * 2 * words + 2 * p;
+        *(ulonglong2 *)row = make_ulonglong2(f[0], f[1]);
+        *(ulonglong2 *)(row + words) = make_ulonglong2(t[0], t[1]);
     }
 }
 
@@ -1566,27 +1586,11 @@ hipError_t launch_step_end(const ChunkArgs &c, const StepEndArgs &a, hipStream_t
     return hipGetLastError();
 }
 
-hipError_t launch_base_apply_dyn(const gss_base_update *u, const int64_t *n, uint64_t *bases,
-                                 int64_t vw, hipStream_t s) {
-    hipLaunchKernelGGL(k_base_apply_dyn, dim3(256), dim3(256), 0, s, u, n, bases, vw);
-    return hipGetLastError();
-}
-
 hipError_t launch_words_load_dyn(const gss_word_load *loads, const int64_t *n,
                                  const uint64_t *bases, int64_t vw, uint64_t *table, int words,
                                  int64_t vars, hipStream_t s) {
     hipLaunchKernelGGL(k_words_load_dyn, dim3(4096), dim3(256), 0, s, loads, n, bases, vw, table,
                        words, vars);
-    return hipGetLastError();
-}
-
-hipError_t launch_words_load_lines(const gss_word_load *loads, const int64_t *n,
-                                   const uint64_t *bases, int64_t vw, uint64_t *table, int words,
-                                   int64_t vars, hipStream_t s) {
-    if (words % 2 || vw != (vars + 63) / 64) return hipErrorInvalidValue;
-    if (vars <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_words_load_lines, dim3((unsigned)vw), dim3(256), 0, s, loads, n, bases,
-                       vw, table, words, vars);
     return hipGetLastError();
 }
 
@@ -1630,17 +1634,11 @@ hipError_t launch_group_by_word(const ChunkArgs &c, uint32_t *counts, void *dens
                                 uint64_t dense_cap, uint64_t *group, uint32_t *out,
                                 uint32_t *halt, hipStream_t s) {
     if (c.rec_words != 1 && c.rec_words != 3) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_word_count, dim3(1024), dim3(256), 0, s, c, counts);
+    hipLaunchKernelGGL(k_word_count, dim3(kGroupBlocks), dim3(256), 0, s, c, counts);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_word_scatter, dim3(1024), dim3(256), 0, s, c, counts,
+    hipLaunchKernelGGL(k_word_scatter, dim3(kGroupBlocks), dim3(256), 0, s, c, counts,
                        counts + GSS_MAX_WORDS, (uint64_t *)dense, dense_cap, group, out, halt);
-    return hipGetLastError();
-}
-
-hipError_t launch_serve_admit(const ServeRing &r, StepHeader *dh, gss_word_load *loads,
-                              ServeReport *report, int words, hipStream_t s) {
-    hipLaunchKernelGGL(k_serve_admit, dim3(1), dim3(64), 0, s, r, dh, loads, report, words);
     return hipGetLastError();
 }
 
@@ -1674,16 +1672,12 @@ hipError_t launch_table_agg_update(const uint64_t *table, const StepHeader *dh,
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_serve_stage_patches(const ServeRing &r, const StepHeader *dh, hipStream_t s) {
-    hipLaunchKernelGGL(k_serve_stage_patches, dim3(1024), dim3(256), 0, s, r, dh);
-    return hipGetLastError();
-}
-
-hipError_t launch_serve_agg(const ServeRing &r, const StepHeader *dh, const gss_word_load *loads,
-                            const uint64_t *bases, int64_t vw, int64_t vars, uint32_t *agg,
-                            uint64_t *agg_words, hipStream_t s) {
-    hipLaunchKernelGGL(k_serve_agg, dim3(2048), dim3(256), 0, s, r, dh, loads, bases, vw, vars,
-                       agg, agg_words);
+hipError_t launch_serve_load(const ServeRing &r, const StepHeader *dh, const gss_word_load *loads,
+                             const uint64_t *bases, int64_t vw, uint64_t *table, int words,
+                             int64_t vars, uint32_t *agg, uint64_t *agg_words, hipStream_t s) {
+    const unsigned blocks = kPatchBlocks + (unsigned)((vars + 63) / 64);
+    hipLaunchKernelGGL(k_serve_load, dim3(blocks), dim3(256), 0, s, r, dh, loads, bases, vw, table,
+                       words, vars, agg, agg_words);
     return hipGetLastError();
 }
 

@@ -246,7 +246,7 @@ void complete_oldest(gss_server *s, std::unique_lock<std::mutex> &lk) {
     const double wait_ms =
         std::chrono::duration<double, std::milli>(Clock::now() - t_wait).count();
     // what the step admitted and where its records of each word start (both
-    // written by the step's graph into pinned memory) are read before the
+    // written by the step into pinned memory) are read before the
     // next step is launched: it reuses this slot's pinned header
     ServeReport rep{};
     if (!rc) rc = gss::step_serve_report(s->e, &rep);
@@ -272,7 +272,7 @@ void complete_oldest(gss_server *s, std::unique_lock<std::mutex> &lk) {
         lk.unlock();
     }
     // the records themselves: waits for their copy to pinned memory, which
-    // the step just launched does not touch (its graph waits for that copy
+    // the step just launched does not touch (it waits for that copy
     // on the device before it reuses the slot's device buffers)
     const uint64_t *raw = nullptr;
     const int rw = s->cfg.records == GSS_RECORDS_IDS ? 1 : 3;
@@ -683,7 +683,7 @@ int gss_server_stats_get(gss_server *s, gss_server_stats *out) {
     out->checks = s->checks;
     out->device_ms = s->device_ms;
     out->host_grouped = s->host_grouped;
-    out->graph_captures = gss::engine_graph_captures(s->e);
+    out->graph_captures = 0;  // steps are launched kernel by kernel
     out->submit_ms_total = s->submit_ms_total;
     out->submit_ms_max = s->submit_ms_max;
     out->wait_ms_max = s->wait_ms_max;

@@ -192,8 +192,7 @@ void EngineClauseSharer::ensure_table() {
 // A run (GpuRunner::startGpuRunAsync, GpuRunner.cu:274-351) is one batched
 // step: the run's new clauses, the solvers' assignment updates, the valid
 // slots and the roll-forward positions are staged into the step's pinned slot
-// (one host-to-device copy, made by the step's first kernel), and one HIP
-// graph appends, applies, checks, rolls forward and compacts the records.
+// and read from there by the step's first kernel, and the step appends, applies, checks, rolls forward and compacts the records.
 // The records are gss_hit_id (clause and solver word, no masks: delivery never
 // reads them); gss_step_wait starts their copy to pinned host memory on the
 // slot's own stream, and deliver() reads them there.

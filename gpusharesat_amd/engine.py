@@ -270,8 +270,8 @@ class Engine:
     # -- batched steps --------------------------------------------------------
     def step_enqueue(self, lits=None, lens=None, ups=None, valid=0, last_pos=None,
                      screen: bool = False) -> np.ndarray:
-        """Enqueues one step (append, apply, sweep, roll forward) as a graph
-        replay; returns the bucket rows of the appended clauses.  screen: the
+        """Enqueues one step (append, apply, sweep, roll forward);
+        returns the bucket rows of the appended clauses.  screen: the
         step screens clauses against the table's aggregate first
         (GSS_STEP_SCREEN; same records)."""
         if screen:

@@ -189,7 +189,7 @@ class ServeResult:
     # (seconds, steps, device ms, clauses) of the server, about every 5 s
     samples: list = field(default_factory=list)
     host_grouped: int = 0    # steps whose records the serving thread grouped itself
-    graph_captures: int = 0  # step graphs the engine captured
+    graph_captures: int = 0  # 0: steps run without captured graphs
     thread: dict = field(default_factory=dict)  # serving thread's submit / wait host times
     lag_ms: np.ndarray = None  # arrival -> published in the ring (this driver's part)
     step_stats: dict = field(default_factory=dict)  # hit-buffer re-runs and size

@@ -265,11 +265,11 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
  * out_rows if non-null) -> apply n_ups updates -> sweep every clause against
  * the slots in valid -> roll forward (last_pos as gss_assig_roll_forward, may
  * be null = none) -> stage the hit counts to pinned host memory.  The device
- * side of a step is one captured HIP graph per ping-pong slot, replayed with
- * new data (the counts are read from device memory), so two steps can be in
- * flight and the host fills one slot while the other runs.  Replaces the
- * per-run sequence of GpuRunner::wholeRun / startGpuRunAsync / launchGpu /
- * gatherGpuRunResults (GpuRunner.cu:211-345,360) with one graph launch.
+ * side of a step is 3 kernels (up to 9 with patches, word loads and screening)
+ * over one of two staging slots, so two steps can be in flight and the host
+ * fills one slot while the other runs.  Replaces the per-run sequence of
+ * GpuRunner::wholeRun / startGpuRunAsync / launchGpu / gatherGpuRunResults
+ * (GpuRunner.cu:211-345,360).
  * Clause literals must have table rows (grow the table before the step). */
 int gss_step_enqueue(gss_engine *e, int64_t n, const uint32_t *lits, const int32_t *lens,
                      uint32_t *out_rows, int64_t n_ups, const gss_var_update *ups,
@@ -327,7 +327,7 @@ int gss_step_submit(gss_engine *e, const gss_step_desc *d);
  * (Assigs.cuh:39-58); here a base is the solver's last assignment, packed. */
 int gss_bases_reset(gss_engine *e, int nbases);
 /* Wait for the oldest step in flight: its number of hit records and the time
- * (ms) between events recorded around its graph launch.  The step's records
+ * (ms) between events recorded around its kernels.  The step's records
  * start travelling to pinned host memory at once, on a stream of the slot's
  * own, while the caller goes on (typically enqueueing the next step); the
  * slot's next step does not overwrite them on the device before that copy is

@@ -84,7 +84,7 @@ typedef struct gss_server_stats {
     double device_ms;         /* sum of the steps' device times */
     int64_t host_grouped;     /* steps whose records outgrew the device grouping buffer and
                                  were grouped by the serving thread */
-    int64_t graph_captures;   /* step graphs captured (a new one whenever buffers grow) */
+    int64_t graph_captures;   /* 0: steps run without captured graphs */
     double submit_ms_total;   /* serving thread: host time staging and launching steps */
     double submit_ms_max;     /* the longest of them */
     double wait_ms_max;       /* the longest wait for a step to end */

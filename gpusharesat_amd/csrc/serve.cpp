@@ -84,7 +84,7 @@ struct Done {
     gss_serve_result r{};
     std::shared_ptr<const StepRecords> step;
     size_t first = 0;                 // its first record in step->words
-    std::vector<gss_serve_hit> recs;  // translated on request (gss_server_records)
+    std::unique_ptr<gss_serve_hit[]> recs;  // translated on request (gss_server_records)
     bool translated = false;
 };
 
@@ -376,7 +376,8 @@ void complete_oldest(gss_server *s, std::unique_lock<std::mutex> &lk) {
     if (step->lent) s->lent.emplace_back(si.index, step);
     if (cnt) {
         const Pending &last = s->pending[cnt - 1];
-        s->patch_completed = last.patch_off + last.n_patches;
+        // (a request without patches may hold a place before the ring's restart)
+        s->patch_completed = std::max(s->patch_completed, last.patch_off + last.n_patches);
     }
     s->pending.erase(s->pending.begin(), s->pending.begin() + cnt);
     s->completed += (uint64_t)cnt;
@@ -565,7 +566,10 @@ int gss_server_submit(gss_server *s, int solver, int k, int64_t n_patches,
     if (solver < 0 || solver >= s->cfg.solvers || k < 1 || k > 64 * s->cfg.words)
         return fail(GSS_E_INVAL, "request solver or size out of range");
     const uint32_t nw = (uint32_t)(k + 63) / 64;
+    bool bad = false;  // no way out of the loop: several patches are checked at a time
     for (int64_t i = 0; i < n_patches; i++)
+        bad |= (patches[i].var >= (uint64_t)s->cfg.var_count) | (patches[i].word >= nw);
+    for (int64_t i = 0; bad && i < n_patches; i++)
         if (patches[i].var >= (uint64_t)s->cfg.var_count || patches[i].word >= nw)
             return fail(GSS_E_INVAL, "patch " + std::to_string(i) + " out of range");
     {
@@ -578,8 +582,15 @@ int gss_server_submit(gss_server *s, int solver, int k, int64_t n_patches,
             (uint64_t)s->cfg.patch_ring)
             return fail(GSS_E_STATE, "patch ring full");
         const uint64_t pcap = (uint64_t)s->cfg.patch_ring;
-        for (int64_t i = 0; i < n_patches; i++)
-            s->patches[(s->patch_published + (uint64_t)i) % pcap] = patches[i];
+        // an empty ring starts over: its first pages are mapped and cached, the
+        // next ones may not be (12 ns per patch there)
+        if (s->patch_published == s->patch_completed)
+            s->patch_published = s->patch_completed = (s->patch_published + pcap - 1) / pcap * pcap;
+        // two copies at most: up to the ring's end, and on from its start
+        const uint64_t at = s->patch_published % pcap;
+        const uint64_t head = std::min<uint64_t>((uint64_t)n_patches, pcap - at);
+        std::copy(patches, patches + head, s->patches + at);
+        std::copy(patches + head, patches + n_patches, s->patches);
         const uint64_t seq = s->published;
         ServeReq q{};
         q.solver = (uint32_t)solver;
@@ -639,23 +650,32 @@ int gss_server_records(gss_server *s, int64_t id, const gss_serve_hit **out, int
     Done &d = it->second;
     if (!d.translated) {
         const int rw = d.step->rw;
-        d.recs.resize((size_t)d.r.n_records);
-        for (int64_t r = 0; r < d.r.n_records; r++) {
-            const uint64_t *src = d.step->data() + (d.first + (size_t)r) * rw;
+        // every field is written below: not cleared first
+        d.recs.reset(new gss_serve_hit[(size_t)d.r.n_records]);
+        const uint64_t *src = d.step->data() + d.first * rw;
+        const uint32_t w0 = d.step->absolute ? (uint32_t)d.r.first_word : 0u;
+        // records of one chunk of hits follow each other: mostly of one length
+        uint32_t at_len = UINT32_MAX;
+        const std::vector<int64_t> none, *ids = &none;
+        for (int64_t r = 0; r < d.r.n_records; r++, src += rw) {
             const uint32_t row = (uint32_t)src[0];
             const uint32_t len = (uint32_t)(src[0] >> 32) & 0xFFFFu;
+            if (len != at_len) {
+                at_len = len;
+                ids = len < s->ids.size() ? &s->ids[len] : &none;
+            }
             gss_serve_hit &h = d.recs[r];
-            h.clause = (len < s->ids.size() && row < s->ids[len].size()) ? s->ids[len][row] : -1;
-            h.word = (uint32_t)(src[0] >> 48) - (d.step->absolute ? (uint32_t)d.r.first_word : 0u);
+            h.clause = row < ids->size() ? (*ids)[row] : -1;
+            h.word = (uint32_t)(src[0] >> 48) - w0;
             h.pad = 0;
             h.false_mask = rw == 3 ? src[1] : 0;
             h.unit_mask = rw == 3 ? src[2] : 0;
         }
         d.translated = true;
         d.step.reset();  // the step's buffer goes once every request has its records
-        d.r.records = d.recs.data();
+        d.r.records = d.recs.get();
     }
-    *out = d.recs.data();
+    *out = d.recs.get();
     *n = d.r.n_records;
     return GSS_OK;
 }

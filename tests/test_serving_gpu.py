@@ -332,6 +332,50 @@ def test_native_loop_one_word_table():
             _same(_as_oracle(recs), _oracle_request(off, lits, N, d, t, k), f"request {rid}")
 
 
+@pytest.mark.parametrize("ring", [97, 256, 701])
+def test_patch_ring_wraps_and_restarts(ring):
+    """Patch rings that hold few requests: requests go round the ring's end, a
+    drained ring starts over, and requests without patches are in between; a
+    request that finds the ring full is sent again."""
+    rng = np.random.default_rng(ring)
+    V, N = 300, 1500
+    lens = rng.integers(1, 10, size=N).astype(np.int32)
+    lits = rng.integers(0, 2 * V, size=int(lens.sum())).astype(np.uint32)
+    off = np.zeros(N + 1, np.int64)
+    np.cumsum(lens, out=off[1:])
+    bd, bt = random_bases(rng, 3, V)
+    with sv.GpuServer(V, 3, words=16, patch_ring=ring) as srv:
+        assert srv.add_clauses(lits, lens) == 0
+        srv.update_base(base_updates(bd, bt))
+        sent, got, refused = [], {}, 0
+
+        def collect():
+            for rid in srv.poll(64, 2_000_000):
+                got[rid] = srv.result(rid)
+                srv.release(rid)
+
+        for i in range(24):
+            s_, k = i % 3, int(rng.integers(1, 130))
+            p = sv.slot_patches(rng, V, k, 6, 0.6)
+            p = p[p["word"] < (k + 63) // 64][:int(rng.integers(0, min(ring, 90)))]
+            p = p[:0] if i % 5 == 4 else p
+            rid = srv.submit(s_, k, p)
+            while rid is None:
+                refused += 1
+                collect()
+                rid = srv.submit(s_, k, p)
+            sent.append((rid, s_, k, p))
+            if i % 8 == 7:  # drained
+                while len(got) < len(sent):
+                    collect()
+        while len(got) < len(sent):
+            collect()
+        for rid, s_, k, p in sent:
+            d, t = _explicit_request(bd[s_], bt[s_], p, k)
+            _same(_as_oracle(got[rid][1]), _oracle_request(off, lits, N, d, t, k),
+                  f"request {rid}, {p.size} patches")
+
+
 @pytest.mark.parametrize("records", [sv.RECORDS_IDS, sv.RECORDS_FULL])
 def test_result_held_across_many_steps_keeps_its_records(records):
     """A client holds a finished request's result unread while 24 more

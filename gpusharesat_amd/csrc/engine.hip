@@ -1515,7 +1515,8 @@ int gss_hits_copy(gss_engine *e, gss_hit *out, int64_t cap, int64_t *n) {
     if (!out) return set_err(GSS_E_INVAL, "null output");
     // The chunks into a dense device buffer, then one D2H.
     if ((rc = e->d_dense.reserve((size_t)e->last_hits))) return rc;
-    HIP_TRY(launch_gather(sweep_chunks(e), e->d_dense.p, e->d_dense.cap, e->stream));
+    HIP_TRY(launch_gather(sweep_chunks(e), (uint64_t)e->last_hits, e->d_dense.p, e->d_dense.cap,
+                          e->stream));
     HIP_TRY(hipMemcpyAsync(out, e->d_dense.p, (size_t)want * sizeof(gss_hit),
                            hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1540,7 +1541,8 @@ int gss_hits_gather(gss_engine *e, gss_hit *d_out, int64_t cap, int64_t *n) {
                        e->last_chunks, kGatherMaxChunks);
     if (!e->last_hits) return GSS_OK;
     // the same kernel as gss_hits_copy, into the caller's array
-    HIP_TRY(launch_gather(sweep_chunks(e), d_out, (uint64_t)cap, e->stream));
+    HIP_TRY(launch_gather(sweep_chunks(e), (uint64_t)e->last_hits, d_out, (uint64_t)cap,
+                          e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
     return GSS_OK;
 }
@@ -1757,7 +1759,8 @@ static int queue_records_copy(gss_engine *e, StepSlot &sl, int64_t total) {
     }
     if ((uint64_t)total > sl.step_dense) {
         if ((rc = sl.d_dense.reserve_async((size_t)total, cs))) return rc;
-        HIP_TRY(launch_gather(step_chunks(sl, rw), sl.d_dense.p, (uint64_t)total, cs));
+        HIP_TRY(launch_gather(step_chunks(sl, rw), (uint64_t)total, sl.d_dense.p, (uint64_t)total,
+                              cs));
         sl.dense_want = std::max<uint64_t>(sl.dense_want, 2 * (uint64_t)total);
     }
     HIP_TRY(hipMemcpyAsync(sl.h_hits().p, sl.d_dense.p, (size_t)total * rw * sizeof(uint64_t),

@@ -267,8 +267,10 @@ hipError_t launch_assig_roll_dyn(const gss_var_update *ups, const int64_t *n, ui
 hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, hipStream_t s);
 // Dense copy of a sweep's records (chunk order, the records of a chunk in
 // place) when they all fit in dense_cap records; counts are read on the
-// device.  Chunk c starts at word c * kHitChunk * rec_words.
-hipError_t launch_gather(const ChunkArgs &c, void *dense, uint64_t dense_cap, hipStream_t s);
+// device (records = how many the host knows of, for the grid).  Chunk c starts
+// at word c * kHitChunk * rec_words.
+hipError_t launch_gather(const ChunkArgs &c, uint64_t records, void *dense, uint64_t dense_cap,
+                         hipStream_t s);
 // Dense copy of a sweep's records grouped by assignment word, ascending:
 // counts = 2 * 64 uint32 of device scratch (zero), group = 66 uint64:
 // group[w] = first record of word w, group[64] = all, group[65] = 1 if they

@@ -865,7 +865,11 @@ __global__ __launch_bounds__(256) void k_step_in(StepInArgs a) {
         if ((r == kRegClauses || r == kRegLits) && a.clauses) continue;
         const uint32_t *src = a.h[r];
         uint32_t *dst = a.d[r];
-        for (int64_t i = tid; i < h.region_words[r]; i += stride) dst[i] = src[i];
+        // short regions by different blocks, beside the updates' and the
+        // clauses': a trip over PCIe takes ~1.5 us, and a block's follow each other
+        int64_t i = tid + r * (stride / kStageRegions);
+        if (i >= stride) i -= stride;
+        for (; i < h.region_words[r]; i += stride) dst[i] = src[i];
     }
     const gss_base_update *bups = (const gss_base_update *)a.h[kRegBaseUps];
     for (int64_t i = tid; i < h.nbups; i += stride) base_update(bups[i], a.bases, a.bases_vw);
@@ -1034,19 +1038,62 @@ __device__ __forceinline__ void sum_fills(const uint32_t *__restrict__ fills, ui
     total = s_sum[1][0] + s_sum[1][1] + s_sum[1][2] + s_sum[1][3];
 }
 
+// Ends of 64 chunks' records (exclusive sums from the first one's start), from
+// a lane's chunk of `fill` records; the first wave writes them.
+__device__ __forceinline__ void fill_ends(uint32_t fill, uint32_t *ends) {
+    if (threadIdx.x < 64) ends[threadIdx.x] = (uint32_t)wave_incl_scan(fill, (int)threadIdx.x);
+}
+
+// The chunk that record i of the 64 is in: the first that ends after it.
+__device__ __forceinline__ uint32_t chunk_of(const uint32_t *ends, uint32_t i) {
+    uint32_t k = 0;
+#pragma unroll
+    for (uint32_t d = 32; d > 0; d >>= 1)
+        if (ends[k + d - 1] <= i) k += d;
+    return k;
+}
+
+// Words [0, m) of 64 chunks' records (ends: fill_ends) to dst, a thread per
+// word and four of them in flight.
+template <uint32_t RW>
+__device__ __forceinline__ void copy_words(const uint64_t *__restrict__ hits, const uint32_t *ends,
+                                           uint32_t m, uint64_t *__restrict__ dst) {
+    for (uint32_t i = threadIdx.x; i < m; i += 256 * 4) {
+        uint64_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t x = i + 256 * u;
+            if (x < m) {
+                const uint32_t k = chunk_of(ends, x / RW);
+                v[u] = hits[(uint64_t)k * kHitChunk * RW + x - (k ? ends[k - 1] : 0u) * RW];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (i + 256 * u < m) dst[i + 256 * u] = v[u];
+    }
+}
+
 // Block `blk` of `blocks` (256 threads) of the dense copy: its share of the
-// chunks, one wave per chunk, each to its place in the dense array.  Every
-// block sums the fills itself (32 KB from L2 for a sweep of ~8,000 waves): an
-// offsets kernel before this one took longer, on one CU, than the sums do.
-// Records go straight to `host` when they take at most host_words there (the
-// wait then has no copy to start), else to `dense` if they fit.
+// chunks to their place in the dense array.  Every block sums the fills itself
+// (32 KB from L2 for a sweep of ~8,000 waves): an offsets kernel before this
+// one took longer, on one CU, than the sums do.  Where chunks hold few records
+// (at most 128 on average: 40 in a screened step of 280,000) a thread copies a
+// word, whatever chunk it is in; with a wave per chunk the block's chunks were
+// a chain of reads (k_step_end of a step of 1,930 records: 10.5 us, now 7.6; of
+// 285,000: 25.9, now 21.6).  Full chunks take a wave each, without the search.  Records go straight to `host` when
+// they take at most host_words there (the wait then has no copy to start),
+// else to `dense` if they fit.
 __device__ __forceinline__ void gather_block(const ChunkArgs &c, uint32_t blk, uint32_t blocks,
                                              uint64_t *dense, uint64_t dense_cap, uint64_t *host,
                                              uint64_t host_words, uint32_t *out) {
+    __shared__ uint32_t s_end[64];
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint32_t n = chunks_held(c);
     const uint32_t per = (n + blocks - 1) / blocks;
     const uint32_t c0 = blk * per < n ? blk * per : n, c1 = c0 + per < n ? c0 + per : n;
     if (blk != 0 && c0 == c1) return;
+    uint32_t fill = c0 + lane < c1 ? c.fills[c0 + lane] : 0u;
     uint64_t at, total;
     sum_fills(c.fills, c0, n, at, total);
     if (out && blk == 0 && threadIdx.x == 0) write_counts(c, total, out);
@@ -1054,24 +1101,38 @@ __device__ __forceinline__ void gather_block(const ChunkArgs &c, uint32_t blk, u
     const uint32_t rw = c.rec_words;
     uint64_t *to = host && total * rw <= host_words ? host : total <= dense_cap ? dense : nullptr;
     if (!to) return;
-    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (uint32_t k = c0; k < c1; k++) {
-        const uint32_t f = c.fills[k];
-        if (f && (k & 3) == wv) {
-            const uint64_t *__restrict__ src = c.hits + (uint64_t)k * kHitChunk * rw;
-            uint64_t *__restrict__ dst = to + at * rw;
-            const uint32_t m = f * rw;
-            uint32_t i = lane;
-            for (; i + 64 * 3 < m; i += 64 * 4) {
-                uint64_t v[4];
+    for (uint32_t k0 = c0; k0 < c1; k0 += 64) {
+        const uint32_t held = c1 - k0 < 64 ? c1 - k0 : 64;
+        fill_ends(fill, s_end);
+        __syncthreads();
+        const uint32_t records = s_end[63];
+        const uint64_t *__restrict__ src = c.hits + (uint64_t)k0 * kHitChunk * rw;
+        uint64_t *__restrict__ dst = to + at * rw;
+        if (records <= 128 * held) {
+            if (rw == 1) copy_words<1>(src, s_end, records, dst);
+            else if (rw == 2) copy_words<2>(src, s_end, records * 2, dst);
+            else copy_words<3>(src, s_end, records * 3, dst);
+        } else {
+            for (uint32_t k = wv; k < held; k += 4) {
+                const uint32_t first = k ? s_end[k - 1] : 0u, m = (s_end[k] - first) * rw;
+                const uint64_t *__restrict__ x = src + (uint64_t)k * kHitChunk * rw;
+                uint64_t *__restrict__ y = dst + (uint64_t)first * rw;
+                uint32_t i = lane;
+                for (; i + 64 * 3 < m; i += 64 * 4) {
+                    uint64_t v[4];
 #pragma unroll
-                for (int u = 0; u < 4; u++) v[u] = src[i + 64 * u];
+                    for (int u = 0; u < 4; u++) v[u] = x[i + 64 * u];
 #pragma unroll
-                for (int u = 0; u < 4; u++) dst[i + 64 * u] = v[u];
+                    for (int u = 0; u < 4; u++) y[i + 64 * u] = v[u];
+                }
+                for (; i < m; i += 64) y[i] = x[i];
             }
-            for (; i < m; i += 64) dst[i] = src[i];
         }
-        at += f;
+        at += records;
+        if (k0 + 64 < c1) {  // more than 64 chunks in the block's share
+            fill = k0 + 64 + lane < c1 ? c.fills[k0 + 64 + lane] : 0u;
+            __syncthreads();  // everyone is done with the ends
+        }
     }
 }
 
@@ -1128,27 +1189,19 @@ __global__ __launch_bounds__(256) void k_step_end(ChunkArgs c, StepEndArgs a) {
 // ---- records grouped by assignment word (serving steps) ----------------------
 
 // f(record) for every record of the block's share of the chunks, a thread per
-// record: with a wave per chunk, the chunks' few records each (thousands of
-// chunks, ~10 records in one) were a chain of reads per wave.
+// record (as in gather_block).
 template <typename F>
 __device__ __forceinline__ void for_records(const ChunkArgs &ch, F &&f) {
-    __shared__ uint32_t s_end[64];  // records up to and with the group's chunk k
+    __shared__ uint32_t s_end[64];
     const uint32_t n = chunks_held(ch), rw = ch.rec_words;
     const uint32_t per = (n + gridDim.x - 1) / gridDim.x;
     const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < n ? c0 + per : n;
     for (uint32_t c = c0; c < c1; c += 64) {
-        if (threadIdx.x < 64) {
-            const uint32_t fill = c + threadIdx.x < c1 ? ch.fills[c + threadIdx.x] : 0u;
-            s_end[threadIdx.x] = (uint32_t)wave_incl_scan(fill, (int)threadIdx.x);
-        }
+        fill_ends(threadIdx.x < 64 && c + threadIdx.x < c1 ? ch.fills[c + threadIdx.x] : 0u, s_end);
         __syncthreads();
         const uint32_t total = s_end[63];
         for (uint32_t i = threadIdx.x; i < total; i += 256) {
-            uint32_t k = 0;  // the first chunk that ends after record i
-#pragma unroll
-            for (uint32_t d = 32; d > 0; d >>= 1)
-                if (s_end[k + d - 1] <= i) k += d;
-            const uint32_t at = i - (k ? s_end[k - 1] : 0u);
+            const uint32_t k = chunk_of(s_end, i), at = i - (k ? s_end[k - 1] : 0u);
             f(ch.hits + ((uint64_t)(c + k) * kHitChunk + at) * rw);
         }
         __syncthreads();
@@ -1624,9 +1677,14 @@ hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *nex
     return hipGetLastError();
 }
 
-hipError_t launch_gather(const ChunkArgs &c, void *dense, uint64_t dense_cap, hipStream_t s) {
+hipError_t launch_gather(const ChunkArgs &c, uint64_t records, void *dense, uint64_t dense_cap,
+                         hipStream_t s) {
     if (c.rec_words < 1 || c.rec_words > 3) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_gather, dim3(2048), dim3(256), 0, s, c, (uint64_t *)dense, dense_cap);
+    // a block per 16 KB of records (each block sums the fills: 28 KB for 7,168
+    // waves), at least one per CU and at most eight
+    const uint64_t want = records * c.rec_words / 2048;
+    const unsigned blocks = (unsigned)(want < 256 ? 256 : want < 2048 ? want : 2048);
+    hipLaunchKernelGGL(k_gather, dim3(blocks), dim3(256), 0, s, c, (uint64_t *)dense, dense_cap);
     return hipGetLastError();
 }
 

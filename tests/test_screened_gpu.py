@@ -1,0 +1,83 @@
+"""Screened steps (GSS_STEP_SCREEN) whose words mostly hold one value in all
+slots, against the oracle: literals known from the screening entries alone,
+true, false or undefined in all slots of a word group, beside literals whose
+rows have to be read, at clause lengths around the positions the check keeps
+apart (31), over steps that change the table and roll it forward.
+"""
+import numpy as np
+import pytest
+
+import _oracle as orc
+from gpusharesat_amd import serving as sv
+from gpusharesat_amd.engine import VAR_UPDATE_DTYPE
+
+pytestmark = pytest.mark.gpu
+
+ALL = np.uint64(0xFFFFFFFFFFFFFFFF)
+V = 400
+
+
+def planes(rng, words, sigma):
+    """Most variables one value in a word (true under sigma, false, undefined),
+    the same in its neighbours more often than not; a few differ in a slot."""
+    d = np.repeat(rng.random((V, (words + 3) // 4)) < 0.95, 4, axis=1)[:, :words]
+    t = np.where(rng.random((V, words)) < 0.99, sigma[:, None], ~sigma[:, None])
+    is_def = np.where(d, ALL, np.uint64(0))
+    is_true = np.where(d & t, ALL, np.uint64(0))
+    bit = np.uint64(1) << rng.integers(0, 64, size=(V, words), dtype=np.uint64)
+    is_def ^= np.where(rng.random((V, words)) < 0.02, bit, np.uint64(0))
+    is_true ^= np.where(rng.random((V, words)) < 0.02, bit, np.uint64(0))
+    return is_def, is_true & is_def
+
+
+@pytest.mark.parametrize("W", [1, 2, 4, 8, 16, 32, 64])
+def test_words_of_one_value(engine_factory, W):
+    rng = np.random.default_rng(500 + W)
+    sigma = rng.random(V) < 0.5
+    lens = np.concatenate([np.full(70, n, np.int32)
+                           for n in [*range(1, 9), 16, 30, 31, 32, 33, 34, 64, 130]])
+    v = rng.integers(0, V, size=int(lens.sum()))
+    false = rng.random(v.size) > 0.5 / np.repeat(lens, lens)
+    lits = (2 * v + (false == sigma[v])).astype(np.uint32)
+    off = np.zeros(lens.size + 1, np.int64)
+    off[1:] = np.cumsum(lens)
+    e = engine_factory()
+    rows = e.append(lits, lens).astype(np.uint64)
+    e.reset_assignments(V, W)
+    is_def, is_true = planes(rng, W, sigma)
+    e.upload(is_def, is_true)
+    units = 0
+    for step in range(4):
+        ups = np.zeros(0, VAR_UPDATE_DTYPE)
+        if step:  # changed words, rolled forward by the step before
+            cells = np.unique(rng.integers(0, V * W, size=V * W // 8))
+            nd, nt = planes(rng, W, sigma)
+            ups = np.zeros(cells.size, VAR_UPDATE_DTYPE)
+            ups["var"], ups["word"] = cells // W, cells % W
+            ups["is_def"], ups["is_true"] = nd.ravel()[cells], nt.ravel()[cells]
+            is_def.ravel()[cells], is_true.ravel()[cells] = ups["is_def"], ups["is_true"]
+        valid = np.full(W, ALL)
+        valid[-1] = np.uint64(0x7FFFFFFFFFFFFF0F)
+        if W > 2:
+            valid[step % W] = 0
+        last = np.full(W, 63, np.int8)
+        last[-1] = 62
+        exp = orc.sweep(off, lits, is_def, is_true, valid)
+        units += int((exp["unit_mask"] != 0).sum())
+        print(f"{W} words, step {step}: {ups.size} updates, {exp.size} records", flush=True)
+        sv.submit(e, valid, ups=ups, last_pos=last, flags=sv.STEP_SCREEN)
+        assert e.step_wait()[0] == exp.size
+        got = e.step_hits_view().view(np.uint64).reshape(-1, 3)
+        want = np.empty((exp.size, 3), np.uint64)
+        c = exp["clause"]
+        want[:, 0] = (rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
+                      | (exp["word"].astype(np.uint64) << np.uint64(48)))
+        want[:, 1], want[:, 2] = exp["false_mask"], exp["unit_mask"]
+        assert np.array_equal(got[np.argsort(got[:, 0])], want[np.argsort(want[:, 0])])
+        for k in range(ups.size):  # the roll forward: the word takes its last slot's value
+            x, w = int(ups["var"][k]), int(ups["word"][k])
+            b = np.uint64(int(last[w]))
+            one = np.uint64(1)
+            is_true[x, w] = ALL if (is_true[x, w] >> b) & one else np.uint64(0)
+            is_def[x, w] = ALL if (is_def[x, w] >> b) & one else np.uint64(0)
+    assert units > 50

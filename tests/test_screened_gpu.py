@@ -30,8 +30,12 @@ def planes(rng, words, sigma):
     return is_def, is_true & is_def
 
 
-@pytest.mark.parametrize("W", [1, 2, 4, 8, 16, 32, 64])
-def test_words_of_one_value(engine_factory, W):
+@pytest.mark.parametrize("W, used", [(1, [1] * 4), (2, [2] * 4), (4, [4] * 4), (8, [8] * 4),
+                                     (16, [16] * 4), (32, [32] * 4), (64, [64] * 4),
+                                     (16, [4, 4, 16, 9, 9]), (32, [17, 17, 8, 32, 32]),
+                                     (64, [3, 3, 34, 34, 20, 64, 64])])
+def test_words_of_one_value(engine_factory, W, used):
+    """`used` = words with valid slots at each step; updates go to any word."""
     rng = np.random.default_rng(500 + W)
     sigma = rng.random(V) < 0.5
     lens = np.concatenate([np.full(70, n, np.int32)
@@ -47,7 +51,7 @@ def test_words_of_one_value(engine_factory, W):
     is_def, is_true = planes(rng, W, sigma)
     e.upload(is_def, is_true)
     units = 0
-    for step in range(4):
+    for step, n_used in enumerate(used):
         ups = np.zeros(0, VAR_UPDATE_DTYPE)
         if step:  # changed words, rolled forward by the step before
             cells = np.unique(rng.integers(0, V * W, size=V * W // 8))
@@ -58,8 +62,9 @@ def test_words_of_one_value(engine_factory, W):
             is_def.ravel()[cells], is_true.ravel()[cells] = ups["is_def"], ups["is_true"]
         valid = np.full(W, ALL)
         valid[-1] = np.uint64(0x7FFFFFFFFFFFFF0F)
-        if W > 2:
-            valid[step % W] = 0
+        valid[n_used:] = 0
+        if n_used > 2:
+            valid[step % n_used] = 0
         last = np.full(W, 63, np.int8)
         last[-1] = 62
         exp = orc.sweep(off, lits, is_def, is_true, valid)

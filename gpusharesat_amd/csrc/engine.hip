@@ -432,7 +432,10 @@ struct gss_engine {
     std::vector<BucketDesc> desc_new, desc_up;
     const BucketDesc *desc_up_at = nullptr;
     std::vector<uint64_t> valid_up;
-    Pinned<uint32_t> h_count;  // [0] = chunks claimed, [1], [2] = records (low, high word)
+    // [0] = chunks claimed, [1], [2] = records (low, high word), [3] = sweep_seq
+    // once the sweep has ended and the others are there
+    Pinned<uint32_t> h_count;
+    uint32_t sweep_seq = 0;
     // host buffers that are only copy endpoints of at least this many bytes
     // are pageable (< 0: no limit); see Pinned
     int64_t page_limit = -1;
@@ -448,6 +451,7 @@ struct gss_engine {
     bool pending = false, waited = false, have_sweep = false;
     int64_t last_hits = 0;
     uint32_t last_chunks = 0;
+    bool time_due = false;  // the last waited sweep's time is still to be read (read_time)
     float last_ms = 0.f;
     double total_ms = 0.0;
     int64_t nsweeps = 0;
@@ -630,7 +634,33 @@ ChunkArgs sweep_chunks(const gss_engine *e) {
 }
 
 // Launches the sweep kernel for the current descriptors (already uploaded).
+// The kernel time of the last waited sweep, from its events.
+int read_time(gss_engine *e) {
+    if (!e->time_due) return GSS_OK;
+    e->time_due = false;
+    float ms = 0.f;
+    HIP_TRY(hipEventSynchronize(e->ev1));
+    HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
+    e->last_ms = ms;
+    e->total_ms += ms;
+    e->nsweeps++;
+    return GSS_OK;
+}
+
+// Waits until the queued sweep's counts are in h_count.
+hipError_t wait_counts(gss_engine *e) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 1;; i++) {
+        if (__atomic_load_n(&e->h_count.p[3], __ATOMIC_ACQUIRE) == e->sweep_seq) return hipSuccess;
+        __builtin_ia32_pause();
+        // long sweeps: the stream's wait, which also reports errors
+        if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2))
+            return hipStreamSynchronize(e->stream);
+    }
+}
+
 int launch_current_sweep(gss_engine *e) {
+    if (const int rc = read_time(e)) return rc;
     e->alloc_at ^= 1;
     e->sweep_waves = e->npasses > 0 ? (uint32_t)e->blocks * 4 : 0;
     HIP_TRY(hipEventRecord(e->ev0, e->stream));
@@ -654,7 +684,7 @@ int launch_current_sweep(gss_engine *e) {
     HIP_TRY(hipEventRecord(e->ev1, e->stream));
     // counts to pinned memory: the wait reads them there
     HIP_TRY(launch_count_records(sweep_chunks(e), e->h_count.p,
-                                 e->d_alloc + 8 * (e->alloc_at ^ 1), e->stream));
+                                 e->d_alloc + 8 * (e->alloc_at ^ 1), ++e->sweep_seq, e->stream));
     return GSS_OK;
 }
 
@@ -663,7 +693,12 @@ int reserve_chunks(gss_engine *e, uint64_t chunks) {
     int rc;
     if ((rc = e->d_hits.reserve((size_t)chunks * kHitChunk))) return rc;
     if ((rc = e->d_fills.reserve((size_t)chunks))) return rc;
-    if ((rc = e->h_count.reserve(4))) return rc;
+    if (!e->h_count.p) {
+        if ((rc = e->h_count.reserve(4))) return rc;
+        // pinned memory comes back with what an engine before left in it, its
+        // sweep number included; this engine's numbers start at 1
+        e->h_count.p[3] = 0;
+    }
     e->chunk_cap = (uint32_t)std::min<size_t>(e->d_fills.cap, e->d_hits.cap / kHitChunk);
     return GSS_OK;
 }
@@ -1461,7 +1496,7 @@ int gss_sweep_wait(gss_engine *e, int64_t *n_hits) {
     if (rc) return rc;
     if (!e->pending) return set_err(GSS_E_STATE, "no sweep in flight");
     for (;;) {
-        HIP_TRY(hipStreamSynchronize(e->stream));
+        HIP_TRY(wait_counts(e));
         const uint32_t used = e->h_count.p[0];
         if (used <= e->chunk_cap) {
             e->last_chunks = used;
@@ -1488,11 +1523,7 @@ int gss_sweep_wait(gss_engine *e, int64_t *n_hits) {
     }
     e->pending = false;
     e->waited = true;
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, e->ev0, e->ev1));
-    e->last_ms = ms;
-    e->total_ms += ms;
-    e->nsweeps++;
+    e->time_due = true;
     const int64_t tot = (int64_t)((uint64_t)e->h_count.p[1] | ((uint64_t)e->h_count.p[2] << 32));
     e->last_hits = tot;
     if (n_hits) *n_hits = tot;
@@ -1549,12 +1580,14 @@ int gss_hits_gather(gss_engine *e, gss_hit *d_out, int64_t cap, int64_t *n) {
 
 int gss_sweep_kernel_ms(gss_engine *e, float *ms) {
     if (!e || !ms) return set_err(GSS_E_INVAL, "null argument");
+    if (const int rc = read_time(e)) return rc;
     *ms = e->last_ms;
     return GSS_OK;
 }
 
 int gss_sweep_kernel_stats(gss_engine *e, double *total_ms, int64_t *count, int reset) {
     if (!e) return set_err(GSS_E_INVAL, "null engine");
+    if (const int rc = read_time(e)) return rc;
     if (total_ms) *total_ms = e->total_ms;
     if (count) *count = e->nsweeps;
     if (reset) {
@@ -1618,6 +1651,7 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
         e->tune_waves_per_cu = c.wpc;
         e->tune_schedule = c.sched;
     };
+    if ((rc = read_time(e))) return rc;
     double total0 = e->total_ms;
     int64_t count0 = e->nsweeps;
     Cfg best_cfg = saved;
@@ -1627,7 +1661,7 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
         apply(c);
         std::vector<float> ts;
         for (int r = 0; r < reps + 1; r++) {
-            if ((rc = gss_sweep(e, valid, nullptr))) {
+            if ((rc = gss_sweep(e, valid, nullptr)) || (rc = read_time(e))) {
                 apply(saved);
                 return rc;
             }

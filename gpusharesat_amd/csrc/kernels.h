@@ -264,7 +264,8 @@ hipError_t launch_assig_roll_dyn(const gss_var_update *ups, const int64_t *n, ui
                                  int words, const int8_t *last_pos, hipStream_t s);
 // Counts of a plain sweep to pinned host memory (write_counts in
 // kernels.hip); next = the counters of the sweep after it, cleared.
-hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, hipStream_t s);
+hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, uint32_t seq,
+                                hipStream_t s);
 // Dense copy of a sweep's records (chunk order, the records of a chunk in
 // place) when they all fit in dense_cap records; counts are read on the
 // device (records = how many the host knows of, for the grid).  Chunk c starts

@@ -1225,8 +1225,10 @@ __global__ __launch_bounds__(256) void k_gather(ChunkArgs c, uint64_t *dense, ui
 
 // Counts of a plain sweep to pinned memory.  The counters are read by the
 // gather after it; the next sweep starts from `next`, cleared here.
-__global__ __launch_bounds__(1024) void k_count_records(ChunkArgs c, uint32_t *out,
-                                                        uint32_t *next) {
+// `seq` goes to out[3] last: the host waits for it there (ending with the
+// stream's own wait instead took 7 us more).
+__global__ __launch_bounds__(1024) void k_count_records(ChunkArgs c, uint32_t *out, uint32_t *next,
+                                                        uint32_t seq) {
     __shared__ uint64_t part[16];
     const uint32_t n = chunks_held(c);
     uint64_t sum = 0;
@@ -1245,6 +1247,7 @@ __global__ __launch_bounds__(1024) void k_count_records(ChunkArgs c, uint32_t *o
         for (int i = 0; i < 16; i++) t += part[i];
         write_counts(c, t, out);
         next[0] = next[1] = 0;
+        __hip_atomic_store(out + 3, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1786,8 +1789,9 @@ hipError_t launch_assig_roll_dyn(const gss_var_update *ups, const int64_t *n, ui
     return hipGetLastError();
 }
 
-hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, hipStream_t s) {
-    hipLaunchKernelGGL(k_count_records, dim3(1), dim3(1024), 0, s, c, out, next);
+hipError_t launch_count_records(const ChunkArgs &c, uint32_t *out, uint32_t *next, uint32_t seq,
+                                hipStream_t s) {
+    hipLaunchKernelGGL(k_count_records, dim3(1), dim3(1024), 0, s, c, out, next, seq);
     return hipGetLastError();
 }
 

@@ -113,3 +113,16 @@ def test_records_around_the_direct_size(engine_factory, form, words):
             assert got.size == m and np.array_equal(rows, np.arange(m)), (k, m)
     assert e.step_wait()[0] == totals[-1]
     assert np.array_equal(np.sort(view()["row"]), np.arange(totals[-1]))
+
+
+def test_first_sweeps_of_engines_in_turn():
+    """Engines that run one sweep each and go: a new engine's first wait must not
+    take what the one before left in the pinned counts it is handed again."""
+    from gpusharesat_amd.engine import Engine
+    for n in (100, 7000, 3, 50000, 1, 900):
+        e = Engine(0)
+        e.reset_assignments(64, 1)
+        e.append(np.full(n, 2, np.uint32), np.ones(n, np.int32))
+        assert e.sweep(np.full(1, ALL)) == n
+        assert np.array_equal(np.sort(e.hits()["row"]), np.arange(n))
+        e.close()

@@ -451,6 +451,12 @@ struct gss_engine {
     bool pending = false, waited = false, have_sweep = false;
     int64_t last_hits = 0;
     uint32_t last_chunks = 0;
+    // plain sweeps that may be screened (k_sweep_choose): entries, the words of
+    // each group ([8]: the choice), and passes of 64 clauses
+    DevBuf<uint32_t> sweep_agg;
+    DevBuf<uint64_t> sweep_agg_words;
+    int screen_passes = 0;
+    bool may_screen = false;
     bool time_due = false;  // the last waited sweep's time is still to be read (read_time)
     float last_ms = 0.f;
     double total_ms = 0.0;
@@ -659,6 +665,21 @@ hipError_t wait_counts(gss_engine *e) {
     }
 }
 
+// Whether a plain sweep may gain from screening, were its words' slots mostly of
+// one value (the device decides that: k_sweep_choose).  In microseconds, with
+// that: the plain kernel reads 2.8 rows a clause (52 per million of one line
+// each), the screened one takes 24 per million clauses after a pass over the
+// table (5.5 TB/s); 12 are kept for the launches.  Measured, plain and screened
+// with its entries: 1M clauses x 8 words x 100K variables 43 and 27, 2M x 16 x
+// 500K 118 and 71, 400K x 64 x 200K 87 and 68.  Where the slots differ the
+// two launches that find out cost 7.
+bool screening_may_pay(const gss_engine *e) {
+    if (e->words < 8 || e->vars <= 0) return false;
+    const double m = (double)e->total_clauses * 1e-6;
+    const double rows = (double)e->vars * 2.0 * e->words * 8.0;
+    return 52.0 * m * std::max(1, e->words / 16) > 24.0 * m + rows / 5.5e6 + 12.0;
+}
+
 int launch_current_sweep(gss_engine *e) {
     if (const int rc = read_time(e)) return rc;
     e->alloc_at ^= 1;
@@ -679,6 +700,18 @@ int launch_current_sweep(gss_engine *e) {
         a.alloc = e->d_alloc + 8 * e->alloc_at;
         a.chunk_cap = e->chunk_cap;
         a.rec_words = 3;
+        if (e->may_screen) {
+            uint32_t *choose = (uint32_t *)(e->sweep_agg_words.p + 8);
+            HIP_TRY(launch_sweep_choose(e->table.p, e->d_valid, e->vars, e->words, e->sweep_agg.p,
+                                        e->sweep_agg_words.p, choose, e->stream));
+            a.choose = choose;
+            SweepArgs b = a;
+            b.npasses = e->screen_passes;
+            b.task_passes = task_passes(e, true);
+            b.agg = e->sweep_agg.p;
+            b.agg_words = e->sweep_agg_words.p;
+            HIP_TRY(launch_sweep(b, e->words, e->blocks, e->stream));
+        }
         HIP_TRY(launch_sweep(a, e->words, e->blocks, e->stream));
     }
     HIP_TRY(hipEventRecord(e->ev1, e->stream));
@@ -799,6 +832,8 @@ int gss_engine_destroy(gss_engine *e) {
     e->table.release();
     e->bases.release();
     e->d_desc.release();
+    e->sweep_agg.release();
+    e->sweep_agg_words.release();
     e->d_hits.release();
     e->d_fills.release();
     e->d_stage.release();
@@ -1408,7 +1443,7 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
         if (e->buckets[len].count) nb++;
     if ((rc = e->h_desc.reserve(std::max(nb, 1))) || (rc = e->d_desc.reserve(std::max(nb, 1))))
         return rc;
-    int64_t passes = 0;
+    int64_t passes = 0, screen_passes = 0;
     e->desc_new.clear();
     const size_t nlen = e->buckets.size();
     for (size_t i = 1; i < nlen; i++) {
@@ -1426,13 +1461,15 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
         d.len = (uint32_t)len;
         d.count = (uint32_t)b.count;
         d.pass_begin = (uint32_t)passes;
-        d.pad = 0;
+        d.screen_begin = (uint32_t)screen_passes;
         e->desc_new.push_back(d);
         passes += (b.count + cpp - 1) / cpp;
+        screen_passes += (b.count + 63) / 64;
     }
     if (passes > 0x7FFFFFFF) return set_err(GSS_E_INVAL, "too many clauses");
     e->nbuckets = nb;
     e->npasses = (int)passes;
+    e->screen_passes = (int)screen_passes;
     int active_words = 0;
     for (int w = 0; w < W; w++)
         if (valid[w]) active_words++;
@@ -1482,6 +1519,13 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
     }
     if (e->tune_max_chunks > 0) chunks = std::min<uint64_t>(chunks, e->tune_max_chunks);
     if (chunks > e->chunk_cap && (rc = reserve_chunks(e, chunks))) return rc;
+    // (no room for the entries: the plain kernel)
+    e->may_screen = screening_may_pay(e);
+    if (e->may_screen && (e->sweep_agg.reserve_async((size_t)e->vars + 1, e->stream) ||
+                          e->sweep_agg_words.reserve_async(9, e->stream))) {
+        e->may_screen = false;
+        (void)hipGetLastError();
+    }
     if ((rc = launch_current_sweep(e))) return rc;
     e->sweep_rows_version = e->rows_version;
     e->sweep_state_version = e->state_version;
@@ -2456,8 +2500,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         d.lits = b.d;
         d.len = (uint32_t)len;
         d.count = (uint32_t)b.count;
-        d.pass_begin = (uint32_t)t;
-        d.pad = 0;
+        d.pass_begin = d.screen_begin = (uint32_t)t;
         t += (b.count + cpp - 1) / cpp;
     }
     StepHeader &h = *sl.h_hdr.p;

@@ -16,8 +16,8 @@ struct BucketDesc {
                            // row offsets (literal << 7)
     uint32_t len;
     uint32_t count;        // rows
-    uint32_t pass_begin;   // first wave pass of this bucket
-    uint32_t pad;
+    uint32_t pass_begin;   // first wave pass of this bucket: plain sweeps (64 / words clauses
+    uint32_t screen_begin; // a pass) and screened ones (64)
 };
 
 struct SweepArgs {
@@ -49,6 +49,9 @@ struct SweepArgs {
     // other words.
     const uint32_t *agg;
     const uint64_t *agg_words;  // [8]
+    // launch_sweep_choose's: the plain kernel runs where it is 0, the screened
+    // one elsewhere (null: whichever is launched)
+    const uint32_t *choose;
 };
 
 // Staged regions of a batched step, read by k_step_in.
@@ -190,6 +193,11 @@ struct StepInArgs {
     ServeReport *report;  // pinned
 };
 
+// Plain sweeps, words >= 8: decides from a sample of the table whether the sweep
+// is screened (*choose), and if so builds the entries and agg_words.
+hipError_t launch_sweep_choose(const uint64_t *table, const uint64_t *valid, int64_t vars,
+                               int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
+                               hipStream_t s);
 // Screening entries of a batched step from the table itself (SweepArgs::agg):
 // group b = words [b * words / 8, (b + 1) * words / 8) (one word per group
 // below 8 words), over every slot of its words (valid or not: what holds in

@@ -168,11 +168,17 @@ __device__ __forceinline__ Lits<W> load_lits(LitPtr cl, int base, int len,
 
 // Bucket of pass p: the last one whose first pass is <= p.  One lane per
 // bucket (a binary search is a chain of 6-9 dependent scalar loads).
+template <bool SCREENED>
+__device__ __forceinline__ uint32_t pass_begin(const BucketDesc &b) {
+    return SCREENED ? b.screen_begin : b.pass_begin;
+}
+
+template <bool SCREENED>
 __device__ __forceinline__ int find_bucket(const BucketDesc *__restrict__ b, int nb, int p,
                                            int lane) {
     int n = 0;
     for (int i = 0; i < nb; i += 64) {
-        const bool le = i + lane < nb && (int)b[i + lane].pass_begin <= p;
+        const bool le = i + lane < nb && (int)pass_begin<SCREENED>(b[i + lane]) <= p;
         n += __popcll(__ballot(le));
     }
     return uniform(n - 1);
@@ -292,21 +298,21 @@ struct Run {
 };
 
 // Calls run(Run) for every run of passes that belongs to this wave.
-template <int CPW, typename F>
+template <int CPW, bool SCREENED, typename F>
 __device__ __forceinline__ void walk(const SweepArgs &a, const Passes &ps, int lane, F &&run) {
     for (int64_t t = ps.gw;; t += ps.nw) {
         const int64_t first = t * ps.tp;
         if (first >= ps.total) break;
         int p = (int)first;
         const int end = ps.total - p < ps.tp ? ps.total : p + ps.tp;
-        int bi = find_bucket(a.buckets, ps.nbuckets, p, lane);
+        int bi = find_bucket<SCREENED>(a.buckets, ps.nbuckets, p, lane);
         while (p < end) {
             const BucketDesc d = a.buckets[bi];
             Run r;
             r.lits = (LitPtr)uniform64((uint64_t)d.lits);
             r.len = uniform((int)d.len);
             r.count = uniform((int)d.count);
-            r.first = p - uniform((int)d.pass_begin);
+            r.first = p - uniform((int)pass_begin<SCREENED>(d));
             const int have = (r.count - 1) / CPW + 1 - r.first;
             r.n = end - p < have ? end - p : have;
             const int n = r.n;
@@ -332,6 +338,7 @@ __device__ __forceinline__ void walk(const SweepArgs &a, const Passes &ps, int l
 // by the number of live lanes read as few rows but spilled: 845 us.
 template <int W, bool CLAUSES>
 __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
+    if (a.choose && *a.choose) return;  // the screened kernel's
     using L = Lits<W>;
     constexpr int CPW = 64 / W;  // clauses per wave pass
     constexpr int H = L::kHeld;
@@ -346,7 +353,7 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
     const Passes ps(a);
     HitWriter out(a, ps);
 
-    walk<CPW>(a, ps, lane, [&](const Run &run) {
+    walk<CPW, false>(a, ps, lane, [&](const Run &run) {
         const int len = run.len, n = run.n;
         const int row0 = run.first * CPW;   // of the run's first pass
         const int left = run.count - row0;  // rows from there on
@@ -638,6 +645,7 @@ __device__ __forceinline__ void check_words(LitPtr cl, int len,
 // idle: a clause survives in one or two of its eight word groups.
 template <int W, bool CLAUSES>
 __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k_sweep_screened(SweepArgs a) {
+    if (a.choose && !*a.choose) return;  // the plain kernel's
     constexpr int P = W == 1 ? 1 : 2;  // words of an item
     __shared__ uint64_t s_valid[W], s_words[4][64], s_hit[4][64];
     __shared__ uint32_t s_start[4][64], s_group[W];
@@ -656,7 +664,7 @@ __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k
     const Passes ps(a);
     HitWriter out(a, ps);
 
-    walk<64>(a, ps, lane, [&](const Run &run) {
+    walk<64, true>(a, ps, lane, [&](const Run &run) {
         const int len = run.len, count = run.count;
         for (int pass = 0; pass < run.n; pass++) {
             const int row0 = (run.first + pass) * 64;
@@ -1402,38 +1410,35 @@ __device__ __forceinline__ void group_fold(const uint64_t *__restrict__ row, int
 // for the narrow tables, whose rows are neighbours), took 490 us for 1 GB; now
 // 185, 5.5 TB/s.
 template <int W>
-__global__ __launch_bounds__(256) void k_table_agg(const uint64_t *__restrict__ table,
-                                                   const StepHeader *__restrict__ dh,
-                                                   int64_t vars, uint32_t *__restrict__ agg) {
-    if (dh->halted) return;  // the aggregate stays the halted step's
-    if constexpr (W <= 8) {
-        for (int64_t v = blockIdx.x * 256ll + threadIdx.x; v < vars; v += gridDim.x * 256ll) {
-            const uint64_t *f = table + (size_t)v * 2 * W, *t = f + W;
+struct TableEntries {
+    static constexpr int VARS = W <= 8 ? 64 : W == 16 ? 8 : 4;  // per turn of a wave
+
+    // Entry of variable v0 + lane * step, in the first VARS lanes.
+    static __device__ __forceinline__ uint32_t turn(const uint64_t *__restrict__ table, int64_t v0,
+                                                    int64_t step, int64_t vars, int lane) {
+        if constexpr (W <= 8) {
+            if (v0 + lane * step >= vars) return 0;
+            const uint64_t *f = table + (size_t)(v0 + lane * step) * 2 * W, *t = f + W;
             uint32_t x = 0;
 #pragma unroll
             for (int b = 0; b < W; b++)
                 x |= ((f[b] == ~0ull ? 1u : 0u) | (t[b] == 0 ? 0x100u : 0u) |
                       (t[b] == ~0ull ? 0x10000u : 0u) | (f[b] == 0 ? 0x1000000u : 0u))
                      << b;
-            agg[v] = x;
-        }
-    } else {
-        constexpr int VARS = W == 16 ? 8 : 4;        // per turn of a wave
-        constexpr int LINES = VARS * 2 * W / 64;     // of 64 words
-        const int lane = (int)__lane_id();
-        const int64_t total = vars * 2 * W;
-        // lane 8 k + b: group b of the entry's field k (literal v non-false /
-        // true, ~v non-false / true)
-        const int k = (lane >> 3) & 3, first = (lane & 7) * (W / 8);
-        const uint64_t words = ((1ull << (W / 8)) - 1ull) << first;
-        for (int64_t v0 = (blockIdx.x * 4ll + (threadIdx.x >> 6)) * VARS; v0 < vars;
-             v0 += gridDim.x * 4ll * VARS) {
+            return x;
+        } else {
+            constexpr int LINES = VARS * 2 * W / 64;  // of 64 words
+            // lane 8 k + b: group b of the entry's field k (literal v non-false /
+            // true, ~v non-false / true)
+            const int k = (lane >> 3) & 3, first = (lane & 7) * (W / 8);
+            const uint64_t words = ((1ull << (W / 8)) - 1ull) << first;
             uint64_t x[LINES];
             uint32_t out = 0;
 #pragma unroll
             for (int l = 0; l < LINES; l++) {
-                const int64_t at = v0 * 2 * W + l * 64 + lane;
-                x[l] = at < total ? table[at] : 0ull;
+                const int o = l * 64 + lane;
+                const int64_t at = (v0 + o / (2 * W) * (step - 1)) * 2 * W + o;
+                x[l] = at < vars * 2 * W ? table[at] : 0ull;
             }
 #pragma unroll
             for (int j = 0; j < VARS; j++) {
@@ -1445,8 +1450,72 @@ __global__ __launch_bounds__(256) void k_table_agg(const uint64_t *__restrict__ 
                 const uint32_t e = (uint32_t)__ballot((~m & words) == 0);
                 if (lane == j) out = e;
             }
-            if (lane < VARS && v0 + lane < vars) agg[v0 + lane] = out;
+            return out;
         }
+    }
+};
+
+template <int W>
+__global__ __launch_bounds__(256) void k_table_agg(const uint64_t *__restrict__ table,
+                                                   const StepHeader *__restrict__ dh,
+                                                   int64_t vars, uint32_t *__restrict__ agg) {
+    if (dh->halted) return;  // the aggregate stays the halted step's
+    constexpr int VARS = TableEntries<W>::VARS;
+    const int lane = (int)__lane_id();
+    for (int64_t v0 = (blockIdx.x * 4ll + (threadIdx.x >> 6)) * VARS; v0 < vars;
+         v0 += gridDim.x * 4ll * VARS) {
+        const uint32_t e = TableEntries<W>::turn(table, v0, 1, vars, lane);
+        if (lane < VARS && v0 + lane < vars) agg[v0 + lane] = e;
+    }
+}
+
+// Whether a plain sweep is screened, and the entries if it is.  The screened
+// kernel pays where entries know what a variable is (true or false in all
+// slots of a group): each block looks at the same 16 to 256 variables spread
+// over the table, and where kScreenKnown in 100 of their groups are known the
+// entries are built and *choose is 1; else *choose is 0 and nothing is.
+// Plain against screened, entries included, by the share that is known: 400K
+// clauses x 4096 slots 89 and 75 us at 58 %, 92 and 83 at 48, 95 and 94 at 38;
+// 1M x 333 slots 55 and 42 at 44 %; 2M x 1024 slots 149 and 94 at 55 %, 119 and
+// 73 at 88; random slots (nothing known) 4M x 1024 615 and 1460.
+constexpr int kScreenKnown = 40;
+template <int W>
+__global__ __launch_bounds__(256) void k_sweep_choose(const uint64_t *__restrict__ table,
+                                                      const uint64_t *__restrict__ valid,
+                                                      int64_t vars, uint32_t *__restrict__ agg,
+                                                      uint64_t *__restrict__ agg_words,
+                                                      uint32_t *choose) {
+    static_assert(W >= 8, "eight groups");
+    constexpr int VARS = TableEntries<W>::VARS;
+    __shared__ int s_known[4], s_of[4];
+    const int lane = (int)__lane_id(), wv = (int)(threadIdx.x >> 6);
+    {
+        const int64_t v0 = vars / 4 * wv, step = vars / (4 * VARS) + (vars < 4 * VARS);
+        const uint32_t e = TableEntries<W>::turn(table, v0, step, vars, lane);
+        const bool in = lane < VARS && v0 + lane * step < vars;
+        int known = in ? __popc(((e >> 8) | (e >> 24)) & 0xFFu) : 0;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) known += __shfl_xor(known, d);
+        const int of = 8 * __popcll(__ballot(in));
+        if (lane == 0) {
+            s_known[wv] = known;
+            s_of[wv] = of;
+        }
+    }
+    __syncthreads();
+    const int known = s_known[0] + s_known[1] + s_known[2] + s_known[3];
+    const bool screen = known * 100 >= kScreenKnown * (s_of[0] + s_of[1] + s_of[2] + s_of[3]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *choose = screen ? 1u : 0u;
+    if (!screen) return;
+    if (blockIdx.x == 0 && threadIdx.x < 8) {
+        uint64_t m = 0;
+        for (int w = (int)threadIdx.x * (W / 8); w < ((int)threadIdx.x + 1) * (W / 8); w++)
+            if (valid[w]) m |= 1ull << w;
+        agg_words[threadIdx.x] = m;
+    }
+    for (int64_t v0 = (blockIdx.x * 4ll + wv) * VARS; v0 < vars; v0 += gridDim.x * 4ll * VARS) {
+        const uint32_t e = TableEntries<W>::turn(table, v0, 1, vars, lane);
+        if (lane < VARS && v0 + lane < vars) agg[v0 + lane] = e;
     }
 }
 
@@ -1830,6 +1899,23 @@ hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t
         return hipGetLastError();                                                           \
     }
     GSS_WORDS(X)
+#undef X
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_sweep_choose(const uint64_t *table, const uint64_t *valid, int64_t vars,
+                               int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
+                               hipStream_t s) {
+    if (vars <= 0 || words < 8) return hipErrorInvalidValue;
+    const int64_t per = words == 8 ? 256 : words == 16 ? 32 : 16;  // variables a block takes
+    const unsigned blocks = (unsigned)std::min<int64_t>((vars + per - 1) / per, 2048);
+#define X(W_)                                                                                \
+    if (words == W_) {                                                                       \
+        hipLaunchKernelGGL(k_sweep_choose<W_>, dim3(blocks), dim3(256), 0, s, table, valid, \
+                           vars, agg, agg_words, choose);                                    \
+        return hipGetLastError();                                                            \
+    }
+    X(8) X(16) X(32) X(64)
 #undef X
     return hipErrorInvalidValue;
 }

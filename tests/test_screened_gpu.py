@@ -2,7 +2,9 @@
 slots, against the oracle: literals known from the screening entries alone,
 true, false or undefined in all slots of a word group, beside literals whose
 rows have to be read, at clause lengths around the positions the check keeps
-apart (31), over steps that change the table and roll it forward.
+apart (31), over steps that change the table and roll it forward.  And plain
+sweeps of so many clauses that they may be screened too, over tables whose slots
+agree, differ, or agree for a share of the variables.
 """
 import numpy as np
 import pytest
@@ -86,3 +88,39 @@ def test_words_of_one_value(engine_factory, W, used):
             is_true[x, w] = ALL if (is_true[x, w] >> b) & one else np.uint64(0)
             is_def[x, w] = ALL if (is_def[x, w] >> b) & one else np.uint64(0)
     assert units > 50
+
+
+@pytest.mark.parametrize("agree", [1.0, 0.42, 0.38, 0.0])
+@pytest.mark.parametrize("W, n", [(8, 450_000), (16, 450_000), (32, 160_000), (64, 80_000)])
+def test_plain_sweeps_that_may_be_screened(engine_factory, W, n, agree):
+    rng = np.random.default_rng(W + int(100 * agree))
+    sigma = rng.random(V) < 0.5
+    lens = rng.integers(1, 6, size=n).astype(np.int32)
+    v = rng.integers(0, V, size=int(lens.sum()))
+    # mostly true literals: few records
+    lits = (2 * v + ((rng.random(v.size) < 0.15) == sigma[v])).astype(np.uint32)
+    off = np.zeros(n + 1, np.int64)
+    off[1:] = np.cumsum(lens)
+    is_def = np.full((V, W), ALL)
+    is_true = np.repeat(np.where(sigma, ALL, np.uint64(0))[:, None], W, axis=1)
+    mixed = rng.random(V) >= agree
+    is_def[mixed] &= rng.integers(0, 1 << 63, size=(int(mixed.sum()), W), dtype=np.uint64)
+    is_true &= is_def
+    valid = np.full(W, ALL)
+    valid[1] = 0
+    valid[-1] = np.uint64(0x7FFFFFFFFFFFFF0F)
+    exp = orc.sweep(off, lits, is_def, is_true, valid)
+    e = engine_factory()
+    rows = e.append(lits, lens).astype(np.uint64)
+    e.reset_assignments(V, W)
+    e.upload(is_def, is_true)
+    print(f"{W} words, {agree} agree: {exp.size} records", flush=True)
+    for _ in range(2):
+        assert e.sweep(valid) == exp.size
+        got = e.hits().view(np.uint64).reshape(-1, 3)
+        want = np.empty((exp.size, 3), np.uint64)
+        c = exp["clause"]
+        want[:, 0] = (rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
+                      | (exp["word"].astype(np.uint64) << np.uint64(48)))
+        want[:, 1], want[:, 2] = exp["false_mask"], exp["unit_mask"]
+        assert np.array_equal(got[np.argsort(got[:, 0])], want[np.argsort(want[:, 0])])

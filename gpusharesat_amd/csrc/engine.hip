@@ -287,6 +287,7 @@ struct StepPlan {
     bool serve = false, screen = false;
     bool agg_full = false;   // screened: the entries are rebuilt from the table
     bool agg_fused = false;  // screened: the applying and rolling kernels refresh them
+    bool may_screen = false;  // not a screened step, but screened where that pays
     bool staged = false;     // clauses are copied by a kernel of their own
     bool loads = false;      // word loads
     bool patches = false;
@@ -673,11 +674,35 @@ hipError_t wait_counts(gss_engine *e) {
 // with its entries: 1M clauses x 8 words x 100K variables 43 and 27, 2M x 16 x
 // 500K 118 and 71, 400K x 64 x 200K 87 and 68.  Where the slots differ the
 // two launches that find out cost 7.
-bool screening_may_pay(const gss_engine *e) {
+// Also false without room for the entries.
+bool screening_may_pay(gss_engine *e, int64_t clauses) {
     if (e->words < 8 || e->vars <= 0) return false;
-    const double m = (double)e->total_clauses * 1e-6;
+    const double m = (double)clauses * 1e-6;
     const double rows = (double)e->vars * 2.0 * e->words * 8.0;
-    return 52.0 * m * std::max(1, e->words / 16) > 24.0 * m + rows / 5.5e6 + 12.0;
+    if (52.0 * m * std::max(1, e->words / 16) <= 24.0 * m + rows / 5.5e6 + 12.0) return false;
+    if (e->sweep_agg.reserve_async((size_t)e->vars + 1, e->stream) ||
+        e->sweep_agg_words.reserve_async(9, e->stream)) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+// Before a sweep a that may be screened: the choice, and the screened kernel if
+// that is it (a is launched after it, and runs if it is not).
+hipError_t launch_screened_choice(gss_engine *e, const uint64_t *valid, SweepArgs &a, int blocks,
+                                  hipStream_t s) {
+    uint32_t *choose = (uint32_t *)(e->sweep_agg_words.p + 8);
+    hipError_t he = launch_sweep_choose(e->table.p, valid, e->vars, e->words, e->sweep_agg.p,
+                                        e->sweep_agg_words.p, choose, s);
+    if (he != hipSuccess) return he;
+    a.choose = choose;
+    SweepArgs b = a;
+    b.npasses = e->screen_passes;
+    b.task_passes = task_passes(e, true);
+    b.agg = e->sweep_agg.p;
+    b.agg_words = e->sweep_agg_words.p;
+    return launch_sweep(b, e->words, blocks, s);
 }
 
 int launch_current_sweep(gss_engine *e) {
@@ -700,18 +725,7 @@ int launch_current_sweep(gss_engine *e) {
         a.alloc = e->d_alloc + 8 * e->alloc_at;
         a.chunk_cap = e->chunk_cap;
         a.rec_words = 3;
-        if (e->may_screen) {
-            uint32_t *choose = (uint32_t *)(e->sweep_agg_words.p + 8);
-            HIP_TRY(launch_sweep_choose(e->table.p, e->d_valid, e->vars, e->words, e->sweep_agg.p,
-                                        e->sweep_agg_words.p, choose, e->stream));
-            a.choose = choose;
-            SweepArgs b = a;
-            b.npasses = e->screen_passes;
-            b.task_passes = task_passes(e, true);
-            b.agg = e->sweep_agg.p;
-            b.agg_words = e->sweep_agg_words.p;
-            HIP_TRY(launch_sweep(b, e->words, e->blocks, e->stream));
-        }
+        if (e->may_screen) HIP_TRY(launch_screened_choice(e, e->d_valid, a, e->blocks, e->stream));
         HIP_TRY(launch_sweep(a, e->words, e->blocks, e->stream));
     }
     HIP_TRY(hipEventRecord(e->ev1, e->stream));
@@ -1519,13 +1533,7 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
     }
     if (e->tune_max_chunks > 0) chunks = std::min<uint64_t>(chunks, e->tune_max_chunks);
     if (chunks > e->chunk_cap && (rc = reserve_chunks(e, chunks))) return rc;
-    // (no room for the entries: the plain kernel)
-    e->may_screen = screening_may_pay(e);
-    if (e->may_screen && (e->sweep_agg.reserve_async((size_t)e->vars + 1, e->stream) ||
-                          e->sweep_agg_words.reserve_async(9, e->stream))) {
-        e->may_screen = false;
-        (void)hipGetLastError();
-    }
+    e->may_screen = screening_may_pay(e, e->total_clauses);
     if ((rc = launch_current_sweep(e))) return rc;
     e->sweep_rows_version = e->rows_version;
     e->sweep_state_version = e->state_version;
@@ -1879,7 +1887,7 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     StepHeader *dh = sl.d_hdr.p;
     SweepArgs a{};
     a.buckets = sl.d_desc.p;
-    a.dyn = &dh->nbuckets;  // {nbuckets, npasses}
+    a.dyn = &dh->nbuckets;  // {nbuckets, npasses, screen_passes}
     a.task_passes = sl.plan.tp;
     a.table = e->table.p;
     a.valid = dh->valid;
@@ -1893,7 +1901,9 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
         (sl.plan.serve && e->serve_prefilter) || sl.plan.screen ? e->serve_agg.p : nullptr;
     a.agg = agg;
     a.agg_words = agg ? e->serve_agg_words.p : nullptr;
-    hipError_t he = launch_sweep(a, e->words, sl.plan.blocks, s);
+    hipError_t he = hipSuccess;
+    if (sl.plan.may_screen) he = launch_screened_choice(e, dh->valid, a, sl.plan.blocks, s);
+    if (he == hipSuccess) he = launch_sweep(a, e->words, sl.plan.blocks, s);
     const ChunkArgs c = step_chunks(sl, sl.rec_words);
     if (sl.plan.serve) {
         if (he == hipSuccess)
@@ -1920,7 +1930,8 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
 }
 
 // The launches of a step of plan sl.plan over the slot's buffers, in order: 3
-// for a plain step, 6 for a serving one, at most 9.  One by one: launching and
+// for a plain step (5 where its sweep may be screened), 6 for a serving one, at
+// most 9.  One by one: launching and
 // waiting for 3 / 5 / 10 small kernels takes 17 / 22 / 38 us so and 37 / 35 / 38
 // us as a captured graph, the host's part 10 / 16 / 30 us and 28 us.
 static hipError_t launch_step(gss_engine *e, StepSlot &sl, hipStream_t cs) {
@@ -2446,6 +2457,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     pl.serve = serve;
     pl.screen = screen;
     pl.agg_full = agg_full;
+    pl.may_screen = !serve && !screen && screening_may_pay(e, e->total_clauses + n);
     // Few literals go straight from the staging to their rows (32-byte reads
     // over PCIe); more are copied first and scattered by a kernel of its own.
     pl.staged = total > kDirectLits;
@@ -2490,7 +2502,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     if (n_loads) std::memcpy(sl.h_loads.p, desc->loads, (size_t)n_loads * sizeof(gss_word_load));
     // descriptors of every non-empty bucket, the step's own inserts included
     int k = 0;
-    int64_t t = 0;
+    int64_t t = 0, t64 = 0;
     const size_t nb_len = e->buckets.size();
     for (size_t i = 1; i < nb_len; i++) {
         const size_t len = e->tune_schedule == 2 ? i : nb_len - i;
@@ -2500,8 +2512,10 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         d.lits = b.d;
         d.len = (uint32_t)len;
         d.count = (uint32_t)b.count;
-        d.pass_begin = d.screen_begin = (uint32_t)t;
+        d.pass_begin = (uint32_t)t;
+        d.screen_begin = (uint32_t)t64;
         t += (b.count + cpp - 1) / cpp;
+        t64 += (b.count + 63) / 64;
     }
     StepHeader &h = *sl.h_hdr.p;
     std::memset(&h, 0, sizeof h);
@@ -2509,6 +2523,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     // with no valid slot every clause starts dead: the sweep has no work (a
     // serving step's admission decides that on the device)
     h.npasses = active_words ? (int32_t)t : 0;
+    h.screen_passes = active_words ? (int32_t)t64 : 0;
     h.nclauses = (int32_t)n;
     h.nups = n_ups;
     h.npatches = n_patches;

@@ -34,7 +34,8 @@ struct SweepArgs {
                              // (wave g starts in chunk g), [1] chunks past chunk_cap with records
     uint32_t chunk_cap;
     uint32_t sentinel;       // stored row offset of the sentinel literal
-    const int32_t *dyn;      // if set, {nbuckets, npasses} are read here (steps)
+    const int32_t *dyn;      // if set, {nbuckets, npasses} and the passes of the
+                             // screened kernel are read here (steps)
     int rec_words;           // 8-byte words per record: 3 (gss_hit), 1 (gss_hit_id) or 2
                              // (gss_hit_clause: one record per clause, its words as a mask)
     // Serving and screened batched steps (null otherwise): for each literal l
@@ -72,6 +73,7 @@ enum StepRegion {
 struct StepHeader {
     int32_t nbuckets;
     int32_t npasses;
+    int32_t screen_passes;  // npasses of a screened sweep (of 64 clauses)
     int32_t nclauses;
     // 1 in the device copy when the step found the engine halted: every
     // count is then 0 and the step does nothing (it is replayed later)

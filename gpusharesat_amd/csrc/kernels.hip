@@ -201,12 +201,12 @@ constexpr int kTaskRounds = 4;
 struct Passes {
     int nbuckets, total, tp, gw, nw;
 
-    __device__ __forceinline__ explicit Passes(const SweepArgs &a) {
+    __device__ __forceinline__ Passes(const SweepArgs &a, bool screened) {
         nbuckets = a.nbuckets;
         total = a.npasses;
         if (a.dyn) {
             nbuckets = uniform(a.dyn[0]);
-            total = uniform(a.dyn[1]);
+            total = uniform(a.dyn[screened ? 2 : 1]);
         }
         gw = uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));  // 256-thread blocks
         nw = (int)gridDim.x * 4;
@@ -350,7 +350,7 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
     const uint32_t w8 = (uint32_t)w * 8u;
     const uint64_t valid = a.valid[w];
     const uint64_t *__restrict__ table = a.table;
-    const Passes ps(a);
+    const Passes ps(a, false);
     HitWriter out(a, ps);
 
     walk<CPW, false>(a, ps, lane, [&](const Run &run) {
@@ -661,7 +661,7 @@ __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k
     uint32_t gdead = 0;  // groups without a word
     for (int b = 0; b < 8; b++)
         if (!a.agg_words[b]) gdead |= 1u << b;
-    const Passes ps(a);
+    const Passes ps(a, true);
     HitWriter out(a, ps);
 
     walk<64, true>(a, ps, lane, [&](const Run &run) {
@@ -897,7 +897,7 @@ __device__ __forceinline__ void serve_admit(const ServePending &p, const ServeRi
         *r.adm_count = (uint32_t)count;
         dh->nloads = (int64_t)total_words;
         dh->npatches = count > 0 ? (int64_t)total_patches : 0;
-        if (count == 0) dh->npasses = 0;  // nothing to check
+        if (count == 0) dh->npasses = dh->screen_passes = 0;  // nothing to check
         *r.tail = p.tail + (uint64_t)count;
         report->first = p.tail;
         report->count = (uint32_t)count;

@@ -115,12 +115,26 @@ def test_plain_sweeps_that_may_be_screened(engine_factory, W, n, agree):
     e.reset_assignments(V, W)
     e.upload(is_def, is_true)
     print(f"{W} words, {agree} agree: {exp.size} records", flush=True)
+    want = np.empty((exp.size, 3), np.uint64)
+    c = exp["clause"]
+    want[:, 0] = (rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
+                  | (exp["word"].astype(np.uint64) << np.uint64(48)))
+    want[:, 1], want[:, 2] = exp["false_mask"], exp["unit_mask"]
+    want = want[np.argsort(want[:, 0])]
     for _ in range(2):
         assert e.sweep(valid) == exp.size
         got = e.hits().view(np.uint64).reshape(-1, 3)
-        want = np.empty((exp.size, 3), np.uint64)
-        c = exp["clause"]
-        want[:, 0] = (rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
-                      | (exp["word"].astype(np.uint64) << np.uint64(48)))
-        want[:, 1], want[:, 2] = exp["false_mask"], exp["unit_mask"]
-        assert np.array_equal(got[np.argsort(got[:, 0])], want[np.argsort(want[:, 0])])
+        assert np.array_equal(got[np.argsort(got[:, 0])], want)
+    # unscreened steps' sweeps may be too
+    sv.submit(e, valid)
+    assert e.step_wait()[0] == exp.size
+    got = e.step_hits_view().view(np.uint64).reshape(-1, 3)
+    assert np.array_equal(got[np.argsort(got[:, 0])], want)
+    sv.submit(e, valid, records=sv.RECORDS_IDS)
+    assert e.step_wait()[0] == exp.size
+    assert np.array_equal(np.sort(e.step_ids_view().view(np.uint64).ravel()), want[:, 0])
+    sv.submit(e, valid, records=sv.RECORDS_CLAUSES)
+    assert e.step_wait()[0] == np.unique(c).size
+    got = e.step_clauses_view().view(np.uint64).reshape(-1, 2)
+    words = np.bitwise_count(got[:, 1]).sum()
+    assert words == exp.size and np.unique(got[:, 0]).size == got.shape[0]

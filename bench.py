@@ -24,7 +24,7 @@ before timing starts.  Prints one JSON line.
   latency_ms     after the timed region: submit -> every hit of the sweep in
                  pinned host memory as the drop-in gpuRun() delivers it (one
                  16-byte record per clause with its solver words), one sweep
-                 in flight, through the step path (graph replay, device
+                 in flight, through the step path (device
                  compaction, PCIe copy); latency_id_records_ms the same with
                  one 8-byte record per (clause, word), latency_full_records_ms
                  with the 24-byte records that also carry the masks
@@ -32,7 +32,7 @@ before timing starts.  Prints one JSON line.
 --workload batched-16 measures the batched form instead: 16 solver streams
 over 1M vars, each step inserting Poisson(16 x 2800) clauses of Pareto(1.5)
 lengths (2..500) and 16 uneven batches of U[16, 256] assignments (64-word
-table, 4096 slots), as one graph-captured step (gss_step_enqueue /
+table, 4096 slots), as one step (gss_step_enqueue /
 gss_step_wait / gss_step_hits_copy, two steps in flight).  The DB grows from
 1M to ~10M clauses over 200 steps; the warmup steps are also replayed through
 the plain entry points on a second engine and their records must be
@@ -264,7 +264,7 @@ def main() -> int:
         f"{achieved:.0f} GB/s algorithmic")
     # Report latency (outside the timed region): submit -> every hit of the
     # sweep in pinned host memory, one sweep in flight, through the step path
-    # (graph replay: sweep, compaction, copy over PCIe); first with the
+    # (sweep, compaction, copy over PCIe); first with the
     # records the solvers receive (clause and solver word), then with the
     # full records.
     from gpusharesat_amd import serving as sv
@@ -284,7 +284,7 @@ def main() -> int:
                 raise RuntimeError(f"step path gave {n_step} records, the sweep {hits}")
             if records not in views:
                 views[records] = view.copy()
-            if k >= 2:  # the first replays capture the graph and size the buffers
+            if k >= 2:  # the first steps size the buffers
                 lat.append((t_rep - t_sub) * 1e3)
         if not lat:
             return None
@@ -320,7 +320,7 @@ def main() -> int:
             raise RuntimeError("clause records differ from the id records grouped by clause")
     # The device's own ceiling for this access pattern: random 128-byte line
     # gathers (independent, 4 in flight per lane) from a table of the same size.
-    kernel_name = "k_sweep<16,1,4,true>"
+    kernel_name = "k_sweep<16,false>"
     tr = measured_traffic(kernel_name) if args.scale == 1.0 else {
         "bytes": None, "note": "not the headline instance"}
     traffic = tr["bytes"]
@@ -365,7 +365,7 @@ def main() -> int:
             "traffic_source": tr,
             "traffic_gbps": traffic / k_avg_s / 1e9 if traffic else None,
             "gather_ceiling_gbps": gather,
-            "kernel": "k_sweep<16,1,4,true>",
+            "kernel": "k_sweep<16,false>",
             "kernel_ms": k_avg_s * 1e3,
             "algorithmic_bytes": alg_bytes,
         },
@@ -502,7 +502,7 @@ def run_batched(args) -> int:
     # travel to the host while the next step is staged, then they are read.
     # With --inflight 1 a step is submitted only once the previous one has
     # left the device (its records still travelling), so no step waits
-    # behind another's graph.
+    # behind another's kernels.
     while todo and len(pending) < args.inflight:
         enqueue_next()
     while pending:

@@ -30,8 +30,10 @@
 //
 // Work mapping.  k_sweep: W lanes check one clause, one table word each, 64 / W
 // clauses per wave pass, literals handed out with DPP (no LDS); k_sweep_screened:
-// one clause per lane against the aggregate, then one surviving (clause, word)
-// per lane.  Waves are persistent and walk the clauses in tasks of passes.
+// one clause per lane against the screening entries, then one surviving clause
+// and two words per lane.  Waves are persistent and walk the clauses in tasks of
+// passes.  Steps are screened on request; other sweeps where a look at the
+// table says that it pays (k_sweep_choose).
 //
 // What bounds it is the row reads: 128-byte lines of a table that the L2s do
 // not hold, ~6.9 TB/s of them at any size past 32 MB.  Measured on one MI355X,
@@ -39,10 +41,10 @@
 // all negated rows of a clause left with a candidate, both rows of every
 // literal up to 4 literals) and now:
 //   16 words, 4M clauses, 1M variables, random values   711 -> 618 us
-//   16 words, 2M clauses, 500k variables, planted       204 -> 119 us
-//   64 words, 400k clauses, 200k variables, planted     140 ->  87 us
-//    8 words, 1M clauses, 100k variables, planted       109 ->  45 us
-//    1 word,  100k clauses, 10k variables, random        32 ->  10 us
+//   16 words, 2M clauses, 500k variables, planted       204 -> 119 us (screened: 73)
+//   64 words, 400k clauses, 200k variables, planted     140 ->  87 us (screened: 72)
+//    8 words, 1M clauses, 100k variables, planted       109 ->  45 us (screened: 32)
+//    1 word,  100k clauses, 10k variables, random        32 ->   8 us
 // Rows read per clause, counted on the CPU: 7.97 -> 6.95 (random), 4.54 -> 2.77
 // (planted).
 //
@@ -1563,6 +1565,10 @@ __global__ void k_table_agg_update(const uint64_t *__restrict__ table,
 // r % 8 = b, from their solvers' bases (a request's words are loaded whole from
 // its base, so until its patches the base value holds in all its slots;
 // k_serve_patch clears what a patch undoes).  Bits of empty groups are not read.
+//
+// What bounds it: the row writes (256 MB at 1M variables and up to 16 words: 53
+// us) or, over few variables, the patches.  Three kernels in a row took 60 us
+// where it takes 45.
 //
 // The first kPatchBlocks blocks copy the admitted requests' patches from the
 // pinned ring (consecutive lanes read consecutive 4-byte words: one pass over

@@ -317,7 +317,9 @@ typedef struct gss_step_desc {
  * loads); else only the entries of the step's updates and patches are
  * refreshed, after they are applied and again after the roll forward.  It
  * pays where the slots of a word group share most of their values
- * (consecutive assignments of one solver). */
+ * (consecutive assignments of one solver).  Without the flag, as in plain
+ * sweeps, a sweep large enough to gain reads the aggregate anew and is screened
+ * where a sample of the table says that it pays. */
 #define GSS_STEP_SCREEN 1
 int gss_step_submit(gss_engine *e, const gss_step_desc *d);
 /* (Re)creates nbases solver base planes over the current variable count,

@@ -138,3 +138,36 @@ def test_plain_sweeps_that_may_be_screened(engine_factory, W, n, agree):
     got = e.step_clauses_view().view(np.uint64).reshape(-1, 2)
     words = np.bitwise_count(got[:, 1]).sum()
     assert words == exp.size and np.unique(got[:, 0]).size == got.shape[0]
+
+
+@pytest.mark.parametrize("variables", [1, 3, 403])
+@pytest.mark.parametrize("W, n", [(8, 450_000), (16, 450_000), (32, 160_000), (64, 80_000)])
+def test_screening_tables_of_odd_sizes(engine_factory, W, n, variables):
+    """Fewer variables than a wave's turn over the table, and a last turn in part:
+    plain sweeps that may be screened, and screened steps."""
+    rng = np.random.default_rng(W + variables)
+    lens = rng.integers(1, 4, size=n).astype(np.int32)
+    lits = rng.integers(0, 2 * variables, size=int(lens.sum())).astype(np.uint32)
+    off = np.zeros(n + 1, np.int64)
+    off[1:] = np.cumsum(lens)
+    is_def = np.full((variables, W), ALL)
+    is_true = np.repeat(np.where(rng.random(variables) < 0.5, ALL, np.uint64(0))[:, None], W, axis=1)
+    is_def[-1, W // 2:] = 0  # the last variable: undefined from half of the words on
+    is_true &= is_def
+    valid = np.zeros(W, np.uint64)
+    valid[[0, W // 2, W - 1]] = [3, 1 << 63, 1]
+    exp = orc.sweep(off, lits, is_def, is_true, valid)
+    e = engine_factory()
+    rows = e.append(lits, lens).astype(np.uint64)
+    e.reset_assignments(variables, W)
+    e.upload(is_def, is_true)
+    c = exp["clause"]
+    want = np.sort(rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
+                   | (exp["word"].astype(np.uint64) << np.uint64(48)))
+    print(f"{W} words, {variables} variables: {exp.size} records", flush=True)
+    assert e.sweep(valid) == exp.size
+    assert np.array_equal(np.sort(e.hits().view(np.uint64).reshape(-1, 3)[:, 0]), want)
+    for flags in (0, sv.STEP_SCREEN):
+        sv.submit(e, valid, records=sv.RECORDS_IDS, flags=flags)
+        assert e.step_wait()[0] == exp.size
+        assert np.array_equal(np.sort(e.step_ids_view().view(np.uint64).ravel()), want)

@@ -370,6 +370,10 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
         auto row = [&]<int J>(const Lits<W> &l) {
             return load_word(table, scale_offset<W>(lit_at<W, J>(l)) | w8);
         };
+        // Clause records wait, one per lane, for W passes' clauses: written pass by
+        // pass they took 13 % of a sweep of 64 words where most clauses have one
+        // (a batched step of random clauses: 1.545 ms, 1.339 now).
+        uint64_t found = 0;
         // One pass: its held literals and first two rows.
         auto check = [&](int pass, const Lits<W> &cur, uint64_t x0, uint64_t x1) {
             const int r = pass * CPW + c;
@@ -461,14 +465,18 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
             const bool hit = (fm | um) != 0;
             if constexpr (CLAUSES) {
                 const unsigned long long bw = __ballot(hit);
-                if (bw) {
-                    const uint64_t wm =
-                        W == 64 ? bw : (bw >> (c * W)) & ((1ull << (W & 63)) - 1ull);
-                    out.clause(w == 0 && wm != 0, (uint32_t)(row0 + r), len, wm, lane);
+                if (bw && pass % W == lane / CPW) {
+                    const int k = lane % CPW;  // its clause of the pass
+                    found = W == 64 ? bw : (bw >> (k * W)) & ((1ull << (W & 63)) - 1ull);
                 }
             } else {
                 out.words(hit, (uint32_t)(row0 + r), len, w, fm, um, a.rec_words, lane);
             }
+        };
+        auto flush = [&](int pass) {
+            if (__ballot(found != 0))
+                out.clause(found != 0, (uint32_t)(row0 + pass / W * 64 + lane), len, found, lane);
+            found = 0;
         };
         // Two passes per turn: the rows of one are in flight while the other
         // is checked, and the literals of the next two (separate registers: a
@@ -481,7 +489,12 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
             check(pass, la, a0, a1);
             a0 = row.template operator()<0>(na);
             a1 = row.template operator()<1>(na);
+            if constexpr (CLAUSES && W == 1) flush(pass);
             if (pass + 1 < n) check(pass + 1, lb, b0, b1);
+            if constexpr (CLAUSES) {
+                if (W == 1 ? pass + 1 < n : (pass + 2) % W == 0 || pass + 2 >= n)
+                    flush(W == 1 ? pass + 1 : pass);
+            }
             la = na;
             lb = nb;
         }

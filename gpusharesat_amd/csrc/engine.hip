@@ -114,6 +114,7 @@ struct Pinned {
             cap = nc;
             return GSS_OK;
         }
+        if (lock) (void)hipGetLastError();  // the refusal is dealt with here
         p = nullptr;
         if (!page_limit)
             return set_err(GSS_E_NOMEM, "pinned host allocation of %zu bytes failed", bytes);
@@ -242,9 +243,11 @@ struct DevBuf {
         size_t nc = std::max(n, cap + cap / 2);
         T *np = nullptr;
         hipError_t e = hipMalloc((void **)&np, nc * sizeof(T));
-        if (e != hipSuccess)
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
             return set_err(GSS_E_NOMEM, "device allocation of %zu bytes failed: %s",
                            nc * sizeof(T), hipGetErrorString(e));
+        }
         if (p) {
             if (keep && cap) {
                 HIP_TRY(hipMemcpyAsync(np, p, cap * sizeof(T), hipMemcpyDeviceToDevice, s));
@@ -263,9 +266,11 @@ struct DevBuf {
         size_t nc = std::max(n, cap * 2);
         T *np = nullptr;
         hipError_t e = hipMallocAsync((void **)&np, nc * sizeof(T), s);
-        if (e != hipSuccess)
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
             return set_err(GSS_E_NOMEM, "device allocation of %zu bytes failed: %s",
                            nc * sizeof(T), hipGetErrorString(e));
+        }
         if (p) HIP_TRY(hipFreeAsync(p, s));
         p = np;
         cap = nc;
@@ -540,8 +545,11 @@ struct gss_engine {
 
 namespace {
 
+// The launches read hipGetLastError: an error that an earlier call of this
+// thread left there is not theirs.
 int check_engine(gss_engine *e) {
     if (!e) return set_err(GSS_E_INVAL, "null engine");
+    (void)hipGetLastError();
     return hipSetDevice(e->device) == hipSuccess ? GSS_OK
                                                  : set_err(GSS_E_HIP, "hipSetDevice failed");
 }
@@ -681,10 +689,8 @@ bool screening_may_pay(gss_engine *e, int64_t clauses) {
     const double rows = (double)e->vars * 2.0 * e->words * 8.0;
     if (52.0 * m * std::max(1, e->words / 16) <= 24.0 * m + rows / 5.5e6 + 12.0) return false;
     if (e->sweep_agg.reserve_async((size_t)e->vars + 1, e->stream) ||
-        e->sweep_agg_words.reserve_async(9, e->stream)) {
-        (void)hipGetLastError();
+        e->sweep_agg_words.reserve_async(9, e->stream))
         return false;
-    }
     return true;
 }
 

@@ -1,0 +1,72 @@
+"""HIP runtime calls that are refused (no memory, a failed event) leave the engine
+as it was: the next call gives what it gives without the refusal.  Each case runs
+in a process of its own, in which tests/cpp/hip_fail.cpp stands in front of the
+runtime and refuses the call; nothing reaches the GPU for it.
+"""
+import pathlib
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = pathlib.Path(__file__).resolve().parent.parent
+
+HEAD = """
+import ctypes, sys
+import numpy as np
+fail = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+fail.hip_fail_set.argtypes = [ctypes.c_int, ctypes.c_size_t, ctypes.c_long, ctypes.c_long]
+fail.hip_fail_calls.restype = ctypes.c_long
+HOST_MALLOC, MALLOC_ASYNC, EVENT_RECORD = range(3)
+from gpusharesat_amd import _lib, engine as en, serving as sv
+
+ALL = np.uint64(0xFFFFFFFFFFFFFFFF)
+
+
+def refused(call):
+    try:
+        call()
+    except _lib.GssError as x:
+        print("refused:", x, flush=True)
+    else:
+        raise SystemExit("the call was not refused")
+
+
+def ones(n):
+    return np.ones(n, np.int32)
+"""
+
+
+def run_case(tmp_path, body):
+    shim = tmp_path / "hip_fail.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared",
+                    str(ROOT / "tests" / "cpp" / "hip_fail.cpp"), "-o", str(shim), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-u", "-c",
+                        textwrap.dedent(HEAD) + textwrap.dedent(body) + "\nprint('ok')", str(shim)],
+                       cwd=ROOT, capture_output=True, text=True, timeout=100)
+    print(r.stdout + r.stderr, flush=True)
+    assert r.returncode == 0 and r.stdout.rstrip().endswith("ok")
+
+
+def test_calls_after_an_error_of_the_callers_own(tmp_path):
+    """An error that another HIP call of the thread has left is not taken for one
+    of the engine's launches."""
+    run_case(tmp_path, """
+        hip = ctypes.CDLL("libamdhip64.so.7")
+        e = en.Engine(0)
+        e.reset_assignments(64, 1)
+        e.append(np.full(100, 2, np.uint32), ones(100))
+        every = np.full(1, ALL)
+        for k in range(7):
+            sv.submit(e, every, records=sv.RECORDS_IDS)
+            assert e.step_wait()[0] == 100
+            if k > 2:
+                assert hip.hipMalloc(None, ctypes.c_size_t(16)) != 0
+        print("steps done", flush=True)
+        for k in range(3):
+            assert e.sweep(every) == 100
+            assert hip.hipMalloc(None, ctypes.c_size_t(16)) != 0
+    """)

@@ -451,6 +451,7 @@ struct gss_engine {
     // (8 words on), cleared by the sweep before it
     uint32_t *d_alloc = nullptr;
     int alloc_at = 0;
+    bool alloc_dirty = false;  // a sweep was not queued whole: either set may hold claims
     uint32_t sweep_waves = 0;  // waves of the last sweep
     uint32_t chunk_cap = 0;
     int nbuckets = 0, npasses = 0, blocks = 0;
@@ -648,7 +649,6 @@ ChunkArgs sweep_chunks(const gss_engine *e) {
     return c;
 }
 
-// Launches the sweep kernel for the current descriptors (already uploaded).
 // The kernel time of the last waited sweep, from its events.
 int read_time(gss_engine *e) {
     if (!e->time_due) return GSS_OK;
@@ -711,8 +711,13 @@ hipError_t launch_screened_choice(gss_engine *e, const uint64_t *valid, SweepArg
     return launch_sweep(b, e->words, blocks, s);
 }
 
+// Launches the sweep kernel for the current descriptors (already uploaded).
 int launch_current_sweep(gss_engine *e) {
     if (const int rc = read_time(e)) return rc;
+    // a set is cleared by the counting kernel of the sweep before; without that
+    // kernel (a call below failed) neither set is known to be clear
+    if (e->alloc_dirty) HIP_TRY(launch_reset_u32(e->d_alloc, 16, e->stream));
+    e->alloc_dirty = true;
     e->alloc_at ^= 1;
     e->sweep_waves = e->npasses > 0 ? (uint32_t)e->blocks * 4 : 0;
     HIP_TRY(hipEventRecord(e->ev0, e->stream));
@@ -738,6 +743,7 @@ int launch_current_sweep(gss_engine *e) {
     // counts to pinned memory: the wait reads them there
     HIP_TRY(launch_count_records(sweep_chunks(e), e->h_count.p,
                                  e->d_alloc + 8 * (e->alloc_at ^ 1), ++e->sweep_seq, e->stream));
+    e->alloc_dirty = false;
     return GSS_OK;
 }
 
@@ -1538,13 +1544,18 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
         chunks = std::min(chunks, std::max<uint64_t>(budget, 1));
     }
     if (e->tune_max_chunks > 0) chunks = std::min<uint64_t>(chunks, e->tune_max_chunks);
-    if (chunks > e->chunk_cap && (rc = reserve_chunks(e, chunks))) return rc;
+    if (chunks > e->chunk_cap) {
+        const gss_hit *old = e->d_hits.p;
+        rc = reserve_chunks(e, chunks);
+        if (e->d_hits.p != old) e->waited = false;  // the last sweep's records are gone
+        if (rc) return rc;
+    }
     e->may_screen = screening_may_pay(e, e->total_clauses);
+    e->waited = false;
     if ((rc = launch_current_sweep(e))) return rc;
     e->sweep_rows_version = e->rows_version;
     e->sweep_state_version = e->state_version;
     e->pending = true;
-    e->waited = false;
     e->have_sweep = true;
     return GSS_OK;
 }

@@ -70,3 +70,25 @@ def test_calls_after_an_error_of_the_callers_own(tmp_path):
             assert e.sweep(every) == 100
             assert hip.hipMalloc(None, ctypes.c_size_t(16)) != 0
     """)
+
+
+def test_sweep_after_a_sweep_that_was_not_queued(tmp_path):
+    """A sweep that claimed chunks past its waves' own, one whose first event is
+    refused, one without a valid slot: none of the first one's claims is left."""
+    run_case(tmp_path, """
+        e = en.Engine(0)
+        e.reset_assignments(64, 1)
+        n = 2_000_000
+        e.append(np.full(n, 2, np.uint32), ones(n))  # undefined: a record per clause
+        e.set_tuning(en.TUNE_WAVES_PER_CU, 4)  # ~2,000 records a wave: two chunks
+        every = np.full(1, ALL)
+        assert e.sweep(every) == n
+        fail.hip_fail_set(EVENT_RECORD, 0, 0, 1)
+        refused(lambda: e.sweep(every))
+        assert e.sweep(np.zeros(1, np.uint64)) == 0
+        assert e.sweep(every) == n
+        assert np.array_equal(np.sort(e.hits()["row"]), np.arange(n))
+        fail.hip_fail_set(EVENT_RECORD, 0, 0, 1)
+        refused(lambda: e.sweep(every))
+        refused(e.hits)
+    """)

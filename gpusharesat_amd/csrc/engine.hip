@@ -2418,12 +2418,13 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         return rc;
     if ((rc = sl.h_out.reserve(4))) return rc;
     // the pinned buffer that takes this step's records if they are few; a
-    // page-locked limit below its size rules it out
-    const int nd = sl.h_n + 1;
-    sl.direct_at = (sl.direct_at + 1) % nd;
+    // page-locked limit below its size rules it out.  direct_at moves on once
+    // the step is launched: a refused submit must not move it past the buffer
+    // after the one whose records are still to be read.
+    const int direct_at = (sl.direct_at + 1) % (sl.h_n + 1);
     const bool can_direct =
         !serve && (e->page_limit < 0 || (int64_t)(kDirectWords * 8) < e->page_limit);
-    if (can_direct && (rc = sl.h_direct[sl.direct_at].reserve(kDirectWords))) return rc;
+    if (can_direct && (rc = sl.h_direct[direct_at].reserve(kDirectWords))) return rc;
     if (serve && (rc = sl.d_wcount.reserve_async(2 * GSS_MAX_WORDS, e->stream))) return rc;
     // a screened step rebuilds the aggregate unless the last change to the
     // table was a screened step's (word loads change whole words: rebuilt)
@@ -2557,7 +2558,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         h.valid[w] = w < W ? valid[w] : 0;
         h.last_pos[w] = (w < W && last_pos) ? last_pos[w] : -1;
     }
-    h.host_rec = can_direct ? sl.h_direct[sl.direct_at].p : nullptr;
+    h.host_rec = can_direct ? sl.h_direct[direct_at].p : nullptr;
     e->state_version++;
     e->table_agg_at = screen ? e->state_version : 0;
     HIP_TRY(hipEventRecord(sl.t0, e->stream));
@@ -2567,6 +2568,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     sl.settled = false;
     sl.records_lost = false;
     sl.serve = serve;
+    sl.direct_at = direct_at;
     // the previous records of this slot stay readable only if their copy
     // was queued (or there were none)
     if (sl.rec_total > 0 && !sl.copy_queued && !sl.direct) sl.results = false;

@@ -92,3 +92,33 @@ def test_sweep_after_a_sweep_that_was_not_queued(tmp_path):
         refused(lambda: e.sweep(every))
         refused(e.hits)
     """)
+
+
+def test_records_held_while_a_submit_is_refused(tmp_path):
+    """A step's records keep their place until its slot is waited for again, also
+    where the slot's next submit is refused first."""
+    run_case(tmp_path, """
+        e = en.Engine(0)
+        e.reset_assignments(64, 1)
+        every = np.full(1, ALL)
+        e.append(np.full(100, 2, np.uint32), ones(100))
+        views = []
+        for _ in range(2):
+            sv.submit(e, every, records=sv.RECORDS_IDS)
+            assert e.step_wait()[0] == 100
+            views.append(e.step_ids_view())
+        held = [v.copy() for v in views]
+        # variable 1 true: of the step's records only the new clauses' are left
+        ups = np.zeros(5000, en.VAR_UPDATE_DTYPE)
+        ups["var"], ups["is_def"], ups["is_true"] = 1, ALL, ALL
+        step = lambda: sv.submit(e, every, lits=np.full(50, 6, np.uint32), lens=ones(50), ups=ups,
+                                 records=sv.RECORDS_IDS)
+        fail.hip_fail_set(MALLOC_ASYNC, 100_000, 0, 1)  # the device copy of the updates
+        refused(step)
+        step()
+        e.sync()
+        for v, h in zip(views, held):
+            assert np.array_equal(v, h)
+        assert e.step_wait()[0] == 50
+        assert np.array_equal(np.sort(e.step_ids_view()["row"]), np.arange(100, 150))
+    """)

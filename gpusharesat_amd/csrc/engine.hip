@@ -2418,13 +2418,14 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
         return rc;
     if ((rc = sl.h_out.reserve(4))) return rc;
     // the pinned buffer that takes this step's records if they are few; a
-    // page-locked limit below its size rules it out.  direct_at moves on once
+    // page-locked limit below its size rules it out, as does a system that
+    // will not lock it (the records are then copied).  direct_at moves on once
     // the step is launched: a refused submit must not move it past the buffer
     // after the one whose records are still to be read.
     const int direct_at = (sl.direct_at + 1) % (sl.h_n + 1);
     const bool can_direct =
-        !serve && (e->page_limit < 0 || (int64_t)(kDirectWords * 8) < e->page_limit);
-    if (can_direct && (rc = sl.h_direct[direct_at].reserve(kDirectWords))) return rc;
+        !serve && (e->page_limit < 0 || (int64_t)(kDirectWords * 8) < e->page_limit) &&
+        sl.h_direct[direct_at].reserve(kDirectWords) == GSS_OK;
     if (serve && (rc = sl.d_wcount.reserve_async(2 * GSS_MAX_WORDS, e->stream))) return rc;
     // a screened step rebuilds the aggregate unless the last change to the
     // table was a screened step's (word loads change whole words: rebuilt)

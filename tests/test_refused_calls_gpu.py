@@ -122,3 +122,21 @@ def test_records_held_while_a_submit_is_refused(tmp_path):
         assert e.step_wait()[0] == 50
         assert np.array_equal(np.sort(e.step_ids_view()["row"]), np.arange(100, 150))
     """)
+
+
+def test_steps_whose_record_buffers_are_not_page_locked(tmp_path):
+    """Neither the buffer of few records nor the one for more: the records are
+    copied, to pageable memory."""
+    run_case(tmp_path, """
+        for times in (1, 1000):
+            e = en.Engine(0)
+            e.reset_assignments(64, 1)
+            e.append(np.full(100, 2, np.uint32), ones(100))
+            fail.hip_fail_set(HOST_MALLOC, 500_000, 0, times)
+            for _ in range(5):
+                sv.submit(e, np.full(1, ALL), records=sv.RECORDS_IDS)
+                assert e.step_wait()[0] == 100
+                assert np.array_equal(np.sort(e.step_ids_view()["row"]), np.arange(100))
+            assert e.sweep(np.full(1, ALL)) == 100
+            e.close()
+    """)

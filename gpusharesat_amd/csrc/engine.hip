@@ -1153,6 +1153,10 @@ int gss::sweep_records(gss_engine *e, const gss_hit **hits, const uint32_t **fil
 
 hipStream_t gss::engine_stream(gss_engine *e) { return e->stream; }
 
+bool gss::engine_may_lock(const gss_engine *e, size_t bytes) {
+    return e->page_limit < 0 || (int64_t)bytes < e->page_limit;
+}
+
 int gss::engine_activate(gss_engine *e) { return check_engine(e); }
 
 extern "C" {
@@ -2424,7 +2428,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     // after the one whose records are still to be read.
     const int direct_at = (sl.direct_at + 1) % (sl.h_n + 1);
     const bool can_direct =
-        !serve && (e->page_limit < 0 || (int64_t)(kDirectWords * 8) < e->page_limit) &&
+        !serve && gss::engine_may_lock(e, kDirectWords * 8) &&
         sl.h_direct[direct_at].reserve(kDirectWords) == GSS_OK;
     if (serve && (rc = sl.d_wcount.reserve_async(2 * GSS_MAX_WORDS, e->stream))) return rc;
     // a screened step rebuilds the aggregate unless the last change to the

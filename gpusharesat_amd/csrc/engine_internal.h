@@ -23,6 +23,9 @@ int db_tag_arrays(gss_engine *e, std::vector<const uint32_t *> &tags);
 int sweep_records(gss_engine *e, const gss_hit **hits, const uint32_t **fills,
                   uint32_t *chunks);
 hipStream_t engine_stream(gss_engine *e);
+// Whether host memory of this size may be page-locked
+// (gss_engine_set_page_locked_limit).
+bool engine_may_lock(const gss_engine *e, size_t bytes);
 // Serving (gss_server): attaches the request and patch rings (fine-grained
 // pinned host memory the host publishes into, head = requests published) to
 // the engine; the device-side admission cursor starts at request 0.

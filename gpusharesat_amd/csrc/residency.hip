@@ -46,6 +46,7 @@ static_assert(OB3 + 1 == P, "parameter layout");
 constexpr int kBuckets = 20000;
 constexpr float kRescale = 1e19f;  // RESCALE_CONST, gpuShareLib/Clauses.cuh:39
 constexpr size_t kGradDirect = 4u << 20;  // floats gss_res_grad passes through pinned memory
+
 int set_err(int code, const char *fmt, ...) {
     char buf[512];
     va_list ap;
@@ -688,6 +689,8 @@ struct gss_res {
     Buf<float> params, mom, partial;
     float *h_in = nullptr, *h_res = nullptr;  // pinned: samples of gss_res_grad, a pass's results
     size_t h_in_cap = 0;
+    Buf<float> d_res;           // a pass's results where h_res is not to be had,
+    float paged_res[kPartial];  // and their copy
     Buf<float> xs, ys, ws;
     Buf<uint32_t> idx;
     // scratch
@@ -712,17 +715,30 @@ int check(gss_res *r) {
     return engine_activate(r->e);
 }
 
+// Page-locked memory for n floats; null where the engine's limit or the system
+// has none (the device's memory and copies take its place).
+float *lock_floats(const gss_res *r, size_t n) {
+    void *p = nullptr;
+    if (!engine_may_lock(r->e, n * sizeof(float))) return nullptr;
+    if (hipHostMalloc(&p, n * sizeof(float), hipHostMallocDefault) == hipSuccess) return (float *)p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // Runs forward/backward + gradient (+ optional SGD step) on n samples x / y /
 // wt (device or pinned memory), in the order of idx (null = identity).  With
-// wait, r->h_res then holds the gradient and, at [P], the mean loss.
+// results, that many floats are there when it returns: the gradient and, at [P],
+// the mean loss.
 int run_batch(gss_res *r, hipStream_t st, const float *x, const float *y, const float *wt,
-              const uint32_t *idx, int64_t n, float w_pos, float w_neg, float lr, bool wait) {
+              const uint32_t *idx, int64_t n, float w_pos, float w_neg, float lr,
+              const float **results) {
     int rc;
     if ((rc = r->partial.reserve((size_t)kMlpBlocks * kPartial))) return rc;
-    if (!r->h_res && hipHostMalloc((void **)&r->h_res, kPartial * sizeof(float),
-                                   hipHostMallocDefault) != hipSuccess) {
-        r->h_res = nullptr;
-        return set_err(GSS_E_NOMEM, "pinned host allocation failed");
+    float *out = nullptr;
+    if (results) {
+        if (!r->h_res) r->h_res = lock_floats(r, kPartial);
+        if (!r->h_res && (rc = r->d_res.reserve(kPartial))) return rc;
+        out = r->h_res ? r->h_res : r->d_res.p;
     }
     const int blocks = (int)std::min<int64_t>((n + kTile - 1) / kTile, kMlpBlocks);
     hipLaunchKernelGGL(k_mlp_pass, dim3(blocks), dim3(256), 0, st, r->params.p, x, y, wt, idx, n,
@@ -730,9 +746,14 @@ int run_batch(gss_res *r, hipStream_t st, const float *x, const float *y, const 
     RES_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_mlp_reduce_step, dim3((kPartial + 63) / 64), dim3(256), 0, st,
                        r->partial.p, blocks, 1.0f / (float)n, r->params.p, r->mom.p, lr, 0.9f,
-                       wait ? r->h_res : (float *)nullptr);
+                       out);
     RES_HIP(hipGetLastError());
-    if (wait) RES_HIP(hipStreamSynchronize(st));
+    if (!results) return GSS_OK;
+    if (!r->h_res) {
+        RES_HIP(hipMemcpyAsync(r->paged_res, out, sizeof r->paged_res, hipMemcpyDeviceToHost, st));
+    }
+    RES_HIP(hipStreamSynchronize(st));
+    *results = r->h_res ? r->h_res : r->paged_res;
     return GSS_OK;
 }
 
@@ -806,7 +827,7 @@ int gss_res_destroy(gss_res *r) {
     if (r->h_in) (void)hipHostFree(r->h_in);
     if (r->h_res) (void)hipHostFree(r->h_res);
     for (auto *b : {&r->ema_f, &r->ema_s, &r->tot, &r->act, &r->score, &r->params, &r->mom,
-                    &r->partial, &r->xs, &r->ys, &r->ws, &r->act_in, &r->fout})
+                    &r->partial, &r->d_res, &r->xs, &r->ys, &r->ws, &r->act_in, &r->fout})
         b->release();
     r->alive_d.release();
     r->keep.release();
@@ -985,11 +1006,11 @@ int gss_res_train(gss_res *r, int32_t round, int horizon, int epochs, int batch,
         int nb = 0;
         for (int64_t b0 = 0; b0 < n; b0 += batch) {
             const int64_t m = std::min<int64_t>(batch, n - b0);
-            const bool wait = ep == epochs - 1;
+            const float *res = nullptr;
             if ((rc = run_batch(r, st, sn.x.p, r->ys.p, r->ws.p, r->idx.p + b0, m, w_pos, w_neg,
-                                lr, wait)))
+                                lr, ep == epochs - 1 ? &res : nullptr)))
                 return rc;
-            if (wait) acc += r->h_res[P];
+            if (res) acc += res[P];
             nb++;
         }
         if (ep == epochs - 1) last = (float)(acc / std::max(nb, 1));
@@ -1124,19 +1145,13 @@ int gss_res_grad(gss_res *r, int64_t n, const float *x, const float *y, const fl
     // their waits took as long as all the kernels)
     const size_t need = (size_t)n * (F + 1 + (wt ? 1 : 0));
     const float *dx, *dy, *dw = nullptr;
-    if (need <= kGradDirect) {
-        if (need > r->h_in_cap) {
-            if (r->h_in) (void)hipHostFree(r->h_in);
-            r->h_in = nullptr;
-            r->h_in_cap = 0;
-            const size_t cap = std::min(kGradDirect, 2 * need);
-            if (hipHostMalloc((void **)&r->h_in, cap * sizeof(float), hipHostMallocDefault) !=
-                hipSuccess) {
-                r->h_in = nullptr;
-                return set_err(GSS_E_NOMEM, "pinned host allocation failed");
-            }
-            r->h_in_cap = cap;
-        }
+    if (need <= kGradDirect && need > r->h_in_cap) {
+        if (r->h_in) (void)hipHostFree(r->h_in);
+        const size_t cap = std::min(kGradDirect, 2 * need);
+        r->h_in = lock_floats(r, cap);
+        r->h_in_cap = r->h_in ? cap : 0;
+    }
+    if (need <= r->h_in_cap) {
         std::memcpy(r->h_in, x, (size_t)n * F * 4);
         std::memcpy(r->h_in + (size_t)n * F, y, (size_t)n * 4);
         if (wt) std::memcpy(r->h_in + (size_t)n * (F + 1), wt, (size_t)n * 4);
@@ -1154,9 +1169,10 @@ int gss_res_grad(gss_res *r, int64_t n, const float *x, const float *y, const fl
         dy = r->ys.p;
         if (wt) dw = r->ws.p;
     }
-    if ((rc = run_batch(r, st, dx, dy, dw, nullptr, n, 1.f, 1.f, 0.f, true))) return rc;
-    std::memcpy(grad, r->h_res, P * 4);
-    if (loss) *loss = r->h_res[P];
+    const float *res = nullptr;
+    if ((rc = run_batch(r, st, dx, dy, dw, nullptr, n, 1.f, 1.f, 0.f, &res))) return rc;
+    std::memcpy(grad, res, P * 4);
+    if (loss) *loss = res[P];
     return GSS_OK;
 }
 

@@ -135,7 +135,8 @@ int gss_engine_cu_count(gss_engine *e, int *out);
 int gss_engine_sync(gss_engine *e);
 /* Host buffers that are only copy endpoints (the plain path's staging, the
  * steps' records on the host) are allocated pageable instead of page-locked
- * when one allocation reaches `bytes`, or when page-locking fails; bytes < 0
+ * when one allocation reaches `bytes`, or when page-locking fails, and the
+ * scorer's samples and results (gss_res_grad) then go through device memory; bytes < 0
  * (the default): no limit.  Replaces maxPageLockedMemory
  * (GpuClauseSharer.h:47, gpuShareLib/CorrespArr.cu:212-235).  Staging that the
  * step's kernels read in place stays page-locked. */

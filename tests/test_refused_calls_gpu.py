@@ -140,3 +140,35 @@ def test_steps_whose_record_buffers_are_not_page_locked(tmp_path):
             assert e.sweep(np.full(1, ALL)) == 100
             e.close()
     """)
+
+
+def test_scorer_pass_without_page_locked_memory(tmp_path):
+    """Samples and results then take the device's memory; so they do where the
+    engine's page-locked limit is below the samples' size."""
+    run_case(tmp_path, """
+        from gpusharesat_amd import residency as rs
+        rng = np.random.default_rng(3)
+        n = 3000
+        x = rng.normal(0, 1, (n, 12)).astype(np.float32)
+        y = (rng.random(n) < 0.3).astype(np.float32)
+        e = en.Engine(0)
+        e.enable_tags()
+        def grad(at_least, times):
+            r = rs.Residency(e, 64, seed=3)
+            fail.hip_fail_set(HOST_MALLOC, at_least, 0, times)
+            out = [r.grad(x[:m], y[:m]) for m in (n // 2, n, 100)]
+            r.close()
+            return out, fail.hip_fail_calls(HOST_MALLOC)
+        want, calls = grad(70_000, 0)
+        assert calls > 0
+        for at_least in (70_000, 1):
+            got, calls = grad(at_least, 1000)
+            assert calls > 0
+            for a, b in zip(got, want):
+                assert a[0] == b[0] and np.array_equal(a[1], b[1])
+        e.set_page_locked_limit(70_000)
+        got, calls = grad(70_000, 0)
+        assert calls == 0
+        for a, b in zip(got, want):
+            assert a[0] == b[0] and np.array_equal(a[1], b[1])
+    """)

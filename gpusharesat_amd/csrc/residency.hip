@@ -454,13 +454,18 @@ __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ para
             for (int c = 0; c < 4; c++)
                 a2[c] = mfma(a, s_w2[(16 * c + lc) * kLd + k + lr], a2[c]);
         }
+        // Rows past n take no part: parameters may be such that only they, which
+        // see the biases alone, overflow (a weight of 0 times infinity is NaN).
+        bool on[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) on[r] = t0 + r0 + 4 * lr + r < n;
         f32x4 z3 = {};
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             const float w3 = s_w3[16 * c + lc];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                a2[c][r] = fmaxf(a2[c][r], 0.f);
+                a2[c][r] = on[r] ? fmaxf(a2[c][r], 0.f) : 0.f;
                 z3[r] = fmaf(w3, a2[c][r], z3[r]);
             }
         }
@@ -472,8 +477,8 @@ __global__ __launch_bounds__(256) void k_mlp_pass(const float *__restrict__ para
             for (int d = 1; d < 16; d <<= 1) z += __shfl_xor(z, d);
             z += b3;
             const float yv = s_y[r0 + 4 * lr + r], sw = s_sw[r0 + 4 * lr + r];
-            d3[r] = sw * (sigmoidf(z) - yv);
-            if (lc == 0) {
+            d3[r] = on[r] ? sw * (sigmoidf(z) - yv) : 0.f;
+            if (lc == 0 && on[r]) {
                 gb3 += d3[r];
                 loss += sw * logistic_loss(z, yv);
             }

@@ -271,3 +271,25 @@ def test_mlp_gradient_at_tile_edges(engine_factory, n, weighted):
           flush=True)
     assert abs(loss - loss_ref) <= 3e-5 * abs(loss_ref)
     assert np.linalg.norm(g - g_ref) <= 3e-5 * np.linalg.norm(g_ref)
+
+
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 100])
+def test_mlp_rows_past_the_samples_take_no_part(engine_factory, n):
+    """Parameters for which a row without a sample, which sees the biases alone,
+    overflows where the samples do not: unit 0 of the second layer is 1e30 on its
+    bias and 0 with the first layer's unit 0, which is 1 for every sample.  The
+    samples' loss is then that of the output bias, an error of a few 2^-24."""
+    _, r = make_res(engine_factory)
+    h, f = rs.HIDDEN, rs.FEATURES
+    p = np.zeros(rs.PARAMS, np.float32)
+    b1, w2 = h * f, h * f + h
+    b2, w3, b3 = w2 + h * h, w2 + h * h + h, w2 + h * h + 2 * h
+    p[b1], p[w2], p[b2], p[w3], p[b3] = 1, -2e30, 1e30, 1e30, 0.1
+    r.params = p
+    rng = np.random.default_rng(n)
+    x = rng.normal(0, 1, (n, 12)).astype(np.float32)
+    y = (rng.random(n) < 0.3).astype(np.float32)
+    loss, g = r.grad(x, y)
+    loss_ref, g_ref = ref.loss_and_grad(p, x, y)
+    assert abs(loss - loss_ref) <= 1e-5 * loss_ref
+    assert np.allclose(g, g_ref, rtol=1e-5, atol=1e-6)

@@ -60,6 +60,7 @@ SIGNATURES: dict[str, list] = {
     "gss_hits_copy": [c_p, c_p, c_i64, c_p],
     "gss_hits_gather": [c_p, c_p, c_i64, c_p],
     "gss_sweep_kernel_ms": [c_p, c_p],
+    "gss_sweep_screened": [c_p, c_p],
     "gss_sweep_kernel_stats": [c_p, c_p, c_p, c_int],
     "gss_set_tuning": [c_p, c_int, c_int],
     "gss_autotune": [c_p, c_p, c_int, c_p, c_p],

@@ -464,6 +464,7 @@ struct gss_engine {
     DevBuf<uint64_t> sweep_agg_words;
     int screen_passes = 0;
     bool may_screen = false;
+    bool chosen = false;  // the last sweep launched, a step's included, had the choice
     bool time_due = false;  // the last waited sweep's time is still to be read (read_time)
     float last_ms = 0.f;
     double total_ms = 0.0;
@@ -677,17 +678,23 @@ hipError_t wait_counts(gss_engine *e) {
 // Whether a plain sweep may gain from screening, were its words' slots mostly of
 // one value (the device decides that: k_sweep_choose).  In microseconds, with
 // that: the plain kernel reads 2.8 rows a clause (52 per million of one line
-// each), the screened one takes 24 per million clauses after a pass over the
+// each, of the row's lines with a valid word), the screened one takes 24 per million clauses after a pass over the
 // table (5.5 TB/s); 12 are kept for the launches.  Measured, plain and screened
 // with its entries: 1M clauses x 8 words x 100K variables 43 and 27, 2M x 16 x
 // 500K 118 and 71, 400K x 64 x 200K 87 and 68.  Where the slots differ the
 // two launches that find out cost 7.
 // Also false without room for the entries.
-bool screening_may_pay(gss_engine *e, int64_t clauses) {
+bool screening_may_pay(gss_engine *e, int64_t clauses, const uint64_t *valid) {
     if (e->words < 8 || e->vars <= 0) return false;
     const double m = (double)clauses * 1e-6;
     const double rows = (double)e->vars * 2.0 * e->words * 8.0;
-    if (52.0 * m * std::max(1, e->words / 16) <= 24.0 * m + rows / 5.5e6 + 12.0) return false;
+    int lines = 0;  // of 16 words
+    for (int w = 0; w < e->words; w += 16) {
+        bool any = false;
+        for (int i = w; i < std::min(w + 16, e->words); i++) any |= valid[i] != 0;
+        lines += any;
+    }
+    if (52.0 * m * lines <= 24.0 * m + rows / 5.5e6 + 12.0) return false;
     if (e->sweep_agg.reserve_async((size_t)e->vars + 1, e->stream) ||
         e->sweep_agg_words.reserve_async(9, e->stream))
         return false;
@@ -699,6 +706,7 @@ bool screening_may_pay(gss_engine *e, int64_t clauses) {
 hipError_t launch_screened_choice(gss_engine *e, const uint64_t *valid, SweepArgs &a, int blocks,
                                   hipStream_t s) {
     uint32_t *choose = (uint32_t *)(e->sweep_agg_words.p + 8);
+    e->chosen = true;
     hipError_t he = launch_sweep_choose(e->table.p, valid, e->vars, e->words, e->sweep_agg.p,
                                         e->sweep_agg_words.p, choose, s);
     if (he != hipSuccess) return he;
@@ -720,6 +728,7 @@ int launch_current_sweep(gss_engine *e) {
     e->alloc_dirty = true;
     e->alloc_at ^= 1;
     e->sweep_waves = e->npasses > 0 ? (uint32_t)e->blocks * 4 : 0;
+    e->chosen = false;
     HIP_TRY(hipEventRecord(e->ev0, e->stream));
     if (e->npasses > 0) {
         SweepArgs a{};
@@ -1554,7 +1563,7 @@ int gss_sweep_async(gss_engine *e, const uint64_t *valid) {
         if (e->d_hits.p != old) e->waited = false;  // the last sweep's records are gone
         if (rc) return rc;
     }
-    e->may_screen = screening_may_pay(e, e->total_clauses);
+    e->may_screen = screening_may_pay(e, e->total_clauses, valid);
     e->waited = false;
     if ((rc = launch_current_sweep(e))) return rc;
     e->sweep_rows_version = e->rows_version;
@@ -1655,6 +1664,20 @@ int gss_sweep_kernel_ms(gss_engine *e, float *ms) {
     if (!e || !ms) return set_err(GSS_E_INVAL, "null argument");
     if (const int rc = read_time(e)) return rc;
     *ms = e->last_ms;
+    return GSS_OK;
+}
+
+int gss_sweep_screened(gss_engine *e, int *out) {
+    int rc = check_engine(e);
+    if (rc) return rc;
+    if (!out) return set_err(GSS_E_INVAL, "null argument");
+    *out = -1;
+    if (!e->chosen) return GSS_OK;
+    uint32_t v = 0;
+    HIP_TRY(hipMemcpyAsync(&v, e->sweep_agg_words.p + 8, sizeof v, hipMemcpyDeviceToHost,
+                           e->stream));
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    *out = v ? 1 : 0;
     return GSS_OK;
 }
 
@@ -1923,6 +1946,7 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     a.agg = agg;
     a.agg_words = agg ? e->serve_agg_words.p : nullptr;
     hipError_t he = hipSuccess;
+    e->chosen = false;
     if (sl.plan.may_screen) he = launch_screened_choice(e, dh->valid, a, sl.plan.blocks, s);
     if (he == hipSuccess) he = launch_sweep(a, e->words, sl.plan.blocks, s);
     const ChunkArgs c = step_chunks(sl, sl.rec_words);
@@ -2480,7 +2504,7 @@ int gss::step_submit_ex(gss_engine *e, const gss_step_desc *desc, bool serve) {
     pl.serve = serve;
     pl.screen = screen;
     pl.agg_full = agg_full;
-    pl.may_screen = !serve && !screen && screening_may_pay(e, e->total_clauses + n);
+    pl.may_screen = !serve && !screen && screening_may_pay(e, e->total_clauses + n, valid);
     // Few literals go straight from the staging to their rows (32-byte reads
     // over PCIe); more are copied first and scattered by a kernel of its own.
     pl.staged = total > kDirectLits;

@@ -244,6 +244,12 @@ class Engine:
         _lib.call("gss_sweep_kernel_ms", self._h, ctypes.byref(v))
         return v.value
 
+    def screened(self) -> int:
+        """Whether the last sweep was screened: 1, 0, or -1 (not considered)."""
+        v = ctypes.c_int()
+        _lib.call("gss_sweep_screened", self._h, ctypes.byref(v))
+        return v.value
+
     def kernel_stats(self, reset: bool = False) -> tuple[float, int]:
         t, c = ctypes.c_double(), ctypes.c_int64()
         _lib.call("gss_sweep_kernel_stats", self._h, ctypes.byref(t), ctypes.byref(c), int(reset))

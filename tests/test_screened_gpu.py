@@ -171,3 +171,45 @@ def test_screening_tables_of_odd_sizes(engine_factory, W, n, variables):
         sv.submit(e, valid, records=sv.RECORDS_IDS, flags=flags)
         assert e.step_wait()[0] == exp.size
         assert np.array_equal(np.sort(e.step_ids_view().view(np.uint64).ravel()), want)
+
+
+@pytest.mark.parametrize("agree", [True, False])
+@pytest.mark.parametrize("W, used", [(8, 1), (16, 2), (16, 3), (32, 4), (64, 8), (64, 17)])
+def test_choice_looks_at_the_words_in_use(engine_factory, W, used, agree):
+    """Few words with a valid slot, whose slots agree beside words that hold
+    nothing, or differ beside words that hold one value: what the other words hold
+    does not count."""
+    rng = np.random.default_rng(70 + W + used)
+    n = 900_000
+    sigma = rng.random(V) < 0.5
+    lens = rng.integers(3, 6, size=n).astype(np.int32)
+    v = rng.integers(0, V, size=int(lens.sum()))
+    lits = (2 * v + ((rng.random(v.size) < 0.15) == sigma[v])).astype(np.uint32)
+    off = np.zeros(n + 1, np.int64)
+    off[1:] = np.cumsum(lens)
+    one = np.repeat(np.where(sigma, ALL, np.uint64(0))[:, None], W, axis=1)
+    is_def, is_true = np.full((V, W), ALL), one.copy()
+    if agree:
+        is_def[:, used:] = 0
+    else:
+        is_true[:, :used] = rng.integers(0, 1 << 63, size=(V, used), dtype=np.uint64)
+    is_true &= is_def
+    valid = np.zeros(W, np.uint64)
+    valid[:used] = ALL
+    valid[used - 1] = np.uint64(0x7FFFFFFFFFFFFF0F)
+    exp = orc.sweep(off, lits, is_def, is_true, valid)
+    e = engine_factory()
+    rows = e.append(lits, lens).astype(np.uint64)
+    e.reset_assignments(V, W)
+    e.upload(is_def, is_true)
+    c = exp["clause"]
+    want = np.sort(rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
+                   | (exp["word"].astype(np.uint64) << np.uint64(48)))
+    print(f"{W} words, {used} in use: {exp.size} records", flush=True)
+    assert e.sweep(valid) == exp.size
+    assert np.array_equal(np.sort(e.hits().view(np.uint64).reshape(-1, 3)[:, 0]), want)
+    assert e.screened() == int(agree)
+    sv.submit(e, valid, records=sv.RECORDS_IDS)
+    assert e.step_wait()[0] == exp.size
+    assert e.screened() == int(agree)
+    assert np.array_equal(np.sort(e.step_ids_view().view(np.uint64).ravel()), want)

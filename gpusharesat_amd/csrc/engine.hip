@@ -702,7 +702,7 @@ bool screening_may_pay(gss_engine *e, int64_t clauses, const uint64_t *valid) {
 }
 
 // Before a sweep a that may be screened: the choice, and the screened kernel if
-// that is it (a is launched after it, and runs if it is not).
+// that is it (a is launched after it, and runs if it is not).  valid: host memory.
 hipError_t launch_screened_choice(gss_engine *e, const uint64_t *valid, SweepArgs &a, int blocks,
                                   hipStream_t s) {
     uint32_t *choose = (uint32_t *)(e->sweep_agg_words.p + 8);
@@ -745,7 +745,8 @@ int launch_current_sweep(gss_engine *e) {
         a.alloc = e->d_alloc + 8 * e->alloc_at;
         a.chunk_cap = e->chunk_cap;
         a.rec_words = 3;
-        if (e->may_screen) HIP_TRY(launch_screened_choice(e, e->d_valid, a, e->blocks, e->stream));
+        if (e->may_screen)
+            HIP_TRY(launch_screened_choice(e, e->valid_up.data(), a, e->blocks, e->stream));
         HIP_TRY(launch_sweep(a, e->words, e->blocks, e->stream));
     }
     HIP_TRY(hipEventRecord(e->ev1, e->stream));
@@ -1947,7 +1948,8 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     a.agg_words = agg ? e->serve_agg_words.p : nullptr;
     hipError_t he = hipSuccess;
     e->chosen = false;
-    if (sl.plan.may_screen) he = launch_screened_choice(e, dh->valid, a, sl.plan.blocks, s);
+    if (sl.plan.may_screen)
+        he = launch_screened_choice(e, sl.h_hdr.p->valid, a, sl.plan.blocks, s);
     if (he == hipSuccess) he = launch_sweep(a, e->words, sl.plan.blocks, s);
     const ChunkArgs c = step_chunks(sl, sl.rec_words);
     if (sl.plan.serve) {

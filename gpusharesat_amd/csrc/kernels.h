@@ -196,7 +196,8 @@ struct StepInArgs {
 };
 
 // Plain sweeps, words >= 8: decides from a sample of the table whether the sweep
-// is screened (*choose), and if so builds the entries and agg_words.
+// is screened (*choose), and if so builds the entries and agg_words.  valid is
+// host memory, read before the launch.
 hipError_t launch_sweep_choose(const uint64_t *table, const uint64_t *valid, int64_t vars,
                                int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
                                hipStream_t s);

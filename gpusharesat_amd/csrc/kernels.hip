@@ -63,6 +63,7 @@
 #include <hipcub/hipcub.hpp>
 #include <utility>
 
+#include "chunks.h"
 #include "kernels.h"
 
 namespace gss {
@@ -833,15 +834,6 @@ __device__ __forceinline__ void base_update(const gss_base_update &x, uint64_t *
     else atomicAnd(tru, ~bit);
 }
 
-__device__ __forceinline__ uint64_t wave_incl_scan(uint64_t x, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t y = __shfl_up(x, d);
-        if (lane >= d) x += y;
-    }
-    return x;
-}
-
 // Admission of a serving step: in sequence order, the published requests whose
 // words fit the table.  One wave reads the ring (two reads over PCIe, one
 // after the other) while the header is on its way, and fills the header in
@@ -1142,21 +1134,6 @@ __device__ __forceinline__ void sum_fills(const uint32_t *__restrict__ fills, ui
     __syncthreads();
     before = s_sum[0][0] + s_sum[0][1] + s_sum[0][2] + s_sum[0][3];
     total = s_sum[1][0] + s_sum[1][1] + s_sum[1][2] + s_sum[1][3];
-}
-
-// Ends of 64 chunks' records (exclusive sums from the first one's start), from
-// a lane's chunk of `fill` records; the first wave writes them.
-__device__ __forceinline__ void fill_ends(uint32_t fill, uint32_t *ends) {
-    if (threadIdx.x < 64) ends[threadIdx.x] = (uint32_t)wave_incl_scan(fill, (int)threadIdx.x);
-}
-
-// The chunk that record i of the 64 is in: the first that ends after it.
-__device__ __forceinline__ uint32_t chunk_of(const uint32_t *ends, uint32_t i) {
-    uint32_t k = 0;
-#pragma unroll
-    for (uint32_t d = 32; d > 0; d >>= 1)
-        if (ends[k + d - 1] <= i) k += d;
-    return k;
 }
 
 // Words [0, m) of 64 chunks' records (ends: fill_ends) to dst, a thread per

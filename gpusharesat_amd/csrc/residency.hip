@@ -28,6 +28,7 @@
 #include <new>
 #include <vector>
 
+#include "chunks.h"
 #include "engine_internal.h"
 #include "errors.h"
 #include "gss.h"
@@ -152,66 +153,75 @@ __global__ void k_res_init(TagState s, const uint32_t *__restrict__ tags,
     s.alive[t] = 1;
 }
 
-// Hit records -> tag state, one 256-thread block per quarter of a claimed
-// chunk (one record per thread: a sweep claims few chunks, so one block per
-// chunk would leave the kernel waiting on four dependent lookup chains in a
-// row).  A clause's records (one per assignment word that hit it) are adjacent in
-// its chunk, so each wave merges runs of equal (len, row): the run's first
-// lane ORs the run's word bits with a segmented suffix scan and issues one
-// atomicAdd of the run length and one atomicOr for the whole run.
+// Hit records -> tag state, a thread per record, whatever chunk it is in: every
+// wave of a sweep owns a chunk (7,168 on a full grid), most of them with few
+// records, so a block takes a run of chunks.  Records of one clause that are
+// neighbours are merged: a run of equal (len, row) ORs its word bits with a
+// segmented suffix scan and issues one atomicAdd of the run length and one
+// atomicOr.
+//
+// Bound by atomics: device-scope ones on one address are serialised (~10 ns
+// each), and each block with a record adds to `pairs`.  With a block per quarter of
+// a chunk, 1M clauses x 16 words, 660,000 records took 94 us, now 22; 300,000 x
+// 64, 790,000 records 83, now 32 (2,048 blocks: 30 and 28).
 constexpr uint32_t kRecBlock = 256;  // k_res_records block size
-constexpr uint32_t kRecParts = kHitChunk / kRecBlock;
-static_assert(kHitChunk % kRecBlock == 0, "a chunk splits into whole blocks");
+constexpr uint32_t kRecBlocks = 1024;
 
-__global__ void k_res_records(const gss_hit *__restrict__ hits, const uint32_t *__restrict__ fills,
-                              uint32_t chunks, const uint32_t *const *__restrict__ tagptr,
-                              int ntagptr, TagState s, unsigned long long *pairs) {
+__global__ __launch_bounds__(256) void k_res_records(const gss_hit *__restrict__ hits,
+                                                     const uint32_t *__restrict__ fills,
+                                                     uint32_t chunks,
+                                                     const uint32_t *const *__restrict__ tagptr,
+                                                     int ntagptr, TagState s,
+                                                     unsigned long long *pairs) {
     __shared__ unsigned long long blk;
+    __shared__ uint32_t s_end[64];
     if (threadIdx.x == 0) blk = 0;
-    __syncthreads();
     const int lane = threadIdx.x & 63;
     unsigned long long mine = 0;
-    const uint64_t parts = (uint64_t)chunks * kRecParts;
-    for (uint64_t g = blockIdx.x; g < parts; g += gridDim.x) {
-        const uint32_t c = (uint32_t)(g / kRecParts);
-        const uint32_t f = fills[c];  // uniform in the block
-        const uint32_t base = (uint32_t)(g % kRecParts) * kRecBlock;
-        if (base >= f) continue;
-        const uint32_t i = base + threadIdx.x;
-        const bool on = i < f;
-        uint32_t row = 0, len = 0xffffffffu;
-        uint64_t bit = 0;
-        const uint32_t *tp = nullptr;
-        if (on) {
-            const gss_hit h = hits[(size_t)c * kHitChunk + i];
-            row = h.row;
-            len = h.len;
-            bit = 1ull << (h.word & 63);
-            tp = (int)len < ntagptr ? tagptr[len] : nullptr;
-            if (tp) mine += (unsigned long long)__popcll(h.false_mask | h.unit_mask);
-        }
-        const uint32_t prow = (uint32_t)__shfl_up((int)row, 1);
-        const uint32_t plen = (uint32_t)__shfl_up((int)len, 1);
-        const bool head = on && (lane == 0 || prow != row || plen != len);
-        // a run ends at the next head or at the first lane past the fill
-        const uint64_t bound = __ballot(head || !on);
-        const uint64_t above = lane == 63 ? 0ull : bound & (~0ull << (lane + 1));
-        const int end = above ? __ffsll((unsigned long long)above) - 1 : 64;
-        uint64_t acc = bit;
+    const uint32_t per = (chunks + gridDim.x - 1) / gridDim.x;
+    const uint32_t c0 = blockIdx.x * per, c1 = c0 + per < chunks ? c0 + per : chunks;
+    for (uint32_t c = c0; c < c1; c += 64) {
+        __syncthreads();  // everyone is done with the ends
+        fill_ends(threadIdx.x < 64 && c + threadIdx.x < c1 ? fills[c + threadIdx.x] : 0u, s_end);
+        __syncthreads();
+        const uint32_t total = s_end[63];
+        for (uint32_t base = 0; base < total; base += kRecBlock) {
+            const uint32_t i = base + threadIdx.x;
+            const bool on = i < total;
+            uint32_t row = 0, len = 0xffffffffu;
+            uint64_t bit = 0;
+            const uint32_t *tp = nullptr;
+            if (on) {
+                const uint32_t k = chunk_of(s_end, i), at = i - (k ? s_end[k - 1] : 0u);
+                const gss_hit h = hits[(size_t)(c + k) * kHitChunk + at];
+                row = h.row;
+                len = h.len;
+                bit = 1ull << (h.word & 63);
+                tp = (int)len < ntagptr ? tagptr[len] : nullptr;
+                if (tp) mine += (unsigned long long)__popcll(h.false_mask | h.unit_mask);
+            }
+            const uint32_t prow = (uint32_t)__shfl_up((int)row, 1);
+            const uint32_t plen = (uint32_t)__shfl_up((int)len, 1);
+            const bool head = on && (lane == 0 || prow != row || plen != len);
+            // a run ends at the next head or at the first lane without a record
+            const uint64_t bound = __ballot(head || !on);
+            const uint64_t above = lane == 63 ? 0ull : bound & (~0ull << (lane + 1));
+            const int end = above ? __ffsll((unsigned long long)above) - 1 : 64;
+            uint64_t acc = bit;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t lo = (uint32_t)__shfl_down((int)(uint32_t)acc, d);
-            const uint32_t hi = (uint32_t)__shfl_down((int)(uint32_t)(acc >> 32), d);
-            if (lane + d < end) acc |= ((uint64_t)hi << 32) | lo;
-        }
-        if (head && tp) {
-            const uint32_t t = tp[row];
-            atomicAdd(&s.cnt[t], (uint32_t)(end - lane));
-            atomicOr((unsigned long long *)&s.solv[t], (unsigned long long)acc);
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t lo = (uint32_t)__shfl_down((int)(uint32_t)acc, d);
+                const uint32_t hi = (uint32_t)__shfl_down((int)(uint32_t)(acc >> 32), d);
+                if (lane + d < end) acc |= ((uint64_t)hi << 32) | lo;
+            }
+            if (head && tp) {
+                const uint32_t t = tp[row];
+                atomicAdd(&s.cnt[t], (uint32_t)(end - lane));
+                atomicOr((unsigned long long *)&s.solv[t], (unsigned long long)acc);
+            }
         }
     }
-    // Device-scope atomics on one address are serialised (~10 ns each):
-    // blocks with nothing to add issue none.
+    __syncthreads();
     if (mine) atomicAdd(&blk, mine);
     __syncthreads();
     if (threadIdx.x == 0 && blk) atomicAdd(pairs, blk);
@@ -915,9 +925,7 @@ int gss_res_account(gss_res *r, int32_t round, int64_t *hit_pairs) {
     RES_HIP(hipMemsetAsync(r->counters.p, 0, 2 * sizeof(unsigned long long), st));
     RES_HIP(hipMemsetAsync(r->maxbits.p, 0, 4, st));
     if (chunks) {
-        const uint64_t parts = (uint64_t)chunks * kRecParts;
-        hipLaunchKernelGGL(k_res_records, dim3((unsigned)std::min<uint64_t>(parts, 1u << 20)),
-                           dim3(kRecBlock), 0,
+        hipLaunchKernelGGL(k_res_records, dim3(std::min(chunks, kRecBlocks)), dim3(kRecBlock), 0,
                            st, hits, fills, chunks, r->tagptr.p, (int)tp.size(), r->state(),
                            r->counters.p);
         RES_HIP(hipGetLastError());

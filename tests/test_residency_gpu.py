@@ -293,3 +293,33 @@ def test_mlp_rows_past_the_samples_take_no_part(engine_factory, n):
     loss_ref, g_ref = ref.loss_and_grad(p, x, y)
     assert abs(loss - loss_ref) <= 1e-5 * loss_ref
     assert np.allclose(g, g_ref, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("W, n, assigned", [(1, 40, 0.9), (1, 70_000, 0.9), (1, 300_000, 0.5),
+                                            (16, 300_000, 0.9), (16, 300_000, 0.3)])
+def test_record_accounting_over_many_chunks(engine_factory, W, n, assigned):
+    """From a few chunks of records to one for each of a full grid's waves and
+    more claimed, with few records each or full."""
+    rng = np.random.default_rng(n + W)
+    V = 500
+    e, r = make_res(engine_factory, max_tags=n)
+    e.reset_assignments(V, W)
+    d = workloads.bernoulli_words(rng, V, W * 64, assigned)
+    e.upload(d, workloads.bernoulli_words(rng, V, W * 64, 0.3) & d)
+    lens = rng.integers(1, 6, size=n).astype(np.int32)
+    lits = rng.integers(0, 2 * V, size=int(lens.sum())).astype(np.uint32)
+    tags = rng.permutation(n).astype(np.uint32)
+    r.add(lits, lens, tags, 0)
+    e.sweep(np.full(W, ALL))
+    hits = e.hits()
+    print(f"{W} words, {n} clauses: {hits.size} records", flush=True)
+    cnt, bits = np.zeros(n, np.int64), np.zeros(n, np.uint64)
+    for length in np.unique(hits["len"]):
+        h = hits[hits["len"] == length]
+        t = e.read_tags(int(length))[h["row"]]
+        np.add.at(cnt, t, 1)
+        np.bitwise_or.at(bits, t, np.uint64(1) << h["word"].astype(np.uint64))
+    assert r.account(1) == int(np.bitwise_count(hits["false_mask"] | hits["unit_mask"]).sum())
+    f = r.features(1, np.arange(n, dtype=np.uint32))
+    assert np.allclose(f[:, 4], np.log1p(cnt) / 6, atol=1e-6)
+    assert np.array_equal(f[:, 10], (np.bitwise_count(bits) / 64).astype(np.float32))

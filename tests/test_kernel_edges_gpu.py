@@ -9,7 +9,8 @@ import pytest
 
 import _oracle as orc
 from gpusharesat_amd import serving as sv
-from gpusharesat_amd.engine import HIT_CLAUSE_DTYPE, HIT_DTYPE, HIT_ID_DTYPE
+from gpusharesat_amd.engine import (HIT_CLAUSE_DTYPE, HIT_DTYPE, HIT_ID_DTYPE, TUNE_SCHEDULE,
+                                    TUNE_TASK_CLAUSES, TUNE_WAVES_PER_CU)
 
 pytestmark = pytest.mark.gpu
 
@@ -126,3 +127,35 @@ def test_first_sweeps_of_engines_in_turn():
         assert e.sweep(np.full(1, ALL)) == n
         assert np.array_equal(np.sort(e.hits()["row"]), np.arange(n))
         e.close()
+
+
+@pytest.mark.parametrize("passes", [1, 2, 3, "W", "W+1", 1000])
+@pytest.mark.parametrize("W", [1, 2, 4, 8, 16, 32, 64])
+def test_passes_a_wave_takes_at_a_time(engine_factory, W, passes):
+    """Runs of one pass, an odd number, W (the passes a clause record is held
+    for) and more, few waves with many tasks, short clauses first: all records
+    as without these settings."""
+    V, lits, lens, is_def, is_true, valid, exp = edge_case(W)
+    e = engine_factory()
+    rows = e.append(lits, lens).astype(np.uint64)
+    e.reset_assignments(V, W)
+    e.upload(is_def, is_true)
+    n = {"W": W, "W+1": W + 1}.get(passes, passes)
+    e.set_tuning(TUNE_TASK_CLAUSES, n * (64 // W))
+    if n != 2:
+        e.set_tuning(TUNE_WAVES_PER_CU, 4)
+    if n % 2:
+        e.set_tuning(TUNE_SCHEDULE, 2)
+    key = rows[exp["clause"]] | (lens[exp["clause"]].astype(np.uint64) << np.uint64(32))
+    ids = np.sort(key | (exp["word"].astype(np.uint64) << np.uint64(48)))
+    clauses, inv = np.unique(key, return_inverse=True)
+    words = np.zeros(clauses.size, np.uint64)
+    np.bitwise_or.at(words, inv, np.uint64(1) << exp["word"].astype(np.uint64))
+    assert e.sweep(valid) == exp.size
+    assert np.array_equal(np.sort(e.hits().view(np.uint64).reshape(-1, 3)[:, 0]), ids)
+    for flags in (0, sv.STEP_SCREEN):
+        sv.submit(e, valid, records=sv.RECORDS_CLAUSES, flags=flags)
+        assert e.step_wait()[0] == clauses.size
+        got = e.step_clauses_view().view(np.uint64).reshape(-1, 2)
+        got = got[np.argsort(got[:, 0])]
+        assert np.array_equal(got[:, 0], clauses) and np.array_equal(got[:, 1], words)

@@ -120,9 +120,8 @@ __device__ __forceinline__ uint64_t load_word(const uint64_t *__restrict__ table
 typedef const __attribute__((address_space(1))) uint32_t *LitPtr;
 
 // A clause is checked by W lanes (lane w: table word w), which share its
-// literals: a literal register holds G = min(W, 16) consecutive literals of
-// the clause, one per lane of each G-lane group, and kRegs of them hold the
-// first kHeld literals.  Wider clauses repeat the group (every 16-lane DPP
+// literals: each lane of a group of G = min(W, 16) holds kRegs consecutive ones,
+// the group the first kHeld.  Wider clauses repeat the group (every 16-lane DPP
 // row holds the same 16 literals), so a literal is always handed out inside
 // one DPP row.
 template <int W>
@@ -138,7 +137,7 @@ struct Lits {
 // 8, quad_perm for 4 and 2), so no LDS.  All 64 lanes must call it.
 template <int W, int J>
 __device__ __forceinline__ uint32_t lit_at(const Lits<W> &l) {
-    constexpr int G = Lits<W>::G, R = J / G, Q = J % G;
+    constexpr int G = Lits<W>::G, R = J % Lits<W>::kRegs, Q = J / Lits<W>::kRegs;
     const int x = (int)l.r[R];
     if constexpr (G == 16) {
         return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x150 + Q, 0xF, 0xF, false);
@@ -154,17 +153,33 @@ __device__ __forceinline__ uint32_t lit_at(const Lits<W> &l) {
     }
 }
 
-// Literals [base, base + kHeld) of the clause whose row starts at cl (lane q
-// of its group holds literals base + q + G * r), the sentinel past its end
-// and for lanes without a clause (on = false).
+// Literals [base, base + kHeld) of the clause whose row starts at cl (lane q of
+// its group holds kRegs of them from base + q * kRegs on), the sentinel past its
+// end and for lanes without a clause (on = false).  One load a lane where they
+// are all there (rows are 4-byte aligned, as these loads may be): the lanes of a
+// narrow table read lines of their own, one each per load (1 word, 150k clauses of
+// 20 to 60 literals: 65 us with a load per literal, 55 so).
 template <int W>
 __device__ __forceinline__ Lits<W> load_lits(LitPtr cl, int base, int len,
                                              int q, bool on, uint32_t sentinel) {
+    constexpr int R = Lits<W>::kRegs;
+    const int j = base + q * R;
     Lits<W> l;
 #pragma unroll
-    for (int r = 0; r < Lits<W>::kRegs; r++) {
-        const int j = base + r * Lits<W>::G + q;
-        l.r[r] = on && j < len ? cl[j] : sentinel;
+    for (int r = 0; r < R; r++) l.r[r] = sentinel;
+    if constexpr (R == 1) {
+        if (on && j < len) l.r[0] = cl[j];
+    } else {
+        typedef uint32_t Vec __attribute__((ext_vector_type(R), aligned(4)));
+        if (on && j + R <= len) {
+            const Vec v = *(const __attribute__((address_space(1))) Vec *)(cl + j);
+#pragma unroll
+            for (int r = 0; r < R; r++) l.r[r] = v[r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (on && j + r < len) l.r[r] = cl[j + r];
+        }
     }
     return l;
 }
@@ -200,6 +215,14 @@ constexpr int kSweepBlocksPerCu = 7;
 // number of clauses (tasks of a fixed 64 clauses left 4.4 tasks per wave on 2M
 // clauses: some waves had 5), and a wave reads its literals in long runs.
 constexpr int kTaskRounds = 4;
+
+// Tables of less than 8 words: rows read per step past a clause's held literals.
+// A row there is part of a line and comes from the L2s, so long clauses are bound
+// by the chain of reads, not by their number; with the literals one step ahead.
+// 200k variables x 1 word, 150k clauses of 20 to 60 literals, nine in ten false:
+// 65 us with two rows per step, 49 with eight; 40k of 150 to 400, 97 in 100 false:
+// 148 and 94 (four rows: 55 and 128).
+constexpr int kTailRows = 8;
 
 struct Passes {
     int nbuckets, total, tp, gw, nw;
@@ -427,7 +450,36 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
                        step1.template operator()<2 + 2 * P2 + I, (2 + 2 * P2 + I < kKeep)>(cur)),
                  ...);
             }(std::make_integer_sequence<int, H - 2 - 2 * P2>{});
-            if (go && len > H) {
+            if constexpr (W < 8) {
+                if (go && len > H) {
+                    constexpr int R = kTailRows / H;
+                    Lits<W> l[R];
+#pragma unroll
+                    for (int s = 0; s < R; s++)
+                        l[s] = load_lits<W>(clause(pass), H + s * H, len, q, on, a.sentinel);
+                    for (int base = H; base < len && go; base += R * H) {
+                        Lits<W> next[R];
+                        uint32_t o[R * H];
+#pragma unroll
+                        for (int s = 0; s < R; s++)
+                            next[s] = load_lits<W>(clause(pass), base + (R + s) * H, len, q, on,
+                                                   a.sentinel);
+                        [&]<int... I>(std::integer_sequence<int, I...>) {
+                            ((o[I] = scale_offset<W>(lit_at<W, I % H>(l[I / H])) | w8), ...);
+                        }(std::make_integer_sequence<int, R * H>{});
+                        if (c2 != ~0ull) {
+                            uint64_t y[R * H];
+#pragma unroll
+                            for (int i = 0; i < R * H; i++) y[i] = load_word(table, o[i]);
+#pragma unroll
+                            for (int i = 0; i < R * H; i++) fold(y[i]);
+                        }
+                        go = __ballot(c2 != ~0ull) != 0;
+#pragma unroll
+                        for (int s = 0; s < R; s++) l[s] = next[s];
+                    }
+                }
+            } else if (go && len > H) {
                 for (int base = H; base < len && go; base += H) {
                     const Lits<W> l = load_lits<W>(clause(pass), base, len, q, on, a.sentinel);
                     [&]<int... I>(std::integer_sequence<int, I...>) {
@@ -453,13 +505,24 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
                     ((rest &= I < len ? ~f[I] : ~0ull), ...);
                     ((um &= t[I]), ...);
                     // positions past the kept rows, for the slots left over
+                    constexpr int R = W < 8 ? kTailRows / H : 1;
                     for (int base = kKeep; base < len && __ballot((rest & um) != 0);
-                         base += kKeep) {
-                        const Lits<W> l = load_lits<W>(clause(pass), base, len, q, on, a.sentinel);
+                         base += R * kKeep) {
+                        Lits<W> l[R];
+                        uint64_t u[R][kKeep];
+#pragma unroll
+                        for (int s = 0; s < R; s++)
+                            l[s] = load_lits<W>(clause(pass), base + s * kKeep, len, q, on,
+                                                a.sentinel);
                         const bool need = (rest & um) != 0;
-                        ((t[I] = base + I < len ? neg_row.template operator()<I>(l, need) : ~0ull),
-                         ...);
-                        ((um &= ~rest | t[I]), ...);
+#pragma unroll
+                        for (int s = 0; s < R; s++)
+                            ((u[s][I] = base + s * kKeep + I < len
+                                            ? neg_row.template operator()<I>(l[s], need)
+                                            : ~0ull),
+                             ...);
+#pragma unroll
+                        for (int s = 0; s < R; s++) ((um &= ~rest | u[s][I]), ...);
                     }
                 }(std::make_integer_sequence<int, kKeep>{});
             }

@@ -159,3 +159,50 @@ def test_passes_a_wave_takes_at_a_time(engine_factory, W, passes):
         got = e.step_clauses_view().view(np.uint64).reshape(-1, 2)
         got = got[np.argsort(got[:, 0])]
         assert np.array_equal(got[:, 0], clauses) and np.array_equal(got[:, 1], words)
+
+
+@pytest.mark.parametrize("W", [1, 2, 4])
+def test_long_clauses_of_narrow_tables(engine_factory, W):
+    """Lengths around the rows read per step past the held literals, most clauses
+    with one or two literals that may be non-false anywhere, the last included."""
+    rng = np.random.default_rng(4600 + W)
+    V = 3000
+    lens = rng.permutation(np.repeat([*range(37, 54), 199, 200, 203, 204, 205, 400], 67))
+    lens = lens.astype(np.int32)
+    off = np.zeros(lens.size + 1, np.int64)
+    off[1:] = np.cumsum(lens)
+    sigma = rng.random(V) < 0.5
+    v = rng.integers(0, V, size=int(off[-1]))
+    false = np.ones(v.size, bool)
+    false[off[:-1] + rng.integers(0, lens)] = rng.random(lens.size) < 0.3
+    false[off[1:] - 1] &= rng.random(lens.size) < 0.8
+    lits = (2 * v + (false == sigma[v])).astype(np.uint32)
+    one = np.where(sigma, ALL, np.uint64(0))
+    is_def, is_true = np.full((V, W), ALL), np.repeat(one[:, None], W, axis=1)
+    bit = np.uint64(1) << rng.integers(0, 64, size=(V, W), dtype=np.uint64)
+    is_def ^= np.where(rng.random((V, W)) < 0.05, bit, np.uint64(0))
+    undef = rng.random(V) < 0.3  # half of them: undefined in the upper slots
+    is_def[undef] &= np.uint64(0xFFFFFFFF)
+    is_true &= is_def
+    valid = np.full(W, ALL)
+    exp = orc.sweep(off, lits, is_def, is_true, valid)
+    assert (exp["unit_mask"] != 0).sum() > 100 and (exp["false_mask"] != 0).sum() > 100
+    e = engine_factory()
+    rows = e.append(lits, lens).astype(np.uint64)
+    e.reset_assignments(V, W)
+    e.upload(is_def, is_true)
+    c = exp["clause"]
+    want = np.empty((exp.size, 3), np.uint64)
+    want[:, 0] = (rows[c] | (lens[c].astype(np.uint64) << np.uint64(32))
+                  | (exp["word"].astype(np.uint64) << np.uint64(48)))
+    want[:, 1], want[:, 2] = exp["false_mask"], exp["unit_mask"]
+    want = want[np.argsort(want[:, 0])]
+    print(f"{W} words: {lens.size} clauses, {exp.size} records", flush=True)
+    assert e.sweep(valid) == exp.size
+    got = e.hits().view(np.uint64).reshape(-1, 3)
+    assert np.array_equal(got[np.argsort(got[:, 0])], want)
+    for flags in (0, sv.STEP_SCREEN):
+        sv.submit(e, valid, flags=flags)
+        assert e.step_wait()[0] == exp.size
+        got = e.step_hits_view().view(np.uint64).reshape(-1, 3)
+        assert np.array_equal(got[np.argsort(got[:, 0])], want)

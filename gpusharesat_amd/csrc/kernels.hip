@@ -30,8 +30,8 @@
 //
 // Work mapping.  k_sweep: W lanes check one clause, one table word each, 64 / W
 // clauses per wave pass, literals handed out with DPP (no LDS); k_sweep_screened:
-// one clause per lane against the screening entries, then one surviving clause
-// and two words per lane.  Waves are persistent and walk the clauses in tasks of
+// one clause per lane against the screening entries, then two words of a surviving
+// clause per lane, or W lanes per clause where most words are left.  Waves are persistent and walk the clauses in tasks of
 // passes.  Steps are screened on request; other sweeps where a look at the
 // table says that it pays (k_sweep_choose).
 //
@@ -216,18 +216,27 @@ constexpr int kSweepBlocksPerCu = 7;
 // clauses: some waves had 5), and a wave reads its literals in long runs.
 constexpr int kTaskRounds = 4;
 
-// Tables of less than 8 words: rows read per step past a clause's held literals.
+// Tables of less than 8 words: kRows rows read per step past a clause's held
+// literals, and kept of these for the negated-row reads.
 // A row there is part of a line and comes from the L2s, so long clauses are bound
 // by the chain of reads, not by their number; with the literals one step ahead.
 // 200k variables x 1 word, 150k clauses of 20 to 60 literals, nine in ten false:
 // 65 us with two rows per step, 49 with eight; 40k of 150 to 400, 97 in 100 false:
 // 148 and 94 (four rows: 55 and 128).
-constexpr int kTailRows = 8;
+constexpr int kRows = 8;
 
+//
+// A pass of a screened sweep is 64 clauses, checked one after the other as far as
+// they survive: where there are fewer passes than waves it is split into up to
+// max_split parts (a power of two, at most the table's words).  A pass of 32 words
+// and more is so much work that three parts per wave are better than one (600k
+// clauses x 64 words, 9,375 passes, nothing known: 1,097 us whole, 956 in halves);
+// four were not (400k: 255 us per sweep whole, 254 in halves, 281 in quarters).
 struct Passes {
     int nbuckets, total, tp, gw, nw;
+    int split = 0;  // log2 of the parts
 
-    __device__ __forceinline__ Passes(const SweepArgs &a, bool screened) {
+    __device__ __forceinline__ Passes(const SweepArgs &a, bool screened, int max_split) {
         nbuckets = a.nbuckets;
         total = a.npasses;
         if (a.dyn) {
@@ -236,7 +245,10 @@ struct Passes {
         }
         gw = uniform((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));  // 256-thread blocks
         nw = (int)gridDim.x * 4;
-        tp = a.task_passes;
+        const int64_t room = max_split > 16 ? 3ll * nw : nw;
+        while ((2 << split) <= max_split && ((int64_t)total << (split + 1)) <= room) split++;
+        total <<= split;
+        tp = a.task_passes << split;
         if (tp <= 0) tp = (total - 1) / (nw * kTaskRounds) + 1;
     }
 };
@@ -317,7 +329,7 @@ struct HitWriter {
     }
 };
 
-// Passes [first, first + n) of one bucket.
+// Passes (parts of them, if split) [first, first + n) of one bucket.
 struct Run {
     LitPtr lits;  // of the bucket
     int len, count, first, n;
@@ -331,15 +343,15 @@ __device__ __forceinline__ void walk(const SweepArgs &a, const Passes &ps, int l
         if (first >= ps.total) break;
         int p = (int)first;
         const int end = ps.total - p < ps.tp ? ps.total : p + ps.tp;
-        int bi = find_bucket<SCREENED>(a.buckets, ps.nbuckets, p, lane);
+        int bi = find_bucket<SCREENED>(a.buckets, ps.nbuckets, p >> ps.split, lane);
         while (p < end) {
             const BucketDesc d = a.buckets[bi];
             Run r;
             r.lits = (LitPtr)uniform64((uint64_t)d.lits);
             r.len = uniform((int)d.len);
             r.count = uniform((int)d.count);
-            r.first = p - uniform((int)pass_begin<SCREENED>(d));
-            const int have = (r.count - 1) / CPW + 1 - r.first;
+            r.first = p - (uniform((int)pass_begin<SCREENED>(d)) << ps.split);
+            const int have = (((r.count - 1) / CPW + 1) << ps.split) - r.first;
             r.n = end - p < have ? end - p : have;
             const int n = r.n;
             run(r);
@@ -349,34 +361,171 @@ __device__ __forceinline__ void walk(const SweepArgs &a, const Passes &ps, int l
     }
 }
 
-// Every clause checked.  W lanes check one clause, one table word per lane,
-// 64 / W clauses per wave pass; a lane stops reading rows once its 64 slots
-// are dead (the line of a row is fetched while any of its lanes is alive) and
-// the pass ends when every lane is.
+// The exact check of one clause per W lanes, one table word per lane: the
+// clause's literals at cl (len, the same in all lanes, of them; cur: those held)
+// and its first two rows of the lane's word.  Slots in dead are not looked at;
+// on = false: no clause.  All 64 lanes call it; a lane stops reading rows once
+// its 64 slots are dead, and the check ends when every lane is.
 //
 // The rows are the traffic (a line per row and 16 words), so the schedule
-// reads few of them: the first two prefetched during the pass before, then two
-// per step up to the sixth, then one (random 1024-slot clauses of 8 literals
-// and more die after the sixth to eighth: 642 us with pairs throughout, 618 so);
-// and, only for lanes left with a slot of exactly one non-false literal, the
-// negated row of that literal alone (the first kKeep literals' rows are kept in
-// registers for it; past those every negated row is read).  A per-step choice
-// by the number of live lanes read as few rows but spilled: 845 us.
+// reads few of them: two per step up to the sixth, then one (random 1024-slot
+// clauses of 8 literals and more die after the sixth to eighth: 642 us with pairs
+// throughout, 618 so); and, only for lanes left with a slot of exactly one
+// non-false literal, the negated row of that literal alone (the first ROWS
+// literals' rows are kept in registers for it; past those every negated row is
+// read).  A per-step choice by the number of live lanes read as few rows but
+// spilled: 845 us.
+//
+// Below 8 words ROWS rows are read per step past the held literals (4 beside the
+// screening code, where 8 would spill).
+template <int W, int ROWS = kRows>
+__device__ __forceinline__ void check_clause(const uint64_t *__restrict__ table, LitPtr cl,
+                                             int len, int q, bool on, uint32_t w8,
+                                             uint32_t sentinel, uint64_t dead, const Lits<W> &cur,
+                                             uint64_t x0, uint64_t x1, uint64_t &fm,
+                                             uint64_t &um) {
+    constexpr int H = Lits<W>::kHeld;
+    constexpr int kKeep = H < ROWS ? H : ROWS;
+    uint64_t c2 = dead, c1 = dead;
+    uint64_t f[kKeep];
+    f[0] = x0;
+    f[1] = x1;
+    auto fold = [&](uint64_t x) {
+        c2 |= c1 & x;
+        c1 |= x;
+    };
+    fold(x0);
+    fold(x1);
+    // two rows from position J of the literals l; rows kept when J is
+    // among the first kKeep of the clause
+    auto step = [&]<int J, bool KEEP>(const Lits<W> &l) {
+        const uint32_t o0 = scale_offset<W>(lit_at<W, J>(l)) | w8;
+        const uint32_t o1 = scale_offset<W>(lit_at<W, J + 1>(l)) | w8;
+        if (c2 != ~0ull) {
+            const uint64_t y0 = load_word(table, o0), y1 = load_word(table, o1);
+            if constexpr (KEEP) {
+                f[J % kKeep] = y0;
+                f[(J + 1) % kKeep] = y1;
+            }
+            fold(y0);
+            fold(y1);
+        }
+        return __ballot(c2 != ~0ull) != 0;
+    };
+    auto step1 = [&]<int J, bool KEEP>(const Lits<W> &l) {
+        const uint32_t o0 = scale_offset<W>(lit_at<W, J>(l)) | w8;
+        if (c2 != ~0ull) {
+            const uint64_t y0 = load_word(table, o0);
+            if constexpr (KEEP) f[J % kKeep] = y0;
+            fold(y0);
+        }
+        return __ballot(c2 != ~0ull) != 0;
+    };
+    bool go = len > 2 && __ballot(c2 != ~0ull) != 0;
+    constexpr int P2 = H / 2 - 1 < 2 ? H / 2 - 1 : 2;
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        ((go = go && 2 * I + 2 < len &&
+               step.template operator()<2 * I + 2, (2 * I + 2 < kKeep)>(cur)),
+         ...);
+    }(std::make_integer_sequence<int, P2>{});
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        ((go = go && 2 + 2 * P2 + I < len &&
+               step1.template operator()<2 + 2 * P2 + I, (2 + 2 * P2 + I < kKeep)>(cur)),
+         ...);
+    }(std::make_integer_sequence<int, H - 2 - 2 * P2>{});
+    if constexpr (W < 8) {
+        if (go && len > H) {
+            constexpr int R = ROWS / H;
+            Lits<W> l[R];
+#pragma unroll
+            for (int s = 0; s < R; s++)
+                l[s] = load_lits<W>(cl, H + s * H, len, q, on, sentinel);
+            for (int base = H; base < len && go; base += R * H) {
+                Lits<W> next[R];
+                uint32_t o[R * H];
+#pragma unroll
+                for (int s = 0; s < R; s++)
+                    next[s] = load_lits<W>(cl, base + (R + s) * H, len, q, on,
+                                           sentinel);
+                [&]<int... I>(std::integer_sequence<int, I...>) {
+                    ((o[I] = scale_offset<W>(lit_at<W, I % H>(l[I / H])) | w8), ...);
+                }(std::make_integer_sequence<int, R * H>{});
+                if (c2 != ~0ull) {
+                    uint64_t y[R * H];
+#pragma unroll
+                    for (int i = 0; i < R * H; i++) y[i] = load_word(table, o[i]);
+#pragma unroll
+                    for (int i = 0; i < R * H; i++) fold(y[i]);
+                }
+                go = __ballot(c2 != ~0ull) != 0;
+#pragma unroll
+                for (int s = 0; s < R; s++) l[s] = next[s];
+            }
+        }
+    } else if (go && len > H) {
+        for (int base = H; base < len && go; base += H) {
+            const Lits<W> l = load_lits<W>(cl, base, len, q, on, sentinel);
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ((go = go && base + 2 * I < len &&
+                       step.template operator()<2 * I, false>(l)),
+                 ...);
+            }(std::make_integer_sequence<int, H / 2>{});
+        }
+    }
+    fm = ~c1;
+    um = c1 & ~c2;  // exactly one non-false literal
+    if (__ballot(um != 0)) {
+        // a slot's one non-false literal must not be true there
+        auto neg_row = [&]<int J>(const Lits<W> &l, bool need) {
+            const uint32_t o = (scale_offset<W>(lit_at<W, J>(l)) ^ neg_bit<W>()) | w8;
+            return need ? load_word(table, o) : ~0ull;
+        };
+        [&]<int... I>(std::integer_sequence<int, I...>) {
+            uint64_t rest = um, t[kKeep];
+            ((t[I] = I < len ? neg_row.template operator()<I>(cur, (f[I] & um) != 0)
+                             : ~0ull),
+             ...);
+            ((rest &= I < len ? ~f[I] : ~0ull), ...);
+            ((um &= t[I]), ...);
+            // positions past the kept rows, for the slots left over
+            constexpr int R = W < 8 ? ROWS / H : 1;
+            for (int base = kKeep; base < len && __ballot((rest & um) != 0);
+                 base += R * kKeep) {
+                Lits<W> l[R];
+                uint64_t u[R][kKeep];
+#pragma unroll
+                for (int s = 0; s < R; s++)
+                    l[s] = load_lits<W>(cl, base + s * kKeep, len, q, on,
+                                        sentinel);
+                const bool need = (rest & um) != 0;
+#pragma unroll
+                for (int s = 0; s < R; s++)
+                    ((u[s][I] = base + s * kKeep + I < len
+                                    ? neg_row.template operator()<I>(l[s], need)
+                                    : ~0ull),
+                     ...);
+#pragma unroll
+                for (int s = 0; s < R; s++) ((um &= ~rest | u[s][I]), ...);
+            }
+        }(std::make_integer_sequence<int, kKeep>{});
+    }
+}
+
+// Every clause checked: W lanes check one clause, one table word per lane, 64 / W
+// clauses per wave pass, the first two rows of each prefetched during the pass
+// before.
 template <int W, bool CLAUSES>
 __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
     if (a.choose && *a.choose) return;  // the screened kernel's
-    using L = Lits<W>;
     constexpr int CPW = 64 / W;  // clauses per wave pass
-    constexpr int H = L::kHeld;
-    constexpr int kKeep = H < 8 ? H : 8;
     const int lane = (int)__lane_id();
     const int c = lane / W;           // clause of the pass
     const int w = lane % W;           // table word
-    const int q = lane % L::G;        // literal of the group's registers
+    const int q = lane % Lits<W>::G;  // literal of the group's registers
     const uint32_t w8 = (uint32_t)w * 8u;
     const uint64_t valid = a.valid[w];
     const uint64_t *__restrict__ table = a.table;
-    const Passes ps(a, false);
+    const Passes ps(a, false, 1);
     HitWriter out(a, ps);
 
     walk<CPW, false>(a, ps, lane, [&](const Run &run) {
@@ -402,130 +551,10 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
         auto check = [&](int pass, const Lits<W> &cur, uint64_t x0, uint64_t x1) {
             const int r = pass * CPW + c;
             const bool on = r < left;
+            uint64_t fm, um;
             // invalid slots (and lanes without a clause) start dead
-            uint64_t c2 = on ? ~valid : ~0ull, c1 = c2;
-            uint64_t f[kKeep];
-            f[0] = x0;
-            f[1] = x1;
-            auto fold = [&](uint64_t x) {
-                c2 |= c1 & x;
-                c1 |= x;
-            };
-            fold(x0);
-            fold(x1);
-            // two rows from position J of the literals l; rows kept when J is
-            // among the first kKeep of the clause
-            auto step = [&]<int J, bool KEEP>(const Lits<W> &l) {
-                const uint32_t o0 = scale_offset<W>(lit_at<W, J>(l)) | w8;
-                const uint32_t o1 = scale_offset<W>(lit_at<W, J + 1>(l)) | w8;
-                if (c2 != ~0ull) {
-                    const uint64_t y0 = load_word(table, o0), y1 = load_word(table, o1);
-                    if constexpr (KEEP) {
-                        f[J % kKeep] = y0;
-                        f[(J + 1) % kKeep] = y1;
-                    }
-                    fold(y0);
-                    fold(y1);
-                }
-                return __ballot(c2 != ~0ull) != 0;
-            };
-            auto step1 = [&]<int J, bool KEEP>(const Lits<W> &l) {
-                const uint32_t o0 = scale_offset<W>(lit_at<W, J>(l)) | w8;
-                if (c2 != ~0ull) {
-                    const uint64_t y0 = load_word(table, o0);
-                    if constexpr (KEEP) f[J % kKeep] = y0;
-                    fold(y0);
-                }
-                return __ballot(c2 != ~0ull) != 0;
-            };
-            bool go = len > 2 && __ballot(c2 != ~0ull) != 0;
-            constexpr int P2 = H / 2 - 1 < 2 ? H / 2 - 1 : 2;
-            [&]<int... I>(std::integer_sequence<int, I...>) {
-                ((go = go && 2 * I + 2 < len &&
-                       step.template operator()<2 * I + 2, (2 * I + 2 < kKeep)>(cur)),
-                 ...);
-            }(std::make_integer_sequence<int, P2>{});
-            [&]<int... I>(std::integer_sequence<int, I...>) {
-                ((go = go && 2 + 2 * P2 + I < len &&
-                       step1.template operator()<2 + 2 * P2 + I, (2 + 2 * P2 + I < kKeep)>(cur)),
-                 ...);
-            }(std::make_integer_sequence<int, H - 2 - 2 * P2>{});
-            if constexpr (W < 8) {
-                if (go && len > H) {
-                    constexpr int R = kTailRows / H;
-                    Lits<W> l[R];
-#pragma unroll
-                    for (int s = 0; s < R; s++)
-                        l[s] = load_lits<W>(clause(pass), H + s * H, len, q, on, a.sentinel);
-                    for (int base = H; base < len && go; base += R * H) {
-                        Lits<W> next[R];
-                        uint32_t o[R * H];
-#pragma unroll
-                        for (int s = 0; s < R; s++)
-                            next[s] = load_lits<W>(clause(pass), base + (R + s) * H, len, q, on,
-                                                   a.sentinel);
-                        [&]<int... I>(std::integer_sequence<int, I...>) {
-                            ((o[I] = scale_offset<W>(lit_at<W, I % H>(l[I / H])) | w8), ...);
-                        }(std::make_integer_sequence<int, R * H>{});
-                        if (c2 != ~0ull) {
-                            uint64_t y[R * H];
-#pragma unroll
-                            for (int i = 0; i < R * H; i++) y[i] = load_word(table, o[i]);
-#pragma unroll
-                            for (int i = 0; i < R * H; i++) fold(y[i]);
-                        }
-                        go = __ballot(c2 != ~0ull) != 0;
-#pragma unroll
-                        for (int s = 0; s < R; s++) l[s] = next[s];
-                    }
-                }
-            } else if (go && len > H) {
-                for (int base = H; base < len && go; base += H) {
-                    const Lits<W> l = load_lits<W>(clause(pass), base, len, q, on, a.sentinel);
-                    [&]<int... I>(std::integer_sequence<int, I...>) {
-                        ((go = go && base + 2 * I < len &&
-                               step.template operator()<2 * I, false>(l)),
-                         ...);
-                    }(std::make_integer_sequence<int, H / 2>{});
-                }
-            }
-            const uint64_t fm = ~c1;
-            uint64_t um = c1 & ~c2;  // exactly one non-false literal
-            if (__ballot(um != 0)) {
-                // a slot's one non-false literal must not be true there
-                auto neg_row = [&]<int J>(const Lits<W> &l, bool need) {
-                    const uint32_t o = (scale_offset<W>(lit_at<W, J>(l)) ^ neg_bit<W>()) | w8;
-                    return need ? load_word(table, o) : ~0ull;
-                };
-                [&]<int... I>(std::integer_sequence<int, I...>) {
-                    uint64_t rest = um, t[kKeep];
-                    ((t[I] = I < len ? neg_row.template operator()<I>(cur, (f[I] & um) != 0)
-                                     : ~0ull),
-                     ...);
-                    ((rest &= I < len ? ~f[I] : ~0ull), ...);
-                    ((um &= t[I]), ...);
-                    // positions past the kept rows, for the slots left over
-                    constexpr int R = W < 8 ? kTailRows / H : 1;
-                    for (int base = kKeep; base < len && __ballot((rest & um) != 0);
-                         base += R * kKeep) {
-                        Lits<W> l[R];
-                        uint64_t u[R][kKeep];
-#pragma unroll
-                        for (int s = 0; s < R; s++)
-                            l[s] = load_lits<W>(clause(pass), base + s * kKeep, len, q, on,
-                                                a.sentinel);
-                        const bool need = (rest & um) != 0;
-#pragma unroll
-                        for (int s = 0; s < R; s++)
-                            ((u[s][I] = base + s * kKeep + I < len
-                                            ? neg_row.template operator()<I>(l[s], need)
-                                            : ~0ull),
-                             ...);
-#pragma unroll
-                        for (int s = 0; s < R; s++) ((um &= ~rest | u[s][I]), ...);
-                    }
-                }(std::make_integer_sequence<int, kKeep>{});
-            }
+            check_clause<W>(table, clause(pass), len, q, on, w8, a.sentinel, on ? ~valid : ~0ull,
+                            cur, x0, x1, fm, um);
             const bool hit = (fm | um) != 0;
             if constexpr (CLAUSES) {
                 const unsigned long long bw = __ballot(hit);
@@ -571,18 +600,41 @@ __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
 // One clause per lane: the groups in which it can report, i.e. where none of
 // its literals (its row of len stored offsets) is true in every valid slot and
 // fewer than two occurrences are non-false in every valid slot (SweepArgs::agg);
-// 0 once none is left.  Two literals and then their entries are read per vote.
+// 0 once none is left.  unknown (where some are): its (literal, group) pairs,
+// groups in gdead aside, whose entry is neither non-false nor false.  Literals
+// are read four at a time, the entries two per vote.
 __device__ __forceinline__ uint32_t lane_agg(LitPtr row, int len,
-                                             const uint16_t *__restrict__ agg, uint32_t gdead) {
+                                             const uint32_t *__restrict__ agg, uint32_t gdead,
+                                             int &unknown) {
+    typedef uint32_t Vec __attribute__((ext_vector_type(4), aligned(4)));
     uint32_t a1 = 0, a2 = gdead;  // groups with a non-false occurrence / that cannot report
-    for (int j = 0; j < len; j += 2) {
-        const uint32_t l0 = row[j], l1 = j + 1 < len ? row[j + 1] : 0u;
-        const uint32_t x0 = agg[l0 >> 7], x1 = j + 1 < len ? agg[l1 >> 7] : 0u;
-        a2 |= (a1 & x0) | (x0 >> 8);
-        a1 |= x0;
-        a2 |= (a1 & x1) | (x1 >> 8);
-        a1 |= x1;
-        if ((a2 & 0xFFu) == 0xFFu) return 0;
+    unknown = 0;
+    for (int j = 0; j < len; j += 4) {
+        uint32_t l[4] = {};
+        if (j + 4 <= len) {
+            const Vec v = *(const __attribute__((address_space(1))) Vec *)(row + j);
+#pragma unroll
+            for (int u = 0; u < 4; u++) l[u] = v[u];
+        } else {
+#pragma unroll
+            for (int u = 0; u < 3; u++)
+                if (j + u < len) l[u] = row[j + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u += 2) {
+            if (j + u >= len) break;
+            const uint32_t e0 = agg[l[u] >> 8], e1 = agg[l[u + 1] >> 8];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                if (j + u + k >= len) break;
+                const uint32_t at = (l[u + k] >> 3) & 16u, e = k ? e1 : e0;
+                const uint32_t x = e >> at, no = e >> (at ^ 16u);
+                a2 |= (a1 & x) | (x >> 8);
+                a1 |= x;
+                unknown += __popc(~(x | (no >> 8) | gdead) & 0xFFu);
+            }
+            if ((a2 & 0xFFu) == 0xFFu) return 0;
+        }
     }
     return ~a2 & 0xFFu;
 }
@@ -715,17 +767,35 @@ __device__ __forceinline__ void check_words(LitPtr cl, int len,
     }
 }
 
-// Clauses screened against a.agg first (serving and screened steps).  A wave
-// screens 64 clauses, one per lane; the words that are left of each are then
-// spread over the wave, two neighbouring ones (16 bytes of a row) per lane,
-// whatever clause they belong to, and checked exactly (a word per lane: 167 us
-// where two take 152).  Giving each surviving
-// clause a group of 16 lanes (as many words each as it takes) kept most lanes
-// idle: a clause survives in one or two of its eight word groups.
+// Clauses screened against a.agg first (serving and screened steps, sweeps where
+// that pays).  A wave screens 64 clauses, one per lane, and checks what is left
+// of them exactly, in one of two ways:
+//
+// Few words left, or rows mostly known from the entries: the words are spread
+// over the wave, two neighbouring ones (16 bytes of a row) per lane, whatever
+// clause they belong to (a word per lane: 167 us where two take 152; a clause per
+// 16 lanes kept most lanes idle, as a clause survives in one or two of its eight
+// word groups).  A lane follows one literal after the other, with the entries.
+//
+// Else, clause after clause as in k_sweep, W lanes each: every row is read, but
+// several at a time and whole lines of it.
+//
+// The first way costs a wave about len * (2 + 8 u) per 64 items, u the share of
+// unknown (literal, group) pairs of the clauses left, the second len * kDense / 10
+// per clause (the two were equal at u = 0.4 with 1 word, 0.25 with 4, 0.15 with 8
+// and 16, 0.4 with 64, clauses of 12 literals nine in ten false).  From 24 literals
+// on the chain of reads decides, and with an eighth of the words left the second
+// way is the faster.  Measured with the first way alone, now, and as a group of
+// 16 lanes per clause did: 2M clauses x 16 words, slots of two in five words
+// differing 1602, 1046, 1137 us; 600k x 64 words 2274, 910, 1006; 40k clauses of
+// 150 to 400 literals x 16 words, which 625 waves checked before passes were split
+// 18061, 1560, 1858; 3M x 1 word 791, 644, 918.
+constexpr int kDenseLen = 24;
 template <int W, bool CLAUSES>
 __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k_sweep_screened(SweepArgs a) {
     if (a.choose && !*a.choose) return;  // the plain kernel's
     constexpr int P = W == 1 ? 1 : 2;  // words of an item
+    constexpr int kDense = W <= 16 ? 50 + 5 * W : 17 * W;
     __shared__ uint64_t s_valid[W], s_words[4][64], s_hit[4][64];
     __shared__ uint32_t s_start[4][64], s_group[W];
     const int lane = (int)__lane_id(), wv = (int)(threadIdx.x >> 6);
@@ -740,19 +810,24 @@ __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k
     uint32_t gdead = 0;  // groups without a word
     for (int b = 0; b < 8; b++)
         if (!a.agg_words[b]) gdead |= 1u << b;
-    const Passes ps(a, true);
+    const int live = 8 - __popc(gdead);
+    const Passes ps(a, true, W);
     HitWriter out(a, ps);
 
+    const int part = 64 >> ps.split;  // clauses at a time
     walk<64, true>(a, ps, lane, [&](const Run &run) {
         const int len = run.len, count = run.count;
+        const float sixteenth = 16.0f / (float)(live * len);
         for (int pass = 0; pass < run.n; pass++) {
-            const int row0 = (run.first + pass) * 64;
+            const int row0 = (run.first + pass) * part;
             const LitPtr cl = run.lits + (size_t)row0 * len;
+            int unknown = 0;
             const uint32_t grp =
-                row0 + lane < count
-                    ? lane_agg(cl + (size_t)lane * len, len, (const uint16_t *)a.agg, gdead)
+                lane < part && row0 + lane < count
+                    ? lane_agg(cl + (size_t)lane * len, len, a.agg, gdead, unknown)
                     : 0u;
-            if (!__ballot(grp != 0)) continue;
+            uint64_t left = __ballot(grp != 0);  // clauses to check
+            if (!left) continue;
             uint64_t m = 0;  // table words to check
 #pragma unroll
             for (int b = 0; b < 8; b++)
@@ -760,18 +835,68 @@ __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k
             // bit w: words w .. w + P - 1 are an item
             const uint64_t items = P == 1 ? m : (m | (m >> 1)) & 0x5555555555555555ull;
             const int cnt = __popcll(items);
-            int incl = cnt;
+            // items in the low half, 16ths of unknown pairs in the upper
+            const int add = cnt | (grp ? (int)((float)unknown * sixteenth) << 16 : 0);
+            int incl = add;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
                 const int y = __shfl_up(incl, d);
                 if (lane >= d) incl += y;
             }
-            const int total = uniform(__shfl(incl, 63));
-            s_start[wv][lane] = (uint32_t)(incl - cnt);
+            const int sums = uniform(__shfl(incl, 63));
+            const int total = sums & 0xFFFF, surv = __popcll(left);
+            incl = (incl - add) & 0xFFFF;
+            s_start[wv][lane] = (uint32_t)incl;
             s_words[wv][lane] = m;
             if constexpr (CLAUSES) s_hit[wv][lane] = 0;
             __builtin_amdgcn_wave_barrier();
-            for (int base = 0; base < total; base += 64) {
+            const bool dense =
+                len >= kDenseLen ? 8 * total >= surv * W
+                                 : 5 * total * (4 * surv + (sums >> 16)) >= surv * surv * kDense;
+            if (dense) {
+                constexpr int CPW = 64 / W;
+                const int c = lane / W, w = lane % W, q = lane % Lits<W>::G;
+                const uint32_t w8 = (uint32_t)w * 8u;
+                // the lane's clause among those left, its literals
+                int i;
+                bool on;
+                Lits<W> held;
+                const auto next = [&] {
+                    on = c < __popcll(left);
+                    i = on ? nth_bit(left, c) : 0;
+                    held = load_lits<W>(cl + (size_t)i * len, 0, len, q, on, a.sentinel);
+                    left = __popcll(left) > CPW ? left & (~0ull << nth_bit(left, CPW)) : 0ull;
+                };
+                next();
+                for (bool more = true; more;) {
+                    const int at = i;
+                    const bool in = on;
+                    const Lits<W> cur = held;
+                    more = left != 0;
+                    if (more) next();
+                    const uint64_t dead =
+                        in && ((s_words[wv][at] >> w) & 1ull) ? ~s_valid[w] : ~0ull;
+                    const uint32_t o0 = scale_offset<W>(lit_at<W, 0>(cur)) | w8;
+                    const uint32_t o1 = scale_offset<W>(lit_at<W, 1>(cur)) | w8;
+                    uint64_t x0 = 0, x1 = 0, fm, um;
+                    if (dead != ~0ull) {
+                        x0 = load_word(a.table, o0);
+                        x1 = load_word(a.table, o1);
+                    }
+                    check_clause<W, 4>(a.table, cl + (size_t)at * len, len, q, in, w8, a.sentinel,
+                                       dead, cur, x0, x1, fm, um);
+                    const bool hit = (fm | um) != 0;
+                    if constexpr (CLAUSES) {
+                        const uint64_t bw = __ballot(hit);
+                        if (in && w == 0)
+                            s_hit[wv][at] =
+                                W == 64 ? bw : (bw >> lane) & ((1ull << (W & 63)) - 1ull);
+                    } else {
+                        out.words(hit, (uint32_t)(row0 + at), len, w, fm, um, a.rec_words, lane);
+                    }
+                }
+            }
+            for (int base = 0; !dense && base < total; base += 64) {
                 const int item = base + lane;
                 const bool on = item < total;
                 // the clause it belongs to: the last one that starts at or before it

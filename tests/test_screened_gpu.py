@@ -238,3 +238,45 @@ def test_choice_follows_the_share_of_known_variables(engine_factory, W, n, varia
         e.upload(is_def, is_true)
         e.sweep(np.full(W, ALL))
         assert e.screened() == k % 2, (k, share)
+
+
+@pytest.mark.parametrize("W, n, known", [(1, 470_000, 0.3), (2, 470_000, 0.9), (4, 3000, 0.3),
+                                         (4, 470_000, 0.6), (8, 20_000, 0.9), (16, 120_000, 0.0),
+                                         (16, 470_000, 0.5), (32, 40_000, 0.7), (64, 30_000, 0.0),
+                                         (64, 100_000, 0.8)])
+def test_screened_steps_of_mostly_false_clauses(engine_factory, W, n, known):
+    """Clauses of 1 to 60 literals, most of them false, that the entries leave open
+    in some groups, most or all, passes of 64 clauses whole and split among the
+    waves: the records of a step that is not screened."""
+    rng = np.random.default_rng(900 + W + n)
+    variables = 5000
+    lens = np.where(rng.random(n) < 0.9, rng.integers(1, 20, size=n),
+                    rng.integers(20, 61, size=n)).astype(np.int32)
+    sigma = rng.random(variables) < 0.5
+    v = rng.integers(0, variables, size=int(lens.sum()))
+    false = rng.random(v.size) < np.repeat(1.0 - 1.0 / (1.0 + lens), lens)
+    lits = (2 * v + (false == sigma[v])).astype(np.uint32)
+    e = engine_factory()
+    e.append(lits, lens)
+    e.reset_assignments(variables, W)
+    is_true = np.repeat(np.where(sigma, ALL, np.uint64(0))[:, None], W, axis=1)
+    is_def = np.full((variables, W), ALL)
+    bit = np.uint64(1) << rng.integers(0, 64, size=(variables, W), dtype=np.uint64)
+    differ = rng.random((variables, W)) >= known
+    is_true ^= np.where(differ, bit, np.uint64(0))
+    is_def ^= np.where(differ & (rng.random((variables, W)) < 0.5), bit, np.uint64(0))
+    e.upload(is_def, is_true & is_def)
+    valid = np.full(W, ALL)
+    valid[-1] = np.uint64(0x7FFFFFFFFFFFFF0F)
+    if W > 2:
+        valid[1] = 0
+    for form, view, words in ((sv.RECORDS_FULL, e.step_hits_view, 3),
+                              (sv.RECORDS_CLAUSES, e.step_clauses_view, 2)):
+        got = []
+        for flags in (0, sv.STEP_SCREEN):
+            sv.submit(e, valid, records=form, flags=flags)
+            e.step_wait()
+            r = view().view(np.uint64).reshape(-1, words).copy()
+            got.append(r[np.argsort(r[:, 0])])
+        print(f"{W} words, {n} clauses: {got[0].shape[0]} records", flush=True)
+        assert got[0].shape[0] > 100 and np.array_equal(got[0], got[1])

@@ -459,7 +459,7 @@ struct gss_engine {
     int64_t last_hits = 0;
     uint32_t last_chunks = 0;
     // plain sweeps that may be screened (k_sweep_choose): entries, the words of
-    // each group ([8]: the choice), and passes of 64 clauses
+    // each group (from [8] on the choice), and passes of 64 clauses
     DevBuf<uint32_t> sweep_agg;
     DevBuf<uint64_t> sweep_agg_words;
     int screen_passes = 0;
@@ -676,13 +676,15 @@ hipError_t wait_counts(gss_engine *e) {
 }
 
 // Whether a plain sweep may gain from screening, were its words' slots mostly of
-// one value (the device decides that: k_sweep_choose).  In microseconds, with
-// that: the plain kernel reads 2.8 rows a clause (52 per million of one line
-// each, of the row's lines with a valid word), the screened one takes 24 per million clauses after a pass over the
-// table (5.5 TB/s); 12 are kept for the launches.  Measured, plain and screened
-// with its entries: 1M clauses x 8 words x 100K variables 43 and 27, 2M x 16 x
-// 500K 118 and 71, 400K x 64 x 200K 87 and 68.  Where the slots differ the
-// two launches that find out cost 7.
+// one value and its clauses mostly closed by that (the device decides these:
+// k_sweep_choose).  In microseconds, with that: the plain kernel reads 2.8 rows a
+// clause (52 per million of one line each, of the row's lines with a valid word), the
+// screened one takes 24 per million clauses after a pass over the table (5.5 TB/s);
+// 12 are kept for the launches.  A line through three instances, clauses of 12
+// literals in the mean: plain and screened with its entries, 1M clauses x 8 words x
+// 100K variables 43 and 27, 2M x 16 x 500K 118 and 71, 400K x 64 x 200K 87 and 68.
+// Where the slots differ the two launches that find out cost 7, where the clauses do
+// the pass over the table too.
 // Also false without room for the entries.
 bool screening_may_pay(gss_engine *e, int64_t clauses, const uint64_t *valid) {
     if (e->words < 8 || e->vars <= 0) return false;
@@ -696,26 +698,39 @@ bool screening_may_pay(gss_engine *e, int64_t clauses, const uint64_t *valid) {
     }
     if (52.0 * m * lines <= 24.0 * m + rows / 5.5e6 + 12.0) return false;
     if (e->sweep_agg.reserve_async((size_t)e->vars + 1, e->stream) ||
-        e->sweep_agg_words.reserve_async(9, e->stream))
+        e->sweep_agg_words.reserve_async(8 + (kChooseWords + 1) / 2, e->stream))
         return false;
     return true;
 }
 
 // Before a sweep a that may be screened: the choice, and the screened kernel if
-// that is it (a is launched after it, and runs if it is not).  valid: host memory.
-hipError_t launch_screened_choice(gss_engine *e, const uint64_t *valid, SweepArgs &a, int blocks,
-                                  hipStream_t s) {
+// that is it (a is launched after it, and runs if it is not).  desc: the sweep's nb
+// buckets, screen_passes passes of 64 clauses; these and valid are host memory.
+hipError_t launch_screened_choice(gss_engine *e, const BucketDesc *desc, int nb,
+                                  int screen_passes, const uint64_t *valid, SweepArgs &a,
+                                  int blocks, hipStream_t s) {
     uint32_t *choose = (uint32_t *)(e->sweep_agg_words.p + 8);
     e->chosen = true;
-    hipError_t he = launch_sweep_choose(e->table.p, valid, e->vars, e->words, e->sweep_agg.p,
-                                        e->sweep_agg_words.p, choose, s);
-    if (he != hipSuccess) return he;
-    a.choose = choose;
+    ClauseSample sample{};
+    constexpr int n = (int)(4 * kOpenBlocks);
+    for (int k = 0, i = 0; k < n; k++) {
+        const uint32_t p = (uint32_t)((int64_t)screen_passes * k / n);
+        while (i + 1 < nb && desc[i + 1].screen_begin <= p) i++;
+        const BucketDesc &d = desc[i];
+        const uint32_t r = std::min((p - d.screen_begin) * 64u + (uint32_t)(k * 37 & 63),
+                                    d.count - 1);
+        sample.row[k] = d.lits + (size_t)r * d.len;
+        sample.len[k] = d.len | std::min(d.count - r, 2u) << 24;
+    }
     SweepArgs b = a;
-    b.npasses = e->screen_passes;
+    b.npasses = screen_passes;
     b.task_passes = task_passes(e, true);
     b.agg = e->sweep_agg.p;
     b.agg_words = e->sweep_agg_words.p;
+    const hipError_t he = launch_sweep_choose(b, sample, valid, e->vars, e->words, e->sweep_agg.p,
+                                              e->sweep_agg_words.p, choose, s);
+    if (he != hipSuccess) return he;
+    a.choose = b.choose = choose;
     return launch_sweep(b, e->words, blocks, s);
 }
 
@@ -746,7 +761,8 @@ int launch_current_sweep(gss_engine *e) {
         a.chunk_cap = e->chunk_cap;
         a.rec_words = 3;
         if (e->may_screen)
-            HIP_TRY(launch_screened_choice(e, e->valid_up.data(), a, e->blocks, e->stream));
+            HIP_TRY(launch_screened_choice(e, e->desc_up.data(), e->nbuckets, e->screen_passes,
+                                           e->valid_up.data(), a, e->blocks, e->stream));
         HIP_TRY(launch_sweep(a, e->words, e->blocks, e->stream));
     }
     HIP_TRY(hipEventRecord(e->ev1, e->stream));
@@ -1674,11 +1690,11 @@ int gss_sweep_screened(gss_engine *e, int *out) {
     if (!out) return set_err(GSS_E_INVAL, "null argument");
     *out = -1;
     if (!e->chosen) return GSS_OK;
-    uint32_t v = 0;
-    HIP_TRY(hipMemcpyAsync(&v, e->sweep_agg_words.p + 8, sizeof v, hipMemcpyDeviceToHost,
+    uint32_t v[kChooseWords] = {};
+    HIP_TRY(hipMemcpyAsync(v, e->sweep_agg_words.p + 8, sizeof v, hipMemcpyDeviceToHost,
                            e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
-    *out = v ? 1 : 0;
+    *out = screen_chosen(v) ? 1 : 0;
     return GSS_OK;
 }
 
@@ -1949,7 +1965,9 @@ static hipError_t launch_step_tail(gss_engine *e, StepSlot &sl, hipStream_t s) {
     hipError_t he = hipSuccess;
     e->chosen = false;
     if (sl.plan.may_screen)
-        he = launch_screened_choice(e, sl.h_hdr.p->valid, a, sl.plan.blocks, s);
+        he = launch_screened_choice(e, sl.h_desc.p, sl.h_hdr.p->nbuckets,
+                                    sl.h_hdr.p->screen_passes, sl.h_hdr.p->valid, a,
+                                    sl.plan.blocks, s);
     if (he == hipSuccess) he = launch_sweep(a, e->words, sl.plan.blocks, s);
     const ChunkArgs c = step_chunks(sl, sl.rec_words);
     if (sl.plan.serve) {

@@ -50,9 +50,29 @@ struct SweepArgs {
     // other words.
     const uint32_t *agg;
     const uint64_t *agg_words;  // [8]
-    // launch_sweep_choose's: the plain kernel runs where it is 0, the screened
+    // launch_sweep_choose's: the screened kernel runs where screen_chosen, the plain
     // one elsewhere (null: whichever is launched)
     const uint32_t *choose;
+};
+
+// What launch_sweep_choose found.  choose[0], of the variables: 0 too few known, 1
+// enough, 2 so many that the clauses need no look; choose[1 ..]: what the sample's
+// 128 clauses cost by its blocks, in 48ths of a row per literal (open_cost in
+// kernels.hip).  Screened where that is at most kOpenCost in 100.
+constexpr unsigned kOpenBlocks = 16;
+constexpr uint32_t kOpenCost = 21, kOpenLimit = 128 * 48 * kOpenCost / 100;
+constexpr int kChooseWords = 1 + (int)kOpenBlocks;
+__host__ __device__ inline bool screen_chosen(const uint32_t *choose) {
+    uint32_t cost = 0;
+    for (unsigned b = 0; b < kOpenBlocks; b++) cost += choose[1 + b];
+    return choose[0] == 2 || (choose[0] == 1 && cost <= kOpenLimit);
+}
+
+// 64 clauses spread over the buckets: a row, its length and, from bit 24 on, how many
+// rows there are from it on (1 or 2, if more).
+struct ClauseSample {
+    const uint32_t *row[4 * kOpenBlocks];
+    uint32_t len[4 * kOpenBlocks];
 };
 
 // Staged regions of a batched step, read by k_step_in.
@@ -195,12 +215,12 @@ struct StepInArgs {
     ServeReport *report;  // pinned
 };
 
-// Plain sweeps, words >= 8: decides from a sample of the table whether the sweep
-// is screened (*choose), and if so builds the entries and agg_words.  valid is
-// host memory, read before the launch.
-hipError_t launch_sweep_choose(const uint64_t *table, const uint64_t *valid, int64_t vars,
-                               int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
-                               hipStream_t s);
+// Plain sweeps, words >= 8: decides from a sample of the table and of the clauses
+// whether sweep a (the screened kernel's) is screened (choose, kChooseWords), and if
+// so builds the entries and agg_words.  valid is host memory, read before the launch.
+hipError_t launch_sweep_choose(const SweepArgs &a, const ClauseSample &sample,
+                               const uint64_t *valid, int64_t vars, int words, uint32_t *agg,
+                               uint64_t *agg_words, uint32_t *choose, hipStream_t s);
 // Screening entries of a batched step from the table itself (SweepArgs::agg):
 // group b = words [b * words / 8, (b + 1) * words / 8) (one word per group
 // below 8 words), over every slot of its words (valid or not: what holds in

@@ -516,7 +516,7 @@ __device__ __forceinline__ void check_clause(const uint64_t *__restrict__ table,
 // before.
 template <int W, bool CLAUSES>
 __global__ GSS_SWEEP_BOUNDS void k_sweep(SweepArgs a) {
-    if (a.choose && *a.choose) return;  // the screened kernel's
+    if (a.choose && screen_chosen(a.choose)) return;  // the screened kernel's
     constexpr int CPW = 64 / W;  // clauses per wave pass
     const int lane = (int)__lane_id();
     const int c = lane / W;           // clause of the pass
@@ -793,7 +793,7 @@ __device__ __forceinline__ void check_words(LitPtr cl, int len,
 constexpr int kDenseLen = 24;
 template <int W, bool CLAUSES>
 __global__ __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256, 7) void k_sweep_screened(SweepArgs a) {
-    if (a.choose && !*a.choose) return;  // the plain kernel's
+    if (a.choose && !screen_chosen(a.choose)) return;  // the plain kernel's
     constexpr int P = W == 1 ? 1 : 2;  // words of an item
     constexpr int kDense = W <= 16 ? 50 + 5 * W : 17 * W;
     __shared__ uint64_t s_valid[W], s_words[4][64], s_hit[4][64];
@@ -1593,12 +1593,12 @@ template <int W>
 struct TableEntries {
     static constexpr int VARS = W <= 8 ? 64 : W == 16 ? 8 : 4;  // per turn of a wave
 
-    // Entry of variable v0 + lane * step, in the first VARS lanes.
+    // Entry of variable v0 + lane, in the first VARS lanes.
     static __device__ __forceinline__ uint32_t turn(const uint64_t *__restrict__ table, int64_t v0,
-                                                    int64_t step, int64_t vars, int lane) {
+                                                    int64_t vars, int lane) {
         if constexpr (W <= 8) {
-            if (v0 + lane * step >= vars) return 0;
-            const uint64_t *f = table + (size_t)(v0 + lane * step) * 2 * W, *t = f + W;
+            if (v0 + lane >= vars) return 0;
+            const uint64_t *f = table + (size_t)(v0 + lane) * 2 * W, *t = f + W;
             uint32_t x = 0;
 #pragma unroll
             for (int b = 0; b < W; b++)
@@ -1616,8 +1616,7 @@ struct TableEntries {
             uint32_t out = 0;
 #pragma unroll
             for (int l = 0; l < LINES; l++) {
-                const int o = l * 64 + lane;
-                const int64_t at = (v0 + o / (2 * W) * (step - 1)) * 2 * W + o;
+                const int64_t at = v0 * 2 * W + l * 64 + lane;
                 x[l] = at < vars * 2 * W ? table[at] : 0ull;
             }
 #pragma unroll
@@ -1644,31 +1643,91 @@ __global__ __launch_bounds__(256) void k_table_agg(const uint64_t *__restrict__ 
     const int lane = (int)__lane_id();
     for (int64_t v0 = (blockIdx.x * 4ll + (threadIdx.x >> 6)) * VARS; v0 < vars;
          v0 += gridDim.x * 4ll * VARS) {
-        const uint32_t e = TableEntries<W>::turn(table, v0, 1, vars, lane);
+        const uint32_t e = TableEntries<W>::turn(table, v0, vars, lane);
         if (lane < VARS && v0 + lane < vars) agg[v0 + lane] = e;
     }
 }
 
+// What the screened kernel would be left with: the wave's clause of the sample and
+// the row after it, each looked at in one word group's valid slots, straight from the
+// table (the entries are not there yet), a lane per word of a literal's two rows, its
+// first 16 literals at once.  A clause that stays open costs the screened kernel its
+// known literals (a third each) and its unknown ones (a row each), here per literal
+// and in 48ths; kOpenCost in 100 is where it takes as long as the plain one.
+// Plain and screened, 2M clauses, mean length 12, by the share of literals that are
+// false and of groups that are known: half and 60 % x 8 words 260 and 183 us, three
+// quarters and 60 % 390 and 373, nine in ten and 90 % 575 and 453, 80 % 606 and 661,
+// 60 % 632 and 696; x 16 words, nine in ten and 96 % 582 and 412, 64 % 692 and 845.
+//
+// A clause per lane of one block, a literal after the other, took longer than the
+// other blocks need for a table of 128 MB (29 us), so the clauses are spread over
+// kOpenBlocks of them.
+template <int W>
+__device__ __forceinline__ uint32_t open_cost(const SweepArgs &a, const ClauseSample &sample,
+                                              uint32_t groups, int gw, int lane) {
+    constexpr int GW = W / 8, PER = 32 / GW, READS = PER < 16 ? 16 / PER : 1;  // literals a read
+    constexpr uint64_t kOwn = ~0ull / ((1ull << (GW < 8 ? 2 * GW : 16)) - 1ull);
+    const uint32_t len = sample.len[gw] & 0xFFFFFFu, rows = sample.len[gw] >> 24;
+    const int n = len < 16u ? (int)len : 16;
+    const int u = lane / (2 * GW);
+    uint64_t x[2][READS], in[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const uint32_t *lits = sample.row[gw] + (c && rows > 1 ? len : 0u);
+        const int w = nth_bit(groups, (2 * gw + c) % __popc(groups)) * GW + lane % GW;
+        in[c] = a.valid[w];
+#pragma unroll
+        for (int r = 0; r < READS; r++) {
+            const int j = r * PER + u;
+            const uint32_t l = lits[j < n ? j : 0] ^ ((lane / GW) & 1 ? 128u : 0u);
+            x[c][r] = load_word(a.table, scale_offset<W>(l) + (uint32_t)w * 8u);
+        }
+    }
+    uint32_t cost = 0;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        int nonfalse = 0, unknown = n;
+        bool tru = false;
+#pragma unroll
+        for (int r = 0; r < READS; r++) {
+            uint64_t f = __ballot((x[c][r] | ~in[c]) == ~0ull), z = __ballot((x[c][r] & in[c]) == 0);
+#pragma unroll
+            for (int d = 1; d < GW; d <<= 1) {
+                f &= f >> d;
+                z &= z >> d;
+            }
+            const uint64_t own = kOwn & __ballot(r * PER + u < n);
+            nonfalse += __popcll(f & own);
+            unknown -= __popcll((f | z) & own);
+            tru |= ((z >> GW) & own) != 0;
+        }
+        if (!tru && nonfalse < 2) cost += 16u + 48u * (uint32_t)unknown / (uint32_t)n;
+    }
+    return cost;
+}
+
 // Whether a plain sweep is screened, and the entries if it is.  The screened
 // kernel pays where entries know what a variable is (true or false in all
-// slots of a group): each block looks at the same kSample variables spread over
-// the table, each in one group, and where kScreenKnown in 100 are known the
-// entries are built and *choose is 1; else *choose is 0 and nothing is.  A
-// variable's groups mostly agree, so one group each of 128 variables tells more
-// (the share to within 4 points, one standard deviation) than all groups of 16
-// (12 points, 7 in 100 tables of 60 % known judged wrong) for as many bytes.
+// slots of a group) and the clauses are mostly closed by that.  Each block but the
+// first kOpenBlocks looks at the same kSample variables spread over the table, each in one
+// group; where kScreenKnown in 100 are known the entries are built, else nothing
+// is.  Meanwhile the first blocks look at the clauses (open_cost), the next one writes
+// what became of the variables: see screen_chosen.  A variable's groups mostly
+// agree, so one group each of 128 variables tells more (the share to within 4
+// points, one standard deviation) than all groups of 16 (12 points, 7 in 100 tables
+// of 60 % known judged wrong) for as many bytes.
 //
 // Only groups with a valid slot count: words of no request hold one value (rolled
 // forward) or none, whatever the others do.  Counted too, 14 such words beside 2
 // mixed ones took 2M clauses to the screened kernel: 330 us, 213 plain.
 //
-// Plain against screened, entries included, by the share that is known: 400K
-// clauses x 4096 slots 89 and 75 us at 58 %, 92 and 83 at 48, 95 and 94 at 38;
-// 1M x 333 slots 55 and 42 at 44 %; 2M x 1024 slots 149 and 94 at 55 %, 119 and
-// 73 at 88; random slots (nothing known) 4M x 1024 615 and 1460.
-constexpr int kScreenKnown = 40, kSample = 128;
+// Plain against screened, entries included, by the share that is known, clauses
+// mostly true: 400K clauses x 4096 slots 89 and 75 us at 58 %, 92 and 83 at 48, 95
+// and 94 at 38; 1M x 333 slots 55 and 42 at 44 %; 2M x 1024 slots 149 and 94 at 55
+// %, 119 and 73 at 88.
+constexpr int kScreenKnown = 40, kScreenSure = 90, kSample = 128;
 template <int W>
-__global__ __launch_bounds__(256) void k_sweep_choose(const uint64_t *__restrict__ table,
+__global__ __launch_bounds__(256) void k_sweep_choose(SweepArgs a, const uint64_t *__restrict__ table, ClauseSample sample,
                                                       uint64_t words, int64_t vars,
                                                       uint32_t *__restrict__ agg,
                                                       uint64_t *__restrict__ agg_words,
@@ -1681,6 +1740,17 @@ __global__ __launch_bounds__(256) void k_sweep_choose(const uint64_t *__restrict
 #pragma unroll
     for (int b = 0; b < 8; b++)
         if ((words >> (b * GW)) & ((1ull << GW) - 1ull)) groups |= 1u << b;
+    if (blockIdx.x < kOpenBlocks) {
+        __shared__ uint32_t s_cost[4];
+        // (a halted step's clauses are not all there)
+        const bool on = groups && (a.dyn ? a.dyn[2] : a.npasses) > 0;
+        if (on) s_cost[wv] = open_cost<W>(a, sample, groups, (int)blockIdx.x * 4 + wv, lane);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            choose[1 + blockIdx.x] =
+                on ? s_cost[0] + s_cost[1] + s_cost[2] + s_cost[3] : kOpenLimit + 1u;
+        return;
+    }
     const int ng = __popc(groups);
     if (ng) {
         // a lane per word: GW lanes of a variable's row f, then GW of its row t
@@ -1703,14 +1773,18 @@ __global__ __launch_bounds__(256) void k_sweep_choose(const uint64_t *__restrict
         if (lane == 0) s_known[wv] = known;
     }
     __syncthreads();
-    const bool screen =
-        ng && (s_known[0] + s_known[1] + s_known[2] + s_known[3]) * 100 >= kScreenKnown * kSample;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *choose = screen ? 1u : 0u;
+    const int in100 =
+        ng ? (s_known[0] + s_known[1] + s_known[2] + s_known[3]) * 100 / kSample : 0;
+    const bool screen = in100 >= kScreenKnown;
+    if (blockIdx.x == kOpenBlocks) {
+        if (threadIdx.x == 0) choose[0] = in100 >= kScreenSure ? 2u : screen ? 1u : 0u;
+        if (threadIdx.x < 8)
+            agg_words[threadIdx.x] = words & (((1ull << GW) - 1ull) << (threadIdx.x * GW));
+    }
     if (!screen) return;
-    if (blockIdx.x == 0 && threadIdx.x < 8)
-        agg_words[threadIdx.x] = words & (((1ull << (W / 8)) - 1ull) << (threadIdx.x * (W / 8)));
-    for (int64_t v0 = (blockIdx.x * 4ll + wv) * VARS; v0 < vars; v0 += gridDim.x * 4ll * VARS) {
-        const uint32_t e = TableEntries<W>::turn(table, v0, 1, vars, lane);
+    for (int64_t v0 = ((blockIdx.x - kOpenBlocks) * 4ll + wv) * VARS; v0 < vars;
+         v0 += (gridDim.x - kOpenBlocks) * 4ll * VARS) {
+        const uint32_t e = TableEntries<W>::turn(table, v0, vars, lane);
         if (lane < VARS && v0 + lane < vars) agg[v0 + lane] = e;
     }
 }
@@ -2103,19 +2177,20 @@ hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_sweep_choose(const uint64_t *table, const uint64_t *valid, int64_t vars,
-                               int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
+hipError_t launch_sweep_choose(const SweepArgs &a, const ClauseSample &sample,
+                               const uint64_t *valid, int64_t vars, int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
                                hipStream_t s) {
     uint64_t used = 0;
     for (int w = 0; w < words; w++)
         if (valid[w]) used |= 1ull << w;
     if (vars <= 0 || words < 8) return hipErrorInvalidValue;
     const int64_t per = words == 8 ? 256 : words == 16 ? 32 : 16;  // variables a block takes
-    const unsigned blocks = (unsigned)std::min<int64_t>((vars + per - 1) / per, 2048);
+    const unsigned blocks =
+        kOpenBlocks + (unsigned)std::min<int64_t>((vars + per - 1) / per, 2048 - kOpenBlocks);
 #define X(W_)                                                                                \
     if (words == W_) {                                                                       \
-        hipLaunchKernelGGL(k_sweep_choose<W_>, dim3(blocks), dim3(256), 0, s, table, used,  \
-                           vars, agg, agg_words, choose);                                    \
+        hipLaunchKernelGGL(k_sweep_choose<W_>, dim3(blocks), dim3(256), 0, s, a, a.table, sample, \
+                           used, vars, agg, agg_words, choose);                              \
         return hipGetLastError();                                                            \
     }
     X(8) X(16) X(32) X(64)

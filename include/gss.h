@@ -232,8 +232,8 @@ int gss_hits_gather(gss_engine *e, gss_hit *d_out, int64_t cap, int64_t *n);
  * HIP events recorded on the engine's stream around the kernel launch. */
 int gss_sweep_kernel_ms(gss_engine *e, float *ms);
 /* Whether the last sweep launched (a plain one, or a step's without
- * GSS_STEP_SCREEN) was screened: 1 where the sample of the table said that it
- * pays, 0 where it said that it does not, -1 where the sweep's size ruled it
+ * GSS_STEP_SCREEN) was screened: 1 where samples of the table and the clauses
+ * said that it pays, 0 where they said that it does not, -1 where the sweep's size ruled it
  * out.  The records do not depend on it.  Synchronous. */
 int gss_sweep_screened(gss_engine *e, int *out);
 /* Sum of sweep-kernel durations (ms) and count since the last reset. */

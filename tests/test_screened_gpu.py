@@ -280,3 +280,30 @@ def test_screened_steps_of_mostly_false_clauses(engine_factory, W, n, known):
             got.append(r[np.argsort(r[:, 0])])
         print(f"{W} words, {n} clauses: {got[0].shape[0]} records", flush=True)
         assert got[0].shape[0] > 100 and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("false, chosen", [(0.1, 1), (0.95, 0)])
+@pytest.mark.parametrize("W, n", [(8, 450_000), (16, 450_000), (32, 160_000), (64, 80_000)])
+def test_choice_looks_at_the_clauses(engine_factory, W, n, false, chosen):
+    """Tables of which 60 % of the variables are known: enough where most literals
+    are true, so that hardly a clause stays open; not where one in twenty is (seven
+    in ten clauses of 8 to 14 literals then do, at 0.4 rows and a third per literal
+    three times the threshold)."""
+    rng = np.random.default_rng(W)
+    variables = 3001
+    lens = rng.integers(8, 15, size=n).astype(np.int32)
+    sigma = rng.random(variables) < 0.5
+    v = rng.integers(0, variables, size=int(lens.sum()))
+    lits = (2 * v + ((rng.random(v.size) < false) == sigma[v])).astype(np.uint32)
+    e = engine_factory()
+    e.append(lits, lens)
+    e.reset_assignments(variables, W)
+    is_true = np.repeat(np.where(sigma, ALL, np.uint64(0))[:, None], W, axis=1)
+    mixed = rng.permutation(variables) >= 0.6 * variables
+    is_true[mixed] = rng.integers(0, 1 << 63, size=(int(mixed.sum()), W), dtype=np.uint64)
+    e.upload(np.full((variables, W), ALL), is_true)
+    valid = np.full(W, ALL)
+    hits = e.sweep(valid)
+    assert e.screened() == chosen
+    sv.submit(e, valid, records=sv.RECORDS_IDS)
+    assert e.step_wait()[0] == hits and e.screened() == chosen

@@ -630,7 +630,6 @@ def run_serving(args) -> int:
                    "records_total": out.records, "max_queue": out.max_queue, "tuned": tuned,
                    "steps_in_flight": cfg.max_inflight, "loop": "native (gss_server)",
                    "prefilter": os.environ.get("GPUSHARESAT_SERVE_PREFILTER", "1") != "0",
-                   "prefilter_vote": int(os.environ.get("GPUSHARESAT_SERVE_VOTE", "2")),
                    "preloaded_clauses": preloaded, "flips": cfg.flips},
         "latency_ms": {"p50": pct[50], "p99": pct[99], "p999": pct[99.9],
                        "max": float(lat.max()),

@@ -43,6 +43,8 @@
 using namespace gss;
 
 // gss_hits_gather takes the records of at most this many claimed hit chunks.
+// Nothing here needs the line; it is part of the call's contract, and callers
+// that are told to take gss_hits_copy past it keep being told so.
 static constexpr uint32_t kGatherMaxChunks = 262144;
 constexpr int kMaxHostRecordBuffers = 4;  // pinned record buffers per step slot
 // records of a step at most this large are written into pinned memory by the
@@ -475,8 +477,6 @@ struct gss_engine {
     int tune_waves_per_cu = 0;
     int tune_task_clauses = 0;
     int tune_max_chunks = 0;
-    int tune_unroll = 0;
-    int tune_fuse_len = 0;  // 0 = default, -1 = no fused schedule
     int tune_schedule = 0;  // 0 = default (long clauses first), 1 = long first, 2 = short first
 
     // staging
@@ -1720,9 +1720,8 @@ int gss_set_tuning(gss_engine *e, int key, int value) {
         case GSS_TUNE_UNROLL:
             if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8)
                 return set_err(GSS_E_INVAL, "unroll must be 0, 1, 2, 4 or 8");
-            e->tune_unroll = value;
-            return GSS_OK;
-        case GSS_TUNE_FUSE_LEN: e->tune_fuse_len = value; return GSS_OK;
+            return GSS_OK;  // no kernel has rows in flight or a fuse length to choose
+        case GSS_TUNE_FUSE_LEN: return GSS_OK;
         case GSS_TUNE_SCHEDULE:
             if (value > 2) return set_err(GSS_E_INVAL, "schedule must be 0, 1 or 2");
             e->tune_schedule = value;
@@ -1747,19 +1746,16 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
     if (!valid || reps < 1) return set_err(GSS_E_INVAL, "bad autotune arguments");
     if (e->pending) return set_err(GSS_E_STATE, "a sweep is in flight");
     struct Cfg {
-        int unroll, fuse, task, wpc, sched;
+        int task, wpc, sched;
     };
     std::vector<Cfg> grid;
     const int tasks[] = {0, 32, 128, 512};
     const int wpcs[] = {0, 20, 24};
     for (int t : tasks)
         for (int w : wpcs)
-            for (int sc = 1; sc <= 2; sc++) grid.push_back({2, -1, t, w, sc});
-    const Cfg saved{e->tune_unroll, e->tune_fuse_len, e->tune_task_clauses, e->tune_waves_per_cu,
-                    e->tune_schedule};
+            for (int sc = 1; sc <= 2; sc++) grid.push_back({t, w, sc});
+    const Cfg saved{e->tune_task_clauses, e->tune_waves_per_cu, e->tune_schedule};
     auto apply = [&](const Cfg &c) {
-        e->tune_unroll = c.unroll;
-        e->tune_fuse_len = c.fuse;
         e->tune_task_clauses = c.task;
         e->tune_waves_per_cu = c.wpc;
         e->tune_schedule = c.sched;
@@ -1793,8 +1789,8 @@ int gss_autotune(gss_engine *e, const uint64_t *valid, int reps, int *best, floa
     e->total_ms = total0;
     e->nsweeps = count0;
     if (best) {
-        best[0] = best_cfg.unroll;
-        best[1] = best_cfg.fuse;
+        best[0] = 2;   // rows in flight and fuse length: fixed
+        best[1] = -1;
         best[2] = best_cfg.task;
         best[3] = best_cfg.wpc;
         best[4] = best_cfg.sched;

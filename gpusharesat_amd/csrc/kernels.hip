@@ -31,9 +31,10 @@
 // Work mapping.  k_sweep: W lanes check one clause, one table word each, 64 / W
 // clauses per wave pass, literals handed out with DPP (no LDS); k_sweep_screened:
 // one clause per lane against the screening entries, then two words of a surviving
-// clause per lane, or W lanes per clause where most words are left.  Waves are persistent and walk the clauses in tasks of
-// passes.  Steps are screened on request; other sweeps where a look at the
-// table says that it pays (k_sweep_choose).
+// clause per lane, or W lanes per clause where most words are left.  Waves are
+// persistent and walk the clauses in tasks of passes.  Steps are screened on
+// request; other sweeps where a look at the table and the clauses says that it
+// pays (k_sweep_choose).
 //
 // What bounds it is the row reads: 128-byte lines of a table that the L2s do
 // not hold, ~6.9 TB/s of them at any size past 32 MB.  Measured on one MI355X,

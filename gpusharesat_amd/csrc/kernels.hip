@@ -209,14 +209,6 @@ __device__ __forceinline__ int find_bucket(const BucketDesc *__restrict__ b, int
 #define GSS_SWEEP_BOUNDS __attribute__((amdgpu_num_sgpr(96))) __launch_bounds__(256)
 constexpr int kSweepBlocksPerCu = 7;
 
-// How a wave walks the clauses: the passes of all buckets (CPW clauses of one
-// length each) form one sequence, cut into tasks of `tp` passes that the
-// persistent waves take round-robin.  tp gives every wave kTaskRounds tasks
-// of the same number of passes, so the waves finish together whatever the
-// number of clauses (tasks of a fixed 64 clauses left 4.4 tasks per wave on 2M
-// clauses: some waves had 5), and a wave reads its literals in long runs.
-constexpr int kTaskRounds = 4;
-
 // Tables of less than 8 words: kRows rows read per step past a clause's held
 // literals, and kept of these for the negated-row reads.
 // A row there is part of a line and comes from the L2s, so long clauses are bound
@@ -226,6 +218,12 @@ constexpr int kTaskRounds = 4;
 // 148 and 94 (four rows: 55 and 128).
 constexpr int kRows = 8;
 
+// How a wave walks the clauses: the passes of all buckets (CPW clauses of one
+// length each) form one sequence, cut into tasks of `tp` passes that the
+// persistent waves take round-robin.  tp gives every wave kTaskRounds tasks
+// of the same number of passes, so the waves finish together whatever the
+// number of clauses (tasks of a fixed 64 clauses left 4.4 tasks per wave on 2M
+// clauses: some waves had 5), and a wave reads its literals in long runs.
 //
 // A pass of a screened sweep is 64 clauses, checked one after the other as far as
 // they survive: where there are fewer passes than waves it is split into up to
@@ -233,6 +231,8 @@ constexpr int kRows = 8;
 // and more is so much work that three parts per wave are better than one (600k
 // clauses x 64 words, 9,375 passes, nothing known: 1,097 us whole, 956 in halves);
 // four were not (400k: 255 us per sweep whole, 254 in halves, 281 in quarters).
+constexpr int kTaskRounds = 4;
+
 struct Passes {
     int nbuckets, total, tp, gw, nw;
     int split = 0;  // log2 of the parts
@@ -1728,8 +1728,10 @@ __device__ __forceinline__ uint32_t open_cost(const SweepArgs &a, const ClauseSa
 // %, 119 and 73 at 88.
 constexpr int kScreenKnown = 40, kScreenSure = 90, kSample = 128;
 template <int W>
-__global__ __launch_bounds__(256) void k_sweep_choose(SweepArgs a, const uint64_t *__restrict__ table, ClauseSample sample,
-                                                      uint64_t words, int64_t vars,
+__global__ __launch_bounds__(256) void k_sweep_choose(SweepArgs a,
+                                                      const uint64_t *__restrict__ table,
+                                                      ClauseSample sample, uint64_t words,
+                                                      int64_t vars,
                                                       uint32_t *__restrict__ agg,
                                                       uint64_t *__restrict__ agg_words,
                                                       uint32_t *choose) {
@@ -2179,8 +2181,8 @@ hipError_t launch_table_agg(const uint64_t *table, const StepHeader *dh, int64_t
 }
 
 hipError_t launch_sweep_choose(const SweepArgs &a, const ClauseSample &sample,
-                               const uint64_t *valid, int64_t vars, int words, uint32_t *agg, uint64_t *agg_words, uint32_t *choose,
-                               hipStream_t s) {
+                               const uint64_t *valid, int64_t vars, int words, uint32_t *agg,
+                               uint64_t *agg_words, uint32_t *choose, hipStream_t s) {
     uint64_t used = 0;
     for (int w = 0; w < words; w++)
         if (valid[w]) used |= 1ull << w;
